@@ -291,7 +291,8 @@ typedef struct lfgpu_pcg_opts {
   int check_every; /* iterations per chunk; the host polls the state
                     * one step behind the device, every 1 to 8 chunks
                     * (sized from the residual history); chunks after
-                    * the stop run empty                             */
+                    * the stop run empty (a one-launch solve takes no
+                    * chunks)                                        */
   /* mixed mode only (0 selects the default):                        */
   double refine_delta;     /* reliable update once ||r|| fell by this  */
                            /* factor since the last one (default 0.3)  */
@@ -303,11 +304,15 @@ typedef struct lfgpu_pcg_opts {
    * preconditioned residual on the fly; 0 = two sweeps with Eigen's own
    * recurrences (default). */
   int single_reduction;
-  /* FP64 two-sweep and row-sweep iterations: 0 = replay each chunk of
-   * check_every iterations from a captured hipGraph below 2^20 rows, where
-   * the solve is bound by the launch rate (default); 1 = always; -1 = never
-   * (plain launches).  The iterates are the same either way.  Up to two
-   * captured chunks are kept per matrix, keyed by the solution vector. */
+  /* FP64 two-sweep and row-sweep iterations: 0 = the whole solve in one
+   * launch with the vectors kept on the chip where the system fits (matrices
+   * on at most 6 diagonals; info->syncs is 1 then), else replay each chunk
+   * of check_every iterations from a captured hipGraph below 2^20 rows,
+   * where the solve is bound by the launch rate (default); 1 = always replay
+   * chunks; -1 = never (plain launches).  1 and -1 give the same iterates;
+   * the one-launch solve runs the same recurrences and stopping test with
+   * its sums in another order.  Up to two captured chunks are kept per
+   * matrix, keyed by the solution vector. */
   int graph;
 } lfgpu_pcg_opts;
 typedef struct lfgpu_pcg_info {
@@ -352,7 +357,8 @@ int lfgpu_pcg_sweep_times(lfgpu_ctx *ctx, const lfgpu_csr *A,
  * (no solver storage is built) and no graph is captured.  Systems of up to
  * 2^21 rows (LFGPU_ERANGE above); other modes and single_reduction are
  * rejected (LFGPU_EINVAL); opts->graph is ignored.  On a matrix that
- * lfgpu_pcg stores as DIA the iterates are lfgpu_pcg's.  All calls on one
+ * lfgpu_pcg stores as DIA the iterates are those of lfgpu_pcg with
+ * opts->graph 1 or -1.  All calls on one
  * GPU share the array: calls that overlap on one GPU (several contexts or
  * threads) race and must be serialised by the caller. */
 int lfgpu_pcg_noalloc(lfgpu_ctx *ctx, const lfgpu_csr *A, const lfgpu_vec *b,

@@ -62,6 +62,7 @@ int exclusive_scan_i32(hipStream_t s, const int32_t *in, int32_t *out, int64_t n
 
 struct lfgpu_ctx {
   int device = 0;
+  int cus = 0;  // compute units (the largest team of a resident solve)
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t evp[2] = {nullptr, nullptr};  // solver polls (no timing)

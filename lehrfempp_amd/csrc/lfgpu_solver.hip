@@ -30,6 +30,7 @@
 
 #include "lfgpu_internal.h"
 #include "lfgpu_reduce.h"
+#include "lfgpu_resident.h"
 
 using namespace lfgpu;
 
@@ -118,6 +119,7 @@ struct lfgpu_solver_cache {
   int32_t blk_n = 0, blk_cap = 0;
   int32_t *blk_srow = nullptr, *blk_smap = nullptr;
   double *blk_t = nullptr;
+  ResidentBufs res;  // resident solves (lfgpu_resident.hip)
 };
 
 namespace lfgpu {
@@ -127,6 +129,7 @@ void solver_cache_free(lfgpu_csr *A) {
   lfgpu_solver_cache *c = A->cache;
   if (!c) return;
   if (c->cg_graphs) cg_graphs_destroy(c->cg_graphs);
+  resident_free(&c->res);
   for (void *p : {(void *)c->slice_off, (void *)c->s_col, (void *)c->s_dcol, (void *)c->val, (void *)c->val32,
                   (void *)c->dinv, (void *)c->dinv32, (void *)c->dinv16, (void *)c->rowsum, (void *)c->rowsum32,
                   (void *)c->r, (void *)c->p, (void *)c->q, (void *)c->r32, (void *)c->p32,
@@ -3664,6 +3667,27 @@ int pcg_finish(lfgpu_ctx *ctx, const PcgState *hs, bool mixed, lfgpu_pcg_info *i
   }
   return LFGPU_OK;
 }
+
+// end of a resident solve: one wait, then as pcg_finish
+int resident_finish(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentState *rs, bool mixed,
+                    lfgpu_pcg_info *info) {
+  LFG_HIP(hipEventRecord(ctx->ev1, ctx->stream));
+  LFG_HIP(hipEventSynchronize(ctx->ev1));
+  if (rs->aborted) {
+    bufs->epoch = 0xffffffffu;  // the next solve clears the words and the flag
+    set_error("resident PCG: a workgroup waited over 4 s for another one's values");
+    return LFGPU_EHIP;
+  }
+  PcgState h{};
+  h.bb = rs->bb;
+  h.rr = rs->rr;
+  h.iter = rs->iter;
+  h.converged = rs->converged;
+  h.refinements = rs->refinements;
+  const int rc = pcg_finish(ctx, &h, mixed, info);
+  if (info) info->syncs = 1;
+  return rc;
+}
 }  // namespace
 
 extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b, lfgpu_vec *x,
@@ -3716,6 +3740,25 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
   // FP64 two-sweep and row-sweep iterations replay a captured graph of each
   // chunk below 2^20 rows (launch-bound sizes), or as the caller asks
   const bool use_graph = opts->graph > 0 || (opts->graph == 0 && n < (1 << 20));
+
+  // FP64 on DIA storage: the resident solve (lfgpu_resident.hip) where the
+  // system fits the chip, unless the caller asked for graph replays or plain
+  // launches of the sweeps
+  if (!mixed && !single && c->fmt == FMT_DIA && c->blk_n == 0 && opts->graph == 0 && !t_timer) {
+    ResidentDia rd;
+    rd.n = n;
+    rd.ndiag = c->ndiag;
+    rd.off = c->off;
+    rd.val = c->val;
+    rd.rowsum = c->rowsum;
+    rd.dinv = c->dinv;
+    rd.sym = c->sym64;
+    ResidentState *rs = reinterpret_cast<ResidentState *>(ctx->pinned);
+    bool taken = false;
+    LFG_HIP(hipEventRecord(ctx->ev0, s));
+    LFG_TRY(resident_pcg_dia(ctx, &c->res, rd, b->d, x->d, opts->rtol, opts->maxit, rs, &taken));
+    if (taken) return resident_finish(ctx, &c->res, rs, false, info);
+  }
 
   if (single && !c->cg1)
     LFG_TRY(dalloc(&c->cg1, (size_t)6 * n, "single-reduction PCG vectors"));
