@@ -573,28 +573,42 @@ int dia_symmetry(lfgpu_ctx *ctx, lfgpu_solver_cache *c, int32_t n) {
   return LFGPU_OK;
 }
 
-// DIA when the off-diagonal offsets of a middle row cover every row and
-// storing whole diagonals wastes at most 25 %.
+// DIA when the off-diagonal offsets of one row cover every row and storing
+// whole diagonals wastes at most 25 %.  The row is the one with the most
+// off-diagonals of three near the middle: the middle row itself starts a line
+// of a structured mesh with an even number of lines, where it lies on the
+// boundary and shows the offsets of an identity row (Dirichlet) or half of
+// them; 37 rows on is inside a line unless lines are short, n / 7 rows on
+// then most likely is.
 int detect_dia(lfgpu_ctx *ctx, const lfgpu_csr *A, DiagSet *ds) {
   hipStream_t s = ctx->stream;
   const int32_t n = A->nrows;
   ds->ndiag = 0;
   if (n < 2 * kSlice) return LFGPU_OK;
-  const int32_t mid = n / 2;
-  int32_t rp[2];
-  LFG_HIP(hipMemcpyAsync(rp, A->row_ptr + mid, 8, hipMemcpyDeviceToHost, s));
+  constexpr int kRows = 3, kMost = 64;
+  const int32_t at[kRows] = {n / 2, n / 2 + std::min(37, n / 4), n / 2 + n / 7};
+  int32_t rp[kRows][2], cols[kRows][kMost];
+  for (int k = 0; k < kRows; ++k)
+    LFG_HIP(hipMemcpyAsync(rp[k], A->row_ptr + at[k], 8, hipMemcpyDeviceToHost, s));
   LFG_HIP(hipStreamSynchronize(s));
-  const int32_t len = rp[1] - rp[0];
-  if (len <= 1 || len > 64) return LFGPU_OK;
-  std::vector<int32_t> cols(len);
-  LFG_HIP(hipMemcpyAsync(cols.data(), A->col + rp[0], len * 4, hipMemcpyDeviceToHost, s));
+  for (int k = 0; k < kRows; ++k) {
+    const int32_t len = std::min(rp[k][1] - rp[k][0], (int32_t)kMost);
+    if (len > 0)
+      LFG_HIP(hipMemcpyAsync(cols[k], A->col + rp[k][0], (size_t)len * 4, hipMemcpyDeviceToHost, s));
+  }
   LFG_HIP(hipStreamSynchronize(s));
   DiagSet cand{};
-  for (int32_t c : cols)
-    if (c != mid) {
-      if (cand.ndiag == kMaxDiag) return LFGPU_OK;
-      cand.off[cand.ndiag++] = c - mid;
-    }
+  for (int k = 0; k < kRows; ++k) {
+    const int32_t len = rp[k][1] - rp[k][0];
+    if (len > kMost) return LFGPU_OK;
+    DiagSet c{};
+    for (int32_t q = 0; q < len; ++q)
+      if (cols[k][q] != at[k]) {
+        if (c.ndiag == kMaxDiag) return LFGPU_OK;
+        c.off[c.ndiag++] = cols[k][q] - at[k];
+      }
+    if (c.ndiag > cand.ndiag) cand = c;
+  }
   if (cand.ndiag == 0) return LFGPU_OK;
   const int64_t offdiag_nnz = A->nnz - n;  // FE matrices carry every diagonal
   if ((double)cand.ndiag * n > 1.25 * (double)std::max<int64_t>(offdiag_nnz, 1)) return LFGPU_OK;
