@@ -305,8 +305,9 @@ typedef struct lfgpu_pcg_opts {
    * recurrences (default). */
   int single_reduction;
   /* FP64 two-sweep and row-sweep iterations: 0 = the whole solve in one
-   * launch with the vectors kept on the chip where the system fits (matrices
-   * on at most 6 diagonals; info->syncs is 1 then), else replay each chunk
+   * launch with the vectors kept on the chip where the system fits (P1
+   * matrices of structured meshes; all modes; info->syncs is 1 then), else
+   * replay each chunk
    * of check_every iterations from a captured hipGraph below 2^20 rows,
    * where the solve is bound by the launch rate (default); 1 = always replay
    * chunks; -1 = never (plain launches).  1 and -1 give the same iterates;

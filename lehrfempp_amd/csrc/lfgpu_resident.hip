@@ -8,22 +8,33 @@
 // thread (1.18M rows on 256 CUs) the matrix stays in registers too and an
 // iteration touches memory only for the boundary values and the team sums;
 // above, the matrix is streamed once an iteration.  Time per iteration, P1,
-// sweeps against this: 64^2 12.5 -> 3.2 us, 512^2 17.9 -> 5.3, 1024^2 32.0
-// -> 10.0, 2048 x 256 21.3 -> 11.7, 1400^2 53.9 -> 21.6, 2048^2 101 -> 52.8.
+// sweeps against this, in us:
+//              64^2   512^2   1023x770   1024^2   2048x256   1400^2   2048^2
+//   FP64     12.6/2.9 17.6/4.9 29.8/6.2 32.0/8.2  20.8/5.6 55.1/21.3  101/44
+//   FP32     15.2/4.0 14.4/5.4 19.6/6.7 21.8/7.3  17.0/6.0 31.6/15.1 57.6/33
+//   FP32 mat 17.4/4.4 16.7/5.4 24.3/6.6 30.5/7.2  21.1/6.0 46.6/14.8 85.3/49
 //
 // One iteration (the recurrences and the stopping test of the two-sweep
 // solver, with one team sum instead of two):
 //   q = A p; team sum of p.q, (q, D^-1 r), (q, D^-1 q) and of ||r||^2 and
 //   (r, D^-1 r) left by the previous update; stop if ||r||^2 < thr;
 //   alpha = rho / p.q, beta from rho' = rho - 2 alpha (q, D^-1 r) +
-//   alpha^2 (q, D^-1 q); x += alpha p, r -= alpha q, p = D^-1 r + beta p,
-//   the boundary values of p published as they are formed.
+//   alpha^2 (q, D^-1 q); x += alpha p, r -= alpha q, p = D^-1 r + beta p.
 // The product that runs beside the stopping test of the last iteration is
 // discarded, x is what the test was made on.
+//
+// The matrix lives on a lattice: S rows a line, L lines, every off-diagonal
+// couples a row to one of its eight lattice neighbours (the P1 matrix of a
+// structured mesh).  A workgroup owns a tile of the lattice.  Runs of
+// consecutive rows would need no lattice, but their halo is two lines a
+// workgroup: at 2048 x 256 (2560 rows and 4100 halo values a workgroup)
+// exchanging them took half of an iteration (11.5 us).
+#include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <cstdio>
+#include <cstdlib>
+#include <vector>
 
 #include "lfgpu_reduce.h"
 #include "lfgpu_resident.h"
@@ -34,20 +45,22 @@ using namespace lfgpu::res;
 
 namespace {
 
-constexpr int kMaxD = 6;
+constexpr int ND = 6;  // off-diagonals of a P1 matrix on a structured mesh
 
-struct DiaArgs {
-  int32_t n, rows;  // rows per workgroup
-  int32_t halo;     // largest |offset|
-  int32_t slots;    // published values per workgroup
-  int32_t lds;      // doubles of LDS
+struct TileArgs {
+  int32_t n;            // rows of the storage (a diagonal's stride)
+  int32_t S, L;         // lattice: rows a line, lines
+  int32_t TW, TH, TX;   // tile width and height, tiles a line
+  int32_t slots;        // values a workgroup publishes, 2 (TW + TH)
+  int32_t ghosts;       // most halo cells of a workgroup
   int ndiag;
-  int32_t off[kMaxD];
+  int32_t off[ND];      // row offset of diagonal d
+  int32_t shift[ND];    // its offset in the padded tile
   const double *__restrict__ val;
   const double *__restrict__ rowsum;
   const double *__restrict__ dinv;
   const double *__restrict__ b;
-  double *__restrict__ x;
+  double *x;
   word_t *halo_words;  // [2][team][2][slots]
   word_t *part, *total;
   int *abort;
@@ -55,12 +68,21 @@ struct DiaArgs {
   double tol2;
   int maxit;
   ResidentState *st;
+  // mixed modes
+  const float *__restrict__ val32;
+  const float *__restrict__ rowsum32;
+  const float *__restrict__ dinv32;
+  const __hip_bfloat16 *__restrict__ dinv16;
+  double *xlo;
+  double delta2;
+  int max_interval;
 };
 
 // A value of an array at a uniform base and a 32-bit byte offset per lane (one
 // address register for all the arrays of a row).
-__device__ __forceinline__ double load_at(const double *base, uint32_t bytes) {
-  return *reinterpret_cast<const double *>(reinterpret_cast<const char *>(base) + bytes);
+template <class T>
+__device__ __forceinline__ T load_at(const T *base, uint32_t bytes) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes);
 }
 // Hides a value from the optimiser, which else keeps every row's addresses
 // and masks in registers across the iterations (several hundred of them).
@@ -68,183 +90,316 @@ __device__ __forceinline__ int32_t opaque(int32_t v) {
   asm volatile("" : "+v"(v));
   return v;
 }
-__device__ __forceinline__ int32_t opaque_uniform(int32_t v) {
-  asm volatile("" : "+s"(v));
-  return v;
-}
 // Keeps a row's result where it is computed (the compiler else sinks whole
 // rows past the next barrier and spills their operands).
-__device__ __forceinline__ void pin(double &v) { asm volatile("" : "+v"(v)); }
+template <class T>
+__device__ __forceinline__ void pin(T &v) {
+  asm volatile("" : "+v"(v));
+}
 
-// The workgroup's rows and its place in the team's halo exchange: local row
-// i (0 <= i < rows) is global row r0 + i; its value sits at lp[halo + i], the
-// `halo` rows before and after at lp[0..halo) and lp[halo + rows ..).
-struct DiaRows {
-  int32_t n, r0, rows, mine, halo, slots, rank, team;
+// The workgroup's tile: tw x th cells of the lattice, padded by one halo cell
+// on each side to lines of P = TW + 2 cells.  Cell i = line * P + c (c = 0 and
+// c > tw are halo cells) is thread i % 512's cell number i / 512; it sits in
+// an LDS array at P + 1 + i, so that every neighbour is at a fixed distance.
+struct Tile {
+  int32_t S, P, tw, th, x0, y0, n, g0;
+  int32_t rank, team, TW, TH, TX, L, slots;
   word_t *words;
   int *abort;
   uint32_t tag;
+  int32_t *gpos, *gsrc, *ppos;  // LDS tables of the exchange
+  int32_t ng, np;
 
-  __device__ __forceinline__ word_t *slot(int32_t owner) const {
-    return words + ((size_t)(tag & 1u) * team + owner) * 2 * slots;
+  __device__ __forceinline__ Tile(const TileArgs &a, int32_t rank_, int32_t team_)
+      : S(a.S), P(a.TW + 2), n(a.n), rank(rank_), team(team_), TW(a.TW), TH(a.TH), TX(a.TX),
+        L(a.L), slots(a.slots), words(a.halo_words), abort(a.abort), tag(a.tag0) {
+    x0 = rank % TX * TW;
+    y0 = rank / TX * TH;
+    tw = min(TW, S - x0);
+    th = min(TH, L - y0);
+    g0 = y0 * S + x0;
+    ng = 2 * (tw + 2) + 2 * th;
+    np = team > 1 ? slots : 0;
+    gpos = gsrc = ppos = nullptr;
   }
-  __device__ __forceinline__ int32_t mine_of(int32_t g) const { return min(rows, n - g * rows); }
-  // fetches the lower (UP = false) or upper halo into dst[0..halo) with the
-  // threads from `first` on; four values' words are in flight per thread
-  // before the first is checked
-  template <bool UP>
-  __device__ __forceinline__ void fetch(double *dst, int first, int *bad) const {
-    const int32_t owner = UP ? rank + 1 : rank - 1;
-    if (owner < 0 || owner >= team) return;
-    const int32_t have = UP ? min(halo, mine_of(owner)) : halo;
-    const int32_t base = UP ? 0 : (rows <= 2 * halo ? rows - halo : halo);
+
+  // Walks this thread's cells in order: column c and row g of cell number j.
+  struct Walk {
+    int32_t c, g, line;
+  };
+  __device__ __forceinline__ Walk first(int32_t t) const {
+    Walk w;
+    w.line = t / P;
+    w.c = t - w.line * P;
+    w.g = g0 + w.line * S + w.c - 1;
+    return w;
+  }
+  __device__ __forceinline__ void next(Walk &w) const {
+    const int32_t lines = kThreads / P, cols = kThreads - lines * P;  // uniform
+    w.c += cols;
+    w.g += lines * S + cols;
+    w.line += lines;
+    if (w.c >= P) {
+      w.c -= P;
+      w.g += S - P;
+      w.line += 1;
+    }
+  }
+  __device__ __forceinline__ bool alive(const Walk &w) const {
+    return w.line < th && w.c >= 1 && w.c <= tw;
+  }
+
+  // Halo cell h: its place in an LDS array and the word its owner publishes
+  // it in (-1: outside the lattice).  Every workgroup publishes the cells of
+  // its tile's rim: top line, bottom line, left and right column; a cell on
+  // two of them is read from the first.
+  __device__ void tables(int32_t t) {
+    for (int32_t h = t; h < ng; h += kThreads) {
+      int32_t line, c;
+      if (h < 2 * (tw + 2)) {
+        line = h < tw + 2 ? -1 : th;
+        c = h < tw + 2 ? h : h - (tw + 2);
+      } else {
+        const int32_t k = h - 2 * (tw + 2);
+        line = k < th ? k : k - th;
+        c = k < th ? 0 : tw + 1;
+      }
+      gpos[h] = P + 1 + line * P + c;
+      const int32_t gx = x0 + c - 1, gy = y0 + line;
+      int32_t src = -1;
+      if (gx >= 0 && gx < S && gy >= 0 && gy < L) {
+        const int32_t ox = gx / TW, oy = gy / TH, lx = gx - ox * TW, ly = gy - oy * TH;
+        const int32_t oth = min(TH, L - oy * TH);
+        const int32_t s = ly == 0 ? lx : ly == oth - 1 ? TW + lx
+                          : lx == 0 ? 2 * TW + ly : 2 * TW + TH + ly;
+        src = (oy * TX + ox) * 2 * slots + s;
+      }
+      gsrc[h] = src;
+    }
+    for (int32_t s = t; s < slots; s += kThreads) {
+      int32_t line, lx;
+      if (s < 2 * TW) {
+        line = s < TW ? 0 : th - 1;
+        lx = s < TW ? s : s - TW;
+      } else {
+        const int32_t k = s - 2 * TW;
+        line = k < TH ? k : k - TH;
+        lx = k < TH ? 0 : tw - 1;
+      }
+      ppos[s] = lx < tw && line < th ? P + 1 + line * P + lx + 1 : -1;
+    }
+  }
+
+  // Publishes the rim cells of src (indexed like an LDS array of the tile),
+  // with the threads from `first` on.
+  template <class VT, class A>
+  __device__ __forceinline__ void publish(const A *src, int first) const {
+    if ((int)threadIdx.x < first) return;
+    word_t *w = words + ((size_t)(tag & 1u) * team + rank) * 2 * slots;
+    for (int32_t s = (int32_t)threadIdx.x - first; s < np; s += kThreads - first) {
+      const int32_t at = ppos[s];
+      if (at < 0) continue;
+      if constexpr (sizeof(VT) == 8) {
+        const double v = (double)src[at];
+        put(&w[s], low_word(v, tag));
+        put(&w[slots + s], high_word(v, tag));
+      } else {
+        put(&w[s], ((word_t)__float_as_uint((float)src[at]) << 32) | tag);
+      }
+    }
+  }
+  // Waits for the halo cells and hands (h, place, value) to fn, two cells per
+  // thread in flight, with the threads from `first` on.
+  template <class VT, class F>
+  __device__ __forceinline__ void fetch(int first, int *bad, F &&fn) const {
+    if (team == 1 || (int)threadIdx.x < first) return;
+    const word_t *w = words + (size_t)(tag & 1u) * team * 2 * slots;
     const int32_t step = kThreads - first;
-    const word_t *w = slot(owner) + base;
-    for (int32_t h0 = (int32_t)threadIdx.x - first; h0 < have; h0 += 4 * step) {
-      word_t lo[4], hi[4];
+    for (int32_t h0 = (int32_t)threadIdx.x - first; h0 < ng; h0 += 2 * step) {
+      int32_t src[2];
+      word_t lo[2], hi[2];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) src[u] = h0 + u * step < ng ? gsrc[h0 + u * step] : -1;
       bool ok;
       Wait wait(abort);
       do {
         ok = true;
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int32_t h = min(h0 + u * step, have - 1);
-          lo[u] = get(&w[h]);
-          hi[u] = get(&w[slots + h]);
-        }
+        for (int u = 0; u < 2; ++u)
+          if (src[u] >= 0) {
+            lo[u] = get(&w[src[u]]);
+            if constexpr (sizeof(VT) == 8) hi[u] = get(&w[src[u] + slots]);
+          }
 #pragma unroll
-        for (int u = 0; u < 4; ++u) ok = ok && tagged(lo[u], tag) && tagged(hi[u], tag);
+        for (int u = 0; u < 2; ++u)
+          if (src[u] >= 0) {
+            ok = ok && tagged(lo[u], tag);
+            if constexpr (sizeof(VT) == 8) ok = ok && tagged(hi[u], tag);
+          }
       } while (!ok && wait.more());
       if (!ok) *bad = 1;
 #pragma unroll
-      for (int u = 0; u < 4; ++u)
-        if (h0 + u * step < have) dst[h0 + u * step] = from_words(lo[u], hi[u]);
+      for (int u = 0; u < 2; ++u)
+        if (src[u] >= 0) {
+          VT v;
+          if constexpr (sizeof(VT) == 8) v = from_words(lo[u], hi[u]);
+          else v = __uint_as_float((uint32_t)(lo[u] >> 32));
+          fn(h0 + u * step, gpos[h0 + u * step], v);
+        }
     }
+  }
+  // The halo of an LDS array whose values are VTs, from the neighbours' rims;
+  // a workgroup barrier has to precede it and to follow it.
+  template <class VT, class A>
+  __device__ __forceinline__ void exchange(A *arr, int *bad) {
+    ++tag;
+    publish<VT>(arr, 0);
+    fetch<VT>(0, bad, [&](int32_t, int32_t at, VT v) { arr[at] = (A)v; });
   }
 };
 
-// The rows that a workgroup publishes in one exchange: the first and the last
-// `halo` (none without a team).
-struct Publisher {
-  int32_t below, from, shift, mine;
-  uint32_t tag;
-  word_t *lo, *hi;
-  __device__ __forceinline__ explicit Publisher(const DiaRows &D)
-      : below(D.team > 1 ? D.halo : 0),
-        from(D.team > 1 ? D.rows - D.halo : 0x7fffffff),
-        shift(max(D.rows - 2 * D.halo, 0)),
-        mine(D.mine),
-        tag(D.tag),
-        lo(D.slot(D.rank)),
-        hi(lo + D.slots) {}
-  // local row i of a wavefront whose first row (uniform) is i0
-  __device__ __forceinline__ void operator()(int32_t i0, int32_t i, double v) const {
-    if (i0 >= below && i0 + 63 < from) return;
-    if ((i < below || i >= from) && i < mine) {
-      const uint32_t at = (uint32_t)(i < below ? i : i - shift);
-      put(lo + at, low_word(v, tag));
-      put(hi + at, high_word(v, tag));
+// How a variant keeps the matrix and the halo.
+//   GHOST: the matrix stays in registers.  The halo cells' r, q, D^-1 and p
+//     are kept here as well and updated by the same operations as their
+//     owners', so that what travels is q: it is published beside the partial
+//     sums and arrives while the team sum runs, which takes the exchange off
+//     the iteration's critical path.
+//   STREAM: the matrix (its upper half: symmetric values) is read from memory
+//     every iteration, the next row's loads in flight while a row is worked
+//     on; p travels between the update and the next product.
+enum { GHOST, STREAM };
+
+// The threads that carry the exchange of q while the others wait for the
+// team sum: all but the first wavefront, or but the four that sum the
+// members' partials.
+__device__ __forceinline__ int exchange_threads(const Team &tm) {
+  return sums_members(tm) ? kMaxTeam : 64;
+}
+
+// From this many cells a thread the GHOST variants keep row sums and D^-1 in
+// LDS (9 cells' r, q, x and six diagonals take 162 of the 256 registers; with
+// the two others in registers too 1024^2 spilled and took 11.7 us an iteration
+// instead of 8.2).
+constexpr int kLdsDiag = 7;
+
+// LDS: p (FP64 in every mode: converting the neighbours' values of an FP32 p
+// in every product costs more than the bytes), q (GHOST) and the exchange's
+// tables.
+template <int KIND, class VT, int RPT>
+struct TileLds {
+  static constexpr bool kDiag = KIND == GHOST && RPT >= kLdsDiag;
+  double *lp;           // padded tile of p (and of the vectors of a reliable update)
+  double *rs, *di;      // kDiag: row sums and D^-1 of cell j of thread t at t + 512 j
+  VT *lq, *gr, *gq, *gd;
+  __device__ __forceinline__ TileLds(double *base, const TileArgs &a, Tile &T) {
+    const int32_t n = cells(a.TW);
+    lp = base;
+    base += n;
+    rs = di = nullptr;
+    if (kDiag) {
+      rs = base;
+      di = rs + RPT * kThreads;
+      base = di + RPT * kThreads;
     }
+    VT *v = reinterpret_cast<VT *>(base);
+    lq = v;
+    gr = gq = gd = nullptr;
+    if (KIND == GHOST) {
+      gr = v + n;
+      gq = gr + a.ghosts;
+      gd = gq + a.ghosts;
+      v = gd + a.ghosts;
+    }
+    T.gpos = reinterpret_cast<int32_t *>(v);
+    T.gsrc = T.gpos + a.ghosts;
+    T.ppos = T.gsrc + a.ghosts;
+  }
+  // cells of one padded array: what any cell number's neighbours reach
+  static __host__ __device__ int32_t cells(int32_t TW) {
+    return (kThreads * RPT + 2 * (TW + 3) + 1) / 2 * 2;
+  }
+  static size_t bytes(const TileArgs &a) {
+    const size_t n = (size_t)cells(a.TW);
+    return n * 8 + (kDiag ? 2 * (size_t)RPT * kThreads * 8 : 0) +
+           (KIND == GHOST ? (n + 3 * (size_t)a.ghosts) * sizeof(VT) : 0) +
+           4 * (2 * (size_t)a.ghosts + a.slots) + 16;
   }
 };
 
-constexpr int ND = 6;  // off-diagonals of a P1 matrix on a structured mesh
-
-// How a variant keeps the neighbours' values of p and the matrix.
-//   GHOST: the matrix stays in registers.  The neighbours' r, q, D^-1 and p
-//     of the halo rows are kept here as well and updated by the same
-//     operations as their owners', so that what travels is q: it is published
-//     with the partial sums and arrives while the team sum runs, which takes
-//     the exchange off the iteration's critical path.
-//   HALO: the matrix stays in registers; p travels, published by the update
-//     and waited for by the next product.
-//   STREAM: p travels as in HALO; the matrix (its upper half: symmetric
-//     values) is read from memory every iteration, the next row's loads in
-//     flight while a row is worked on.  The upper halo takes the lower one's
-//     place for the second half of the rows, which is what lets 16401 rows
-//     with offsets of 2050 fit 160 KB.
-enum { GHOST, HALO, STREAM };
-
-// RPT: rows per thread (thread t of a workgroup owns its local rows t + 512 j).
-// XR: the rows j < XR keep their x in a register, the others' is read and
-// written in every update (as many as the registers hold without spills).
-template <int KIND, int RPT, int XR>
-__global__ __launch_bounds__(kThreads) void k_res_dia(DiaArgs a) {
+// RPT: cells per thread.  XR: the cells j < XR keep their x in a register, the
+// others' is read and written in every update (as many as the registers hold
+// without spills).  AHEAD: rows of a stream in flight.
+template <int KIND, int RPT, int XR, int AHEAD = 1>
+__global__ __launch_bounds__(kThreads) void k_res_tile(TileArgs a) {
   constexpr bool kStream = KIND == STREAM, kGhost = KIND == GHOST;
-  constexpr int kHalf = (RPT + 1) / 2;  // STREAM: rows before the upper halo's turn
-  extern __shared__ double lp[];
+  extern __shared__ double dyn[];
   __shared__ SumLds sh;
   const int t = threadIdx.x;
-  const int32_t w0 = __builtin_amdgcn_readfirstlane(t & ~63);  // the wavefront's first row
-  DiaRows D;
-  D.n = a.n;
-  D.rank = blockIdx.x;
-  D.team = gridDim.x;
-  D.rows = a.rows;
-  D.r0 = D.rank * a.rows;
-  D.mine = D.mine_of(D.rank);
-  D.halo = a.halo;
-  D.slots = a.slots;
-  D.words = a.halo_words;
-  D.abort = a.abort;
-  D.tag = a.tag0;
-  Team tm{D.rank, D.team, a.part, a.total, a.abort, a.tag0};
+  Tile T(a, blockIdx.x, gridDim.x);
+  typedef TileLds<KIND, double, RPT> Lds;
+  const Lds M(dyn, a, T);
+  constexpr bool kRegDiag = !kStream && !Lds::kDiag;
+  double *const lp = M.lp;
+  Team tm{T.rank, T.team, a.part, a.total, a.abort, a.tag0};
   if (t == 0) sh.bad = 0;
-  const int32_t mine = D.mine, H = a.halo;
-  for (int32_t i = t; i < a.lds; i += kThreads) lp[i] = 0.0;
-  double *const up = lp + (kStream ? 0 : H + a.rows);  // the upper halo
-  // GHOST: r, q and D^-1 of the halo rows
-  double *const gr = lp + 2 * H + RPT * kThreads, *const gq = gr + 2 * H, *const gd = gq + 2 * H;
+  T.tables(t);
+  const int32_t cells = Lds::cells(a.TW);
+  for (int32_t i = t; i < cells; i += kThreads) lp[i] = 0.0;
+  if constexpr (kGhost)
+    for (int32_t h = t; h < T.ng; h += kThreads) M.gr[h] = M.gq[h] = M.gd[h] = 0.0;
+  const int32_t at0 = T.P + 1 + t;  // LDS place of the thread's first cell
 
   double x[XR > 0 ? XR : 1], r[RPT], q[RPT];
-  double v[kStream ? 1 : RPT][ND], rs[kStream ? 1 : RPT], di[kStream ? 1 : RPT];
-  const double *rowsum = a.rowsum + D.r0, *dinv = a.dinv + D.r0;
-  double *xg = a.x + D.r0;
+  double v[kStream ? 1 : RPT][ND], rs[kRegDiag ? RPT : 1], di[kRegDiag ? RPT : 1];
+  uint64_t live = 0;  // the thread's cells that are rows of the tile
   __syncthreads();
-  // x0 and its boundary values
-  ++D.tag;
-  const Publisher pub0(D);
+  {
+    Tile::Walk w = T.first(t);
 #pragma unroll
-  for (int j = 0; j < RPT; ++j) {
-    const int32_t i = t + j * kThreads;
-    r[j] = q[j] = 0.0;
-    if (j < XR) x[j] = 0.0;
-    if constexpr (!kStream) {
-      rs[j] = di[j] = 0.0;
-#pragma unroll
-      for (int d = 0; d < ND; ++d) v[j][d] = 0.0;
-    }
-    if (i < mine) {
-      const double xi = xg[i];
-      if (j < XR) x[j] = xi;
-      lp[H + i] = xi;
-      pub0(w0 + j * kThreads, i, xi);
+    for (int j = 0; j < RPT; ++j) {
+      r[j] = q[j] = 0.0;
+      if (j < XR) x[j] = 0.0;
       if constexpr (!kStream) {
-        rs[j] = rowsum[i];
-        di[j] = dinv[i];
+        if constexpr (kRegDiag) rs[j] = di[j] = 0.0;
+        else M.rs[t + j * kThreads] = M.di[t + j * kThreads] = 0.0;
 #pragma unroll
-        for (int d = 0; d < ND; ++d)
-          if (d < a.ndiag) v[j][d] = a.val[(int64_t)d * a.n + D.r0 + i];
+        for (int d = 0; d < ND; ++d) v[j][d] = 0.0;
       }
+      if (T.alive(w)) {
+        live |= 1ull << j;
+        const double xi = a.x[w.g];
+        if (j < XR) x[j] = xi;
+        lp[at0 + j * kThreads] = xi;
+        if constexpr (!kStream) {
+          if constexpr (kRegDiag) {
+            rs[j] = a.rowsum[w.g];
+            di[j] = a.dinv[w.g];
+          } else {
+            M.rs[t + j * kThreads] = a.rowsum[w.g];
+            M.di[t + j * kThreads] = a.dinv[w.g];
+          }
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+            if (d < a.ndiag) v[j][d] = a.val[(int64_t)d * a.n + w.g];
+        }
+      }
+      T.next(w);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_barrier(0);
   }
-  if constexpr (kGhost) {
-    for (int32_t h = t; h < 2 * H; h += kThreads) {
-      const int32_t g = h < H ? D.r0 - H + h : D.r0 + D.rows + h - H;
-      if (g >= 0 && g < a.n) gd[h] = a.dinv[g];
-    }
-  }
+  __syncthreads();
+  T.template exchange<double>(lp, &sh.bad);
+  __syncthreads();
 
   // q_j = (A p)_i in difference form from LDS, handed to fn with p_i and
-  // D^-1_i; the rows past the workgroup's end give q = 0
+  // D^-1_i; cells that are no rows give q = 0
   auto sweep = [&](auto &&fn) {
-    const int32_t ti = opaque(t);
-    const double *lc = lp + H + ti;
+    const double *lc = lp + opaque(at0);
     const double *bp[ND];
 #pragma unroll
-    for (int d = 0; d < ND; ++d) bp[d] = lc + a.off[d];
+    for (int d = 0; d < ND; ++d) bp[d] = lc + a.shift[d];
     if constexpr (!kStream) {
+      const double *lrs = M.rs + opaque(t), *ldi = M.di + opaque(t);
 #pragma unroll
       for (int j = 0; j < RPT; ++j) {
         // every LDS read of the row before the first use
@@ -252,115 +407,112 @@ __global__ __launch_bounds__(kThreads) void k_res_dia(DiaArgs a) {
         double c[ND], acc = 0.0;
 #pragma unroll
         for (int d = 0; d < ND; ++d) c[d] = bp[d][j * kThreads];
+        const double s = kRegDiag ? rs[kRegDiag ? j : 0] : lrs[j * kThreads];
+        const double dv = kRegDiag ? di[kRegDiag ? j : 0] : ldi[j * kThreads];
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int d = 0; d < ND; ++d) acc = __builtin_fma(v[j][d], c[d] - pi, acc);
-        q[j] = __builtin_fma(rs[j], pi, acc);
+        q[j] = __builtin_fma(s, pi, acc);
         pin(q[j]);
-        fn(j, pi, di[j]);
+        fn(j, pi, dv);
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      // the next row of the stream: the diagonals (the lower ones as the
-      // mirrored upper ones), row sum and D^-1
-      double nv[ND], ns, nd;
+      // the next rows of the stream: the diagonals (the lower ones as the
+      // mirrored upper ones: zero before the first row), row sum and D^-1
+      double nv[AHEAD][ND], ns[AHEAD], nd[AHEAD];
+      Tile::Walk w = T.first(opaque(t));
       auto load_row = [&](int j) {
-        const uint32_t at = (uint32_t)min(ti + j * kThreads, mine - 1) * 8u;
+        const int k = j % AHEAD;
+        const int32_t g = (live >> j) & 1 ? w.g : T.g0;
+        const uint32_t at = (uint32_t)g * 8u;
 #pragma unroll
         for (int d = 0; d < ND; ++d) {
-          const double *m = a.val + (int64_t)(d < ND / 2 ? ND - 1 - d : d) * a.n + D.r0;
-          if (d < ND / 2) {
-            m += a.off[d];
-            // (only the first workgroup's first rows have no such neighbour)
-            if (j < kHalf) {
-              const int32_t from = -(D.r0 + a.off[d]) * 8;
-              const double w = load_at(m, (uint32_t)max((int32_t)at, from));
-              nv[d] = (int32_t)at >= from ? w : 0.0;
-            } else {
-              nv[d] = load_at(m, at);
-            }
-          } else {
-            nv[d] = load_at(m, at);
-          }
+          if (d < ND / 2)
+            nv[k][d] =
+                load_at(a.val + (int64_t)(ND - 1 - d) * a.n, (uint32_t)max(g + a.off[d], 0) * 8u);
+          else
+            nv[k][d] = load_at(a.val + (int64_t)d * a.n, at);
         }
-        ns = load_at(rowsum, at);
-        nd = load_at(dinv, at);
+        if (T.y0 == 0) {
+#pragma unroll
+          for (int d = 0; d < ND / 2; ++d)
+            if (g + a.off[d] < 0) nv[k][d] = 0.0;
+        }
+        ns[k] = load_at(a.rowsum, at);
+        nd[k] = load_at(a.dinv, at);
+        T.next(w);
       };
-      load_row(0);
-      D.template fetch<false>(lp, 0, &sh.bad);
-      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) load_row(j);
 #pragma unroll
       for (int j = 0; j < RPT; ++j) {
-        if (j == kHalf) {
-          __syncthreads();
-          D.template fetch<true>(up, 0, &sh.bad);
-          __syncthreads();
-        }
         double vr[ND];
 #pragma unroll
-        for (int d = 0; d < ND; ++d) vr[d] = nv[d];
-        const double s = ns, dv = nd;
-        // every LDS read of the row and the next row's loads before the first use
+        for (int d = 0; d < ND; ++d) vr[d] = nv[j % AHEAD][d];
+        const double s = ns[j % AHEAD], dv = nd[j % AHEAD];
         const double pi = lc[j * kThreads];
         double c[ND], acc = 0.0;
 #pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          const double *p = bp[d] + j * kThreads;
-          // past the last row: the upper halo in the lower one's place
-          if (j >= kHalf && d >= ND / 2)
-            if (ti >= a.rows - a.off[d] - j * kThreads) p -= H + a.rows;
-          c[d] = *p;
-        }
-        if (j + 1 < RPT) load_row(j + 1);
+        for (int d = 0; d < ND; ++d) c[d] = bp[d][j * kThreads];
+        if (AHEAD == 1 && j + 1 < RPT) load_row(j + 1);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int d = 0; d < ND; ++d) acc = __builtin_fma(vr[d], c[d] - pi, acc);
         const double qi = __builtin_fma(s, pi, acc);
-        q[j] = ti + j * kThreads < mine ? qi : 0.0;
+        q[j] = (live >> j) & 1 ? qi : 0.0;
         pin(q[j]);
         fn(j, pi, dv);
         __builtin_amdgcn_sched_barrier(0);
+        if (AHEAD > 1 && j + AHEAD < RPT) load_row(j + AHEAD);
       }
     }
   };
 
   double rr = 0.0, rz = 0.0, bb = 0.0;
-  if constexpr (!kStream) {
-    D.template fetch<false>(lp, 0, &sh.bad);
-    D.template fetch<true>(up, 0, &sh.bad);
-    __syncthreads();
-  }
   sweep([&](int, double, double) {});
   __syncthreads();
-  // r = b - A x, p = D^-1 r; r (GHOST) or p travels
-  ++D.tag;
-  const Publisher pub1(D);
+  // r = b - A x, p = D^-1 r
+  {
+    Tile::Walk w = T.first(opaque(t));
 #pragma unroll
-  for (int j = RPT - 1; j >= 0; --j) {
-    const int32_t i = t + j * kThreads;
-    if (i < mine) {
-      const double bi = a.b[D.r0 + i];
-      r[j] = bi - q[j];
-      const double z = (kStream ? dinv[i] : di[kStream ? 0 : j]) * r[j];
-      lp[H + i] = z;
-      pub1(w0 + j * kThreads, i, kGhost ? r[j] : z);
-      bb += bi * bi;
-      rr += r[j] * r[j];
-      rz += r[j] * z;
+    for (int j = 0; j < RPT; ++j) {
+      if ((live >> j) & 1) {
+        const double bi = a.b[w.g];
+        r[j] = bi - q[j];
+        const double z =
+            (kRegDiag ? di[kRegDiag ? j : 0] : kStream ? a.dinv[w.g] : M.di[t + j * kThreads]) *
+            r[j];
+        lp[at0 + j * kThreads] = z;
+        if constexpr (kGhost) M.lq[at0 + j * kThreads] = r[j];
+        bb = __builtin_fma(bi, bi, bb);
+        rr = __builtin_fma(r[j], r[j], rr);
+        rz = __builtin_fma(r[j], z, rz);
+      }
+      T.next(w);
+      __builtin_amdgcn_sched_barrier(0);
     }
-    __builtin_amdgcn_sched_barrier(0);
+  }
+  if constexpr (kGhost) {
+    // the halo cells' r, D^-1 and p = D^-1 r
+    __syncthreads();
+    ++T.tag;
+    T.template publish<double>(M.lq, 0);
+    T.template fetch<double>(0, &sh.bad, [&](int32_t h, int32_t at, double rv) {
+      const int32_t cell = at - T.P - 1 + T.P;  // from the line above the tile
+      const int32_t line = cell / T.P - 1, c = cell - (line + 1) * T.P;
+      const double d = a.dinv[T.g0 + line * T.S + c - 1];
+      M.gr[h] = rv;
+      M.gd[h] = d;
+      lp[at] = d * rv;
+    });
   }
   int iter = 0, converged = 0;
   bool run = true, ok;
   double thr, rr_out;
   {
     double s[2] = {bb, rr};
-    ok = team_sum(tm, sh, s, [&] {
-      if constexpr (kGhost) {
-        D.template fetch<false>(gr, kIdle, &sh.bad);
-        D.template fetch<true>(gr + H, kIdle, &sh.bad);
-      }
-    });
+    ok = team_sum(tm, sh, s, [] {});
     bb = s[0];
     rr_out = s[1];
     thr = a.tol2 * bb;
@@ -372,34 +524,29 @@ __global__ __launch_bounds__(kThreads) void k_res_dia(DiaArgs a) {
       run = false;
     }
   }
-  if constexpr (kGhost) {
-    for (int32_t h = t; h < 2 * H; h += kThreads) lp[h < H ? h : D.rows + h] = gd[h] * gr[h];
-  }
   for (int k = 0; run && ok; ++k) {
     double s[5] = {0.0, 0.0, 0.0, rr, rz};
-    if constexpr (KIND == HALO) {
-      D.template fetch<false>(lp, 0, &sh.bad);
-      D.template fetch<true>(up, 0, &sh.bad);
+    __syncthreads();
+    if constexpr (kStream) {
+      T.template exchange<double>(lp, &sh.bad);
+      __syncthreads();
     }
-    if constexpr (kGhost) ++D.tag;
-    if constexpr (!kStream) __syncthreads();
-    {
-      const int32_t wi = opaque_uniform(w0);
-      const int32_t tp = opaque(t);
-      const Publisher pub(D);
-      sweep([&](int j, double pi, double dv) {
-        if constexpr (kGhost) pub(wi + j * kThreads, tp + j * kThreads, q[j]);
-        const double dq = dv * q[j];
-        s[0] = __builtin_fma(pi, q[j], s[0]);
-        s[1] = __builtin_fma(dq, r[j], s[1]);
-        s[2] = __builtin_fma(dq, q[j], s[2]);
-        pin(s[0]), pin(s[1]), pin(s[2]);
-      });
-    }
+    double *lqc = M.lq + opaque(at0);
+    sweep([&](int j, double pi, double dv) {
+      if constexpr (kGhost) lqc[j * kThreads] = q[j];
+      const double dq = dv * q[j];
+      s[0] = __builtin_fma(pi, q[j], s[0]);
+      s[1] = __builtin_fma(dq, r[j], s[1]);
+      s[2] = __builtin_fma(dq, q[j], s[2]);
+      pin(s[0]), pin(s[1]), pin(s[2]);
+    });
+    if constexpr (kGhost) ++T.tag;
     ok = team_sum(tm, sh, s, [&] {
       if constexpr (kGhost) {
-        D.template fetch<false>(gq, kIdle, &sh.bad);
-        D.template fetch<true>(gq + H, kIdle, &sh.bad);
+        const int first = exchange_threads(tm);
+        T.template publish<double>(M.lq, first);
+        T.template fetch<double>(first, &sh.bad,
+                                 [&](int32_t h, int32_t, double qv) { M.gq[h] = qv; });
       }
     });
     if (!ok) break;
@@ -415,27 +562,33 @@ __global__ __launch_bounds__(kThreads) void k_res_dia(DiaArgs a) {
     const double rho_next = rho - 2.0 * alpha * s[1] + alpha * alpha * s[2];
     const double beta = rho_next / rho;
     rr = rz = 0.0;
-    if constexpr (!kGhost) ++D.tag;
-    const Publisher pub(D);
-    const int32_t ti = opaque(t), wi = opaque_uniform(w0);
-    double *lc = lp + H + ti;
+    double *lc = lp + opaque(at0);
     // the next row's streamed values
     double nd = 0.0, nx = 0.0;
+    Tile::Walk w = T.first(opaque(t));
+    uint32_t xat = 0, nxat = 0;
     auto load_update = [&](int j) {
-      const uint32_t at = (uint32_t)min(ti + j * kThreads, mine - 1) * 8u;
-      if constexpr (kStream) nd = load_at(dinv, at);
-      if (j >= XR) nx = load_at(xg, at);
+      if constexpr (kStream) {
+        nxat = (uint32_t)((live >> j) & 1 ? w.g : T.g0) * 8u;
+        nd = load_at(a.dinv, nxat);
+        if (j >= XR) nx = load_at(a.x, nxat);
+        T.next(w);
+      }
     };
-    load_update(RPT - 1);
+    load_update(0);
+    const double *ldi = M.di + opaque(t);
+    double np = lc[0];
 #pragma unroll
-    for (int j = RPT - 1; j >= 0; --j) {
-      const int32_t i = ti + j * kThreads;
-      const double dv = kStream ? nd : di[kStream ? 0 : j];
+    for (int j = 0; j < RPT; ++j) {
+      const double dv = kRegDiag ? di[kRegDiag ? j : 0] : kStream ? nd : ldi[j * kThreads];
       const double xi = j < XR ? x[j < XR ? j : 0] : nx;
-      if (j > 0) load_update(j - 1);
-      // (the rows past the end: q, r and their sums stay zero; what they
-      // read of p is finite where the solve is)
-      const double pi = lc[j * kThreads];
+      xat = nxat;
+      const double pi = np;
+      if (j + 1 < RPT) {
+        load_update(j + 1);
+        np = lc[(j + 1) * kThreads];
+      }
+      // (cells that are no rows: r, q and so their sums stay zero)
       const double xn = __builtin_fma(alpha, pi, xi);
       if (j < XR) x[j < XR ? j : 0] = xn;
       r[j] = __builtin_fma(-alpha, q[j], r[j]);
@@ -443,40 +596,408 @@ __global__ __launch_bounds__(kThreads) void k_res_dia(DiaArgs a) {
       const double p = __builtin_fma(beta, pi, z);
       rr = __builtin_fma(r[j], r[j], rr);
       rz = __builtin_fma(r[j], z, rz);
-      if (i < mine) {
+      if ((live >> j) & 1) {
         lc[j * kThreads] = p;
-        if (j >= XR) xg[i] = xn;
+        if (j >= XR) *reinterpret_cast<double *>(reinterpret_cast<char *>(a.x) + xat) = xn;
       }
-      if constexpr (!kGhost) pub(wi + j * kThreads, i, p);
       pin(r[j]), pin(rr), pin(rz);
       __builtin_amdgcn_sched_barrier(0);
     }
     if constexpr (kGhost) {
-      for (int32_t h = t; h < 2 * H; h += kThreads) {
-        const double rn = __builtin_fma(-alpha, gq[h], gr[h]);
-        gr[h] = rn;
-        const int32_t at = h < H ? h : D.rows + h;
-        lp[at] = __builtin_fma(beta, lp[at], gd[h] * rn);
+      for (int32_t h = t; h < T.ng; h += kThreads) {
+        const int32_t at = T.gpos[h];
+        const double rn = __builtin_fma(-alpha, M.gq[h], M.gr[h]);
+        M.gr[h] = rn;
+        lp[at] = __builtin_fma(beta, lp[at], M.gd[h] * rn);
       }
     }
   }
   if (ok) {
+    Tile::Walk w = T.first(opaque(t));
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
-      const int32_t i = t + j * kThreads;
-      if (i < mine) {
-        if (bb == 0.0) xg[i] = 0.0;
-        else if (j < XR) xg[i] = x[j < XR ? j : 0];
+      if ((live >> j) & 1) {
+        if (bb == 0.0) a.x[w.g] = 0.0;
+        else if (j < XR) a.x[w.g] = x[j < XR ? j : 0];
       }
+      T.next(w);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if (D.rank == 0 && t == 0) {
+  if (T.rank == 0 && t == 0) {
     a.st->rr = rr_out;
     a.st->bb = bb;
     a.st->iter = iter;
     a.st->converged = converged;
     a.st->refinements = 0;
+    a.st->aborted = ok ? 0 : 1;
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Mixed precision: the reliable-update scheme of k_mx_a / k_mx_b
+// (lfgpu_solver.hip).  Matrix values and row sums in FP32, the Krylov vectors
+// in VT (float: D^-1 in bfloat16; double: D^-1 in FP32), row sums and dot
+// products in FP64.  x (high part) and its low part stay in memory: they are
+// touched by the reliable updates only.  A reliable update forms
+// b - A x - A xa - A xlo in FP64 with the FP64 matrix read from memory, the
+// three vectors passing through LDS one after the other (p waits in the
+// registers of q), folds xa into (x, xlo) by TwoSum and replaces r by the
+// true residual, p by p + M (r_true - r).  The first residual b - A x is the
+// same code.
+// ---------------------------------------------------------------------------
+template <class VT>
+__device__ __forceinline__ float mixed_dinv(const TileArgs &a, int32_t g) {
+  if constexpr (sizeof(VT) == 4) return __bfloat162float(a.dinv16[g]);
+  else return a.dinv32[g];
+}
+
+template <int KIND, class VT, int RPT, int AHEAD = 1>
+__global__ __launch_bounds__(kThreads) void k_res_tile_mixed(TileArgs a) {
+  constexpr bool kStream = KIND == STREAM, kGhost = KIND == GHOST;
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  const int t = threadIdx.x;
+  Tile T(a, blockIdx.x, gridDim.x);
+  typedef TileLds<KIND, VT, RPT> Lds;
+  const Lds M(dyn, a, T);
+  constexpr bool kRegDiag = !kStream && !Lds::kDiag;
+  double *const lp = M.lp;
+  Team tm{T.rank, T.team, a.part, a.total, a.abort, a.tag0};
+  if (t == 0) sh.bad = 0;
+  T.tables(t);
+  const int32_t cells = Lds::cells(a.TW);
+  for (int32_t i = t; i < cells; i += kThreads) lp[i] = 0.0;
+  const int32_t at0 = T.P + 1 + t;
+
+  VT r[RPT], q[RPT], xa[RPT];
+  // (the FP32 values, widened once)
+  double v[kStream ? 1 : RPT][ND], rs[kRegDiag ? RPT : 1];
+  VT di[kRegDiag ? RPT : 1];
+  uint64_t live = 0;
+  {
+    Tile::Walk w = T.first(t);
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      r[j] = q[j] = xa[j] = (VT)0;
+      if constexpr (!kStream) {
+        if constexpr (kRegDiag) rs[j] = 0.0, di[j] = (VT)0;
+        else M.rs[t + j * kThreads] = M.di[t + j * kThreads] = 0.0;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) v[j][d] = 0.0;
+      }
+      if (T.alive(w)) {
+        live |= 1ull << j;
+        a.xlo[w.g] = 0.0;
+        if constexpr (!kStream) {
+          if constexpr (kRegDiag) {
+            rs[j] = a.rowsum32[w.g];
+            di[j] = mixed_dinv<VT>(a, w.g);
+          } else {
+            M.rs[t + j * kThreads] = a.rowsum32[w.g];
+            M.di[t + j * kThreads] = mixed_dinv<VT>(a, w.g);
+          }
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+            if (d < a.ndiag) v[j][d] = a.val32[(int64_t)d * a.n + w.g];
+        }
+      }
+      T.next(w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if constexpr (kGhost)
+    for (int32_t h = t; h < T.ng; h += kThreads) M.gr[h] = M.gq[h] = M.gd[h] = (VT)0;
+
+  // q = A32 p, each row's q, p and D^-1 handed to fn
+  auto sweep = [&](auto &&fn) {
+    const double *lc = lp + opaque(at0);
+    const double *bp[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) bp[d] = lc + a.shift[d];
+    const double *lrs = M.rs + opaque(t), *ldi = M.di + opaque(t);
+    float nv[AHEAD][ND], ns[AHEAD], nd[AHEAD];  // the next rows of a stream
+    Tile::Walk w = T.first(opaque(t));
+    auto load_row = [&](int j) {
+      const int k = j % AHEAD;
+      const int32_t g = (live >> j) & 1 ? w.g : T.g0;
+      const uint32_t at = (uint32_t)g * 4u;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        if (d < ND / 2)
+          nv[k][d] =
+              load_at(a.val32 + (int64_t)(ND - 1 - d) * a.n, (uint32_t)max(g + a.off[d], 0) * 4u);
+        else
+          nv[k][d] = load_at(a.val32 + (int64_t)d * a.n, at);
+      }
+      if (T.y0 == 0) {
+#pragma unroll
+        for (int d = 0; d < ND / 2; ++d)
+          if (g + a.off[d] < 0) nv[k][d] = 0.0f;
+      }
+      ns[k] = load_at(a.rowsum32, at);
+      nd[k] = mixed_dinv<VT>(a, g);
+      T.next(w);
+    };
+    if constexpr (kStream)
+#pragma unroll
+      for (int j = 0; j < AHEAD; ++j) load_row(j);
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      const int k = j % AHEAD;
+      double vr[ND];
+#pragma unroll
+      for (int d = 0; d < ND; ++d) vr[d] = kStream ? (double)nv[k][d] : v[kStream ? 0 : j][d];
+      const double pi = lc[j * kThreads];
+      double c[ND], acc = 0.0;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) c[d] = bp[d][j * kThreads];
+      const double s = kRegDiag ? rs[kRegDiag ? j : 0]
+                       : kStream ? (double)ns[k] : lrs[j * kThreads];
+      const VT dv = kRegDiag ? di[kRegDiag ? j : 0]
+                    : kStream ? (VT)nd[k] : (VT)ldi[j * kThreads];
+      if (kStream && AHEAD == 1 && j + 1 < RPT) load_row(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) acc = __builtin_fma(vr[d], c[d] - pi, acc);
+      VT qi = (VT)__builtin_fma(s, pi, acc);
+      if (kStream) qi = (live >> j) & 1 ? qi : (VT)0;
+      q[j] = qi;
+      pin(q[j]);
+      fn(j, pi, dv);
+      __builtin_amdgcn_sched_barrier(0);
+      if (kStream && AHEAD > 1 && j + AHEAD < RPT) load_row(j + AHEAD);
+    }
+  };
+
+  bool first = true, ok = true;
+  int itp = 0, last_refine = 0, refinements = 0, converged = 0;
+  double rr = 0.0, rz = 0.0, bb = 0.0, thr = 0.0, rr_ref = 0.0, rr_out = 0.0;
+  for (;;) {
+    double s[5] = {0.0, 0.0, 0.0, rr, rz};
+    bool refine = first;
+    if (!first) {
+      __syncthreads();
+      if constexpr (kStream) {
+        T.template exchange<VT>(lp, &sh.bad);
+        __syncthreads();
+      }
+      VT *lqc = M.lq + opaque(at0);
+      sweep([&](int j, double pi, VT dv) {
+        if constexpr (kGhost) lqc[j * kThreads] = q[j];
+        const double qd = (double)q[j], dq = (double)(dv * q[j]);
+        s[0] = __builtin_fma(pi, qd, s[0]);
+        s[1] = __builtin_fma(dq, (double)r[j], s[1]);
+        s[2] = __builtin_fma(dq, qd, s[2]);
+        pin(s[0]), pin(s[1]), pin(s[2]);
+      });
+      if constexpr (kGhost) ++T.tag;
+      ok = team_sum(tm, sh, s, [&] {
+        if constexpr (kGhost) {
+          const int from = exchange_threads(tm);
+          T.template publish<VT>(M.lq, from);
+          T.template fetch<VT>(from, &sh.bad, [&](int32_t h, int32_t, VT qv) { M.gq[h] = qv; });
+        }
+      });
+      if (!ok) break;
+      // (a step between two reliable updates, so that the loop ends)
+      refine = itp > last_refine && (s[3] < thr || s[3] < a.delta2 * rr_ref ||
+                                     itp - last_refine >= a.max_interval || itp >= a.maxit);
+    }
+    if (!refine) {
+      itp += 1;
+      const double rho = s[4], alpha = rho / s[0];
+      const double rho_next = rho - 2.0 * alpha * s[1] + alpha * alpha * s[2];
+      const VT fa = (VT)alpha, fb = (VT)(rho_next / rho);
+      rr = rz = 0.0;
+      double *lc = lp + opaque(at0);
+      const double *ldi = M.di + opaque(t);
+      Tile::Walk w = T.first(opaque(t));
+      constexpr int kAhead = AHEAD > 1 ? 2 * AHEAD : 1;  // rows of D^-1 in flight
+      float nd[kAhead];
+      auto load_update = [&](int j) {
+        if constexpr (kStream) {
+          nd[j % kAhead] = mixed_dinv<VT>(a, (live >> j) & 1 ? w.g : T.g0);
+          T.next(w);
+        }
+      };
+#pragma unroll
+      for (int j = 0; j < kAhead; ++j) load_update(j);
+      double np = lc[0];
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) {
+        const VT dv = kRegDiag ? di[kRegDiag ? j : 0]
+                      : kStream ? (VT)nd[j % kAhead] : (VT)ldi[j * kThreads];
+        if (j + kAhead < RPT) load_update(j + kAhead);
+        const VT pi = (VT)np;
+        if (j + 1 < RPT) np = lc[(j + 1) * kThreads];
+        xa[j] = xa[j] + fa * pi;
+        r[j] = r[j] - fa * q[j];
+        const VT z = dv * r[j];
+        const VT p = z + fb * pi;
+        const double rd = (double)r[j];
+        rr = __builtin_fma(rd, rd, rr);
+        rz = __builtin_fma(rd, (double)z, rz);
+        if ((live >> j) & 1) lc[j * kThreads] = (double)p;
+        pin(r[j]), pin(xa[j]), pin(rr), pin(rz);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if constexpr (kGhost) {
+        for (int32_t h = t; h < T.ng; h += kThreads) {
+          const int32_t at = T.gpos[h];
+          const VT rn = M.gr[h] - fa * M.gq[h];
+          M.gr[h] = rn;
+          lp[at] = (double)(M.gd[h] * rn + fb * (VT)lp[at]);
+        }
+      }
+      continue;
+    }
+    // reliable update (or the first residual): r64 = b - A x - A xa - A xlo
+    double r64[RPT];
+    {
+      Tile::Walk w = T.first(opaque(t));
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) {
+        const bool in = (live >> j) & 1;
+        r64[j] = in ? a.b[w.g] : 0.0;
+        if (!first) q[j] = (VT)lp[at0 + j * kThreads];  // p
+        T.next(w);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if (first) {
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) bb = __builtin_fma(r64[j], r64[j], bb);
+    }
+    for (int part = 0; part < (first ? 1 : 3); ++part) {
+      __syncthreads();  // the last readers of LDS are done
+      {
+        Tile::Walk w = T.first(opaque(t));
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+          if ((live >> j) & 1)
+            lp[at0 + j * kThreads] =
+                part == 0 ? a.x[w.g] : part == 1 ? (double)xa[j] : a.xlo[w.g];
+          T.next(w);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+      __syncthreads();
+      T.template exchange<double>(lp, &sh.bad);
+      __syncthreads();
+      {
+        Tile::Walk w = T.first(opaque(t));
+        const double *lc = lp + opaque(at0);
+#pragma unroll
+        for (int j = 0; j < RPT; ++j) {
+          const int32_t g = (live >> j) & 1 ? w.g : T.g0;
+          const double yi = lc[j * kThreads];
+          double acc = 0.0;
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+            if (d < a.ndiag)
+              acc = __builtin_fma(a.val[(int64_t)d * a.n + g], lc[j * kThreads + a.shift[d]] - yi,
+                                  acc);
+          acc = __builtin_fma(a.rowsum[g], yi, acc);
+          if ((live >> j) & 1) r64[j] -= acc;
+          pin(r64[j]);
+          T.next(w);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    double u[2] = {0.0, bb};
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) u[0] = __builtin_fma(r64[j], r64[j], u[0]);
+    ok = team_sum(tm, sh, u, [] {});
+    if (!ok) break;
+    rr_out = u[0];
+    bool stop;
+    if (first) {
+      bb = u[1];
+      thr = a.tol2 * bb;
+      thr = thr > 2.2250738585072014e-308 ? thr : 2.2250738585072014e-308;
+      converged = bb == 0.0 || u[0] < thr ? 1 : 0;
+      stop = converged || a.maxit <= 0;
+    } else {
+      refinements += 1;
+      last_refine = itp;
+      converged = u[0] < thr ? 1 : 0;
+      stop = converged || itp >= a.maxit;
+      Tile::Walk w = T.first(opaque(t));
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) {
+        if ((live >> j) & 1) {
+          const double hi = a.x[w.g], dx = (double)xa[j];
+          const double sm = hi + dx, bp = sm - hi;
+          const double err = (hi - (sm - bp)) + (dx - bp);
+          a.x[w.g] = sm;
+          a.xlo[w.g] += err;
+        }
+        xa[j] = (VT)0;
+        T.next(w);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    rr_ref = u[0];
+    if (stop) break;
+    // r = r64, p += M (r64 - r); the first p is M r64
+    rr = rz = 0.0;
+    {
+      Tile::Walk w = T.first(opaque(t));
+#pragma unroll
+      for (int j = 0; j < RPT; ++j) {
+        if ((live >> j) & 1) {
+          const VT rn = (VT)r64[j];
+          const VT m = kRegDiag ? di[kRegDiag ? j : 0]
+                       : kStream ? (VT)mixed_dinv<VT>(a, w.g) : (VT)M.di[t + j * kThreads];
+          const VT z = m * rn;
+          lp[at0 + j * kThreads] = (double)(first ? z : q[j] + m * (rn - r[j]));
+          r[j] = rn;
+          if constexpr (kGhost) M.lq[at0 + j * kThreads] = rn;
+          // (the first rho, as the sweeps take it: with the FP64 D^-1 and residual)
+          const double rd = first ? r64[j] : (double)rn;
+          const double zd = first ? a.dinv[w.g] * rd : (double)z;
+          rr = __builtin_fma(rd, rd, rr);
+          rz = __builtin_fma(rd, zd, rz);
+        }
+        T.next(w);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    if constexpr (kGhost) {
+      // the halo cells' p and r
+      __syncthreads();
+      T.template exchange<VT>(lp, &sh.bad);
+      __syncthreads();  // no r before every thread has its p
+      ++T.tag;
+      T.template publish<VT>(M.lq, 0);
+      T.template fetch<VT>(0, &sh.bad, [&](int32_t h, int32_t at, VT rv) {
+        M.gr[h] = rv;
+        if (first) {
+          const int32_t cell = at - 1;  // from the line above the tile
+          const int32_t line = cell / T.P - 1, c = cell - (line + 1) * T.P;
+          M.gd[h] = (VT)mixed_dinv<VT>(a, T.g0 + line * T.S + c - 1);
+        }
+      });
+    }
+    first = false;
+  }
+  if (ok) {
+    Tile::Walk w = T.first(opaque(t));
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      if ((live >> j) & 1) a.x[w.g] = bb == 0.0 ? 0.0 : a.x[w.g] + a.xlo[w.g];
+      T.next(w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (T.rank == 0 && t == 0) {
+    a.st->rr = rr_out;
+    a.st->bb = bb;
+    a.st->iter = itp;
+    a.st->converged = converged;
+    a.st->refinements = refinements;
     a.st->aborted = ok ? 0 : 1;
   }
 }
@@ -490,25 +1011,77 @@ __global__ void k_zero_words(word_t *p, size_t n) {
 constexpr size_t kPartWords = (size_t)2 * 2 * kSums * kMaxTeam;
 constexpr size_t kTotalWords = (size_t)2 * kLeaders * 2 * kSums;
 constexpr size_t kLdsBytes = 160 * 1024;
-// LDS of the team sums, rounded up (static, beside the dynamic lp array)
+// LDS of the team sums, rounded up (static, beside the dynamic arrays)
 constexpr size_t kLdsStatic = (sizeof(SumLds) + 1023) / 1024 * 1024;
 
-typedef void (*DiaKernel)(DiaArgs);
-struct DiaVariant {
+// The variants in order of preference (the smallest number of cells per
+// thread with which the team and its LDS fit): FP64, FP32 vectors, FP64
+// vectors with the FP32 matrix.
+struct TileVariant {
   int kind, rpt;
-  DiaKernel fn;
+  size_t (*lds)(const TileArgs &);
+  void (*fn)(TileArgs);
 };
+#define LFG_TILE(K, R, ...) \
+  {K, R, &TileLds<K, double, R>::bytes, &k_res_tile<K, R, __VA_ARGS__>}
+#define LFG_TILEM(K, T, R, A) {K, R, &TileLds<K, T, R>::bytes, &k_res_tile_mixed<K, T, R, A>}
+const std::vector<TileVariant> kTileVariants[3] = {
+    {LFG_TILE(GHOST, 1, 1), LFG_TILE(GHOST, 3, 3), LFG_TILE(GHOST, 5, 5), LFG_TILE(GHOST, 7, 7),
+     LFG_TILE(GHOST, 9, 9), LFG_TILE(STREAM, 17, 17, 2), LFG_TILE(STREAM, 25, 13, 2),
+     LFG_TILE(STREAM, 33, 0, 2)},
+    {LFG_TILEM(GHOST, float, 1, 1), LFG_TILEM(GHOST, float, 3, 1), LFG_TILEM(GHOST, float, 5, 1),
+     LFG_TILEM(GHOST, float, 7, 1), LFG_TILEM(GHOST, float, 9, 1), LFG_TILEM(STREAM, float, 17, 4),
+     LFG_TILEM(STREAM, float, 25, 4), LFG_TILEM(STREAM, float, 33, 4)},
+    {LFG_TILEM(GHOST, double, 1, 1), LFG_TILEM(GHOST, double, 3, 1),
+     LFG_TILEM(GHOST, double, 5, 1), LFG_TILEM(GHOST, double, 7, 1),
+     LFG_TILEM(GHOST, double, 9, 1), LFG_TILEM(STREAM, double, 17, 4),
+     LFG_TILEM(STREAM, double, 25, 3), LFG_TILEM(STREAM, double, 33, 2)},
+};
+#undef LFG_TILE
+#undef LFG_TILEM
 
-// In order of preference: the smallest number of rows per thread with which
-// the team and its LDS fit.
-const DiaVariant kDiaVariants[] = {
-    {GHOST, 1, k_res_dia<GHOST, 1, 1>},   {GHOST, 3, k_res_dia<GHOST, 3, 3>},
-    {GHOST, 5, k_res_dia<GHOST, 5, 5>},   {GHOST, 7, k_res_dia<GHOST, 7, 7>},
-    {GHOST, 9, k_res_dia<GHOST, 9, 9>},   {HALO, 9, k_res_dia<HALO, 9, 9>},
-    {STREAM, 17, k_res_dia<STREAM, 17, 17>},
-    {STREAM, 25, k_res_dia<STREAM, 25, 17>},
-    {STREAM, 33, k_res_dia<STREAM, 33, 8>},
-};
+// Splits the lattice into at most cus tiles for the first variant that takes
+// them; among the splits, the one with the shortest rim (the halo travels
+// every iteration) and, where one workgroup sums all members' partials, the
+// smallest team.  STREAM: lines of a tile are read in 128-byte pieces,
+// two of which at their ends another tile reads too, so a tile line counts
+// as 16 cells more.  Returns the variant or nullptr.
+const TileVariant *tile_plan(TileArgs &a, int mode, bool sym, int cus, int *team) {
+  for (const TileVariant &v : kTileVariants[mode]) {
+    if (v.kind == STREAM && !(sym && a.ndiag == ND)) continue;
+    const int64_t cap = (int64_t)v.rpt * kThreads;
+    if ((int64_t)a.S * a.L > cap * cus) continue;
+    int64_t best = -1;
+    TileArgs pick = a;
+    for (int32_t tx = 1; tx <= cus && tx <= a.S; ++tx) {
+      const int32_t TW = (a.S + tx - 1) / tx, TX = (a.S + TW - 1) / TW;
+      const int32_t most = (int32_t)std::min<int64_t>(cap / (TW + 2), a.L);  // lines a tile
+      if (most < 1 || TX > cus) continue;
+      int32_t TY = (a.L + most - 1) / most;
+      if ((int64_t)TX * TY > cus) continue;
+      const int32_t TH = (a.L + TY - 1) / TY;
+      TY = (a.L + TH - 1) / TH;
+      TileArgs c = a;
+      c.TW = TW;
+      c.TH = TH;
+      c.TX = TX;
+      c.slots = 2 * (TW + TH);
+      c.ghosts = (2 * (TW + 2) + 2 * TH + 1) / 2 * 2;
+      if (v.lds(c) + kLdsStatic > kLdsBytes) continue;
+      const int32_t wgs = TX * TY;
+      int64_t cost = wgs == 1 ? 0 : 2 * (TW + TH) + 7 * std::min(wgs, kFlatTeam);
+      if (v.kind == STREAM) cost += 16 * (int64_t)TH;
+      if (best >= 0 && cost >= best) continue;
+      best = cost;
+      pick = c;
+      *team = TX * TY;
+    }
+    if (best < 0) continue;
+    a = pick;
+    return &v;
+  }
+  return nullptr;
+}
 
 }  // namespace
 
@@ -521,41 +1094,26 @@ void resident_free(ResidentBufs *b) {
   *b = ResidentBufs{};
 }
 
-int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A, const double *b,
-                     double *x, double rtol, int maxit, ResidentState *st, bool *taken) {
+int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
+                     const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
+                     bool *taken) {
   *taken = false;
-  if (A.n <= 0 || A.ndiag > ND) return LFGPU_OK;
-  int32_t H = 0;
-  for (int d = 0; d < A.ndiag; ++d) H = std::max(H, std::abs(A.off[d]));
-  const int cus = std::min(ctx->cus, kMaxTeam);
-  const DiaVariant *pick = nullptr;
+  if (A.n <= 0 || A.width <= 0 || A.ndiag > ND) return LFGPU_OK;
+  TileArgs a{};
+  a.n = A.n;
+  a.S = A.width;
+  a.L = A.n / A.width;
+  a.ndiag = A.ndiag;
   int team = 0;
-  int32_t rows = 0;
-  size_t lds = 0;  // in doubles
-  for (const DiaVariant &v : kDiaVariants) {
-    if (v.kind == STREAM && !(A.sym && A.ndiag == ND)) continue;
-    const int64_t cap = (int64_t)v.rpt * kThreads;
-    team = (int)((A.n + cap - 1) / cap);
-    if (team > cus) continue;
-    // rows in 128-byte steps, evenly over the team
-    rows = (int32_t)(((A.n + team - 1) / team + 15) / 16 * 16);
-    rows = (int32_t)std::min<int64_t>(rows, cap);
-    team = (int)((A.n + rows - 1) / rows);
-    if (team > 1 && H > rows) continue;
-    // STREAM: the first half's rows must not read the upper halo nor the
-    // second half's the lower one (they share their place)
-    const int32_t half = (v.rpt + 1) / 2 * kThreads;
-    if (v.kind == STREAM && (half < H || half > rows - H)) continue;
-    // p with both halos (STREAM: one) and, for GHOST, three more halo arrays;
-    // the rows up to rpt * 512 are read
-    lds = (size_t)cap + (v.kind == GHOST ? 8 : v.kind == HALO ? 2 : 1) * (size_t)H;
-    if (lds * sizeof(double) + kLdsStatic > kLdsBytes) continue;
-    pick = &v;
-    break;
+  const TileVariant *v = tile_plan(a, opts.mode, A.sym, std::min(ctx->cus, kMaxTeam), &team);
+  if (!v) return LFGPU_OK;
+  for (int d = 0; d < A.ndiag; ++d) {
+    a.off[d] = A.off[d];
+    // off = dy S + dx with |dx|, |dy| <= 1
+    const int32_t dy = A.off[d] > 1 ? 1 : A.off[d] < -1 ? -1 : 0;
+    a.shift[d] = dy * (a.TW + 2) + (A.off[d] - dy * a.S);
   }
-  if (!pick) return LFGPU_OK;
-  const int32_t slots = std::min(rows, 2 * H);
-  const size_t words = (size_t)2 * team * 2 * std::max(slots, 1);
+  const size_t words = (size_t)2 * team * 2 * a.slots;
   hipStream_t s = ctx->stream;
   if (!bufs->sums) {
     LFG_TRY(dalloc(&bufs->sums, kPartWords + kTotalWords, "resident PCG sums"));
@@ -571,8 +1129,9 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A, c
     bufs->halo_words = words;
     bufs->epoch = 0xffffffffu;
   }
-  // tags of this solve: one exchange and one sum an iteration and two more
-  const uint64_t need = (uint64_t)maxit + 4;
+  // tags of this solve: one exchange and one sum an iteration, six for a
+  // reliable update (at most one an iteration), and a few at the start
+  const uint64_t need = (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 7) + 16;
   if (bufs->epoch + need > 0xfffffff0ull) {
     hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, s, bufs->halo, bufs->halo_words);
     hipLaunchKernelGGL(k_zero_words, dim3(8), dim3(256), 0, s, bufs->sums,
@@ -583,15 +1142,6 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A, c
     LFG_HIP(hipGetLastError());
     bufs->epoch = 0;
   }
-  DiaArgs a{};
-  a.n = A.n;
-  a.rows = rows;
-  a.halo = H;
-  a.slots = std::max(slots, 1);
-  a.lds = (int32_t)lds;
-  lds *= sizeof(double);
-  a.ndiag = A.ndiag;
-  for (int d = 0; d < kMaxD; ++d) a.off[d] = d < A.ndiag ? A.off[d] : 0;
   a.val = A.val;
   a.rowsum = A.rowsum;
   a.dinv = A.dinv;
@@ -602,25 +1152,33 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A, c
   a.total = bufs->sums + kPartWords;
   a.abort = bufs->abort;
   a.tag0 = bufs->epoch;
-  a.tol2 = rtol * rtol;
-  a.maxit = maxit;
+  a.tol2 = opts.rtol * opts.rtol;
+  a.maxit = opts.maxit;
   a.st = bufs->state;
-  const void *fn = reinterpret_cast<const void *>(pick->fn);
+  a.val32 = A.val32;
+  a.rowsum32 = A.rowsum32;
+  a.dinv32 = A.dinv32;
+  a.dinv16 = static_cast<const __hip_bfloat16 *>(A.dinv16);
+  a.xlo = A.xlo;
+  a.delta2 = opts.refine_delta > 0.0 ? opts.refine_delta * opts.refine_delta : 0.09;
+  a.max_interval = opts.refine_max_interval > 0 ? opts.refine_max_interval : 2147483647;
+  const size_t lds = v->lds(a);
+  const void *fn = reinterpret_cast<const void *>(v->fn);
   LFG_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   void *args[] = {&a};
   if (team == 1) {
     LFG_HIP(hipLaunchKernel(fn, dim3(1), dim3(kThreads), args, lds, s));
   } else {
     // all workgroups of the team must run at once
-    const hipError_t e = hipLaunchCooperativeKernel(fn, dim3(team), dim3(kThreads), args,
-                                                    (unsigned)lds, s);
+    const hipError_t e =
+        hipLaunchCooperativeKernel(fn, dim3(team), dim3(kThreads), args, (unsigned)lds, s);
     if (e == hipErrorCooperativeLaunchTooLarge) {
       (void)hipGetLastError();
       return LFGPU_OK;
     }
     LFG_HIP(e);
   }
-  bufs->epoch += (uint32_t)need;
+  bufs->epoch = (uint32_t)std::min<uint64_t>(bufs->epoch + need, 0xffffffffull);
   LFG_HIP(hipMemcpyAsync(st, bufs->state, sizeof(ResidentState), hipMemcpyDeviceToHost, s));
   *taken = true;
   return LFGPU_OK;

@@ -33,8 +33,9 @@ constexpr int kMaxTeam = 256;  // workgroups of a team (one leader thread per me
 constexpr int kSums = 5;       // values of one team sum
 // Teams of fewer workgroups read every member's partial sums in every
 // workgroup (one hop); larger ones let kLeaders workgroups sum them and
-// publish the totals (two hops, but 256 workgroups polling 256 x 10 words
-// each measured 5.0 us for the hop against 1.3 us)
+// publish the totals (two hops).  One hop costs 2.6 us with one workgroup (to
+// memory and back, five values), 3.9 with 64, 5.0 with 128 and 6.6 with 256,
+// which poll 256 x 10 words each; the second hop costs about 1.7.
 constexpr int kFlatTeam = 64;
 constexpr int kLeaders = 8;
 constexpr uint64_t kWaitTicks = 400000000ull;  // 4 s of the 100 MHz real-time clock
@@ -117,10 +118,14 @@ struct Team {
 // the same bits: wavefronts in order within a workgroup, then the members'
 // partials in a fixed tree over their ranks.  Returns false when the team has
 // been aborted (in every thread of the workgroup).  Contains workgroup
-// barriers: LDS written before the call is visible after it.  The threads
-// from kIdle on, which have no part in the sum once the workgroup's partials
-// are out, run `meanwhile` while the others wait for the team.
-constexpr int kIdle = kMaxTeam;
+// barriers: LDS written before the call is visible after it.  All threads run
+// `meanwhile` between the first of them, when the workgroup's partials are
+// about to go out, and the wait for the team; it must leave to itself the
+// threads that have a part in the sum: the first wavefront, and the first
+// kMaxTeam threads where sums_members() holds.
+__device__ __forceinline__ bool sums_members(const Team &tm) {
+  return tm.size < kFlatTeam || tm.rank < kLeaders;
+}
 template <int K, class F>
 __device__ __forceinline__ bool team_sum(Team &tm, SumLds &sh, double (&v)[K], F &&meanwhile) {
   static_assert(K <= kSums, "too many sums");
@@ -151,9 +156,9 @@ __device__ __forceinline__ bool team_sum(Team &tm, SumLds &sh, double (&v)[K], F
     for (int q = 1; q < kWaves; ++q) s += sh.part[par][q][k];
     put(&pb[(size_t)t * tm.size + tm.rank], (t & 1) ? high_word(s, tag) : low_word(s, tag));
   }
-  if (t >= kIdle) meanwhile();
+  meanwhile();
   const bool flat = tm.size < kFlatTeam;
-  if (flat || tm.rank < kLeaders) {
+  if (sums_members(tm)) {
     if (t < kMaxTeam) {
       double r[K];
 #pragma unroll

@@ -75,6 +75,7 @@ struct lfgpu_solver_cache {
   int fmt = FMT_ELL;
   int ndiag = 0;
   int off[kMaxDiag] = {0};
+  int32_t width = 0;             // DIA: rows a line of the lattice (0: none)
   int32_t nslices = 0;
   int64_t mlen = 0;              // stored off-diagonal slots
   int32_t *slice_off = nullptr;  // ELL: [nslices + 1] element offsets
@@ -629,6 +630,63 @@ int detect_dia(lfgpu_ctx *ctx, const lfgpu_csr *A, DiagSet *ds) {
   return LFGPU_OK;
 }
 
+// flag |= 1 if some off-diagonal entry does not couple lattice neighbours
+// (width rows a line)
+__global__ void k_lattice_check(const int32_t *row_ptr, const int32_t *col, int32_t n,
+                                int32_t width, int *flag) {
+  const int32_t r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= n) return;
+  const int32_t y = r / width, x = r - y * width;
+  for (int32_t p = row_ptr[r]; p < row_ptr[r + 1]; ++p) {
+    const int32_t cy = col[p] / width, cx = col[p] - cy * width;
+    if (abs(cx - x) > 1 || abs(cy - y) > 1) {
+      atomicOr(flag, 1);
+      return;
+    }
+  }
+}
+
+// The lattice of a DIA matrix (for the resident solves): c->width rows a line
+// when the offsets are among +-1, +-width, +-(width +- 1), the lines are
+// whole and no entry wraps around a line's end; else 0.  A tridiagonal
+// matrix is one line.
+int dia_lattice(lfgpu_ctx *ctx, const lfgpu_csr *A, lfgpu_solver_cache *c) {
+  c->width = 0;
+  const int32_t n = A->nrows;
+  int32_t most = 0;
+  for (int d = 0; d < c->ndiag; ++d) most = std::max(most, std::abs(c->off[d]));
+  for (int32_t w : {most - 1, most, most + 1}) {
+    if (most <= 1) w = n;
+    if (w < 4 || n % w != 0) continue;
+    bool fits = true;
+    for (int d = 0; d < c->ndiag; ++d) {
+      const int32_t o = std::abs(c->off[d]);
+      fits = fits && (o == 1 || std::abs(o - w) <= 1);
+    }
+    if (!fits) continue;
+    int *flag = nullptr;
+    LFG_TRY(dalloc(&flag, 1, "lattice flag"));
+    int h = 1;
+    hipStream_t s = ctx->stream;
+    hipError_t e = hipMemsetAsync(flag, 0, 4, s);
+    if (e == hipSuccess) {
+      hipLaunchKernelGGL(k_lattice_check, dim3(grid_for(n, 256)), dim3(256), 0, s, A->row_ptr,
+                         A->col, n, w, flag);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpyAsync(&h, flag, 4, hipMemcpyDeviceToHost, s);
+    if (e == hipSuccess) e = hipStreamSynchronize(s);
+    dfree(flag);
+    if (e != hipSuccess) return hip_fail(e, "lattice check");
+    if (h == 0) {
+      c->width = w;
+      return LFGPU_OK;
+    }
+    if (most <= 1) break;
+  }
+  return LFGPU_OK;
+}
+
 // Locality order of the rows of a sliced-ELL matrix.  Rows are ordered by
 // their locality key (k_row_key2: the smallest column among the row and its
 // neighbours' rows) in windows of 2^kEllWindowBits columns and, inside a
@@ -792,6 +850,7 @@ int ensure_cache(lfgpu_ctx *ctx, lfgpu_csr *A, bool need32, bool allow_perm) {
       c->ndiag = ds.ndiag;
       for (int d = 0; d < kMaxDiag; ++d) c->off[d] = d < ds.ndiag ? ds.off[d] : 0;
       c->mlen = (int64_t)ds.ndiag * n;
+      LFG_TRY(dia_lattice(ctx, A, c));
     } else {
       c->fmt = FMT_ELL;
       if (allow_perm && n > 0) LFG_TRY(ell_locality_order(ctx, A, c));
@@ -3755,23 +3814,29 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
   // chunk below 2^20 rows (launch-bound sizes), or as the caller asks
   const bool use_graph = opts->graph > 0 || (opts->graph == 0 && n < (1 << 20));
 
-  // FP64 on DIA storage: the resident solve (lfgpu_resident.hip) where the
-  // system fits the chip, unless the caller asked for graph replays or plain
+  // on DIA storage: the resident solve (lfgpu_resident.hip) where the system
+  // fits the chip, unless the caller asked for graph replays or plain
   // launches of the sweeps
-  if (!mixed && !single && c->fmt == FMT_DIA && c->blk_n == 0 && opts->graph == 0 && !t_timer) {
+  if (!single && c->fmt == FMT_DIA && c->blk_n == 0 && opts->graph == 0 && !t_timer) {
     ResidentDia rd;
     rd.n = n;
+    rd.width = c->width;
     rd.ndiag = c->ndiag;
     rd.off = c->off;
     rd.val = c->val;
     rd.rowsum = c->rowsum;
     rd.dinv = c->dinv;
     rd.sym = c->sym64;
+    rd.val32 = c->val32;
+    rd.rowsum32 = c->rowsum32;
+    rd.dinv32 = c->dinv32;
+    rd.dinv16 = c->dinv16;
+    rd.xlo = c->xlo;
     ResidentState *rs = reinterpret_cast<ResidentState *>(ctx->pinned);
     bool taken = false;
     LFG_HIP(hipEventRecord(ctx->ev0, s));
-    LFG_TRY(resident_pcg_dia(ctx, &c->res, rd, b->d, x->d, opts->rtol, opts->maxit, rs, &taken));
-    if (taken) return resident_finish(ctx, &c->res, rs, false, info);
+    LFG_TRY(resident_pcg_dia(ctx, &c->res, rd, *opts, b->d, x->d, rs, &taken));
+    if (taken) return resident_finish(ctx, &c->res, rs, mixed, info);
   }
 
   if (single && !c->cg1)

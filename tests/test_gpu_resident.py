@@ -2,13 +2,13 @@
 
 opts->graph = -1 runs the sweeps, 0 (the default) the resident solve where
 the system fits the chip.  Both run the same recurrences and stop on the same
-test with sums in another order.  Iteration counts: a solve of k iterations
-to rtol 1e-10 gains ln(1e10) / k an iteration on average, and the residual
-norm oscillates about that trend by tens of percent, at places that rounding
-moves: 2 % of k (at least 2) is a factor of 1.6 in the residual.  Solutions to
-100 rtol: each is within about kappa(D^-1 A)^(1/2) rtol of the exact one in
-the energy norm, and the measured errors of such solves against direct ones
-stay below 20 rtol.
+test with sums in another order.  Where the recurrence has lost
+orthogonality (chains here take more iterations than they have rows) rounding
+moves the count, so counts are compared over three iterations only.
+Solutions: the
+matrices here have no eigenvalue below 1e-3, so two converged solutions differ
+by at most 2 rtol ||b|| / 1e-3 (a tenth more for the recurrence residual's
+distance from the true one).
 """
 import numpy as np
 import pytest
@@ -17,6 +17,8 @@ from lehrfempp_amd import capi
 
 pytestmark = pytest.mark.gpu
 
+MODES = [capi.PCG_FP64, capi.PCG_MIXED, capi.PCG_MIXED_MATRIX]
+
 
 @pytest.fixture(scope="module")
 def ctx():
@@ -24,29 +26,31 @@ def ctx():
         yield c
 
 
-def _band_system(n, offs, seed, symmetric=True):
-    """Triplets of a diagonally dominant matrix with the given off-diagonal
-    offsets, values random, a reaction term that makes it positive definite."""
+def _lattice_system(S, L, steps, seed, symmetric=True):
+    """Triplets of a lattice Laplacian (S rows a line, L lines, neighbours
+    (dx, dy) in steps and their opposites) with random weights plus 1e-3."""
     rng = np.random.default_rng(seed)
+    n = S * L
+    y, x = np.divmod(np.arange(n), S)
     rows, cols, vals, diag = [], [], [], np.full(n, 1e-3)
-    for o in offs:
-        if o >= n:
-            continue
-        i = np.arange(n - o)
-        w = np.exp(rng.standard_normal(n - o))
-        rows += [i, i + o]
-        cols += [i + o, i]
-        vals += [-w, -w if symmetric else -w * (1.0 + 1e-15 * rng.integers(0, 2, n - o))]
-        diag[: n - o] += w
-        diag[o:] += w
+    for dx, dy in steps:
+        i = np.nonzero((x + dx >= 0) & (x + dx < S) & (y + dy < L))[0]
+        j = i + dy * S + dx
+        w = np.exp(rng.standard_normal(i.size))
+        rows += [i, j]
+        cols += [j, i]
+        vals += [-w, -w if symmetric else -w * (1.0 + 1e-15 * rng.integers(0, 2, i.size))]
+        np.add.at(diag, i, w)
+        np.add.at(diag, j, w)
     rows.append(np.arange(n))
     cols.append(np.arange(n))
     vals.append(diag)
-    return np.concatenate(rows), np.concatenate(cols), np.concatenate(vals)
+    return np.concatenate(rows), np.concatenate(cols), np.concatenate(vals), n
 
 
-def _compare(ctx, A, n, mode, seed, x0=None, maxit=None, rtol=1e-10):
-    b = capi.Vec(ctx, np.random.default_rng(seed).standard_normal(n))
+def _compare(ctx, A, n, mode, seed, x0=None, maxit=20000, rtol=1e-10):
+    bh = np.random.default_rng(seed).standard_normal(n)
+    b, bn = capi.Vec(ctx, bh), np.linalg.norm(bh)
     out = []
     for graph in (-1, 0):
         x = capi.Vec(ctx, np.zeros(n) if x0 is None else x0)
@@ -57,64 +61,84 @@ def _compare(ctx, A, n, mode, seed, x0=None, maxit=None, rtol=1e-10):
     b.close()
     (ia, xa), (ib, xb) = out
     assert ia.converged == ib.converged
-    assert abs(ia.iters - ib.iters) <= max(2, 0.02 * ia.iters), (ia.iters, ib.iters)
-    assert np.linalg.norm(xa - xb) <= 100 * rtol * np.linalg.norm(xa)
+    if ia.converged:
+        bound = 2.2 * rtol * bn / 1e-3
+        assert np.linalg.norm(xa - xb) <= bound, (np.linalg.norm(xa - xb), bound)
     return out
 
 
-# rows at the edges of the workgroup's and the team's splits: one workgroup
-# (n <= 512), one row more, rows per thread 1, 3, 5, 9 and their limits,
-# offsets as long as a workgroup's rows
-@pytest.mark.parametrize("n, offs", [
-    (128, (1,)), (511, (1, 20)), (512, (1, 20, 21)), (513, (1, 20, 21)), (1537, (1, 700)),
-    (4096, (1, 511, 512)), (5000, (1, 512, 513)), (131072, (1, 362, 363)),
-    (131073, (1, 362, 363)), (393217, (1, 1535, 1536)), (400000, (2, 1999, 2001)),
+P1 = ((1, 0), (0, 1), (1, 1))
+
+
+# one workgroup and one line more, tiles of one line and of one column, the
+# limits of 1, 3, 5, 7 and 9 cells a thread, the other diagonal, five-point and
+# tridiagonal stencils (which have fewer off-diagonals than the kernel holds)
+@pytest.mark.parametrize("S, L, steps", [
+    (128, 1, ((1, 0),)), (700, 1, ((1, 0),)), (20, 21, P1), (21, 24, P1), (4, 300, P1),
+    (1500, 3, P1), (64, 64, ((1, 0), (0, 1))), (65, 65, ((1, 0), (0, 1), (-1, 1))),
+    (362, 363, P1), (513, 513, P1), (640, 631, P1), (2049, 257, P1), (1025, 1025, P1),
 ])
 @pytest.mark.parametrize("symmetric", [True, False])
-def test_resident_pcg_on_dia(ctx, n, offs, symmetric):
-    r, c, v = _band_system(n, offs, n, symmetric)
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_pcg_on_a_lattice(ctx, S, L, steps, symmetric, mode):
+    r, c, v, n = _lattice_system(S, L, steps, S + L, symmetric)
     A = capi.coo_to_csr(ctx, r, c, v, n, n)
-    out = _compare(ctx, A, n, capi.PCG_FP64, n + 1)
-    if capi.solver_storage(A)[0] == capi.STORAGE_DIA:  # (one case pads too much for DIA)
+    out = _compare(ctx, A, n, mode, n + 1)
+    if capi.solver_storage(A)[0] == capi.STORAGE_DIA:
         assert out[1][0].syncs == 1  # the resident solve ran
     # a nonzero start, and the iteration cap
     x0 = np.random.default_rng(5).standard_normal(n)
-    _compare(ctx, A, n, capi.PCG_FP64, n + 2, x0=x0)
-    out = _compare(ctx, A, n, capi.PCG_FP64, n + 2, x0=x0, maxit=3, rtol=1e-14)
+    _compare(ctx, A, n, mode, n + 2, x0=x0)
+    out = _compare(ctx, A, n, mode, n + 2, x0=x0, maxit=3, rtol=1e-14)
     assert out[0][0].iters == out[1][0].iters == 3
-    assert np.linalg.norm(out[0][1] - out[1][1]) <= 1e-13 * np.linalg.norm(out[0][1])
+    # three steps of the recurrence: its precision, and the start's rounding
+    eps = 1e-13 if mode == capi.PCG_FP64 else 1e-5 if mode == capi.PCG_MIXED else 1e-12
+    assert np.linalg.norm(out[0][1] - out[1][1]) <= eps * np.linalg.norm(out[0][1])
     A.close()
 
 
-# the streamed matrix: rows per thread 17 and 33, the last with the shared halo
-@pytest.mark.parametrize("n, offs", [
-    (1300000, (1, 1140, 1141)), (2097152, (1, 1448, 1449)), (2300001, (1, 1516, 1517)),
-    (4198401, (1, 2049, 2050)),
-])
-def test_resident_pcg_on_large_dia(ctx, n, offs):
-    r, c, v = _band_system(n, offs, 3)
-    v = v.copy()
+# the streamed matrix: 17, 25 and 33 cells a thread
+@pytest.mark.parametrize("S, L", [(1141, 1140), (1449, 1448), (1400, 1900), (2049, 2049),
+                                  (3000, 500)])
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_pcg_on_large_lattices(ctx, S, L, mode):
+    r, c, v, n = _lattice_system(S, L, P1, 3)
     v[-n:] += 1.0  # well conditioned: a few dozen iterations
     A = capi.coo_to_csr(ctx, r, c, v, n, n)
-    out = _compare(ctx, A, n, capi.PCG_FP64, 4)
+    out = _compare(ctx, A, n, mode, 4)
     assert out[1][0].syncs == 1 and out[1][0].converged
     A.close()
 
 
-def test_resident_pcg_is_deterministic_and_zero_rhs(ctx):
-    n = 70000
-    r, c, v = _band_system(n, (1, 264, 265), 9)
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_pcg_is_deterministic_and_zero_rhs(ctx, mode):
+    r, c, v, n = _lattice_system(264, 265, P1, 9)
     A = capi.coo_to_csr(ctx, r, c, v, n, n)
     b, x = capi.Vec(ctx, np.random.default_rng(2).standard_normal(n)), capi.Vec(ctx, n)
     got = []
     for _ in range(3):
         x.fill(0.0)
-        capi.pcg(ctx, A, b, x)
+        capi.pcg(ctx, A, b, x, mode=mode)
         got.append(x.numpy())
     assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
     b.fill(0.0)
     x.fill(2.0)
-    info = capi.pcg(ctx, A, b, x)
+    info = capi.pcg(ctx, A, b, x, mode=mode)
     assert info.converged and info.iters == 0 and not x.numpy().any()
     for h in (x, b, A):
         h.close()
+
+
+def test_wrapped_band_matrix_keeps_the_sweeps(ctx):
+    # the offsets of a lattice, but entries across the lines' ends
+    n, S = 4096, 64
+    i = np.arange(n)
+    rows, cols, vals = [i], [i], [np.full(n, 7.0)]
+    for o in (1, S, S + 1):
+        rows += [i[:-o], i[o:]]
+        cols += [i[o:], i[:-o]]
+        vals += [np.full(n - o, -1.0)] * 2
+    A = capi.coo_to_csr(ctx, np.concatenate(rows), np.concatenate(cols), np.concatenate(vals), n, n)
+    out = _compare(ctx, A, n, capi.PCG_FP64, 1)
+    assert np.array_equal(out[0][1], out[1][1])  # graph replay against plain launches
+    A.close()
