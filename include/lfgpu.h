@@ -304,16 +304,14 @@ typedef struct lfgpu_pcg_opts {
    * preconditioned residual on the fly; 0 = two sweeps with Eigen's own
    * recurrences (default). */
   int single_reduction;
-  /* FP64 two-sweep and row-sweep iterations: 0 = the whole solve in one
-   * launch with the vectors kept on the chip where the system fits (P1
-   * matrices of structured meshes; all modes; info->syncs is 1 then), else
-   * replay each chunk
-   * of check_every iterations from a captured hipGraph below 2^20 rows,
-   * where the solve is bound by the launch rate (default); 1 = always replay
-   * chunks; -1 = never (plain launches).  1 and -1 give the same iterates;
-   * the one-launch solve runs the same recurrences and stopping test with
-   * its sums in another order.  Up to two captured chunks are kept per
-   * matrix, keyed by the solution vector. */
+  /* 0 (default) = the whole solve in one launch with the vectors kept on
+   * the chip where the system fits (any mode; info->syncs is 1 then), else
+   * plain launches, or in FP64 below 2^20 rows, where the solve is bound by
+   * the launch rate, replays of each chunk of check_every iterations from a
+   * captured hipGraph; 1 = always replay chunks (FP64); -1 = plain launches.
+   * 1 and -1 give the same iterates; the one-launch solve runs the same
+   * recurrences and stopping test with its sums in another order.  Up to two
+   * captured chunks are kept per matrix, keyed by the solution vector. */
   int graph;
 } lfgpu_pcg_opts;
 typedef struct lfgpu_pcg_info {

@@ -24,6 +24,15 @@ struct ResidentBufs {
   uint32_t epoch = 0;
 };
 void resident_free(ResidentBufs *b);
+// Buffers for a solve that exchanges through `words` words and uses at most
+// `need` tags; *tag0 the tag before its first.
+int resident_prepare(hipStream_t s, ResidentBufs *bufs, size_t words, uint64_t need,
+                     uint32_t *tag0);
+// Queues kernel fn (one argument struct) on `team` workgroups that all run at
+// once, and the copy of its outcome to *st; *taken = false where the chip
+// does not hold them.
+int resident_launch(hipStream_t s, ResidentBufs *bufs, const void *fn, int team, void *args,
+                    size_t lds, ResidentState *st, bool *taken);
 
 // A matrix on DIA storage (val[d * n + row], offsets ascending) whose rows
 // form a lattice: `width` rows a line, n / width lines, no entry but between
@@ -48,5 +57,36 @@ struct ResidentDia {
 int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
                      const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
                      bool *taken);
+
+// Sliced-ELL storage split over a team for the resident solves: workgroup g
+// owns the storage rows [g rows, (g + 1) rows) and keeps their p in LDS, with
+// the values of the rows it reads of others behind them.
+struct ResidentEllPlan {
+  bool tried = false;
+  int team = 0, rpt = 0;
+  int32_t rows = 0;            // rows per workgroup, a multiple of 64
+  int32_t most = 0;            // most outside rows of a workgroup
+  int32_t *ext = nullptr;      // [team x stride] the outside rows, ascending
+  int32_t *ext_n = nullptr;    // [team]
+  int32_t stride = 0;
+  uint16_t *lcol = nullptr;    // per slot: the column's place in the workgroup's LDS
+  uint8_t *needed = nullptr;   // per row: some other workgroup reads it
+};
+void resident_ell_free(ResidentEllPlan *p);
+
+// A matrix on sliced-ELL storage with 16-bit column offsets.
+struct ResidentEll {
+  int32_t n = 0, nslices = 0;
+  int64_t slots = 0;
+  const int32_t *slice_off = nullptr, *perm = nullptr;  // perm: storage row -> row of x, b
+  const int16_t *dcol = nullptr;
+  const double *val = nullptr, *rowsum = nullptr, *dinv = nullptr;
+  const float *val32 = nullptr, *rowsum32 = nullptr, *dinv32 = nullptr;
+  const void *dinv16 = nullptr;
+  double *xlo = nullptr;
+};
+int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *plan,
+                     const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b, double *x,
+                     ResidentState *st, bool *taken);
 
 }  // namespace lfgpu

@@ -78,25 +78,6 @@ struct TileArgs {
   int max_interval;
 };
 
-// A value of an array at a uniform base and a 32-bit byte offset per lane (one
-// address register for all the arrays of a row).
-template <class T>
-__device__ __forceinline__ T load_at(const T *base, uint32_t bytes) {
-  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes);
-}
-// Hides a value from the optimiser, which else keeps every row's addresses
-// and masks in registers across the iterations (several hundred of them).
-__device__ __forceinline__ int32_t opaque(int32_t v) {
-  asm volatile("" : "+v"(v));
-  return v;
-}
-// Keeps a row's result where it is computed (the compiler else sinks whole
-// rows past the next barrier and spills their operands).
-template <class T>
-__device__ __forceinline__ void pin(T &v) {
-  asm volatile("" : "+v"(v));
-}
-
 // The workgroup's tile: tw x th cells of the lattice, padded by one halo cell
 // on each side to lines of P = TW + 2 cells.  Cell i = line * P + c (c = 0 and
 // c > tw are halo cells) is thread i % 512's cell number i / 512; it sits in
@@ -1008,12 +989,6 @@ __global__ void k_zero_words(word_t *p, size_t n) {
     p[i] = 0;
 }
 
-constexpr size_t kPartWords = (size_t)2 * 2 * kSums * kMaxTeam;
-constexpr size_t kTotalWords = (size_t)2 * kLeaders * 2 * kSums;
-constexpr size_t kLdsBytes = 160 * 1024;
-// LDS of the team sums, rounded up (static, beside the dynamic arrays)
-constexpr size_t kLdsStatic = (sizeof(SumLds) + 1023) / 1024 * 1024;
-
 // The variants in order of preference (the smallest number of cells per
 // thread with which the team and its LDS fit): FP64, FP32 vectors, FP64
 // vectors with the FP32 matrix.
@@ -1067,7 +1042,7 @@ const TileVariant *tile_plan(TileArgs &a, int mode, bool sym, int cus, int *team
       c.TX = TX;
       c.slots = 2 * (TW + TH);
       c.ghosts = (2 * (TW + 2) + 2 * TH + 1) / 2 * 2;
-      if (v.lds(c) + kLdsStatic > kLdsBytes) continue;
+      if (v.lds(c) > kLdsDynamic) continue;
       const int32_t wgs = TX * TY;
       int64_t cost = wgs == 1 ? 0 : 2 * (TW + TH) + 7 * std::min(wgs, kFlatTeam);
       if (v.kind == STREAM) cost += 16 * (int64_t)TH;
@@ -1094,6 +1069,58 @@ void resident_free(ResidentBufs *b) {
   *b = ResidentBufs{};
 }
 
+int resident_prepare(hipStream_t s, ResidentBufs *bufs, size_t words, uint64_t need,
+                     uint32_t *tag0) {
+  if (!bufs->sums) {
+    LFG_TRY(dalloc(&bufs->sums, kPartWords + kTotalWords, "resident PCG sums"));
+    LFG_TRY(dalloc(&bufs->state, 2, "resident PCG state"));
+    bufs->abort = reinterpret_cast<int *>(bufs->state + 1);
+    bufs->epoch = 0xffffffffu;  // forces the clearing below
+  }
+  if (words > bufs->halo_words) {
+    dfree(bufs->halo);
+    bufs->halo = nullptr;
+    bufs->halo_words = 0;
+    LFG_TRY(dalloc(&bufs->halo, words, "resident PCG halo"));
+    bufs->halo_words = words;
+    bufs->epoch = 0xffffffffu;
+  }
+  if (bufs->epoch + need > 0xfffffff0ull) {
+    hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, s, bufs->halo, bufs->halo_words);
+    hipLaunchKernelGGL(k_zero_words, dim3(8), dim3(256), 0, s, bufs->sums,
+                       kPartWords + kTotalWords);
+    hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s,
+                       reinterpret_cast<word_t *>(bufs->state),
+                       2 * sizeof(ResidentState) / sizeof(word_t));
+    LFG_HIP(hipGetLastError());
+    bufs->epoch = 0;
+  }
+  *tag0 = bufs->epoch;
+  bufs->epoch = (uint32_t)std::min<uint64_t>(bufs->epoch + need, 0xffffffffull);
+  return LFGPU_OK;
+}
+
+int resident_launch(hipStream_t s, ResidentBufs *bufs, const void *fn, int team, void *args,
+                    size_t lds, ResidentState *st, bool *taken) {
+  LFG_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  void *argv[] = {args};
+  if (team == 1) {
+    LFG_HIP(hipLaunchKernel(fn, dim3(1), dim3(kThreads), argv, lds, s));
+  } else {
+    // all workgroups of the team must run at once
+    const hipError_t e =
+        hipLaunchCooperativeKernel(fn, dim3(team), dim3(kThreads), argv, (unsigned)lds, s);
+    if (e == hipErrorCooperativeLaunchTooLarge) {
+      (void)hipGetLastError();
+      return LFGPU_OK;
+    }
+    LFG_HIP(e);
+  }
+  LFG_HIP(hipMemcpyAsync(st, bufs->state, sizeof(ResidentState), hipMemcpyDeviceToHost, s));
+  *taken = true;
+  return LFGPU_OK;
+}
+
 int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
                      const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
                      bool *taken) {
@@ -1113,35 +1140,12 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
     const int32_t dy = A.off[d] > 1 ? 1 : A.off[d] < -1 ? -1 : 0;
     a.shift[d] = dy * (a.TW + 2) + (A.off[d] - dy * a.S);
   }
-  const size_t words = (size_t)2 * team * 2 * a.slots;
-  hipStream_t s = ctx->stream;
-  if (!bufs->sums) {
-    LFG_TRY(dalloc(&bufs->sums, kPartWords + kTotalWords, "resident PCG sums"));
-    LFG_TRY(dalloc(&bufs->state, 2, "resident PCG state"));
-    bufs->abort = reinterpret_cast<int *>(bufs->state + 1);
-    bufs->epoch = 0xffffffffu;  // forces the clearing below
-  }
-  if (words > bufs->halo_words) {
-    dfree(bufs->halo);
-    bufs->halo = nullptr;
-    bufs->halo_words = 0;
-    LFG_TRY(dalloc(&bufs->halo, words, "resident PCG halo"));
-    bufs->halo_words = words;
-    bufs->epoch = 0xffffffffu;
-  }
   // tags of this solve: one exchange and one sum an iteration, six for a
   // reliable update (at most one an iteration), and a few at the start
-  const uint64_t need = (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 7) + 16;
-  if (bufs->epoch + need > 0xfffffff0ull) {
-    hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, s, bufs->halo, bufs->halo_words);
-    hipLaunchKernelGGL(k_zero_words, dim3(8), dim3(256), 0, s, bufs->sums,
-                       kPartWords + kTotalWords);
-    hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s,
-                       reinterpret_cast<word_t *>(bufs->state),
-                       2 * sizeof(ResidentState) / sizeof(word_t));
-    LFG_HIP(hipGetLastError());
-    bufs->epoch = 0;
-  }
+  hipStream_t s = ctx->stream;
+  LFG_TRY(resident_prepare(s, bufs, (size_t)2 * team * 2 * a.slots,
+                           (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 7) + 16,
+                           &a.tag0));
   a.val = A.val;
   a.rowsum = A.rowsum;
   a.dinv = A.dinv;
@@ -1151,7 +1155,6 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
   a.part = bufs->sums;
   a.total = bufs->sums + kPartWords;
   a.abort = bufs->abort;
-  a.tag0 = bufs->epoch;
   a.tol2 = opts.rtol * opts.rtol;
   a.maxit = opts.maxit;
   a.st = bufs->state;
@@ -1162,26 +1165,8 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
   a.xlo = A.xlo;
   a.delta2 = opts.refine_delta > 0.0 ? opts.refine_delta * opts.refine_delta : 0.09;
   a.max_interval = opts.refine_max_interval > 0 ? opts.refine_max_interval : 2147483647;
-  const size_t lds = v->lds(a);
-  const void *fn = reinterpret_cast<const void *>(v->fn);
-  LFG_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  void *args[] = {&a};
-  if (team == 1) {
-    LFG_HIP(hipLaunchKernel(fn, dim3(1), dim3(kThreads), args, lds, s));
-  } else {
-    // all workgroups of the team must run at once
-    const hipError_t e =
-        hipLaunchCooperativeKernel(fn, dim3(team), dim3(kThreads), args, (unsigned)lds, s);
-    if (e == hipErrorCooperativeLaunchTooLarge) {
-      (void)hipGetLastError();
-      return LFGPU_OK;
-    }
-    LFG_HIP(e);
-  }
-  bufs->epoch = (uint32_t)std::min<uint64_t>(bufs->epoch + need, 0xffffffffull);
-  LFG_HIP(hipMemcpyAsync(st, bufs->state, sizeof(ResidentState), hipMemcpyDeviceToHost, s));
-  *taken = true;
-  return LFGPU_OK;
+  return resident_launch(s, bufs, reinterpret_cast<const void *>(v->fn), team, &a, v->lds(a), st,
+                         taken);
 }
 
 }  // namespace lfgpu

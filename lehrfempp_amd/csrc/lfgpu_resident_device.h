@@ -57,6 +57,25 @@ __device__ __forceinline__ double from_words(word_t lo, word_t hi) {
 }
 __device__ __forceinline__ bool tagged(word_t w, uint32_t tag) { return (uint32_t)w == tag; }
 
+// A value of an array at a uniform base and a 32-bit byte offset per lane (one
+// address register for all the arrays of a row).
+template <class T>
+__device__ __forceinline__ T load_at(const T *base, uint32_t bytes) {
+  return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + bytes);
+}
+// Hides a value from the optimiser, which else keeps every row's addresses
+// and masks in registers across the iterations (several hundred of them).
+__device__ __forceinline__ int32_t opaque(int32_t v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+// Keeps a row's result where it is computed (the compiler else sinks whole
+// rows past the next barrier and spills their operands).
+template <class T>
+__device__ __forceinline__ void pin(T &v) {
+  asm volatile("" : "+v"(v));
+}
+
 // A bounded wait: returns false once the team has been aborted.
 struct Wait {
   int *abort;
@@ -104,6 +123,12 @@ struct SumLds {
   double total[2][kSums];
   int bad;
 };
+
+// words of the team sums' buffers
+constexpr size_t kPartWords = (size_t)2 * 2 * kSums * kMaxTeam;
+constexpr size_t kTotalWords = (size_t)2 * kLeaders * 2 * kSums;
+// LDS a resident kernel may take dynamically (beside SumLds)
+constexpr size_t kLdsDynamic = 160 * 1024 - (sizeof(SumLds) + 1023) / 1024 * 1024;
 
 // The team as one workgroup sees it.
 struct Team {

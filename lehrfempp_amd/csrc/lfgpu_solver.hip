@@ -121,6 +121,7 @@ struct lfgpu_solver_cache {
   int32_t *blk_srow = nullptr, *blk_smap = nullptr;
   double *blk_t = nullptr;
   ResidentBufs res;  // resident solves (lfgpu_resident.hip)
+  ResidentEllPlan res_ell;
 };
 
 namespace lfgpu {
@@ -131,6 +132,7 @@ void solver_cache_free(lfgpu_csr *A) {
   if (!c) return;
   if (c->cg_graphs) cg_graphs_destroy(c->cg_graphs);
   resident_free(&c->res);
+  resident_ell_free(&c->res_ell);
   for (void *p : {(void *)c->slice_off, (void *)c->s_col, (void *)c->s_dcol, (void *)c->val, (void *)c->val32,
                   (void *)c->dinv, (void *)c->dinv32, (void *)c->dinv16, (void *)c->rowsum, (void *)c->rowsum32,
                   (void *)c->r, (void *)c->p, (void *)c->q, (void *)c->r32, (void *)c->p32,
@@ -3814,28 +3816,46 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
   // chunk below 2^20 rows (launch-bound sizes), or as the caller asks
   const bool use_graph = opts->graph > 0 || (opts->graph == 0 && n < (1 << 20));
 
-  // on DIA storage: the resident solve (lfgpu_resident.hip) where the system
-  // fits the chip, unless the caller asked for graph replays or plain
-  // launches of the sweeps
-  if (!single && c->fmt == FMT_DIA && c->blk_n == 0 && opts->graph == 0 && !t_timer) {
-    ResidentDia rd;
-    rd.n = n;
-    rd.width = c->width;
-    rd.ndiag = c->ndiag;
-    rd.off = c->off;
-    rd.val = c->val;
-    rd.rowsum = c->rowsum;
-    rd.dinv = c->dinv;
-    rd.sym = c->sym64;
-    rd.val32 = c->val32;
-    rd.rowsum32 = c->rowsum32;
-    rd.dinv32 = c->dinv32;
-    rd.dinv16 = c->dinv16;
-    rd.xlo = c->xlo;
+  // the resident solve (lfgpu_resident*.hip) where the system fits the chip,
+  // unless the caller asked for graph replays or plain launches of the sweeps
+  if (!single && c->blk_n == 0 && opts->graph == 0 && !t_timer) {
     ResidentState *rs = reinterpret_cast<ResidentState *>(ctx->pinned);
     bool taken = false;
     LFG_HIP(hipEventRecord(ctx->ev0, s));
-    LFG_TRY(resident_pcg_dia(ctx, &c->res, rd, *opts, b->d, x->d, rs, &taken));
+    if (c->fmt == FMT_DIA) {
+      ResidentDia rd;
+      rd.n = n;
+      rd.width = c->width;
+      rd.ndiag = c->ndiag;
+      rd.off = c->off;
+      rd.val = c->val;
+      rd.rowsum = c->rowsum;
+      rd.dinv = c->dinv;
+      rd.sym = c->sym64;
+      rd.val32 = c->val32;
+      rd.rowsum32 = c->rowsum32;
+      rd.dinv32 = c->dinv32;
+      rd.dinv16 = c->dinv16;
+      rd.xlo = c->xlo;
+      LFG_TRY(resident_pcg_dia(ctx, &c->res, rd, *opts, b->d, x->d, rs, &taken));
+    } else {
+      ResidentEll re;
+      re.n = n;
+      re.nslices = c->nslices;
+      re.slots = c->mlen;
+      re.slice_off = c->slice_off;
+      re.perm = c->perm;
+      re.dcol = c->s_dcol;
+      re.val = c->val;
+      re.rowsum = c->rowsum;
+      re.dinv = c->dinv;
+      re.val32 = c->val32;
+      re.rowsum32 = c->rowsum32;
+      re.dinv32 = c->dinv32;
+      re.dinv16 = c->dinv16;
+      re.xlo = c->xlo;
+      LFG_TRY(resident_pcg_ell(ctx, &c->res, &c->res_ell, re, *opts, b->d, x->d, rs, &taken));
+    }
     if (taken) return resident_finish(ctx, &c->res, rs, mixed, info);
   }
 

@@ -129,6 +129,42 @@ def test_resident_pcg_is_deterministic_and_zero_rhs(ctx, mode):
         h.close()
 
 
+# sliced ELL: lattices whose squares are cut along random diagonals; fewer rows
+# than a slice, one workgroup, teams summed in one and in two hops, 2, 3, 5, 8
+# and 11 rows a thread
+@pytest.mark.parametrize("S, L", [(7, 8), (22, 23), (40, 64), (181, 182), (363, 362), (450, 451),
+                                  (512, 513), (800, 801), (1025, 1024), (1150, 1151)])
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_pcg_on_ell(ctx, S, L, mode):
+    r, c, v, n = _lattice_system(S, L, P1, S)
+    # half of the diagonal couplings move to the square's other diagonal
+    rng = np.random.default_rng(L)
+    d = np.nonzero(c - r == S + 1)[0]
+    d = d[rng.random(d.size) < 0.5]
+    back = np.nonzero(r - c == S + 1)[0]
+    pos = np.zeros(n, np.int64)
+    pos[c[back]] = back  # (c + S + 1, c) by its column
+    r2, c2 = r.copy(), c.copy()
+    r2[d], c2[d] = r[d] + 1, c[d] - 1
+    r2[pos[r[d]]], c2[pos[r[d]]] = c[d] - 1, r[d] + 1
+    # (row sums move with the couplings: keep the matrix a Laplacian + 1e-3)
+    diag = np.full(n, 1e-3)
+    off = r2 != c2
+    np.subtract.at(diag, r2[off], v[off])
+    v2 = v.copy()
+    v2[~off] = diag[r2[~off]]
+    A = capi.coo_to_csr(ctx, r2, c2, v2, n, n)
+    out = _compare(ctx, A, n, mode, n + 1)
+    assert capi.solver_storage(A)[0] == capi.STORAGE_ELL16
+    assert out[1][0].syncs == 1  # the resident solve ran
+    x0 = np.random.default_rng(5).standard_normal(n)
+    out = _compare(ctx, A, n, mode, n + 2, x0=x0, maxit=3, rtol=1e-14)
+    assert out[0][0].iters == out[1][0].iters == 3
+    eps = 1e-13 if mode == capi.PCG_FP64 else 1e-5 if mode == capi.PCG_MIXED else 1e-12
+    assert np.linalg.norm(out[0][1] - out[1][1]) <= eps * np.linalg.norm(out[0][1])
+    A.close()
+
+
 def test_wrapped_band_matrix_keeps_the_sweeps(ctx):
     # the offsets of a lattice, but entries across the lines' ends
     n, S = 4096, 64
