@@ -376,15 +376,18 @@ int lfgpu_pcg_noalloc(lfgpu_ctx *ctx, const lfgpu_csr *A, const lfgpu_vec *b,
  * counterpart: a batch replaces nprob separate solve calls.
  * lfgpu_batch_create checks on the device that every entry of A lies inside
  * its row's problem block and returns LFGPU_EINVAL otherwise.
- * opts->graph: >= 0 replays the captured chunk (default); -1 launches each
- * chunk's kernels directly (the same iterates, no graph is captured). */
+ * opts->graph: 0 (default) solves all problems in one launch, and one more for
+ * those that are no structured P1 meshes, with their vectors kept on the chip
+ * (see lfgpu_pcg_opts.graph; summary->syncs is 1 then), where every problem
+ * fits; else, and with 1, replays the captured chunk; -1 launches each
+ * chunk's kernels directly (the same iterates as 1, no graph is captured). */
 typedef struct lfgpu_batch lfgpu_batch;
 int lfgpu_batch_create(lfgpu_ctx *ctx, lfgpu_csr *A, int nprob,
                        const int32_t *row_offsets, lfgpu_batch **out);
 int lfgpu_batch_destroy(lfgpu_batch *bt);
 /* infos: nprob entries (or NULL); summary: iters = max over problems,
  * converged = all converged, relres = worst, refinements = the tuned rows
- * per workgroup, ms = device time.  All three modes of lfgpu_pcg: in the
+ * per workgroup (0 while only one-launch solves have run), ms = device time.  All three modes of lfgpu_pcg: in the
  * mixed modes every problem runs its own reliable updates and stops on its
  * FP64 true residual (infos[p].refinements counts them). */
 int lfgpu_batch_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, const lfgpu_vec *b,
@@ -403,12 +406,14 @@ int lfgpu_batch_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, const lfgpu_vec *b,
 int lfgpu_batch_storage(const lfgpu_batch *bt, int *storage);
 /* lfgpu_assemble_galerkin of plan p (without prescribed Dirichlet values)
  * followed by lfgpu_batch_pcg on the batch created over p's matrix, with the
- * same results bit for bit.  The first call with a set of arguments runs the
- * two calls and captures a graph holding the assembly, the refresh of the
- * solver's copy of the values, the solve's set-up and its first chunk of
- * iterations; later calls with the same arguments (handles, coefficient
- * descriptors, vectors and options; the coefficient data may change) replay
- * it as one launch and continue with the captured chunks, polled as in
+ * same results bit for bit.  Where the batch solves in one launch
+ * (opts->graph 0, above) the two calls are made as they are.  Else the first
+ * call with a set of arguments runs the two calls and captures a graph
+ * holding the assembly, the refresh of the solver's copy of the values, the
+ * solve's set-up and its first chunk of iterations; later calls with the same
+ * arguments (handles, coefficient descriptors, vectors and options; the
+ * coefficient data may change) replay it as one launch and continue with the
+ * captured chunks, polled as in
  * lfgpu_batch_pcg (summary->syncs).  summary->ms covers assembly and solve.
  * The batched form of the north-star pipeline (assemble, then solve, per
  * problem; no single reference counterpart: AssembleMatrixLocally +

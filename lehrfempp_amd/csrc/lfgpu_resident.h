@@ -2,6 +2,7 @@
 #pragma once
 
 #include <cstdint>
+#include <vector>
 
 #include "lfgpu_internal.h"
 
@@ -28,6 +29,11 @@ void resident_free(ResidentBufs *b);
 // `need` tags; *tag0 the tag before its first.
 int resident_prepare(hipStream_t s, ResidentBufs *bufs, size_t words, uint64_t need,
                      uint32_t *tag0);
+// Whether resident_prepare would clear the buffers.
+bool resident_will_clear(const ResidentBufs *bufs, size_t words, uint64_t need);
+int resident_clear(hipStream_t s, unsigned long long *words, size_t n);
+int resident_launch_team(hipStream_t s, const void *fn, int team, void *args, size_t lds,
+                         bool *taken);
 // Queues kernel fn (one argument struct) on `team` workgroups that all run at
 // once, and the copy of its outcome to *st; *taken = false where the chip
 // does not hold them.
@@ -58,35 +64,53 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
                      const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
                      bool *taken);
 
-// Sliced-ELL storage split over a team for the resident solves: workgroup g
-// owns the storage rows [g rows, (g + 1) rows) and keeps their p in LDS, with
-// the values of the rows it reads of others behind them.
-struct ResidentEllPlan {
-  bool tried = false;
-  int team = 0, rpt = 0;
-  int32_t rows = 0;            // rows per workgroup, a multiple of 64
-  int32_t most = 0;            // most outside rows of a workgroup
-  int32_t *ext = nullptr;      // [team x stride] the outside rows, ascending
-  int32_t *ext_n = nullptr;    // [team]
-  int32_t stride = 0;
-  uint16_t *lcol = nullptr;    // per slot: the column's place in the workgroup's LDS
-  uint8_t *needed = nullptr;   // per row: some other workgroup reads it
+// The lattice problems of a batch, side by side in one launch.  st (device)
+// receives the outcome of problem `index` at st[index].
+struct ResidentProblem {
+  int32_t index, lo, n, width, ndiag;
+  int32_t off[8];
 };
+struct ResidentTiles;
+int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &probs, int mode,
+                        ResidentTiles **out);
+bool resident_tiles_fit(const ResidentTiles *p);
+void resident_tiles_free(ResidentTiles *p);
+// After an aborted solve: the next one clears the words.
+void resident_tiles_reset(ResidentTiles *p);
+// (A.width, A.ndiag and A.off are the problems' own)
+int resident_tiles_run(lfgpu_ctx *ctx, ResidentTiles *p, const ResidentDia &A,
+                       const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
+                       bool *taken);
+
+// Sliced-ELL storage split over a team for the resident solves: a workgroup
+// owns a run of storage rows and keeps their p in LDS, with the values of the
+// rows it reads of others behind them (lfgpu_resident_ell.hip).
+struct ResidentEllPlan;
 void resident_ell_free(ResidentEllPlan *p);
+bool resident_ell_fits(const ResidentEllPlan *p);
 
 // A matrix on sliced-ELL storage with 16-bit column offsets.
 struct ResidentEll {
-  int32_t n = 0, nslices = 0;
+  int32_t n = 0;  // storage rows
   int64_t slots = 0;
-  const int32_t *slice_off = nullptr, *perm = nullptr;  // perm: storage row -> row of x, b
+  // perm: storage row -> row of x and b (-1: an empty row); null: the same
+  const int32_t *slice_off = nullptr, *perm = nullptr;
   const int16_t *dcol = nullptr;
   const double *val = nullptr, *rowsum = nullptr, *dinv = nullptr;
   const float *val32 = nullptr, *rowsum32 = nullptr, *dinv32 = nullptr;
   const void *dinv16 = nullptr;
-  double *xlo = nullptr;
+  double *xlo = nullptr;  // in storage order
 };
-int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *plan,
+// As resident_pcg_dia; *plan is built by the first call.
+int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **plan,
                      const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b, double *x,
                      ResidentState *st, bool *taken);
+// The problems of a batch that are no lattices: problem q owns the storage
+// rows from q.lo (a multiple of 64) on, q.n of them.
+int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
+                            const std::vector<ResidentProblem> &probs, ResidentEllPlan **out);
+int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *plan,
+                           const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b,
+                           double *x, ResidentState *st, bool *taken);
 
 }  // namespace lfgpu

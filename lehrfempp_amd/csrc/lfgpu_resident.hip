@@ -33,6 +33,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <vector>
 
@@ -46,6 +47,14 @@ using namespace lfgpu::res;
 namespace {
 
 constexpr int ND = 6;  // off-diagonals of a P1 matrix on a structured mesh
+
+// One problem of a batch: its lattice, tiles and place in the buffers.
+struct TileJob {
+  int32_t index, lo;  // problem number, first row
+  int32_t S, L, TW, TH, TX, team, slots, ghosts, ndiag;
+  int32_t off[ND], shift[ND];
+  uint32_t halo_at, sums_at;  // words
+};
 
 struct TileArgs {
   int32_t n;            // rows of the storage (a diagonal's stride)
@@ -76,6 +85,12 @@ struct TileArgs {
   double *xlo;
   double delta2;
   int max_interval;
+  // batches: the jobs, each slot's job and rank in its team, and the counter
+  // that hands out the slots
+  const TileJob *__restrict__ jobs;
+  const int2 *__restrict__ job_slots;
+  int nslots;
+  int *ticket;
 };
 
 // The workgroup's tile: tw x th cells of the lattice, padded by one halo cell
@@ -310,17 +325,18 @@ struct TileLds {
 // RPT: cells per thread.  XR: the cells j < XR keep their x in a register, the
 // others' is read and written in every update (as many as the registers hold
 // without spills).  AHEAD: rows of a stream in flight.
-template <int KIND, int RPT, int XR, int AHEAD = 1>
-__global__ __launch_bounds__(kThreads) void k_res_tile(TileArgs a) {
+template <int KIND, int RPT, int XR, int AHEAD, bool BATCH>
+__device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team, double *dyn,
+                                           SumLds &sh) {
   constexpr bool kStream = KIND == STREAM, kGhost = KIND == GHOST;
-  extern __shared__ double dyn[];
-  __shared__ SumLds sh;
   const int t = threadIdx.x;
-  Tile T(a, blockIdx.x, gridDim.x);
+  Tile T(a, rank, team);
   typedef TileLds<KIND, double, RPT> Lds;
   const Lds M(dyn, a, T);
   constexpr bool kRegDiag = !kStream && !Lds::kDiag;
   double *const lp = M.lp;
+  // (a batch's smaller tiles leave the last cell numbers empty)
+  const int nj = BATCH ? (T.th * T.P + kThreads - 1) / kThreads : RPT;
   Team tm{T.rank, T.team, a.part, a.total, a.abort, a.tag0};
   if (t == 0) sh.bad = 0;
   T.tables(t);
@@ -383,6 +399,7 @@ __global__ __launch_bounds__(kThreads) void k_res_tile(TileArgs a) {
       const double *lrs = M.rs + opaque(t), *ldi = M.di + opaque(t);
 #pragma unroll
       for (int j = 0; j < RPT; ++j) {
+        if (BATCH && j >= nj) break;
         // every LDS read of the row before the first use
         const double pi = lc[j * kThreads];
         double c[ND], acc = 0.0;
@@ -561,6 +578,7 @@ __global__ __launch_bounds__(kThreads) void k_res_tile(TileArgs a) {
     double np = lc[0];
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
+      if (BATCH && j >= nj) break;
       const double dv = kRegDiag ? di[kRegDiag ? j : 0] : kStream ? nd : ldi[j * kThreads];
       const double xi = j < XR ? x[j < XR ? j : 0] : nx;
       xat = nxat;
@@ -613,6 +631,70 @@ __global__ __launch_bounds__(kThreads) void k_res_tile(TileArgs a) {
     a.st->refinements = 0;
     a.st->aborted = ok ? 0 : 1;
   }
+  return ok;
+}
+
+template <int KIND, int RPT, int XR, int AHEAD = 1>
+__global__ __launch_bounds__(kThreads) void k_res_tile(TileArgs a) {
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  (void)tile_solve<KIND, RPT, XR, AHEAD, false>(a, blockIdx.x, gridDim.x, dyn, sh);
+}
+
+// A batch: the workgroups take slots (a problem and a rank in its team) from
+// a counter, in order.  A problem's slots are consecutive and a team has at
+// most as many members as there are workgroups, all of which run, so the
+// first unfinished problem always gets its team together.
+template <class F>
+__device__ __forceinline__ void batch_loop(const TileArgs &base, F &&solve) {
+  __shared__ int slot;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) slot = atomicAdd(base.ticket, 1);
+    __syncthreads();
+    const int k = __builtin_amdgcn_readfirstlane(slot);
+    if (k >= base.nslots) return;
+    const int2 jr = base.job_slots[k];
+    const TileJob &jb = base.jobs[jr.x];
+    TileArgs a = base;
+    a.S = jb.S;
+    a.L = jb.L;
+    a.TW = jb.TW;
+    a.TH = jb.TH;
+    a.TX = jb.TX;
+    a.slots = jb.slots;
+    a.ghosts = jb.ghosts;
+    a.ndiag = jb.ndiag;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      a.off[d] = jb.off[d];
+      a.shift[d] = jb.shift[d];
+    }
+    a.val += jb.lo;
+    a.rowsum += jb.lo;
+    a.dinv += jb.lo;
+    a.b += jb.lo;
+    a.x += jb.lo;
+    a.val32 += jb.lo;
+    a.rowsum32 += jb.lo;
+    a.dinv32 += jb.lo;
+    a.dinv16 += jb.lo;
+    a.xlo += jb.lo;
+    a.halo_words += jb.halo_at;
+    a.part += jb.sums_at;
+    a.total = a.part + (size_t)2 * 2 * kSums * jb.team;
+    a.st += jb.index;
+    if (!solve(a, jr.y, jb.team)) return;
+  }
+}
+
+template <int RPT>
+__global__ __launch_bounds__(kThreads) void k_res_tile_batch(TileArgs base) {
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  batch_loop(base, [&](const TileArgs &a, int rank, int team) {
+    return tile_solve<GHOST, RPT, RPT, 1, true>(a, rank, team, dyn, sh);
+  });
 }
 
 // ---------------------------------------------------------------------------
@@ -633,16 +715,16 @@ __device__ __forceinline__ float mixed_dinv(const TileArgs &a, int32_t g) {
   else return a.dinv32[g];
 }
 
-template <int KIND, class VT, int RPT, int AHEAD = 1>
-__global__ __launch_bounds__(kThreads) void k_res_tile_mixed(TileArgs a) {
+template <int KIND, class VT, int RPT, int AHEAD, bool BATCH>
+__device__ __forceinline__ bool tile_solve_mixed(const TileArgs &a, int rank, int team,
+                                                 double *dyn, SumLds &sh) {
   constexpr bool kStream = KIND == STREAM, kGhost = KIND == GHOST;
-  extern __shared__ double dyn[];
-  __shared__ SumLds sh;
   const int t = threadIdx.x;
-  Tile T(a, blockIdx.x, gridDim.x);
+  Tile T(a, rank, team);
   typedef TileLds<KIND, VT, RPT> Lds;
   const Lds M(dyn, a, T);
   constexpr bool kRegDiag = !kStream && !Lds::kDiag;
+  const int nj = BATCH ? (T.th * T.P + kThreads - 1) / kThreads : RPT;
   double *const lp = M.lp;
   Team tm{T.rank, T.team, a.part, a.total, a.abort, a.tag0};
   if (t == 0) sh.bad = 0;
@@ -725,6 +807,7 @@ __global__ __launch_bounds__(kThreads) void k_res_tile_mixed(TileArgs a) {
       for (int j = 0; j < AHEAD; ++j) load_row(j);
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
+      if (BATCH && j >= nj) break;
       const int k = j % AHEAD;
       double vr[ND];
 #pragma unroll
@@ -807,6 +890,7 @@ __global__ __launch_bounds__(kThreads) void k_res_tile_mixed(TileArgs a) {
       double np = lc[0];
 #pragma unroll
       for (int j = 0; j < RPT; ++j) {
+        if (BATCH && j >= nj) break;
         const VT dv = kRegDiag ? di[kRegDiag ? j : 0]
                       : kStream ? (VT)nd[j % kAhead] : (VT)ldi[j * kThreads];
         if (j + kAhead < RPT) load_update(j + kAhead);
@@ -981,6 +1065,23 @@ __global__ __launch_bounds__(kThreads) void k_res_tile_mixed(TileArgs a) {
     a.st->refinements = refinements;
     a.st->aborted = ok ? 0 : 1;
   }
+  return ok;
+}
+
+template <int KIND, class VT, int RPT, int AHEAD = 1>
+__global__ __launch_bounds__(kThreads) void k_res_tile_mixed(TileArgs a) {
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  (void)tile_solve_mixed<KIND, VT, RPT, AHEAD, false>(a, blockIdx.x, gridDim.x, dyn, sh);
+}
+
+template <class VT, int RPT>
+__global__ __launch_bounds__(kThreads) void k_res_tile_mixed_batch(TileArgs base) {
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  batch_loop(base, [&](const TileArgs &a, int rank, int team) {
+    return tile_solve_mixed<GHOST, VT, RPT, 1, true>(a, rank, team, dyn, sh);
+  });
 }
 
 __global__ void k_zero_words(word_t *p, size_t n) {
@@ -1015,48 +1116,81 @@ const std::vector<TileVariant> kTileVariants[3] = {
 #undef LFG_TILE
 #undef LFG_TILEM
 
-// Splits the lattice into at most cus tiles for the first variant that takes
-// them; among the splits, the one with the shortest rim (the halo travels
-// every iteration) and, where one workgroup sums all members' partials, the
-// smallest team.  STREAM: lines of a tile are read in 128-byte pieces,
-// two of which at their ends another tile reads too, so a tile line counts
-// as 16 cells more.  Returns the variant or nullptr.
+// Splits the lattice a.S x a.L into at most `most` tiles of at most cap padded
+// cells whose LDS fits; among the splits, the one with the shortest rim (the
+// halo travels every iteration) and, where every workgroup sums all members'
+// partials, the smallest team.  STREAM: lines of a tile are read in 128-byte
+// pieces, two of which at their ends another tile reads too, so a tile line
+// counts as 16 cells more.  Returns the team, 0 if there is no such split.
+int tile_split(TileArgs &a, int64_t cap, int most, bool stream, size_t (*lds)(const TileArgs &)) {
+  int64_t best = -1;
+  int team = 0;
+  TileArgs pick = a;
+  for (int32_t tx = 1; tx <= most && tx <= a.S; ++tx) {
+    const int32_t TW = (a.S + tx - 1) / tx, TX = (a.S + TW - 1) / TW;
+    const int32_t lines = (int32_t)std::min<int64_t>(cap / (TW + 2), a.L);  // lines a tile
+    if (lines < 1 || TX > most) continue;
+    int32_t TY = (a.L + lines - 1) / lines;
+    if ((int64_t)TX * TY > most) continue;
+    const int32_t TH = (a.L + TY - 1) / TY;
+    TY = (a.L + TH - 1) / TH;
+    TileArgs c = a;
+    c.TW = TW;
+    c.TH = TH;
+    c.TX = TX;
+    c.slots = 2 * (TW + TH);
+    c.ghosts = (2 * (TW + 2) + 2 * TH + 1) / 2 * 2;
+    if (lds(c) > kLdsDynamic) continue;
+    const int32_t wgs = TX * TY;
+    int64_t cost = wgs == 1 ? 0 : 2 * (TW + TH) + 7 * std::min(wgs, kFlatTeam);
+    if (stream) cost += 16 * (int64_t)TH;
+    if (best >= 0 && cost >= best) continue;
+    best = cost;
+    team = wgs;
+    pick = c;
+  }
+  if (team > 0) a = pick;
+  return team;
+}
+
+// Row offsets to offsets in the padded tile: off = dy S + dx with |dx|, |dy|
+// <= 1.  (An offset that no row of this lattice has gets 0: its values are
+// zero.)
+template <class J>
+void tile_shifts(J &a) {
+  for (int d = 0; d < ND; ++d) {
+    const int32_t o = d < a.ndiag ? a.off[d] : 0;
+    const int32_t dy = o > 1 ? 1 : o < -1 ? -1 : 0, dx = o - dy * a.S;
+    a.shift[d] = std::abs(dx) <= 1 ? dy * (a.TW + 2) + dx : 0;
+  }
+}
+
+// the first variant that takes the lattice, or nullptr
 const TileVariant *tile_plan(TileArgs &a, int mode, bool sym, int cus, int *team) {
   for (const TileVariant &v : kTileVariants[mode]) {
     if (v.kind == STREAM && !(sym && a.ndiag == ND)) continue;
     const int64_t cap = (int64_t)v.rpt * kThreads;
     if ((int64_t)a.S * a.L > cap * cus) continue;
-    int64_t best = -1;
-    TileArgs pick = a;
-    for (int32_t tx = 1; tx <= cus && tx <= a.S; ++tx) {
-      const int32_t TW = (a.S + tx - 1) / tx, TX = (a.S + TW - 1) / TW;
-      const int32_t most = (int32_t)std::min<int64_t>(cap / (TW + 2), a.L);  // lines a tile
-      if (most < 1 || TX > cus) continue;
-      int32_t TY = (a.L + most - 1) / most;
-      if ((int64_t)TX * TY > cus) continue;
-      const int32_t TH = (a.L + TY - 1) / TY;
-      TY = (a.L + TH - 1) / TH;
-      TileArgs c = a;
-      c.TW = TW;
-      c.TH = TH;
-      c.TX = TX;
-      c.slots = 2 * (TW + TH);
-      c.ghosts = (2 * (TW + 2) + 2 * TH + 1) / 2 * 2;
-      if (v.lds(c) > kLdsDynamic) continue;
-      const int32_t wgs = TX * TY;
-      int64_t cost = wgs == 1 ? 0 : 2 * (TW + TH) + 7 * std::min(wgs, kFlatTeam);
-      if (v.kind == STREAM) cost += 16 * (int64_t)TH;
-      if (best >= 0 && cost >= best) continue;
-      best = cost;
-      pick = c;
-      *team = TX * TY;
-    }
-    if (best < 0) continue;
-    a = pick;
-    return &v;
+    *team = tile_split(a, cap, cus, v.kind == STREAM, v.lds);
+    if (*team > 0) return &v;
   }
   return nullptr;
 }
+
+// Batches: up to 3 and up to 7 (FP64 vectors) or 9 cells a thread.
+struct BatchVariant {
+  int rpt;
+  size_t (*lds)(const TileArgs &);
+  void (*fn)(TileArgs);
+};
+const BatchVariant kBatchVariants[3][2] = {
+    {{3, &TileLds<GHOST, double, 3>::bytes, &k_res_tile_batch<3>},
+     {7, &TileLds<GHOST, double, 7>::bytes, &k_res_tile_batch<7>}},
+    {{3, &TileLds<GHOST, float, 3>::bytes, &k_res_tile_mixed_batch<float, 3>},
+     {9, &TileLds<GHOST, float, 9>::bytes, &k_res_tile_mixed_batch<float, 9>}},
+    {{3, &TileLds<GHOST, double, 3>::bytes, &k_res_tile_mixed_batch<double, 3>},
+     {7, &TileLds<GHOST, double, 7>::bytes, &k_res_tile_mixed_batch<double, 7>}},
+};
 
 }  // namespace
 
@@ -1067,6 +1201,36 @@ void resident_free(ResidentBufs *b) {
   dfree(b->sums);
   dfree(b->state);
   *b = ResidentBufs{};
+}
+
+static void fill_args(TileArgs &a, const ResidentDia &A, const lfgpu_pcg_opts &opts,
+                      const double *b, double *x) {
+  a.n = A.n;
+  a.val = A.val;
+  a.rowsum = A.rowsum;
+  a.dinv = A.dinv;
+  a.b = b;
+  a.x = x;
+  a.tol2 = opts.rtol * opts.rtol;
+  a.maxit = opts.maxit;
+  a.val32 = A.val32;
+  a.rowsum32 = A.rowsum32;
+  a.dinv32 = A.dinv32;
+  a.dinv16 = static_cast<const __hip_bfloat16 *>(A.dinv16);
+  a.xlo = A.xlo;
+  a.delta2 = opts.refine_delta > 0.0 ? opts.refine_delta * opts.refine_delta : 0.09;
+  a.max_interval = opts.refine_max_interval > 0 ? opts.refine_max_interval : 2147483647;
+}
+
+int resident_clear(hipStream_t s, unsigned long long *words, size_t n) {
+  hipLaunchKernelGGL(k_zero_words, dim3((unsigned)std::min<size_t>(256, (n + 255) / 256)),
+                     dim3(256), 0, s, words, n);
+  LFG_HIP(hipGetLastError());
+  return LFGPU_OK;
+}
+
+bool resident_will_clear(const ResidentBufs *bufs, size_t words, uint64_t need) {
+  return !bufs->sums || words > bufs->halo_words || bufs->epoch + need > 0xfffffff0ull;
 }
 
 int resident_prepare(hipStream_t s, ResidentBufs *bufs, size_t words, uint64_t need,
@@ -1100,8 +1264,8 @@ int resident_prepare(hipStream_t s, ResidentBufs *bufs, size_t words, uint64_t n
   return LFGPU_OK;
 }
 
-int resident_launch(hipStream_t s, ResidentBufs *bufs, const void *fn, int team, void *args,
-                    size_t lds, ResidentState *st, bool *taken) {
+int resident_launch_team(hipStream_t s, const void *fn, int team, void *args, size_t lds,
+                         bool *taken) {
   LFG_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   void *argv[] = {args};
   if (team == 1) {
@@ -1116,8 +1280,15 @@ int resident_launch(hipStream_t s, ResidentBufs *bufs, const void *fn, int team,
     }
     LFG_HIP(e);
   }
-  LFG_HIP(hipMemcpyAsync(st, bufs->state, sizeof(ResidentState), hipMemcpyDeviceToHost, s));
   *taken = true;
+  return LFGPU_OK;
+}
+
+int resident_launch(hipStream_t s, ResidentBufs *bufs, const void *fn, int team, void *args,
+                    size_t lds, ResidentState *st, bool *taken) {
+  LFG_TRY(resident_launch_team(s, fn, team, args, lds, taken));
+  if (*taken)
+    LFG_HIP(hipMemcpyAsync(st, bufs->state, sizeof(ResidentState), hipMemcpyDeviceToHost, s));
   return LFGPU_OK;
 }
 
@@ -1134,39 +1305,187 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
   int team = 0;
   const TileVariant *v = tile_plan(a, opts.mode, A.sym, std::min(ctx->cus, kMaxTeam), &team);
   if (!v) return LFGPU_OK;
-  for (int d = 0; d < A.ndiag; ++d) {
-    a.off[d] = A.off[d];
-    // off = dy S + dx with |dx|, |dy| <= 1
-    const int32_t dy = A.off[d] > 1 ? 1 : A.off[d] < -1 ? -1 : 0;
-    a.shift[d] = dy * (a.TW + 2) + (A.off[d] - dy * a.S);
-  }
+  for (int d = 0; d < A.ndiag; ++d) a.off[d] = A.off[d];
+  tile_shifts(a);
   // tags of this solve: one exchange and one sum an iteration, six for a
   // reliable update (at most one an iteration), and a few at the start
   hipStream_t s = ctx->stream;
   LFG_TRY(resident_prepare(s, bufs, (size_t)2 * team * 2 * a.slots,
                            (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 7) + 16,
                            &a.tag0));
-  a.val = A.val;
-  a.rowsum = A.rowsum;
-  a.dinv = A.dinv;
-  a.b = b;
-  a.x = x;
+  fill_args(a, A, opts, b, x);
   a.halo_words = bufs->halo;
   a.part = bufs->sums;
   a.total = bufs->sums + kPartWords;
   a.abort = bufs->abort;
-  a.tol2 = opts.rtol * opts.rtol;
-  a.maxit = opts.maxit;
   a.st = bufs->state;
-  a.val32 = A.val32;
-  a.rowsum32 = A.rowsum32;
-  a.dinv32 = A.dinv32;
-  a.dinv16 = static_cast<const __hip_bfloat16 *>(A.dinv16);
-  a.xlo = A.xlo;
-  a.delta2 = opts.refine_delta > 0.0 ? opts.refine_delta * opts.refine_delta : 0.09;
-  a.max_interval = opts.refine_max_interval > 0 ? opts.refine_max_interval : 2147483647;
   return resident_launch(s, bufs, reinterpret_cast<const void *>(v->fn), team, &a, v->lds(a), st,
                          taken);
+}
+
+
+// ---------------------------------------------------------------------------
+// batches
+// ---------------------------------------------------------------------------
+struct ResidentTiles {
+  bool fits = false;
+  int nslots = 0, variant = 0;
+  size_t lds = 0;
+  size_t halo_words = 0, sums_words = 0;
+  TileJob *jobs = nullptr;
+  int2 *slots = nullptr;
+  word_t *words = nullptr;  // sums, then halos
+  int *ticket = nullptr;    // followed by the abort flag
+  uint32_t epoch = 0xffffffffu;
+};
+
+void resident_tiles_free(ResidentTiles *p) {
+  if (!p) return;
+  dfree(p->jobs);
+  dfree(p->slots);
+  dfree(p->words);
+  dfree(p->ticket);
+  delete p;
+}
+
+// Team sizes: the problems run side by side, so that the batch takes as long
+// as its longest problem while all teams fit the chip; iterations grow with
+// the square root of the rows, an iteration takes about 4.5 us and 0.8 ns a
+// cell of a workgroup.  The cells a workgroup takes follow from the smallest
+// common finishing time with which the teams fit; where none does, every
+// workgroup takes as many as it can hold and the longest problems go first.
+int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &probs, int mode,
+                        ResidentTiles **out) {
+  ResidentTiles *p = new ResidentTiles();
+  *out = p;
+  const int cus = std::min(ctx->cus, kMaxTeam);
+  const BatchVariant &big = kBatchVariants[mode][1];
+  const int64_t cap = (int64_t)big.rpt * kThreads;
+  const size_t np = probs.size();
+  if (np == 0) return LFGPU_OK;
+  auto iterations = [&](const ResidentProblem &q) { return std::sqrt((double)q.n); };
+  auto split = [&](const ResidentProblem &q, int64_t cells, TileArgs &a) {
+    a = TileArgs{};
+    a.S = q.width;
+    a.L = q.n / q.width;
+    return tile_split(a, cells, cus, false, big.lds);
+  };
+  // teams for a common finishing time tau; 0 if one does not fit
+  std::vector<int> team(np);
+  std::vector<TileArgs> geo(np);
+  auto total = [&](double tau) {
+    int64_t sum = 0;
+    for (size_t k = 0; k < np; ++k) {
+      const double c = tau > 0.0 ? (tau / iterations(probs[k]) - 4.5) / 0.0008 : (double)cap;
+      const int64_t cells = (int64_t)std::min<double>((double)cap, std::max(c, 128.0));
+      team[k] = split(probs[k], cells, geo[k]);
+      if (team[k] == 0) team[k] = split(probs[k], cap, geo[k]);
+      if (team[k] == 0) return (int64_t)-1;
+      sum += team[k];
+    }
+    return sum;
+  };
+  int64_t all = total(0.0);
+  if (all < 0) return LFGPU_OK;
+  if (all <= cus) {
+    double hi = 0.0;
+    for (const ResidentProblem &q : probs)
+      hi = std::max(hi, iterations(q) * (4.5 + 0.0008 * (double)cap));
+    double lo = 0.0;
+    for (int step = 0; step < 10; ++step) {
+      const double mid = 0.5 * (lo + hi);
+      if (total(mid) <= cus) hi = mid;
+      else lo = mid;
+    }
+    all = total(hi);
+  }
+  std::vector<size_t> order(np);
+  for (size_t k = 0; k < np; ++k) order[k] = k;
+  auto cost = [&](size_t k) {
+    return iterations(probs[k]) * (4.5 + 0.0008 * (geo[k].TW + 2) * geo[k].TH);
+  };
+  std::stable_sort(order.begin(), order.end(),
+                   [&](size_t i, size_t j) { return cost(i) > cost(j); });
+  std::vector<TileJob> jobs(np);
+  std::vector<int2> slots;
+  int64_t most = 0;
+  for (size_t o = 0; o < np; ++o) {
+    const size_t k = order[o];
+    const ResidentProblem &q = probs[k];
+    const TileArgs &g = geo[k];
+    TileJob &j = jobs[o];
+    j.index = q.index;
+    j.lo = q.lo;
+    j.S = g.S;
+    j.L = g.L;
+    j.TW = g.TW;
+    j.TH = g.TH;
+    j.TX = g.TX;
+    j.team = team[k];
+    j.slots = g.slots;
+    j.ghosts = g.ghosts;
+    j.ndiag = q.ndiag;
+    for (int d = 0; d < ND; ++d) j.off[d] = d < q.ndiag ? q.off[d] : 0;
+    tile_shifts(j);
+    j.halo_at = (uint32_t)p->halo_words;
+    j.sums_at = (uint32_t)p->sums_words;
+    p->halo_words += (size_t)2 * j.team * 2 * j.slots;
+    p->sums_words += (size_t)2 * 2 * kSums * j.team + kTotalWords;
+    most = std::max<int64_t>(most, (int64_t)(g.TW + 2) * g.TH);
+    for (int r = 0; r < j.team; ++r) slots.push_back(int2{(int)o, r});
+  }
+  p->variant = most <= (int64_t)kBatchVariants[mode][0].rpt * kThreads ? 0 : 1;
+  for (size_t k = 0; k < np; ++k)
+    p->lds = std::max(p->lds, kBatchVariants[mode][p->variant].lds(geo[k]));
+  p->nslots = (int)slots.size();
+  hipStream_t s = ctx->stream;
+  LFG_TRY(dalloc(&p->jobs, np, "resident batch jobs"));
+  LFG_TRY(dalloc(&p->slots, slots.size(), "resident batch slots"));
+  LFG_TRY(dalloc(&p->words, p->sums_words + p->halo_words, "resident batch words"));
+  LFG_TRY(dalloc(&p->ticket, 4, "resident batch counter"));
+  LFG_HIP(hipMemcpyAsync(p->jobs, jobs.data(), np * sizeof(TileJob), hipMemcpyHostToDevice, s));
+  LFG_HIP(hipMemcpyAsync(p->slots, slots.data(), slots.size() * sizeof(int2),
+                         hipMemcpyHostToDevice, s));
+  LFG_HIP(hipStreamSynchronize(s));
+  p->fits = true;
+  return LFGPU_OK;
+}
+
+bool resident_tiles_fit(const ResidentTiles *p) { return p && p->fits; }
+
+void resident_tiles_reset(ResidentTiles *p) { p->epoch = 0xffffffffu; }
+
+int resident_tiles_run(lfgpu_ctx *ctx, ResidentTiles *p, const ResidentDia &A,
+                       const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
+                       bool *taken) {
+  *taken = false;
+  hipStream_t s = ctx->stream;
+  const uint64_t need = (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 7) + 16;
+  if (p->epoch + need > 0xfffffff0ull) {
+    hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, s, p->words,
+                       p->sums_words + p->halo_words);
+    p->epoch = 0;
+  }
+  // the counter and the abort flag
+  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s, reinterpret_cast<word_t *>(p->ticket),
+                     (size_t)2);
+  LFG_HIP(hipGetLastError());
+  TileArgs a{};
+  fill_args(a, A, opts, b, x);
+  a.halo_words = p->words + p->sums_words;
+  a.part = p->words;
+  a.abort = p->ticket + 2;
+  a.tag0 = p->epoch;
+  a.st = st;
+  a.jobs = p->jobs;
+  a.job_slots = p->slots;
+  a.nslots = p->nslots;
+  a.ticket = p->ticket;
+  p->epoch = (uint32_t)std::min<uint64_t>(p->epoch + need, 0xffffffffull);
+  const int team = std::min(p->nslots, std::min(ctx->cus, kMaxTeam));
+  return resident_launch_team(
+      s, reinterpret_cast<const void *>(kBatchVariants[opts.mode][p->variant].fn), team, &a,
+      p->lds, taken);
 }
 
 }  // namespace lfgpu

@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "lfgpu_reduce.h"
@@ -24,8 +25,20 @@ using namespace lfgpu::res;
 
 namespace {
 
+// One workgroup's share: storage rows [r0, r1), LDS places 0.. for them and
+// from `rows` on for the `outside` rows listed at ext[at..].
+struct EllPart {
+  int32_t r0, r1, rows, outside;
+  int64_t at;
+};
+// One problem of a batch.
+struct EllJob {
+  int32_t index, team;
+  uint32_t sums_at;
+};
+
 struct EllArgs {
-  int32_t n, rows, nslices;
+  int32_t n;  // storage rows
   const int32_t *__restrict__ slice_off;
   const uint16_t *__restrict__ lcol;
   const double *__restrict__ val;
@@ -35,10 +48,9 @@ struct EllArgs {
   const double *__restrict__ dinv;
   const float *__restrict__ dinv32;
   const __hip_bfloat16 *__restrict__ dinv16;
-  const int32_t *__restrict__ perm;  // may be null
+  const int32_t *__restrict__ perm;  // storage row -> row of x, b; -1: none; may be null
+  const EllPart *__restrict__ parts;
   const int32_t *__restrict__ ext;
-  const int32_t *__restrict__ ext_n;
-  int32_t stride;
   const uint8_t *__restrict__ needed;
   const double *__restrict__ b;
   double *x;
@@ -52,6 +64,11 @@ struct EllArgs {
   double delta2;
   int max_interval;
   ResidentState *st;
+  // batches
+  const EllJob *__restrict__ jobs;
+  const int2 *__restrict__ job_slots;  // slot (= part) -> job, rank in its team
+  int nslots;
+  int *ticket;
 };
 
 // the precision modes: FP64; FP32 vectors; FP64 vectors with the FP32 matrix
@@ -116,20 +133,19 @@ __device__ __forceinline__ double ell_lds_row(const MT *__restrict__ vp,
 // 64 (wave + 8 j) + lane, so a wavefront works on whole slices.  DREG: D^-1
 // and row sums in registers (else read every iteration).
 template <int MODE, int RPT, bool DREG>
-__global__ __launch_bounds__(kThreads) void k_res_ell(EllArgs a) {
+__device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int rank, int team,
+                                          double *lp, SumLds &sh) {
   typedef typename Mode<MODE>::VT VT;
   typedef typename Mode<MODE>::MT MT;
   constexpr bool kMixed = MODE != LFGPU_PCG_FP64;
-  extern __shared__ double lp[];
-  __shared__ SumLds sh;
   const int t = threadIdx.x;
-  const int32_t rank = blockIdx.x, team = gridDim.x;
   Team tm{rank, team, a.part, a.total, a.abort, a.tag0};
   uint32_t tag = a.tag0;
   if (t == 0) sh.bad = 0;
-  const int32_t r0 = rank * a.rows, mine = min(a.rows, a.n - r0);
-  const int32_t next = a.ext_n[rank];
-  const int32_t *ext = a.ext + (size_t)rank * a.stride;
+  const EllPart &part = a.parts[slot];
+  const int32_t r0 = part.r0, mine = part.r1 - part.r0, place = part.rows;
+  const int32_t next = part.outside;
+  const int32_t *ext = a.ext + part.at;
   const int32_t s0 = (r0 >> 6) + __builtin_amdgcn_readfirstlane(t >> 6);
   const int32_t slices = (mine + 63) >> 6;
 
@@ -181,15 +197,14 @@ __global__ __launch_bounds__(kThreads) void k_res_ell(EllArgs a) {
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         if (e0 + u * kThreads < next) {
-          if constexpr (kTwo) lp[a.rows + e0 + u * kThreads] = from_words(lo[u], hi[u]);
-          else
-            lp[a.rows + e0 + u * kThreads] = (double)__uint_as_float((uint32_t)(lo[u] >> 32));
+          if constexpr (kTwo) lp[place + e0 + u * kThreads] = from_words(lo[u], hi[u]);
+          else lp[place + e0 + u * kThreads] = (double)__uint_as_float((uint32_t)(lo[u] >> 32));
         }
     }
   };
 
   // (places past the last row are read and have to be finite)
-  for (int32_t i = t; i < a.rows; i += kThreads) lp[i] = 0.0;
+  for (int32_t i = t; i < place; i += kThreads) lp[i] = 0.0;
 
   // x: the solution (FP64) or the mixed modes' increment
   VT x[RPT], r[RPT], q[RPT], di[DREG ? RPT : 1];
@@ -203,7 +218,7 @@ __global__ __launch_bounds__(kThreads) void k_res_ell(EllArgs a) {
       rs[j] = 0.0;
       di[j] = (VT)0;
     }
-    if (i < mine) {
+    if (i < mine && at(r0 + i) >= 0) {
       live |= 1u << j;
       if (a.needed[r0 + i]) needed |= 1u << j;
       if constexpr (DREG) {
@@ -321,8 +336,8 @@ __global__ __launch_bounds__(kThreads) void k_res_ell(EllArgs a) {
 #pragma unroll
       for (int j = 0; j < RPT; ++j) bb = __builtin_fma(r64[j], r64[j], bb);
     }
-    for (int part = 0; part < (first ? 1 : 3); ++part) {
-      if (part == 0) {
+    for (int turn = 0; turn < (first ? 1 : 3); ++turn) {
+      if (turn == 0) {
         __syncthreads();  // the last readers of LDS are done
       } else {
         // nor does a workgroup overwrite words that another still waits for
@@ -337,7 +352,7 @@ __global__ __launch_bounds__(kThreads) void k_res_ell(EllArgs a) {
       for (int j = 0; j < RPT; ++j) {
         const int32_t i = ti + j * kThreads;
         if ((live >> j) & 1) {
-          const double y = part == 0 ? a.x[at(r0 + i)] : part == 1 ? (double)x[j] : a.xlo[r0 + i];
+          const double y = turn == 0 ? a.x[at(r0 + i)] : turn == 1 ? (double)x[j] : a.xlo[r0 + i];
           if (!kMixed) x[j] = (VT)y;
           lp[i] = y;
           if ((needed >> j) & 1) publish(i, y);
@@ -433,6 +448,37 @@ __global__ __launch_bounds__(kThreads) void k_res_ell(EllArgs a) {
     a.st->refinements = refinements;
     a.st->aborted = ok ? 0 : 1;
   }
+  return ok;
+}
+
+template <int MODE, int RPT, bool DREG>
+__global__ __launch_bounds__(kThreads) void k_res_ell(EllArgs a) {
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  (void)ell_solve<MODE, RPT, DREG>(a, blockIdx.x, blockIdx.x, gridDim.x, dyn, sh);
+}
+
+// A batch: the workgroups take slots from a counter, in order (batch_loop in
+// lfgpu_resident.hip says why that ends).
+template <int MODE, int RPT>
+__global__ __launch_bounds__(kThreads) void k_res_ell_batch(EllArgs base) {
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  __shared__ int slot;
+  for (;;) {
+    __syncthreads();
+    if (threadIdx.x == 0) slot = atomicAdd(base.ticket, 1);
+    __syncthreads();
+    const int k = __builtin_amdgcn_readfirstlane(slot);
+    if (k >= base.nslots) return;
+    const int2 jr = base.job_slots[k];
+    const EllJob &jb = base.jobs[jr.x];
+    EllArgs a = base;
+    a.part += jb.sums_at;
+    a.total = a.part + (size_t)2 * 2 * kSums * jb.team;
+    a.st += jb.index;
+    if (!ell_solve<MODE, RPT, true>(a, k, jr.y, jb.team, dyn, sh)) return;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -440,21 +486,24 @@ __global__ __launch_bounds__(kThreads) void k_res_ell(EllArgs a) {
 // ---------------------------------------------------------------------------
 // One workgroup per part: a bitmap of the outside columns over the window
 // that 16-bit offsets reach, its prefix sums as their places behind the own
-// rows, and every slot's place.  ext_n[g] = number of outside rows; a part
-// with more than `room` writes nothing else.
+// rows, and every slot's place.  parts[g].outside = number of outside rows; a
+// part with more than `room` writes nothing else.
 constexpr int kSplitThreads = 512;
-__global__ __launch_bounds__(kSplitThreads) void k_ell_split(
-    int32_t n, int32_t rows, const int32_t *slice_off, const int16_t *dcol, int32_t room,
-    int32_t *ext, int32_t stride, int32_t *ext_n, uint16_t *lcol, uint8_t *needed) {
+__global__ __launch_bounds__(kSplitThreads) void k_ell_split(const int32_t *slice_off,
+                                                             const int16_t *dcol, int32_t room,
+                                                             EllPart *parts, int32_t *ext,
+                                                             uint16_t *lcol, uint8_t *needed) {
   extern __shared__ uint32_t map[];
   __shared__ int32_t sums[kSplitThreads];
   const int t = threadIdx.x;
-  const int32_t g = blockIdx.x, r0 = g * rows, r1 = min(r0 + rows, n);
+  EllPart &part = parts[blockIdx.x];
+  const int32_t r0 = part.r0, r1 = part.r1, rows = part.rows;
+  int32_t *list = ext + part.at;
   const int32_t words = (rows + 65536) / 32;
   for (int32_t k = t; k < words; k += kSplitThreads) map[k] = 0;
   __syncthreads();
   for (int32_t r = r0 + t; r < r1; r += kSplitThreads) {
-    const int32_t o = slice_off[r >> 6] + (r & 63), w = (slice_off[(r >> 6) + 1] - slice_off[r >> 6]) >> 6;
+    const int32_t s = r >> 6, o = slice_off[s] + (r & 63), w = (slice_off[s + 1] - slice_off[s]) >> 6;
     for (int32_t k = 0; k < w; ++k) {
       const int32_t c = r + dcol[o + 64 * k];
       if (c < r0 || c >= r1) {
@@ -476,19 +525,19 @@ __global__ __launch_bounds__(kSplitThreads) void k_ell_split(
     if (q < t) before += sums[q];
     all += sums[q];
   }
-  if (t == 0) ext_n[g] = all;
-  if (all > room) return;
+  if (t == 0) part.outside = all;
+  if (all > room - rows) return;
   int32_t e = before;
   for (int32_t k = k0; k < k1; ++k)
     for (uint32_t m = map[k]; m; m &= m - 1) {
       const int32_t c = r0 - 32768 + 32 * k + (__ffs(m) - 1);
-      ext[(size_t)g * stride + e++] = c;
+      list[e++] = c;
       needed[c] = 1;
     }
   __syncthreads();
   const int32_t s1 = (r1 + 63) >> 6;
   for (int32_t r = r0 + t; r < s1 * 64; r += kSplitThreads) {
-    const int32_t o = slice_off[r >> 6] + (r & 63), w = (slice_off[(r >> 6) + 1] - slice_off[r >> 6]) >> 6;
+    const int32_t s = r >> 6, o = slice_off[s] + (r & 63), w = (slice_off[s + 1] - slice_off[s]) >> 6;
     for (int32_t k = 0; k < w; ++k) {
       int32_t at = 0;  // (lanes past the last row)
       if (r < r1) {
@@ -498,7 +547,6 @@ __global__ __launch_bounds__(kSplitThreads) void k_ell_split(
         } else {
           // place of c among the outside rows: binary search in the list
           int32_t lo = 0, hi = all - 1;
-          const int32_t *list = ext + (size_t)g * stride;
           while (lo < hi) {
             const int32_t m = (lo + hi) >> 1;
             if (list[m] < c) lo = m + 1;
@@ -526,75 +574,96 @@ const std::vector<EllVariant> kEllVariants = {LFG_ELL(1, true),  LFG_ELL(2, true
                                               LFG_ELL(15, false), LFG_ELL(19, false)};
 #undef LFG_ELL
 
-int ell_split(hipStream_t s, ResidentEllPlan *p, const ResidentEll &A, int cus) {
-  p->tried = true;
-  const size_t cap = kLdsDynamic / sizeof(double);
-  for (const EllVariant &v : kEllVariants) {
-    const int64_t most = (int64_t)v.rpt * kThreads;
-    const int64_t want = std::min<int64_t>((A.n + most - 1) / most, 0x7fffffff);
-    if (want > cus) continue;
-    const int32_t rows = (int32_t)(((A.n + want - 1) / want + 63) / 64 * 64);
-    const int team = (int)((A.n + rows - 1) / rows);
-    const int32_t room = (int32_t)std::min<int64_t>((int64_t)cap, 65536) - rows;
-    if (room < 1) continue;
-    if (!p->lcol) {
-      LFG_TRY(dalloc(&p->lcol, (size_t)std::max<int64_t>(A.slots, 1), "resident ELL places"));
-      LFG_TRY(dalloc(&p->needed, (size_t)A.n, "resident ELL flags"));
-      LFG_TRY(dalloc(&p->ext_n, (size_t)cus, "resident ELL counts"));
-    }
-    dfree(p->ext);
-    p->ext = nullptr;
-    LFG_TRY(dalloc(&p->ext, (size_t)team * room, "resident ELL outside rows"));
-    LFG_HIP(hipMemsetAsync(p->needed, 0, (size_t)A.n, s));
-    const size_t map = (size_t)(rows + 65536) / 32 * 4;
-    hipLaunchKernelGGL(k_ell_split, dim3(team), dim3(kSplitThreads), map, s, A.n, rows,
-                       A.slice_off, A.dcol, room, p->ext, room, p->ext_n, p->lcol, p->needed);
-    LFG_HIP(hipGetLastError());
-    std::vector<int32_t> h(team);
-    LFG_HIP(hipMemcpyAsync(h.data(), p->ext_n, (size_t)team * 4, hipMemcpyDeviceToHost, s));
-    LFG_HIP(hipStreamSynchronize(s));
-    const int32_t big = *std::max_element(h.begin(), h.end());
-    if (big > room) continue;
-    p->team = team;
-    p->rpt = v.rpt;
-    p->rows = rows;
-    p->most = big;
-    p->stride = room;
-    break;
-  }
-  return LFGPU_OK;
-}
+const void *const kEllBatch[2][3] = {
+    {reinterpret_cast<const void *>(&k_res_ell_batch<LFGPU_PCG_FP64, 2>),
+     reinterpret_cast<const void *>(&k_res_ell_batch<LFGPU_PCG_MIXED, 2>),
+     reinterpret_cast<const void *>(&k_res_ell_batch<LFGPU_PCG_MIXED_MATRIX, 2>)},
+    {reinterpret_cast<const void *>(&k_res_ell_batch<LFGPU_PCG_FP64, 8>),
+     reinterpret_cast<const void *>(&k_res_ell_batch<LFGPU_PCG_MIXED, 8>),
+     reinterpret_cast<const void *>(&k_res_ell_batch<LFGPU_PCG_MIXED_MATRIX, 8>)}};
 
 }  // namespace
 
 namespace lfgpu {
+struct ResidentEllPlan {
+  int rpt = 0, nparts = 0;  // rpt 0: does not fit
+  int32_t most = 0;         // most places (own and outside rows) of a workgroup
+  EllPart *parts = nullptr;
+  int32_t *ext = nullptr;     // the outside rows of every part, ascending
+  uint16_t *lcol = nullptr;   // per slot: the column's place in the workgroup's LDS
+  uint8_t *needed = nullptr;  // per row: some other workgroup reads it
+  // batches
+  EllJob *jobs = nullptr;
+  int2 *slots = nullptr;
+  word_t *sums = nullptr;
+  size_t sums_words = 0;
+  int *ticket = nullptr;  // followed by the abort flag
+};
 
 void resident_ell_free(ResidentEllPlan *p) {
+  if (!p) return;
+  dfree(p->parts);
   dfree(p->ext);
-  dfree(p->ext_n);
   dfree(p->lcol);
   dfree(p->needed);
-  *p = ResidentEllPlan{};
+  dfree(p->jobs);
+  dfree(p->slots);
+  dfree(p->sums);
+  dfree(p->ticket);
+  delete p;
+}
+bool resident_ell_fits(const ResidentEllPlan *p) { return p && p->rpt > 0; }
+}  // namespace lfgpu
+
+namespace {
+
+// Splits the storage into the given parts (r0, r1, rows filled in); *fits
+// tells whether every part's places fit the LDS.
+int ell_split(hipStream_t s, ResidentEllPlan *p, const ResidentEll &A, std::vector<EllPart> &parts,
+              bool *fits) {
+  const int32_t room = (int32_t)std::min<size_t>(kLdsDynamic / sizeof(double), 65536);
+  *fits = false;
+  int64_t at = 0;
+  int32_t rows = 0;
+  for (EllPart &q : parts) {
+    if (q.rows >= room) return LFGPU_OK;
+    q.at = at;
+    at += room - q.rows;
+    rows = std::max(rows, q.rows);
+  }
+  if (!p->lcol) {
+    LFG_TRY(dalloc(&p->lcol, (size_t)std::max<int64_t>(A.slots, 1), "resident ELL places"));
+    LFG_TRY(dalloc(&p->needed, (size_t)A.n, "resident ELL flags"));
+  }
+  dfree(p->ext);
+  dfree(p->parts);
+  p->ext = nullptr;
+  p->parts = nullptr;
+  LFG_TRY(dalloc(&p->ext, (size_t)at, "resident ELL outside rows"));
+  LFG_TRY(dalloc(&p->parts, parts.size(), "resident ELL parts"));
+  LFG_HIP(hipMemcpyAsync(p->parts, parts.data(), parts.size() * sizeof(EllPart),
+                         hipMemcpyHostToDevice, s));
+  LFG_HIP(hipMemsetAsync(p->needed, 0, (size_t)A.n, s));
+  const size_t map = (size_t)(rows + 65536) / 32 * 4;
+  hipLaunchKernelGGL(k_ell_split, dim3((unsigned)parts.size()), dim3(kSplitThreads), map, s,
+                     A.slice_off, A.dcol, room, p->parts, p->ext, p->lcol, p->needed);
+  LFG_HIP(hipGetLastError());
+  LFG_HIP(hipMemcpyAsync(parts.data(), p->parts, parts.size() * sizeof(EllPart),
+                         hipMemcpyDeviceToHost, s));
+  LFG_HIP(hipStreamSynchronize(s));
+  p->most = 0;
+  for (const EllPart &q : parts) {
+    if (q.outside > room - q.rows) return LFGPU_OK;
+    p->most = std::max(p->most, q.rows + q.outside);
+  }
+  p->nparts = (int)parts.size();
+  *fits = true;
+  return LFGPU_OK;
 }
 
-int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *plan,
-                     const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b, double *x,
-                     ResidentState *st, bool *taken) {
-  *taken = false;
-  if (A.n <= 0 || !A.dcol) return LFGPU_OK;
-  hipStream_t s = ctx->stream;
-  if (!plan->tried) LFG_TRY(ell_split(s, plan, A, std::min(ctx->cus, kMaxTeam)));
-  if (plan->team == 0) return LFGPU_OK;
-  const EllVariant *v = nullptr;
-  for (const EllVariant &k : kEllVariants)
-    if (k.rpt == plan->rpt) v = &k;
-  EllArgs a{};
-  LFG_TRY(resident_prepare(s, bufs, (size_t)4 * A.n,
-                           (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 5) + 16,
-                           &a.tag0));
+void fill_args(EllArgs &a, const ResidentEllPlan *plan, const ResidentEll &A,
+               const lfgpu_pcg_opts &opts, const double *b, double *x) {
   a.n = A.n;
-  a.rows = plan->rows;
-  a.nslices = A.nslices;
   a.slice_off = A.slice_off;
   a.lcol = plan->lcol;
   a.val = A.val;
@@ -605,24 +674,171 @@ int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *plan,
   a.dinv32 = A.dinv32;
   a.dinv16 = static_cast<const __hip_bfloat16 *>(A.dinv16);
   a.perm = A.perm;
+  a.parts = plan->parts;
   a.ext = plan->ext;
-  a.ext_n = plan->ext_n;
-  a.stride = plan->stride;
   a.needed = plan->needed;
   a.b = b;
   a.x = x;
   a.xlo = A.xlo;
-  a.words = bufs->halo;
-  a.part = bufs->sums;
-  a.total = bufs->sums + kPartWords;
-  a.abort = bufs->abort;
   a.tol2 = opts.rtol * opts.rtol;
   a.maxit = opts.maxit;
   a.delta2 = opts.refine_delta > 0.0 ? opts.refine_delta * opts.refine_delta : 0.09;
   a.max_interval = opts.refine_max_interval > 0 ? opts.refine_max_interval : 2147483647;
+}
+
+// tags of a solve: one exchange and one sum an iteration, four for a
+// reliable update (at most one an iteration), and a few at the start
+uint64_t ell_tags(const lfgpu_pcg_opts &opts) {
+  return (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 5) + 16;
+}
+
+}  // namespace
+
+namespace lfgpu {
+
+int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan,
+                     const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b, double *x,
+                     ResidentState *st, bool *taken) {
+  *taken = false;
+  if (A.n <= 0 || !A.dcol) return LFGPU_OK;
+  hipStream_t s = ctx->stream;
+  const int cus = std::min(ctx->cus, kMaxTeam);
+  if (!*pplan) {
+    ResidentEllPlan *p = *pplan = new ResidentEllPlan();
+    for (const EllVariant &v : kEllVariants) {
+      const int64_t want = (A.n + (int64_t)v.rpt * kThreads - 1) / ((int64_t)v.rpt * kThreads);
+      if (want > cus) continue;
+      const int32_t rows = (int32_t)(((A.n + want - 1) / want + 63) / 64 * 64);
+      std::vector<EllPart> parts((A.n + rows - 1) / rows);
+      for (size_t g = 0; g < parts.size(); ++g)
+        parts[g] = EllPart{(int32_t)g * rows, std::min((int32_t)(g + 1) * rows, A.n), rows, 0, 0};
+      bool fits = false;
+      LFG_TRY(ell_split(s, p, A, parts, &fits));
+      if (!fits) continue;
+      p->rpt = v.rpt;
+      break;
+    }
+  }
+  const ResidentEllPlan *plan = *pplan;
+  if (plan->rpt == 0) return LFGPU_OK;
+  const EllVariant *v = nullptr;
+  for (const EllVariant &k : kEllVariants)
+    if (k.rpt == plan->rpt) v = &k;
+  EllArgs a{};
+  LFG_TRY(resident_prepare(s, bufs, (size_t)4 * A.n, ell_tags(opts), &a.tag0));
+  fill_args(a, plan, A, opts, b, x);
+  a.words = bufs->halo;
+  a.part = bufs->sums;
+  a.total = bufs->sums + kPartWords;
+  a.abort = bufs->abort;
   a.st = bufs->state;
-  const size_t lds = ((size_t)plan->rows + plan->most) * sizeof(double);
-  return resident_launch(s, bufs, v->fn[opts.mode], plan->team, &a, lds, st, taken);
+  return resident_launch(s, bufs, v->fn[opts.mode], plan->nparts, &a,
+                         (size_t)plan->most * sizeof(double), st, taken);
+}
+
+// Team sizes as for the lattice problems (resident_tiles_plan): an iteration
+// takes about 6 us and 0.3 ns a slot of a workgroup's rows.
+int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
+                            const std::vector<ResidentProblem> &probs, ResidentEllPlan **out) {
+  ResidentEllPlan *p = *out = new ResidentEllPlan();
+  hipStream_t s = ctx->stream;
+  const int cus = std::min(ctx->cus, kMaxTeam);
+  const size_t np = probs.size();
+  if (np == 0 || !A.dcol) return LFGPU_OK;
+  const int32_t cap = 8 * kThreads;
+  const double row_us = 0.0003 * (double)A.slots / std::max(A.n, 1);
+  auto iterations = [&](const ResidentProblem &q) { return std::sqrt((double)q.n); };
+  std::vector<int32_t> rows(np);
+  auto total = [&](double tau) {
+    int64_t sum = 0;
+    for (size_t k = 0; k < np; ++k) {
+      const double c = tau > 0.0 ? (tau / iterations(probs[k]) - 6.0) / row_us : (double)cap;
+      const int32_t want = (int32_t)std::min<double>((double)cap, std::max(c, 64.0));
+      const int32_t n = (probs[k].n + 63) / 64 * 64;
+      // evenly over the team, whole slices, at most kMaxTeam members
+      const int32_t team = std::min((n + want - 1) / want, cus);
+      rows[k] = ((n + team - 1) / team + 63) / 64 * 64;
+      if (rows[k] > cap) return (int64_t)-1;
+      sum += (n + rows[k] - 1) / rows[k];
+    }
+    return sum;
+  };
+  const int64_t all = total(0.0);
+  if (all < 0) return LFGPU_OK;
+  if (all <= cus) {
+    double lo = 0.0, hi = 0.0;
+    for (const ResidentProblem &q : probs)
+      hi = std::max(hi, iterations(q) * (6.0 + row_us * cap));
+    for (int step = 0; step < 12; ++step) {
+      const double mid = 0.5 * (lo + hi);
+      const int64_t n = total(mid);
+      if (n >= 0 && n <= cus) hi = mid;
+      else lo = mid;
+    }
+    (void)total(hi);
+  }
+  std::vector<size_t> order(np);
+  for (size_t k = 0; k < np; ++k) order[k] = k;
+  auto cost = [&](size_t k) { return iterations(probs[k]) * (6.0 + row_us * rows[k]); };
+  std::stable_sort(order.begin(), order.end(),
+                   [&](size_t i, size_t j) { return cost(i) > cost(j); });
+  std::vector<EllJob> jobs(np);
+  std::vector<EllPart> parts;
+  std::vector<int2> slots;
+  int32_t most = 0;
+  for (size_t o = 0; o < np; ++o) {
+    const ResidentProblem &q = probs[order[o]];
+    const int32_t R = rows[order[o]], end = q.lo + (q.n + 63) / 64 * 64;
+    EllJob &j = jobs[o];
+    j.index = q.index;
+    j.team = (end - q.lo + R - 1) / R;
+    j.sums_at = (uint32_t)p->sums_words;
+    p->sums_words += (size_t)2 * 2 * kSums * j.team + kTotalWords;
+    most = std::max(most, R);
+    for (int r = 0; r < j.team; ++r) {
+      parts.push_back(EllPart{q.lo + r * R, std::min(q.lo + (r + 1) * R, end), R, 0, 0});
+      slots.push_back(int2{(int)o, r});
+    }
+  }
+  bool fits = false;
+  LFG_TRY(ell_split(s, p, A, parts, &fits));
+  if (!fits) return LFGPU_OK;
+  LFG_TRY(dalloc(&p->jobs, np, "resident batch jobs"));
+  LFG_TRY(dalloc(&p->slots, slots.size(), "resident batch slots"));
+  LFG_TRY(dalloc(&p->sums, p->sums_words, "resident batch sums"));
+  LFG_TRY(dalloc(&p->ticket, 4, "resident batch counter"));
+  LFG_HIP(hipMemcpyAsync(p->jobs, jobs.data(), np * sizeof(EllJob), hipMemcpyHostToDevice, s));
+  LFG_HIP(hipMemcpyAsync(p->slots, slots.data(), slots.size() * sizeof(int2),
+                         hipMemcpyHostToDevice, s));
+  LFG_HIP(hipStreamSynchronize(s));
+  p->rpt = most <= 2 * kThreads ? 2 : 8;
+  return LFGPU_OK;
+}
+
+int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *plan,
+                           const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b,
+                           double *x, ResidentState *st, bool *taken) {
+  *taken = false;
+  hipStream_t s = ctx->stream;
+  EllArgs a{};
+  // (the problems' sums have their own words; they are cleared with the rest)
+  const bool fresh = resident_will_clear(bufs, (size_t)4 * A.n, ell_tags(opts));
+  LFG_TRY(resident_prepare(s, bufs, (size_t)4 * A.n, ell_tags(opts), &a.tag0));
+  if (fresh) LFG_TRY(resident_clear(s, plan->sums, plan->sums_words));
+  // the counter and the abort flag
+  LFG_TRY(resident_clear(s, reinterpret_cast<unsigned long long *>(plan->ticket), 2));
+  fill_args(a, plan, A, opts, b, x);
+  a.words = bufs->halo;
+  a.part = plan->sums;
+  a.abort = plan->ticket + 2;
+  a.st = st;
+  a.jobs = plan->jobs;
+  a.job_slots = plan->slots;
+  a.nslots = plan->nparts;
+  a.ticket = plan->ticket;
+  return resident_launch_team(s, kEllBatch[plan->rpt == 2 ? 0 : 1][opts.mode],
+                              std::min(plan->nparts, std::min(ctx->cus, kMaxTeam)), &a,
+                              (size_t)plan->most * sizeof(double), taken);
 }
 
 }  // namespace lfgpu

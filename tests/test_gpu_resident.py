@@ -48,6 +48,26 @@ def _lattice_system(S, L, steps, seed, symmetric=True):
     return np.concatenate(rows), np.concatenate(cols), np.concatenate(vals), n
 
 
+def _flipped_system(S, L, seed):
+    """_lattice_system with half of the squares cut along the other diagonal."""
+    r, c, v, n = _lattice_system(S, L, ((1, 0), (0, 1), (1, 1)), seed)
+    rng = np.random.default_rng(seed + 1)
+    d = np.nonzero(c - r == S + 1)[0]
+    d = d[rng.random(d.size) < 0.5]
+    back = np.nonzero(r - c == S + 1)[0]
+    pos = np.zeros(n, np.int64)
+    pos[c[back]] = back  # the entry (i + S + 1, i) by i
+    r2, c2 = r.copy(), c.copy()
+    r2[d], c2[d] = r[d] + 1, c[d] - 1
+    r2[pos[r[d]]], c2[pos[r[d]]] = c[d] - 1, r[d] + 1
+    diag = np.full(n, 1e-3)  # (row sums move with the couplings)
+    off = r2 != c2
+    np.subtract.at(diag, r2[off], v[off])
+    v2 = v.copy()
+    v2[~off] = diag[r2[~off]]
+    return r2, c2, v2, n
+
+
 def _compare(ctx, A, n, mode, seed, x0=None, maxit=20000, rtol=1e-10):
     bh = np.random.default_rng(seed).standard_normal(n)
     b, bn = capi.Vec(ctx, bh), np.linalg.norm(bh)
@@ -136,23 +156,7 @@ def test_resident_pcg_is_deterministic_and_zero_rhs(ctx, mode):
                                   (512, 513), (800, 801), (1025, 1024), (1150, 1151)])
 @pytest.mark.parametrize("mode", MODES)
 def test_resident_pcg_on_ell(ctx, S, L, mode):
-    r, c, v, n = _lattice_system(S, L, P1, S)
-    # half of the diagonal couplings move to the square's other diagonal
-    rng = np.random.default_rng(L)
-    d = np.nonzero(c - r == S + 1)[0]
-    d = d[rng.random(d.size) < 0.5]
-    back = np.nonzero(r - c == S + 1)[0]
-    pos = np.zeros(n, np.int64)
-    pos[c[back]] = back  # (c + S + 1, c) by its column
-    r2, c2 = r.copy(), c.copy()
-    r2[d], c2[d] = r[d] + 1, c[d] - 1
-    r2[pos[r[d]]], c2[pos[r[d]]] = c[d] - 1, r[d] + 1
-    # (row sums move with the couplings: keep the matrix a Laplacian + 1e-3)
-    diag = np.full(n, 1e-3)
-    off = r2 != c2
-    np.subtract.at(diag, r2[off], v[off])
-    v2 = v.copy()
-    v2[~off] = diag[r2[~off]]
+    r2, c2, v2, n = _flipped_system(S, L, S)
     A = capi.coo_to_csr(ctx, r2, c2, v2, n, n)
     out = _compare(ctx, A, n, mode, n + 1)
     assert capi.solver_storage(A)[0] == capi.STORAGE_ELL16
@@ -178,3 +182,46 @@ def test_wrapped_band_matrix_keeps_the_sweeps(ctx):
     out = _compare(ctx, A, n, capi.PCG_FP64, 1)
     assert np.array_equal(out[0][1], out[1][1])  # graph replay against plain launches
     A.close()
+
+
+# more teams than the chip holds at once, 5 x 5 to 90 x 90 problems and in FP64
+# single rows (on which the reliable updates fail: the one step exhausts the
+# Krylov space, and the old direction that they keep is no longer conjugate);
+# all lattices, none, and both (which take a launch each)
+@pytest.mark.parametrize("kind", ["lattice", "flipped", "both"])
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_batch(ctx, kind, mode):
+    rng = np.random.default_rng(17)
+    parts, off = [], [0]
+    for k in range(300):
+        S, L = (int(q) for q in rng.integers(5, 60 if k else 91, 2))
+        if k % 50 == 7 and mode == capi.PCG_FP64:
+            r, c, v, n = np.array([0]), np.array([0]), np.array([2.0]), 1
+        elif kind == "lattice" or (kind == "both" and k % 3):
+            r, c, v, n = _lattice_system(S, L, P1, k)
+        else:
+            r, c, v, n = _flipped_system(S, L, k)
+        parts.append((r + off[-1], c + off[-1], v))
+        off.append(off[-1] + n)
+    n = off[-1]
+    A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n, n)
+    bh = rng.standard_normal(n)
+    bh[off[3]:off[4]] = 0.0  # a zero right-hand side
+    b = capi.Vec(ctx, bh)
+    batch = capi.Batch(ctx, A, np.array(off, np.int32))
+    out = []
+    for graph in (1, 0, 0):
+        x = capi.Vec(ctx, np.ones(n))
+        summ, infos = batch.pcg(b, x, rtol=1e-10, maxit=20000, mode=mode, graph=graph)
+        out.append((summ, infos, x.numpy()))
+        x.close()
+    assert all(s.converged for s, _, _ in out)
+    assert out[1][0].syncs == 1  # the resident solve ran
+    assert np.array_equal(out[1][2], out[2][2])
+    assert out[1][1][3].iters == 0 and not out[1][2][off[3]:off[4]].any()
+    for k in range(300):
+        xa, xb = (o[2][off[k]:off[k + 1]] for o in out[:2])
+        bound = 2.2e-10 * np.linalg.norm(bh[off[k]:off[k + 1]]) / 1e-3
+        assert np.linalg.norm(xa - xb) <= bound, k
+    for h in (batch, b, A):
+        h.close()
