@@ -10,9 +10,9 @@
 // above, the matrix is streamed once an iteration.  Time per iteration, P1,
 // sweeps against this, in us:
 //              64^2   512^2   1023x770   1024^2   2048x256   1400^2   2048^2
-//   FP64     12.6/2.9 17.6/4.9 29.8/6.2 32.0/8.2  20.8/5.6 55.1/21.3  101/44
-//   FP32     15.2/4.0 14.4/5.4 19.6/6.7 21.8/7.3  17.0/6.0 31.6/15.1 57.6/33
-//   FP32 mat 17.4/4.4 16.7/5.4 24.3/6.6 30.5/7.2  21.1/6.0 46.6/14.8 85.3/49
+//   FP64     12.6/2.4 17.6/3.4 29.8/4.8 32.0/6.3  20.8/4.0 55.1/20.0  101/43
+//   FP32     15.2/3.5 14.4/4.1 19.6/5.3 21.8/6.1  17.0/4.7 31.6/13.9 57.6/28
+//   FP32 mat 17.4/3.8 16.7/4.2 24.3/5.4 30.5/6.4  21.1/4.7 46.6/13.6 85.3/49
 //
 // One iteration (the recurrences and the stopping test of the two-sweep
 // solver, with one team sum instead of two):
@@ -264,13 +264,6 @@ struct Tile {
 //     every iteration, the next row's loads in flight while a row is worked
 //     on; p travels between the update and the next product.
 enum { GHOST, STREAM };
-
-// The threads that carry the exchange of q while the others wait for the
-// team sum: all but the first wavefront, or but the four that sum the
-// members' partials.
-__device__ __forceinline__ int exchange_threads(const Team &tm) {
-  return sums_members(tm) ? kMaxTeam : 64;
-}
 
 // From this many cells a thread the GHOST variants keep row sums and D^-1 in
 // LDS (9 cells' r, q, x and six diagonals take 162 of the 256 registers; with
@@ -541,7 +534,7 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
     if constexpr (kGhost) ++T.tag;
     ok = team_sum(tm, sh, s, [&] {
       if constexpr (kGhost) {
-        const int first = exchange_threads(tm);
+        const int first = sums_threads(tm);
         T.template publish<double>(M.lq, first);
         T.template fetch<double>(first, &sh.bad,
                                  [&](int32_t h, int32_t, double qv) { M.gq[h] = qv; });
@@ -682,7 +675,7 @@ __device__ __forceinline__ void batch_loop(const TileArgs &base, F &&solve) {
     a.xlo += jb.lo;
     a.halo_words += jb.halo_at;
     a.part += jb.sums_at;
-    a.total = a.part + (size_t)2 * 2 * kSums * jb.team;
+    a.total = a.part + part_words(jb.team);
     a.st += jb.index;
     if (!solve(a, jr.y, jb.team)) return;
   }
@@ -858,7 +851,7 @@ __device__ __forceinline__ bool tile_solve_mixed(const TileArgs &a, int rank, in
       if constexpr (kGhost) ++T.tag;
       ok = team_sum(tm, sh, s, [&] {
         if constexpr (kGhost) {
-          const int from = exchange_threads(tm);
+          const int from = sums_threads(tm);
           T.template publish<VT>(M.lq, from);
           T.template fetch<VT>(from, &sh.bad, [&](int32_t h, int32_t, VT qv) { M.gq[h] = qv; });
         }
@@ -1177,7 +1170,8 @@ const TileVariant *tile_plan(TileArgs &a, int mode, bool sym, int cus, int *team
   return nullptr;
 }
 
-// Batches: up to 3 and up to 7 (FP64 vectors) or 9 cells a thread.
+// Batches: up to 3 and up to 7 cells a thread (with 9 FP32 cells 55 registers
+// spill and 64 problems of 32 to 512 lines take 59 ms instead of 46).
 struct BatchVariant {
   int rpt;
   size_t (*lds)(const TileArgs &);
@@ -1187,7 +1181,7 @@ const BatchVariant kBatchVariants[3][2] = {
     {{3, &TileLds<GHOST, double, 3>::bytes, &k_res_tile_batch<3>},
      {7, &TileLds<GHOST, double, 7>::bytes, &k_res_tile_batch<7>}},
     {{3, &TileLds<GHOST, float, 3>::bytes, &k_res_tile_mixed_batch<float, 3>},
-     {9, &TileLds<GHOST, float, 9>::bytes, &k_res_tile_mixed_batch<float, 9>}},
+     {7, &TileLds<GHOST, float, 7>::bytes, &k_res_tile_mixed_batch<float, 7>}},
     {{3, &TileLds<GHOST, double, 3>::bytes, &k_res_tile_mixed_batch<double, 3>},
      {7, &TileLds<GHOST, double, 7>::bytes, &k_res_tile_mixed_batch<double, 7>}},
 };
@@ -1350,7 +1344,7 @@ void resident_tiles_free(ResidentTiles *p) {
 
 // Team sizes: the problems run side by side, so that the batch takes as long
 // as its longest problem while all teams fit the chip; iterations grow with
-// the square root of the rows, an iteration takes about 4.5 us and 0.8 ns a
+// the square root of the rows, an iteration takes about 2.5 us and 0.8 ns a
 // cell of a workgroup.  The cells a workgroup takes follow from the smallest
 // common finishing time with which the teams fit; where none does, every
 // workgroup takes as many as it can hold and the longest problems go first.
@@ -1376,7 +1370,7 @@ int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &prob
   auto total = [&](double tau) {
     int64_t sum = 0;
     for (size_t k = 0; k < np; ++k) {
-      const double c = tau > 0.0 ? (tau / iterations(probs[k]) - 4.5) / 0.0008 : (double)cap;
+      const double c = tau > 0.0 ? (tau / iterations(probs[k]) - 2.5) / 0.0008 : (double)cap;
       const int64_t cells = (int64_t)std::min<double>((double)cap, std::max(c, 128.0));
       team[k] = split(probs[k], cells, geo[k]);
       if (team[k] == 0) team[k] = split(probs[k], cap, geo[k]);
@@ -1390,7 +1384,7 @@ int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &prob
   if (all <= cus) {
     double hi = 0.0;
     for (const ResidentProblem &q : probs)
-      hi = std::max(hi, iterations(q) * (4.5 + 0.0008 * (double)cap));
+      hi = std::max(hi, iterations(q) * (2.5 + 0.0008 * (double)cap));
     double lo = 0.0;
     for (int step = 0; step < 10; ++step) {
       const double mid = 0.5 * (lo + hi);
@@ -1402,7 +1396,7 @@ int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &prob
   std::vector<size_t> order(np);
   for (size_t k = 0; k < np; ++k) order[k] = k;
   auto cost = [&](size_t k) {
-    return iterations(probs[k]) * (4.5 + 0.0008 * (geo[k].TW + 2) * geo[k].TH);
+    return iterations(probs[k]) * (2.5 + 0.0008 * (geo[k].TW + 2) * geo[k].TH);
   };
   std::stable_sort(order.begin(), order.end(),
                    [&](size_t i, size_t j) { return cost(i) > cost(j); });
@@ -1430,7 +1424,7 @@ int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &prob
     j.halo_at = (uint32_t)p->halo_words;
     j.sums_at = (uint32_t)p->sums_words;
     p->halo_words += (size_t)2 * j.team * 2 * j.slots;
-    p->sums_words += (size_t)2 * 2 * kSums * j.team + kTotalWords;
+    p->sums_words += part_words(j.team) + kTotalWords;
     most = std::max<int64_t>(most, (int64_t)(g.TW + 2) * g.TH);
     for (int r = 0; r < j.team; ++r) slots.push_back(int2{(int)o, r});
   }

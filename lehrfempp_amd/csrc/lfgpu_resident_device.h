@@ -32,10 +32,14 @@ constexpr int kWaves = kThreads / 64;
 constexpr int kMaxTeam = 256;  // workgroups of a team (one leader thread per member)
 constexpr int kSums = 5;       // values of one team sum
 // Teams of fewer workgroups read every member's partial sums in every
-// workgroup (one hop); larger ones let kLeaders workgroups sum them and
-// publish the totals (two hops).  One hop costs 2.6 us with one workgroup (to
-// memory and back, five values), 3.9 with 64, 5.0 with 128 and 6.6 with 256,
-// which poll 256 x 10 words each; the second hop costs about 1.7.
+// workgroup (one hop: 32 members a wavefront); in larger ones each of kLeaders
+// workgroups sums a group of the members and every workgroup reads the
+// leaders' sums (two hops).  A member's leader is the one of the same rank
+// modulo 8, which puts a group on one XCD when the ranks are the workgroup
+// numbers.  A sum of five values, workgroup's part included, takes 1.3 us
+// with 2 members, 1.8 with 32, 2.0 with 63, 2.3 with 64 and 2.5 with 256 (8
+// leaders that poll all 256 members, five separate wavefront sums and 40 LDS
+// reads a thread took 3.9).
 constexpr int kFlatTeam = 64;
 constexpr int kLeaders = 8;
 constexpr uint64_t kWaitTicks = 400000000ull;  // 4 s of the 100 MHz real-time clock
@@ -95,155 +99,210 @@ struct Wait {
   }
 };
 
-// One step of a wavefront sum: v + (v of the lane that CTRL names, 0 where
-// there is none or ROWS masks the row out).
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_add(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, ROWS, 0xf, false);
-  return v + __hiloint2double(hi, lo);
+// Lane l's 32 bits from the lane that the DPP control CTRL names.
+template <int CTRL>
+__device__ __forceinline__ double dpp(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, false);
+  return __hiloint2double(hi, lo);
 }
-// Sum over the wavefront, valid in lane 63 (row shifts by 1, 2, 4, 8, then
-// the row broadcasts; a fixed order).  Register moves only: the shuffle form
-// goes through LDS and costs about 0.3 us for five values.
-__device__ __forceinline__ double wave_sum63(double v) {
-  v = dpp_add<0x111, 0xf>(v);
-  v = dpp_add<0x112, 0xf>(v);
-  v = dpp_add<0x114, 0xf>(v);
-  v = dpp_add<0x118, 0xf>(v);
-  v = dpp_add<0x142, 0xa>(v);
-  v = dpp_add<0x143, 0xc>(v);
-  return v;
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppRor8 = 0x128;
+
+// a summed over lane pairs (l, l + 32) in the lower half of the result, b in
+// the upper half; and the same over (l, l + 16) in the even and odd rows.
+__device__ __forceinline__ double fold32(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(a),
+                                                   (unsigned)__double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(a),
+                                                   (unsigned)__double2hiint(b), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ double fold16(double a, double b) {
+  const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(a),
+                                                   (unsigned)__double2loint(b), false, false);
+  const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(a),
+                                                   (unsigned)__double2hiint(b), false, false);
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// Up to five values summed over the wavefront in a fixed order, the values
+// folded into one register on the way (35 instructions; five separate DPP
+// sums take 90).  PAIRS: both lanes of a pair (2i, 2i + 1) hold the same, one
+// of them counts.  The result of value wave_value(l) is in lane l; every
+// value is in the two lanes of which wave_owner(l) >= 0 (0 and 1).
+template <bool PAIRS, int K>
+__device__ __forceinline__ double wave_sums(const double (&v)[K]) {
+  static_assert(K <= kSums, "too many sums");
+  auto val = [&](int k) { return k < K ? v[k < K ? k : 0] : 0.0; };
+  const double a = fold32(val(0), K > 1 ? val(1) : val(0));
+  const double b = K > 2 ? fold32(val(2), K > 3 ? val(3) : val(2)) : a;
+  double d = fold16(a, b);
+  if constexpr (K > 4) {
+    double c = fold32(val(4), val(4));
+    c = fold16(c, c);
+    const bool up = (threadIdx.x & 8) != 0;
+    d = (up ? c : d) + dpp<kDppRor8>(up ? d : c);
+  } else {
+    d += dpp<kDppRor8>(d);
+  }
+  d += dpp<kDppHalfMirror>(d);
+  d += dpp<kDppXor2>(d);
+  if constexpr (!PAIRS) d += dpp<kDppXor1>(d);
+  return d;
+}
+__device__ __forceinline__ int wave_value(int l) {
+  return (l & 8) ? 4 : (l >> 4 & 1) * 2 + (l >> 5);
+}
+__device__ __forceinline__ int wave_owner(int l) {
+  return (l & 14) == 0 || (l & 62) == 8 ? l & 1 : -1;
+}
+
+// The value whose low and high words the lanes 2i and 2i + 1 hold.
+__device__ __forceinline__ double join_words(word_t w) {
+  const int mine = (int)(w >> 32);
+  const int other = __builtin_amdgcn_update_dpp(0, mine, kDppXor1, 0xf, 0xf, false);
+  return (threadIdx.x & 1) ? __hiloint2double(mine, other) : __hiloint2double(other, mine);
 }
 
 // Workgroup-shared scratch of the team sums.
 struct SumLds {
   double part[2][kWaves][kSums];
-  double lead[2][4][kSums];
-  double total[2][kSums];
+  double total[2][2][kSums];
   int bad;
 };
 
-// words of the team sums' buffers
-constexpr size_t kPartWords = (size_t)2 * 2 * kSums * kMaxTeam;
-constexpr size_t kTotalWords = (size_t)2 * kLeaders * 2 * kSums;
+// words of the team sums' buffers: a line of 16 (10 in use) per member and
+// per leader
+constexpr int kLine = 16;
+constexpr size_t part_words(int team) { return (size_t)2 * kLine * team; }
+constexpr size_t kPartWords = part_words(kMaxTeam);
+constexpr size_t kTotalWords = (size_t)2 * kLine * kLeaders;
 // LDS a resident kernel may take dynamically (beside SumLds)
 constexpr size_t kLdsDynamic = 160 * 1024 - (sizeof(SumLds) + 1023) / 1024 * 1024;
 
 // The team as one workgroup sees it.
 struct Team {
   int rank, size;
-  word_t *part;   // [2][2 kSums][size] partial sums of every member
-  word_t *total;  // [2][kLeaders][2 kSums] totals, one copy per leader
+  word_t *part;   // [2][size][kLine] partial sums of every member
+  word_t *total;  // [2][kLeaders][kLine] sums over a leader's group
   int *abort;
   uint32_t tag;   // number of the last team sum
 };
 
-// Sums v over all threads of the team; every thread of every workgroup gets
-// the same bits: wavefronts in order within a workgroup, then the members'
-// partials in a fixed tree over their ranks.  Returns false when the team has
-// been aborted (in every thread of the workgroup).  Contains workgroup
-// barriers: LDS written before the call is visible after it.  All threads run
-// `meanwhile` between the first of them, when the workgroup's partials are
-// about to go out, and the wait for the team; it must leave to itself the
-// threads that have a part in the sum: the first wavefront, and the first
-// kMaxTeam threads where sums_members() holds.
-__device__ __forceinline__ bool sums_members(const Team &tm) {
-  return tm.size < kFlatTeam || tm.rank < kLeaders;
+// The first sums_threads() threads of a workgroup carry a team sum, the
+// others are free between its barriers.
+__device__ __forceinline__ int sums_threads(const Team &tm) {
+  return tm.size > 32 && tm.size < kFlatTeam ? 128 : 64;
 }
+
+// Polls N words per lane (word u at src + u * step; lanes that are not `in`
+// count as arrived) until all of the wavefront's carry the tag.  (A second
+// poll in flight half a round trip behind gains 1 %.)
+template <int N>
+__device__ __forceinline__ bool poll_words(const word_t *src, int step, bool in, uint32_t tag,
+                                           int *abort, word_t (&a)[N]) {
+  Wait wait(abort);
+  for (;;) {
+#pragma unroll
+    for (int u = 0; u < N; ++u) a[u] = get(src + u * step);
+    bool ok = true;
+#pragma unroll
+    for (int u = 0; u < N; ++u) ok = ok && tagged(a[u], tag);
+    if (__all(ok || !in)) return true;
+    if (!wait.more()) return false;
+  }
+}
+
+// Sums v over all threads of the team; every thread of every workgroup gets
+// the same bits: every step adds in a fixed order.  Returns false when the
+// team has been aborted (in every thread of the workgroup).  Contains
+// workgroup barriers: LDS written before the call is visible after it.  All
+// threads run `meanwhile` between the first of them, when the workgroup's
+// partials are about to go out, and the wait for the team; it must leave the
+// first sums_threads() threads to themselves.
 template <int K, class F>
 __device__ __forceinline__ bool team_sum(Team &tm, SumLds &sh, double (&v)[K], F &&meanwhile) {
-  static_assert(K <= kSums, "too many sums");
   const int t = threadIdx.x, w = t >> 6, l = t & 63;
   const uint32_t tag = ++tm.tag;
   const int par = (int)(tag & 1u);
-#pragma unroll
-  for (int k = 0; k < K; ++k) v[k] = wave_sum63(v[k]);
-  if (l == 63)
-#pragma unroll
-    for (int k = 0; k < K; ++k) sh.part[par][w][k] = v[k];
+  {
+    const double s = wave_sums<false>(v);
+    if (wave_owner(l) == 0 && wave_value(l) < K) sh.part[par][w][wave_value(l)] = s;
+  }
   __syncthreads();
+  // the workgroup's sums: waves in a fixed tree
+  auto group = [&](int k) {
+    const double(*p)[kSums] = sh.part[par];
+    return ((p[0][k] + p[1][k]) + (p[2][k] + p[3][k])) +
+           ((p[4][k] + p[5][k]) + (p[6][k] + p[7][k]));
+  };
   if (tm.size == 1) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      double s = sh.part[par][0][k];
-#pragma unroll
-      for (int q = 1; q < kWaves; ++q) s += sh.part[par][q][k];
-      v[k] = s;
-    }
+    for (int k = 0; k < K; ++k) v[k] = group(k);
     return true;
   }
-  word_t *pb = tm.part + (size_t)par * 2 * kSums * tm.size;
+  word_t *pb = tm.part + (size_t)par * kLine * tm.size;
   if (t < 2 * K) {
-    const int k = t >> 1;
-    double s = sh.part[par][0][k];
-#pragma unroll
-    for (int q = 1; q < kWaves; ++q) s += sh.part[par][q][k];
-    put(&pb[(size_t)t * tm.size + tm.rank], (t & 1) ? high_word(s, tag) : low_word(s, tag));
+    const double s = group(t >> 1);
+    put(&pb[tm.rank * kLine + t], (t & 1) ? high_word(s, tag) : low_word(s, tag));
   }
   meanwhile();
   const bool flat = tm.size < kFlatTeam;
-  if (sums_members(tm)) {
-    if (t < kMaxTeam) {
-      double r[K];
+  // sums over a group of up to 32 members: lane 2i + h holds word h of member i
+  auto members = [&](int first, int stride, int count) {
+    word_t a[K];
+    const int i = l >> 1;
+    const bool in = i < count;
+    const word_t *src = pb + (in ? first + i * stride : first) * kLine + (l & 1);
+    if (!poll_words(src, 2, in, tag, tm.abort, a)) sh.bad = 1;
+    double r[K];
 #pragma unroll
-      for (int k = 0; k < K; ++k) r[k] = 0.0;
-      if (t < tm.size) {
-        word_t a[2 * K];
-        Wait wait(tm.abort);
-        bool ok;
-        do {
-          ok = true;
-#pragma unroll
-          for (int k = 0; k < 2 * K; ++k) a[k] = get(&pb[(size_t)k * tm.size + t]);
-#pragma unroll
-          for (int k = 0; k < 2 * K; ++k) ok = ok && tagged(a[k], tag);
-        } while (!ok && wait.more());
-        if (!ok) sh.bad = 1;
-#pragma unroll
-        for (int k = 0; k < K; ++k) r[k] = from_words(a[2 * k], a[2 * k + 1]);
-      }
-#pragma unroll
-      for (int k = 0; k < K; ++k) r[k] = wave_sum63(r[k]);
-      if (l == 63)
-#pragma unroll
-        for (int k = 0; k < K; ++k) sh.lead[par][w][k] = r[k];
+    for (int k = 0; k < K; ++k) {
+      r[k] = join_words(a[k]);
+      r[k] = in ? r[k] : 0.0;
+    }
+    return wave_sums<true>(r);
+  };
+  const int k = wave_value(l);
+  if (flat) {
+    if (w < 2 && w * 32 < tm.size) {
+      const double s = members(w * 32, 1, tm.size - w * 32);
+      if (wave_owner(l) == 0 && k < K) sh.total[par][w][k] = s;
     }
     __syncthreads();
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      double s = sh.lead[par][0][k];
+    for (int q = 0; q < K; ++q) v[q] = sh.total[par][0][q];
+    if (tm.size > 32)
 #pragma unroll
-      for (int q = 1; q < kMaxTeam / 64; ++q) s += sh.lead[par][q][k];
-      v[k] = s;
-    }
-    if (!flat && t < 2 * K) {
-      double s = v[0];
-#pragma unroll
-      for (int k = 1; k < K; ++k)
-        if ((t >> 1) == k) s = v[k];
-      put(&tm.total[((size_t)par * kLeaders + tm.rank) * 2 * kSums + t],
-          (t & 1) ? high_word(s, tag) : low_word(s, tag));
-    }
+      for (int q = 0; q < K; ++q) v[q] += sh.total[par][1][q];
     return sh.bad == 0;
   }
-  if (t < 2 * K) {
-    const word_t *src =
-        &tm.total[((size_t)par * kLeaders + (tm.rank & (kLeaders - 1))) * 2 * kSums + t];
-    word_t a;
-    Wait wait(tm.abort);
-    bool ok;
-    do {
-      a = get(src);
-      ok = tagged(a, tag);
-    } while (!ok && wait.more());
-    if (!ok) sh.bad = 1;
-    // the payload halves of one value sit in neighbouring lanes
-    reinterpret_cast<uint32_t *>(&sh.total[par][0])[t] = (uint32_t)(a >> 32);
+  if (w == 0) {
+    word_t *tb = tm.total + (size_t)par * kLine * kLeaders;
+    if (tm.rank < kLeaders) {
+      const double s =
+          members(tm.rank, kLeaders, (tm.size - tm.rank + kLeaders - 1) / kLeaders);
+      const int h = wave_owner(l);
+      if (h >= 0 && k < K)
+        put(&tb[tm.rank * kLine + 2 * k + h], h ? high_word(s, tag) : low_word(s, tag));
+    }
+    // lane 8 g + j: word j of leader g, and word 8 + j % 2 (the fifth value's)
+    double r[2] = {0.0, 0.0};
+    const int j = l & 7;
+    word_t a[K > 4 ? 2 : 1];
+    if (!poll_words(tb + (l >> 3) * kLine + j, 8 - (j & 6), j < 2 * K, tag, tm.abort, a))
+      sh.bad = 1;
+    r[0] = join_words(a[0]);
+    if constexpr (K > 4) r[1] = join_words(a[1]);
+    double s = fold32(r[0], r[1]);
+    s = fold16(s, s);
+    s += dpp<kDppRor8>(s);
+    if ((l & 57) == 0 && (l >> 1) < K) sh.total[par][0][l >> 1] = s;
+    if (K > 4 && l == 32) sh.total[par][0][K > 4 ? 4 : 0] = s;
   }
   __syncthreads();
 #pragma unroll
-  for (int k = 0; k < K; ++k) v[k] = sh.total[par][k];
+  for (int q = 0; q < K; ++q) v[q] = sh.total[par][0][q];
   return sh.bad == 0;
 }
 

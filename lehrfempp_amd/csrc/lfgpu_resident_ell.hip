@@ -475,7 +475,7 @@ __global__ __launch_bounds__(kThreads) void k_res_ell_batch(EllArgs base) {
     const EllJob &jb = base.jobs[jr.x];
     EllArgs a = base;
     a.part += jb.sums_at;
-    a.total = a.part + (size_t)2 * 2 * kSums * jb.team;
+    a.total = a.part + part_words(jb.team);
     a.st += jb.index;
     if (!ell_solve<MODE, RPT, true>(a, k, jr.y, jb.team, dyn, sh)) return;
   }
@@ -793,7 +793,7 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
     j.index = q.index;
     j.team = (end - q.lo + R - 1) / R;
     j.sums_at = (uint32_t)p->sums_words;
-    p->sums_words += (size_t)2 * 2 * kSums * j.team + kTotalWords;
+    p->sums_words += part_words(j.team) + kTotalWords;
     most = std::max(most, R);
     for (int r = 0; r < j.team; ++r) {
       parts.push_back(EllPart{q.lo + r * R, std::min(q.lo + (r + 1) * R, end), R, 0, 0});

@@ -117,6 +117,22 @@ def test_resident_pcg_on_a_lattice(ctx, S, L, steps, symmetric, mode):
     A.close()
 
 
+# teams of 1, 2, 31 to 33 (one wavefront or two sum the members), 63 to 65 (one
+# hop or two) and 256 workgroups: 64 lines of 6 cells each; tolerance as above
+@pytest.mark.parametrize("team", [1, 2, 31, 32, 33, 63, 64, 65, 256])
+@pytest.mark.parametrize("mode", MODES)
+def test_team_sums(ctx, team, mode):
+    r, c, v, n = _lattice_system(6, 64 * team, P1, team)
+    A = capi.coo_to_csr(ctx, r, c, v, n, n)
+    x0 = np.random.default_rng(5).standard_normal(n)
+    out = _compare(ctx, A, n, mode, team + 2, x0=x0, maxit=3, rtol=1e-14)
+    assert out[0][0].iters == out[1][0].iters == 3
+    assert abs(out[0][0].relres - out[1][0].relres) <= 1e-4 * out[0][0].relres
+    eps = 1e-13 if mode == capi.PCG_FP64 else 1e-5 if mode == capi.PCG_MIXED else 1e-12
+    assert np.linalg.norm(out[0][1] - out[1][1]) <= eps * np.linalg.norm(out[0][1])
+    A.close()
+
+
 # the streamed matrix: 17, 25 and 33 cells a thread
 @pytest.mark.parametrize("S, L", [(1141, 1140), (1449, 1448), (1400, 1900), (2049, 2049),
                                   (3000, 500)])
