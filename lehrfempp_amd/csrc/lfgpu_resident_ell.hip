@@ -3,12 +3,13 @@
 // others is a compact neighbourhood), keeps their x, r and q in registers and
 // their p in LDS, followed by the p of the outside rows that it reads.  The
 // columns are stored once more as places in that LDS array (16 bits).  The
-// matrix is streamed every iteration (10 B a slot in FP64, 6 in FP32): what
-// the row sweeps spend beside it (two reduction launches, the vectors' trips,
-// the gathers' L2 misses) is gone.  Time per iteration, sweeps against this,
-// FP64: P1 on 300 x 260 unstructured squares 20.8 -> 7.4 us, 600^2 30.3 ->
-// 12.2; P3 on 37 x 29 19.6 -> 7.5, 200^2 35.9 -> 18.6, 384^2 86 -> 45 (226 MB
-// of matrix); FP32 matrix, P3 384^2: 64 -> 38.
+// matrix is streamed every iteration (10 B a slot in FP64, 6 in FP32) unless
+// a thread has one to three rows: then their first 40, 16 or 8 slots stay in
+// registers and an iteration is the exchange, the team sum and the gathers.
+// Time per iteration, sweeps against this, FP64: P1 on 300 x 260 unstructured
+// squares 20.8 -> 4.1 us, 600^2 30.3 -> 6.7, 900^2 45 -> 17; P3 on 37 x 29
+// 19.6 -> 3.5, 200^2 35.9 -> 10.6, 384^2 84 -> 43 (226 MB of matrix, 28 us of
+// it at 8 TB/s); FP32 matrix, P3 384^2: 64 -> 36.
 #include <hip/hip_bf16.h>
 #include <hip/hip_runtime.h>
 
@@ -25,10 +26,12 @@ using namespace lfgpu::res;
 
 namespace {
 
-// One workgroup's share: storage rows [r0, r1), LDS places 0.. for them and
-// from `rows` on for the `outside` rows listed at ext[at..].
+// One workgroup's share: the `slices` slices listed at slist[first..], which
+// lie in the storage rows [r0, r1) (and are all of them where the kernel
+// takes no list), LDS places 0.. for their rows and from 64 * slices on for
+// the `outside` rows listed at ext[at..].
 struct EllPart {
-  int32_t r0, r1, rows, outside;
+  int32_t r0, r1, slices, first, outside;
   int64_t at;
 };
 // One problem of a batch.
@@ -50,12 +53,13 @@ struct EllArgs {
   const __hip_bfloat16 *__restrict__ dinv16;
   const int32_t *__restrict__ perm;  // storage row -> row of x, b; -1: none; may be null
   const EllPart *__restrict__ parts;
+  const int32_t *__restrict__ slist;
   const int32_t *__restrict__ ext;
   const uint8_t *__restrict__ needed;
   const double *__restrict__ b;
   double *x;
   double *xlo;  // storage order
-  word_t *words;  // [2][2][n]
+  word_t *words;  // [2][planes(rpt)][n]
   word_t *part, *total;
   int *abort;
   uint32_t tag0;
@@ -90,15 +94,18 @@ struct Mode<LFGPU_PCG_MIXED_MATRIX> {
   typedef float MT;
 };
 
-// sum over a row's w slots of v_k (p_{c_k} - pi) from LDS; vp and cp point at
-// the row's first slot, a row's slots are 64 apart.  Eight, then four slots'
-// loads are issued before the first use.
+// acc + the sum over a row's slots k.. of w of v_k (p_{c_k} - pi) from LDS; vp
+// and cp point at the row's first slot, a row's slots are 64 apart.  Eight
+// slots' loads are issued before the first use, and the up to seven last ones'
+// of an FP64 matrix (four and then one after the other: P1 on 900 x 900
+// unstructured squares takes 21.3 us an iteration instead of 17.1, P3 on
+// 200 x 200 11.4 instead of 10.6; with FP32 values 64 P3 problems of 8 to 64
+// cells take 26.2 ms that way and 30.3 this way).
 template <class MT>
 __device__ __forceinline__ double ell_lds_row(const MT *__restrict__ vp,
-                                              const uint16_t *__restrict__ cp, int32_t w,
-                                              const double *lp, double pi) {
-  double acc = 0.0;
-  int32_t k = 0;
+                                              const uint16_t *__restrict__ cp, int32_t k,
+                                              int32_t w, const double *lp, double pi,
+                                              double acc) {
   for (; k + 8 <= w; k += 8) {
     MT v[8];
     uint16_t c[8];
@@ -113,21 +120,54 @@ __device__ __forceinline__ double ell_lds_row(const MT *__restrict__ vp,
 #pragma unroll
     for (int u = 0; u < 8; ++u) acc = __builtin_fma((double)v[u], y[u] - pi, acc);
   }
-  if (k + 4 <= w) {
-    MT v[4];
-    uint16_t c[4];
+  if constexpr (sizeof(MT) < 8) {
+    if (k + 4 <= w) {
+      MT v[4];
+      uint16_t c[4];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      c[u] = cp[64 * (k + u)];
-      v[u] = vp[64 * (k + u)];
+      for (int u = 0; u < 4; ++u) {
+        c[u] = cp[64 * (k + u)];
+        v[u] = vp[64 * (k + u)];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc = __builtin_fma((double)v[u], lp[c[u]] - pi, acc);
+      k += 4;
+    }
+    for (; k < w; ++k) acc = __builtin_fma((double)vp[64 * k], lp[cp[64 * k]] - pi, acc);
+    return acc;
+  }
+  const int32_t left = __builtin_amdgcn_readfirstlane(w - k);
+  if (left > 0) {
+    MT v[7];
+    uint16_t c[7];
+#pragma unroll
+    for (int u = 0; u < 7; ++u) {
+      c[u] = 0;
+      v[u] = (MT)0;
+      if (u < left) {
+        c[u] = cp[64 * (k + u)];
+        v[u] = vp[64 * (k + u)];
+      }
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) acc = __builtin_fma((double)v[u], lp[c[u]] - pi, acc);
-    k += 4;
+    for (int u = 0; u < 7; ++u)
+      if (u < left) acc = __builtin_fma((double)v[u], lp[c[u]] - pi, acc);
   }
-  for (; k < w; ++k) acc = __builtin_fma((double)vp[64 * k], lp[cp[64 * k]] - pi, acc);
   return acc;
 }
+
+// Up to this many rows a thread a part is small: its slices come from a list,
+// the first held_slots() slots of every row stay in registers, and the outside
+// rows' r, q, D^-1 and p are kept here and updated by their owners'
+// operations, so that what travels is q, during the team sum (as GHOST in
+// lfgpu_resident.hip).  Above, LDS and registers do not hold that, and the
+// exchange of p is a tenth of an iteration.
+constexpr int kSmallRows = 3;
+constexpr int held_slots(int rpt) {
+  return rpt == 1 ? 40 : rpt == 2 ? 16 : rpt <= kSmallRows ? 8 : 0;
+}
+// words per row and parity: two of p or q, and two of r (small parts)
+constexpr int planes(int rpt) { return rpt <= kSmallRows ? 4 : 2; }
 
 // RPT: rows per thread: thread t = 64 wave + lane owns the local rows
 // 64 (wave + 8 j) + lane, so a wavefront works on whole slices.  DREG: D^-1
@@ -138,16 +178,29 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
   typedef typename Mode<MODE>::VT VT;
   typedef typename Mode<MODE>::MT MT;
   constexpr bool kMixed = MODE != LFGPU_PCG_FP64;
+  constexpr bool kSmall = RPT <= kSmallRows;
+  constexpr int kHeld = held_slots(RPT);
   const int t = threadIdx.x;
   Team tm{rank, team, a.part, a.total, a.abort, a.tag0};
   uint32_t tag = a.tag0;
   if (t == 0) sh.bad = 0;
   const EllPart &part = a.parts[slot];
-  const int32_t r0 = part.r0, mine = part.r1 - part.r0, place = part.rows;
-  const int32_t next = part.outside;
-  const int32_t *ext = a.ext + part.at;
-  const int32_t s0 = (r0 >> 6) + __builtin_amdgcn_readfirstlane(t >> 6);
-  const int32_t slices = (mine + 63) >> 6;
+  const int32_t slices = part.slices, place = 64 * slices, next = part.outside;
+  const int32_t wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int32_t s0 = (part.r0 >> 6) + wave;
+  // small parts: the outside rows' r, q, D^-1 and storage rows
+  VT *const gr = reinterpret_cast<VT *>(lp + place + next), *const gq = gr + next,
+     *const gd = gq + next;
+  int32_t *const gsrc = reinterpret_cast<int32_t *>(gd + next);
+  const int32_t *const ext = a.ext + part.at;
+  // the wavefront's slice number j, and its thread's storage row there
+  int32_t list[kSmall ? RPT : 1];
+  if constexpr (kSmall)
+#pragma unroll
+    for (int j = 0; j < RPT; ++j)
+      list[j] = wave + j * kWaves < slices ? a.slist[part.first + wave + j * kWaves] : 0;
+  auto slice = [&](int j) { return kSmall ? list[kSmall ? j : 0] : s0 + j * kWaves; };
+  auto row = [&](int j) { return 64 * slice(j) + (t & 63); };
 
   auto dinv_of = [&](int32_t g) -> VT {
     if constexpr (MODE == LFGPU_PCG_FP64) return a.dinv[g];
@@ -159,10 +212,11 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
     else return a.rowsum[g];
   };
   auto at = [&](int32_t g) { return a.perm ? a.perm[g] : g; };
-  // Publishes row r0 + i's value (VT or, for reliable updates, double) and
-  // fetches the outside rows' into LDS, four in flight per thread.
-  auto publish = [&](int32_t i, auto v) {
-    word_t *w = a.words + (size_t)(tag & 1u) * 2 * a.n + r0 + i;
+  // Publishes storage row g's value (VT or, for reliable updates, double) in
+  // a plane's words, and hands the outside rows' e = 0.. to fn(e, value),
+  // four in flight for each of the threads from `from` on.
+  auto publish = [&](int32_t g, auto v, int plane) {
+    word_t *w = a.words + ((size_t)(tag & 1u) * planes(RPT) + plane) * a.n + g;
     if constexpr (sizeof(v) == 8) {
       put(w, low_word(v, tag));
       put(w + a.n, high_word(v, tag));
@@ -170,14 +224,20 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
       put(w, ((word_t)__float_as_uint(v) << 32) | tag);
     }
   };
-  auto fetch = [&](auto like) {
+  auto fetch = [&](auto like, int plane, int from, auto &&fn) {
+    typedef decltype(like) FT;
     constexpr bool kTwo = sizeof(like) == 8;
-    const word_t *w = a.words + (size_t)(tag & 1u) * 2 * a.n;
-    for (int32_t e0 = t; e0 < next; e0 += 4 * kThreads) {
+    if (t < from) return;
+    const word_t *w = a.words + ((size_t)(tag & 1u) * planes(RPT) + plane) * a.n;
+    const int32_t step = kThreads - from;
+    for (int32_t e0 = t - from; e0 < next; e0 += 4 * step) {
       int32_t src[4];
       word_t lo[4], hi[4];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) src[u] = ext[min(e0 + u * kThreads, next - 1)];
+      for (int u = 0; u < 4; ++u) {
+        const int32_t e = min(e0 + u * step, next - 1);
+        src[u] = kSmall ? gsrc[e] : ext[e];
+      }
       bool ok;
       Wait wait(a.abort);
       do {
@@ -196,36 +256,66 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
       if (!ok) sh.bad = 1;
 #pragma unroll
       for (int u = 0; u < 4; ++u)
-        if (e0 + u * kThreads < next) {
-          if constexpr (kTwo) lp[place + e0 + u * kThreads] = from_words(lo[u], hi[u]);
-          else lp[place + e0 + u * kThreads] = (double)__uint_as_float((uint32_t)(lo[u] >> 32));
+        if (e0 + u * step < next) {
+          FT v;
+          if constexpr (kTwo) v = from_words(lo[u], hi[u]);
+          else v = __uint_as_float((uint32_t)(lo[u] >> 32));
+          fn(e0 + u * step, v);
         }
     }
   };
+  auto to_lds = [&](int32_t e, auto v) { lp[place + e] = (double)v; };
 
   // (places past the last row are read and have to be finite)
   for (int32_t i = t; i < place; i += kThreads) lp[i] = 0.0;
+  if constexpr (kSmall)
+    for (int32_t e = t; e < next; e += kThreads) {
+      const int32_t g = ext[e];
+      gsrc[e] = g;
+      gd[e] = dinv_of(g);
+      gr[e] = gq[e] = (VT)0;
+      lp[place + e] = 0.0;
+    }
 
   // x: the solution (FP64) or the mixed modes' increment
   VT x[RPT], r[RPT], q[RPT], di[DREG ? RPT : 1];
   double rs[DREG ? RPT : 1];
+  // the held slots: values (0 past the row's end) and LDS places, two a word
+  MT hv[kSmall ? RPT : 1][kSmall ? kHeld : 1];
+  uint32_t hc[kSmall ? RPT : 1][kSmall ? kHeld / 2 : 1];
   uint32_t live = 0, needed = 0;
 #pragma unroll
   for (int j = 0; j < RPT; ++j) {
-    const int32_t i = t + j * kThreads;
+    const int32_t g = row(j), i = t + j * kThreads;
     x[j] = r[j] = q[j] = (VT)0;
     if constexpr (DREG) {
       rs[j] = 0.0;
       di[j] = (VT)0;
     }
-    if (i < mine && at(r0 + i) >= 0) {
+    if (i < place && g < a.n && at(g) >= 0) {
       live |= 1u << j;
-      if (a.needed[r0 + i]) needed |= 1u << j;
+      if (a.needed[g]) needed |= 1u << j;
       if constexpr (DREG) {
-        rs[j] = rowsum_of(r0 + i);
-        di[j] = dinv_of(r0 + i);
+        rs[j] = rowsum_of(g);
+        di[j] = dinv_of(g);
       }
-      if constexpr (kMixed) a.xlo[r0 + i] = 0.0;
+      if constexpr (kMixed) a.xlo[g] = 0.0;
+    }
+    if constexpr (kSmall) {
+      const bool in = wave + j * kWaves < slices;
+      const int32_t o = in ? a.slice_off[slice(j)] : 0;
+      const int32_t w = in ? (a.slice_off[slice(j) + 1] - o) >> 6 : 0;
+      const MT *vp;
+      if constexpr (kMixed) vp = a.val32;
+      else vp = a.val;
+#pragma unroll
+      for (int k = 0; k < kHeld; ++k) {
+        const int32_t l = o + 64 * k + (t & 63);
+        hv[j][k] = k < w ? vp[l] : (MT)0;
+        const uint32_t c = k < w ? (uint32_t)a.lcol[l] : (uint32_t)(in ? i : 0);
+        if (k % 2) hc[j][k / 2] |= c << 16;
+        else hc[j][k / 2] = c;
+      }
     }
     __builtin_amdgcn_sched_barrier(0);
   }
@@ -235,13 +325,42 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
     const int32_t ti = opaque(t);
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
-      const int32_t s = s0 + j * kWaves;
-      if (s - (r0 >> 6) < slices) {
-        const int32_t i = ti + j * kThreads;
+      if (wave + j * kWaves < slices) {
+        const int32_t s = slice(j), i = ti + j * kThreads;
         const int32_t o = a.slice_off[s], w = (a.slice_off[s + 1] - o) >> 6;
         const double pi = lp[i];
         const int32_t l = o + (ti & 63);
-        fn(j, i, ell_lds_row(val + l, a.lcol + l, w, lp, pi), pi);
+        fn(j, 64 * s + (ti & 63), ell_lds_row(val + l, a.lcol + l, 0, w, lp, pi, 0.0), pi);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  // the same with the held slots, eight gathers in flight
+  auto held_rows = [&](const MT *val, auto &&fn) {
+    const int32_t ti = opaque(t);
+#pragma unroll
+    for (int j = 0; j < (kSmall ? RPT : 0); ++j) {
+      if (wave + j * kWaves < slices) {
+        const int32_t s = slice(j), i = ti + j * kThreads;
+        const int32_t o = a.slice_off[s], w = (a.slice_off[s + 1] - o) >> 6;
+        const double pi = lp[i];
+        double acc = 0.0;
+#pragma unroll
+        for (int k = 0; k < kHeld; k += 8)
+          if (k < w) {
+            double y[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+              const uint32_t c = hc[j][(k + u) / 2];
+              y[u] = lp[u % 2 ? c >> 16 : c & 0xffffu];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+              acc = __builtin_fma((double)hv[j][k + u], y[u] - pi, acc);
+          }
+        const int32_t l = o + (ti & 63);
+        if (w > kHeld) acc = ell_lds_row(val + l, a.lcol + l, kHeld, w, lp, pi, acc);
+        fn(j, 64 * s + (ti & 63), acc, pi);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -254,23 +373,32 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
     double s[5] = {0.0, 0.0, 0.0, rr, rz};
     bool refine = first;
     if (!first) {
-      fetch((VT)0);
+      if constexpr (kSmall) ++tag;
+      else fetch((VT)0, 0, 0, to_lds);
       __syncthreads();
-      auto product = [&](int j, int32_t i, double acc, double pi) {
-        const double ri = DREG ? rs[DREG ? j : 0] : rowsum_of(r0 + min(i, mine - 1));
-        const VT dv = DREG ? di[DREG ? j : 0] : dinv_of(r0 + min(i, mine - 1));
+      auto product = [&](int j, int32_t g, double acc, double pi) {
+        const double ri = DREG ? rs[DREG ? j : 0] : rowsum_of(min(g, a.n - 1));
+        const VT dv = DREG ? di[DREG ? j : 0] : dinv_of(min(g, a.n - 1));
         VT qi = (VT)__builtin_fma(ri, pi, acc);
         qi = (live >> j) & 1 ? qi : (VT)0;
         q[j] = qi;
+        if constexpr (kSmall)
+          if ((needed >> j) & 1) publish(g, qi, 0);
         const double qd = (double)qi, dq = (double)(dv * qi);
         s[0] = __builtin_fma(pi, qd, s[0]);
         s[1] = __builtin_fma(dq, (double)r[j], s[1]);
         s[2] = __builtin_fma(dq, qd, s[2]);
         pin(q[j]), pin(s[0]), pin(s[1]), pin(s[2]);
       };
-      if constexpr (kMixed) rows(a.val32, product);
-      else rows(a.val, product);
-      ok = team_sum(tm, sh, s, [] {});
+      const MT *val;
+      if constexpr (kMixed) val = a.val32;
+      else val = a.val;
+      if constexpr (kSmall) held_rows(val, product);
+      else rows(val, product);
+      ok = team_sum(tm, sh, s, [&] {
+        if constexpr (kSmall)
+          fetch((VT)0, 0, sums_threads(tm), [&](int32_t e, VT v) { gq[e] = v; });
+      });
       if (!ok) break;
       if constexpr (kMixed) {
         // (a step between two reliable updates, so that the loop ends)
@@ -291,36 +419,48 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
       const double rho = s[4], alpha = rho / s[0];
       const double rho_next = rho - 2.0 * alpha * s[1] + alpha * alpha * s[2];
       const VT fa = (VT)alpha, fb = (VT)(rho_next / rho);
+      // z and the next p of a row
+      auto step = [&](VT dv, VT qi, VT pi, VT &ri, VT &z) {
+        if constexpr (MODE == LFGPU_PCG_FP64) {
+          ri = __builtin_fma(-fa, qi, ri);
+          z = dv * ri;
+          return __builtin_fma(fb, pi, z);
+        } else {
+          ri = ri - fa * qi;
+          z = dv * ri;
+          return z + fb * pi;
+        }
+      };
       rr = rz = 0.0;
-      ++tag;
+      if constexpr (!kSmall) ++tag;
       const int32_t ti = opaque(t);
 #pragma unroll
       for (int j = 0; j < RPT; ++j) {
         const int32_t i = ti + j * kThreads;
         if ((live >> j) & 1) {
-          const VT dv = DREG ? di[DREG ? j : 0] : dinv_of(r0 + i);
+          const int32_t g = 64 * slice(j) + (ti & 63);
+          const VT dv = DREG ? di[DREG ? j : 0] : dinv_of(g);
           const VT pi = (VT)lp[i];
-          VT z, p;
-          if constexpr (MODE == LFGPU_PCG_FP64) {
-            x[j] = __builtin_fma(fa, pi, x[j]);
-            r[j] = __builtin_fma(-fa, q[j], r[j]);
-            z = dv * r[j];
-            p = __builtin_fma(fb, pi, z);
-          } else {
-            x[j] = x[j] + fa * pi;
-            r[j] = r[j] - fa * q[j];
-            z = dv * r[j];
-            p = z + fb * pi;
-          }
+          VT z;
+          if constexpr (MODE == LFGPU_PCG_FP64) x[j] = __builtin_fma(fa, pi, x[j]);
+          else x[j] = x[j] + fa * pi;
+          const VT p = step(dv, q[j], pi, r[j], z);
           const double rd = (double)r[j];
           rr = __builtin_fma(rd, rd, rr);
           rz = __builtin_fma(rd, (double)z, rz);
           lp[i] = (double)p;
-          if ((needed >> j) & 1) publish(i, p);
+          if constexpr (!kSmall)
+            if ((needed >> j) & 1) publish(g, p, 0);
         }
         pin(r[j]), pin(x[j]), pin(rr), pin(rz);
         __builtin_amdgcn_sched_barrier(0);
       }
+      if constexpr (kSmall)
+        for (int32_t e = ti; e < next; e += kThreads) {
+          VT z, rn = gr[e];
+          lp[place + e] = (double)step(gd[e], gq[e], (VT)lp[place + e], rn, z);
+          gr[e] = rn;
+        }
       continue;
     }
     // the first residual b - A x, or a reliable update's b - A x - A xa - A xlo
@@ -328,7 +468,7 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
       const int32_t i = t + j * kThreads;
-      r64[j] = (live >> j) & 1 ? a.b[at(r0 + i)] : 0.0;
+      r64[j] = (live >> j) & 1 ? a.b[at(row(j))] : 0.0;
       if (!first && ((live >> j) & 1)) q[j] = (VT)lp[i];  // p
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -352,17 +492,18 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
       for (int j = 0; j < RPT; ++j) {
         const int32_t i = ti + j * kThreads;
         if ((live >> j) & 1) {
-          const double y = turn == 0 ? a.x[at(r0 + i)] : turn == 1 ? (double)x[j] : a.xlo[r0 + i];
+          const int32_t g = 64 * slice(j) + (ti & 63);
+          const double y = turn == 0 ? a.x[at(g)] : turn == 1 ? (double)x[j] : a.xlo[g];
           if (!kMixed) x[j] = (VT)y;
           lp[i] = y;
-          if ((needed >> j) & 1) publish(i, y);
+          if ((needed >> j) & 1) publish(g, y, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
-      fetch(0.0);
+      fetch(0.0, 0, 0, to_lds);
       __syncthreads();
-      rows(a.val, [&](int j, int32_t i, double acc, double yi) {
-        if ((live >> j) & 1) r64[j] -= __builtin_fma(a.rowsum[r0 + i], yi, acc);
+      rows(a.val, [&](int j, int32_t g, double acc, double yi) {
+        if ((live >> j) & 1) r64[j] -= __builtin_fma(a.rowsum[g], yi, acc);
         pin(r64[j]);
       });
     }
@@ -387,14 +528,13 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
       stop = converged || itp >= a.maxit;
 #pragma unroll
       for (int j = 0; j < RPT; ++j) {
-        const int32_t i = t + j * kThreads;
         if ((live >> j) & 1) {
-          const int32_t g = at(r0 + i);
+          const int32_t g = at(row(j));
           const double hi = a.x[g], dx = (double)x[j];
           const double sm = hi + dx, bp = sm - hi;
           const double err = (hi - (sm - bp)) + (dx - bp);
           a.x[g] = sm;
-          a.xlo[r0 + i] += err;
+          a.xlo[row(j)] += err;
         }
         x[j] = (VT)0;
         __builtin_amdgcn_sched_barrier(0);
@@ -411,30 +551,37 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
       const int32_t i = ti + j * kThreads;
       if ((live >> j) & 1) {
         const VT rn = (VT)r64[j];
-        const VT m = DREG ? di[DREG ? j : 0] : dinv_of(r0 + i);
+        const int32_t g = 64 * slice(j) + (ti & 63);
+        const VT m = DREG ? di[DREG ? j : 0] : dinv_of(g);
         const VT z = m * rn;
         const VT p = first ? z : q[j] + m * (rn - r[j]);
         r[j] = rn;
         lp[i] = (double)p;
-        if ((needed >> j) & 1) publish(i, p);
+        if ((needed >> j) & 1) {
+          publish(g, p, 0);
+          if constexpr (kSmall) publish(g, rn, 2);
+        }
         // (the first rho, as the sweeps take it: with the FP64 D^-1 and residual)
         const double rd = first ? r64[j] : (double)rn;
-        const double zd = first ? a.dinv[r0 + i] * rd : (double)z;
+        const double zd = first ? a.dinv[g] * rd : (double)z;
         rr = __builtin_fma(rd, rd, rr);
         rz = __builtin_fma(rd, zd, rz);
       }
       __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (kSmall) {
+      fetch((VT)0, 0, 0, to_lds);
+      fetch((VT)0, 2, 0, [&](int32_t e, VT v) { gr[e] = v; });
     }
     first = false;
   }
   if (ok) {
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
-      const int32_t i = t + j * kThreads;
       if ((live >> j) & 1) {
-        const int32_t g = at(r0 + i);
+        const int32_t g = at(row(j));
         if (bb == 0.0) a.x[g] = 0.0;
-        else if (kMixed) a.x[g] = a.x[g] + a.xlo[r0 + i];
+        else if (kMixed) a.x[g] = a.x[g] + a.xlo[row(j)];
         else if (!first) a.x[g] = (double)x[j];
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -486,27 +633,30 @@ __global__ __launch_bounds__(kThreads) void k_res_ell_batch(EllArgs base) {
 // ---------------------------------------------------------------------------
 // One workgroup per part: a bitmap of the outside columns over the window
 // that 16-bit offsets reach, its prefix sums as their places behind the own
-// rows, and every slot's place.  parts[g].outside = number of outside rows; a
-// part with more than `room` writes nothing else.
+// rows, and every slot's place.  home: every slice's part and number in it.
+// parts[g].outside = number of outside rows; a part with more than `room`
+// places writes nothing else.
 constexpr int kSplitThreads = 512;
-__global__ __launch_bounds__(kSplitThreads) void k_ell_split(const int32_t *slice_off,
-                                                             const int16_t *dcol, int32_t room,
-                                                             EllPart *parts, int32_t *ext,
-                                                             uint16_t *lcol, uint8_t *needed) {
+__global__ __launch_bounds__(kSplitThreads) void k_ell_split(
+    int32_t n, const int32_t *slice_off, const int16_t *dcol, const int32_t *slist,
+    const int2 *home, int32_t room, EllPart *parts, int32_t *ext, uint16_t *lcol,
+    uint8_t *needed) {
   extern __shared__ uint32_t map[];
   __shared__ int32_t sums[kSplitThreads];
-  const int t = threadIdx.x;
-  EllPart &part = parts[blockIdx.x];
-  const int32_t r0 = part.r0, r1 = part.r1, rows = part.rows;
+  const int t = threadIdx.x, me = blockIdx.x;
+  EllPart &part = parts[me];
+  const int32_t r0 = part.r0, rows = 64 * part.slices;
+  slist += part.first;
   int32_t *list = ext + part.at;
-  const int32_t words = (rows + 65536) / 32;
+  const int32_t words = (part.r1 - r0 + 65567) / 32;
   for (int32_t k = t; k < words; k += kSplitThreads) map[k] = 0;
   __syncthreads();
-  for (int32_t r = r0 + t; r < r1; r += kSplitThreads) {
-    const int32_t s = r >> 6, o = slice_off[s] + (r & 63), w = (slice_off[s + 1] - slice_off[s]) >> 6;
-    for (int32_t k = 0; k < w; ++k) {
+  for (int32_t i = t; i < rows; i += kSplitThreads) {
+    const int32_t s = slist[i >> 6], r = 64 * s + (i & 63);
+    const int32_t o = slice_off[s] + (i & 63), w = (slice_off[s + 1] - slice_off[s]) >> 6;
+    for (int32_t k = 0; k < w && r < n; ++k) {
       const int32_t c = r + dcol[o + 64 * k];
-      if (c < r0 || c >= r1) {
+      if (home[c >> 6].x != me) {
         const int32_t b = c - r0 + 32768;
         atomicOr(&map[b >> 5], 1u << (b & 31));
       }
@@ -535,15 +685,16 @@ __global__ __launch_bounds__(kSplitThreads) void k_ell_split(const int32_t *slic
       needed[c] = 1;
     }
   __syncthreads();
-  const int32_t s1 = (r1 + 63) >> 6;
-  for (int32_t r = r0 + t; r < s1 * 64; r += kSplitThreads) {
-    const int32_t s = r >> 6, o = slice_off[s] + (r & 63), w = (slice_off[s + 1] - slice_off[s]) >> 6;
+  for (int32_t i = t; i < rows; i += kSplitThreads) {
+    const int32_t s = slist[i >> 6], r = 64 * s + (i & 63);
+    const int32_t o = slice_off[s] + (i & 63), w = (slice_off[s + 1] - slice_off[s]) >> 6;
     for (int32_t k = 0; k < w; ++k) {
       int32_t at = 0;  // (lanes past the last row)
-      if (r < r1) {
+      if (r < n) {
         const int32_t c = r + dcol[o + 64 * k];
-        if (c >= r0 && c < r1) {
-          at = c - r0;
+        const int2 h = home[c >> 6];
+        if (h.x == me) {
+          at = 64 * h.y + (c & 63);
         } else {
           // place of c among the outside rows: binary search in the list
           int32_t lo = 0, hi = all - 1;
@@ -587,8 +738,9 @@ const void *const kEllBatch[2][3] = {
 namespace lfgpu {
 struct ResidentEllPlan {
   int rpt = 0, nparts = 0;  // rpt 0: does not fit
-  int32_t most = 0;         // most places (own and outside rows) of a workgroup
+  size_t lds = 0;           // most bytes of a workgroup
   EllPart *parts = nullptr;
+  int32_t *slist = nullptr;   // the parts' slices
   int32_t *ext = nullptr;     // the outside rows of every part, ascending
   uint16_t *lcol = nullptr;   // per slot: the column's place in the workgroup's LDS
   uint8_t *needed = nullptr;  // per row: some other workgroup reads it
@@ -603,6 +755,7 @@ struct ResidentEllPlan {
 void resident_ell_free(ResidentEllPlan *p) {
   if (!p) return;
   dfree(p->parts);
+  dfree(p->slist);
   dfree(p->ext);
   dfree(p->lcol);
   dfree(p->needed);
@@ -617,19 +770,115 @@ bool resident_ell_fits(const ResidentEllPlan *p) { return p && p->rpt > 0; }
 
 namespace {
 
-// Splits the storage into the given parts (r0, r1, rows filled in); *fits
-// tells whether every part's places fit the LDS.
-int ell_split(hipStream_t s, ResidentEllPlan *p, const ResidentEll &A, std::vector<EllPart> &parts,
+// The parts of a split, their slices one after the other.
+struct Split {
+  std::vector<EllPart> parts;
+  std::vector<int32_t> slist;
+  void add(const std::vector<int32_t> &slices, int32_t n) {
+    EllPart q{};
+    q.r0 = 64 * slices.front();
+    q.r1 = std::min(64 * (slices.back() + 1), n);
+    q.slices = (int32_t)slices.size();
+    q.first = (int32_t)slist.size();
+    slist.insert(slist.end(), slices.begin(), slices.end());
+    parts.push_back(q);
+  }
+};
+
+// Splits the slices [s0, s1) into runs of `each` slices.  (Runs of equally
+// many slots on all 256 CUs: P3 on 384 x 384 takes 44.8 instead of 42.5 us an
+// iteration, its parts read more outside rows.)
+void split_runs(Split &out, int32_t s0, int32_t s1, int each, int32_t n) {
+  std::vector<int32_t> part;
+  for (int32_t s = s0; s < s1; s += each) {
+    part.clear();
+    for (int32_t k = s; k < std::min(s + each, s1); ++k) part.push_back(k);
+    out.add(part, n);
+  }
+}
+
+// The locality order sorts its windows' rows by length: on a third-order
+// mesh, the cells', the edges' and then the vertices' rows.  Runs of a few
+// slices are of one kind, so that some parts have four times the slots of
+// others and read rows all over the window (37 x 29 cells: 600 outside rows in
+// a part of edges, 3200 in one of vertices).  Where the windows hold several
+// parts, every part gets its share of every length in the window.  Returns
+// false if the windows are too small for that, or too many parts result.
+bool split_windows(Split &out, const std::vector<int32_t> &off, int32_t s0, int32_t s1, int cap,
+                   int most, int32_t n) {
+  auto width = [&](int32_t s) { return off[s + 1] - off[s]; };
+  std::vector<int32_t> starts{s0};  // of the runs of ascending lengths
+  for (int32_t s = s0 + 1; s < s1; ++s)
+    if (width(s) < width(s - 1)) starts.push_back(s);
+  starts.push_back(s1);
+  if (2 * (int64_t)(s1 - s0) < 3 * (int64_t)cap * (int64_t)(starts.size() - 1)) return false;
+  const size_t had = out.parts.size(), had_slices = out.slist.size();
+  auto fail = [&] {
+    out.parts.resize(had);
+    out.slist.resize(had_slices);
+    return false;
+  };
+  for (size_t k = 0; k + 1 < starts.size(); ++k) {
+    const int32_t u = starts[k], v = starts[k + 1];
+    if (v - u > 1024) return fail();  // (the outside rows' bitmap covers a window)
+    const int fewest = (v - u + cap - 1) / cap;
+    bool done = false;
+    for (int m = fewest; m <= fewest + fewest / 8 + 1 && !done; ++m) {
+      // slice number k of a length's L goes to the part in which (k + phase) / L
+      // of the window lies; the phase spreads lengths of few slices
+      std::vector<std::vector<int32_t>> deal(m);
+      double phase = 0.5;
+      for (int32_t a = u; a < v;) {
+        int32_t b = a + 1;
+        while (b < v && width(b) == width(a)) ++b;
+        for (int32_t s = a; s < b; ++s)
+          deal[std::min(m - 1, (int)((s - a + phase) / (b - a) * m))].push_back(s);
+        phase = std::fmod(phase + 0.6180339887498949, 1.0);
+        a = b;
+      }
+      // what a part has above its cap goes to the next one with room
+      std::vector<int32_t> over;
+      for (auto &d : deal)
+        for (; (int)d.size() > cap; d.pop_back()) over.push_back(d.back());
+      for (auto &d : deal)
+        for (; (int)d.size() < cap && !over.empty(); over.pop_back()) d.push_back(over.back());
+      if (!over.empty()) continue;
+      for (auto &d : deal) {
+        if (d.empty()) continue;
+        std::sort(d.begin(), d.end());
+        out.add(d, n);
+      }
+      done = true;
+    }
+    if (!done) return fail();
+    if ((int64_t)(out.parts.size() - had) > most) return fail();
+  }
+  return true;
+}
+
+// LDS of a part
+size_t lds_bytes(const EllPart &q, int rpt) {
+  const size_t places = 64 * (size_t)q.slices + q.outside;
+  return (places + (rpt <= kSmallRows ? 3 * (size_t)q.outside : 0)) * 8 +
+         (rpt <= kSmallRows ? 4 * (size_t)q.outside : 0);
+}
+
+// Builds the places of a split; *fits tells whether every part fits the LDS.
+int ell_split(hipStream_t s, ResidentEllPlan *p, const ResidentEll &A, Split &split, int rpt,
               bool *fits) {
   const int32_t room = (int32_t)std::min<size_t>(kLdsDynamic / sizeof(double), 65536);
   *fits = false;
   int64_t at = 0;
-  int32_t rows = 0;
-  for (EllPart &q : parts) {
-    if (q.rows >= room) return LFGPU_OK;
+  int32_t span = 0;
+  std::vector<int2> home((size_t)(A.n + 63) / 64, int2{-1, 0});
+  for (size_t g = 0; g < split.parts.size(); ++g) {
+    EllPart &q = split.parts[g];
+    if (64 * q.slices >= room) return LFGPU_OK;
     q.at = at;
-    at += room - q.rows;
-    rows = std::max(rows, q.rows);
+    at += room - 64 * q.slices;
+    span = std::max(span, q.r1 - q.r0);
+    for (int32_t k = 0; k < q.slices; ++k)
+      home[split.slist[(size_t)q.first + k]] = int2{(int)g, k};
   }
   if (!p->lcol) {
     LFG_TRY(dalloc(&p->lcol, (size_t)std::max<int64_t>(A.slots, 1), "resident ELL places"));
@@ -637,27 +886,52 @@ int ell_split(hipStream_t s, ResidentEllPlan *p, const ResidentEll &A, std::vect
   }
   dfree(p->ext);
   dfree(p->parts);
+  dfree(p->slist);
   p->ext = nullptr;
   p->parts = nullptr;
+  p->slist = nullptr;
   LFG_TRY(dalloc(&p->ext, (size_t)at, "resident ELL outside rows"));
-  LFG_TRY(dalloc(&p->parts, parts.size(), "resident ELL parts"));
-  LFG_HIP(hipMemcpyAsync(p->parts, parts.data(), parts.size() * sizeof(EllPart),
-                         hipMemcpyHostToDevice, s));
-  LFG_HIP(hipMemsetAsync(p->needed, 0, (size_t)A.n, s));
-  const size_t map = (size_t)(rows + 65536) / 32 * 4;
-  hipLaunchKernelGGL(k_ell_split, dim3((unsigned)parts.size()), dim3(kSplitThreads), map, s,
-                     A.slice_off, A.dcol, room, p->parts, p->ext, p->lcol, p->needed);
-  LFG_HIP(hipGetLastError());
-  LFG_HIP(hipMemcpyAsync(parts.data(), p->parts, parts.size() * sizeof(EllPart),
-                         hipMemcpyDeviceToHost, s));
-  LFG_HIP(hipStreamSynchronize(s));
-  p->most = 0;
-  for (const EllPart &q : parts) {
-    if (q.outside > room - q.rows) return LFGPU_OK;
-    p->most = std::max(p->most, q.rows + q.outside);
+  LFG_TRY(dalloc(&p->parts, split.parts.size(), "resident ELL parts"));
+  LFG_TRY(dalloc(&p->slist, split.slist.size(), "resident ELL slices"));
+  int2 *dhome = nullptr;
+  LFG_TRY(dalloc(&dhome, home.size(), "resident ELL slices"));
+  hipError_t e = hipMemcpyAsync(dhome, home.data(), home.size() * sizeof(int2),
+                                hipMemcpyHostToDevice, s);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(p->parts, split.parts.data(), split.parts.size() * sizeof(EllPart),
+                       hipMemcpyHostToDevice, s);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(p->slist, split.slist.data(), split.slist.size() * 4,
+                       hipMemcpyHostToDevice, s);
+  if (e == hipSuccess) e = hipMemsetAsync(p->needed, 0, (size_t)A.n, s);
+  if (e == hipSuccess) {
+    const size_t map = (size_t)(span + 65567) / 32 * 4;
+    hipLaunchKernelGGL(k_ell_split, dim3((unsigned)split.parts.size()), dim3(kSplitThreads), map,
+                       s, A.n, A.slice_off, A.dcol, p->slist, dhome, room, p->parts, p->ext,
+                       p->lcol, p->needed);
+    e = hipGetLastError();
   }
-  p->nparts = (int)parts.size();
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(split.parts.data(), p->parts, split.parts.size() * sizeof(EllPart),
+                       hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  dfree(dhome);
+  if (e != hipSuccess) return hip_fail(e, "resident ELL split");
+  p->lds = 0;
+  for (const EllPart &q : split.parts) {
+    if (q.outside > room - 64 * q.slices || lds_bytes(q, rpt) > kLdsDynamic) return LFGPU_OK;
+    p->lds = std::max(p->lds, lds_bytes(q, rpt));
+  }
+  p->nparts = (int)split.parts.size();
   *fits = true;
+  return LFGPU_OK;
+}
+
+// the slices' offsets
+int slice_offsets(hipStream_t s, const ResidentEll &A, std::vector<int32_t> &off) {
+  off.resize((size_t)(A.n + 63) / 64 + 1);
+  LFG_HIP(hipMemcpyAsync(off.data(), A.slice_off, off.size() * 4, hipMemcpyDeviceToHost, s));
+  LFG_HIP(hipStreamSynchronize(s));
   return LFGPU_OK;
 }
 
@@ -675,6 +949,7 @@ void fill_args(EllArgs &a, const ResidentEllPlan *plan, const ResidentEll &A,
   a.dinv16 = static_cast<const __hip_bfloat16 *>(A.dinv16);
   a.perm = A.perm;
   a.parts = plan->parts;
+  a.slist = plan->slist;
   a.ext = plan->ext;
   a.needed = plan->needed;
   a.b = b;
@@ -705,15 +980,17 @@ int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan
   const int cus = std::min(ctx->cus, kMaxTeam);
   if (!*pplan) {
     ResidentEllPlan *p = *pplan = new ResidentEllPlan();
+    std::vector<int32_t> off;
+    LFG_TRY(slice_offsets(s, A, off));
+    const int32_t slices = (int32_t)off.size() - 1;
     for (const EllVariant &v : kEllVariants) {
-      const int64_t want = (A.n + (int64_t)v.rpt * kThreads - 1) / ((int64_t)v.rpt * kThreads);
+      const int cap = v.rpt * kWaves, want = (slices + cap - 1) / cap;
       if (want > cus) continue;
-      const int32_t rows = (int32_t)(((A.n + want - 1) / want + 63) / 64 * 64);
-      std::vector<EllPart> parts((A.n + rows - 1) / rows);
-      for (size_t g = 0; g < parts.size(); ++g)
-        parts[g] = EllPart{(int32_t)g * rows, std::min((int32_t)(g + 1) * rows, A.n), rows, 0, 0};
+      Split split;
+      if (v.rpt > kSmallRows || !split_windows(split, off, 0, slices, cap, cus, A.n))
+        split_runs(split, 0, slices, (slices + want - 1) / want, A.n);
       bool fits = false;
-      LFG_TRY(ell_split(s, p, A, parts, &fits));
+      LFG_TRY(ell_split(s, p, A, split, v.rpt, &fits));
       if (!fits) continue;
       p->rpt = v.rpt;
       break;
@@ -725,19 +1002,20 @@ int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan
   for (const EllVariant &k : kEllVariants)
     if (k.rpt == plan->rpt) v = &k;
   EllArgs a{};
-  LFG_TRY(resident_prepare(s, bufs, (size_t)4 * A.n, ell_tags(opts), &a.tag0));
+  LFG_TRY(resident_prepare(s, bufs, (size_t)2 * planes(plan->rpt) * A.n, ell_tags(opts),
+                           &a.tag0));
   fill_args(a, plan, A, opts, b, x);
   a.words = bufs->halo;
   a.part = bufs->sums;
   a.total = bufs->sums + kPartWords;
   a.abort = bufs->abort;
   a.st = bufs->state;
-  return resident_launch(s, bufs, v->fn[opts.mode], plan->nparts, &a,
-                         (size_t)plan->most * sizeof(double), st, taken);
+  return resident_launch(s, bufs, v->fn[opts.mode], plan->nparts, &a, plan->lds, st, taken);
 }
 
 // Team sizes as for the lattice problems (resident_tiles_plan): an iteration
 // takes about 6 us and 0.3 ns a slot of a workgroup's rows.
+constexpr double kFixedUs = 6.0, kSlotUs = 0.0003;
 int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
                             const std::vector<ResidentProblem> &probs, ResidentEllPlan **out) {
   ResidentEllPlan *p = *out = new ResidentEllPlan();
@@ -745,21 +1023,23 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
   const int cus = std::min(ctx->cus, kMaxTeam);
   const size_t np = probs.size();
   if (np == 0 || !A.dcol) return LFGPU_OK;
-  const int32_t cap = 8 * kThreads;
-  const double row_us = 0.0003 * (double)A.slots / std::max(A.n, 1);
+  const int kCap = 8 * kWaves, kSmallCap = 2 * kWaves;  // slices
+  std::vector<int32_t> off;
+  LFG_TRY(slice_offsets(s, A, off));
+  const double slice_us = 64 * kSlotUs * (double)A.slots / std::max(A.n, 1);
   auto iterations = [&](const ResidentProblem &q) { return std::sqrt((double)q.n); };
-  std::vector<int32_t> rows(np);
+  auto slices = [&](const ResidentProblem &q) { return (q.n + 63) / 64; };
+  std::vector<int32_t> take(np);  // slices a workgroup
   auto total = [&](double tau) {
     int64_t sum = 0;
     for (size_t k = 0; k < np; ++k) {
-      const double c = tau > 0.0 ? (tau / iterations(probs[k]) - 6.0) / row_us : (double)cap;
-      const int32_t want = (int32_t)std::min<double>((double)cap, std::max(c, 64.0));
-      const int32_t n = (probs[k].n + 63) / 64 * 64;
-      // evenly over the team, whole slices, at most kMaxTeam members
-      const int32_t team = std::min((n + want - 1) / want, cus);
-      rows[k] = ((n + team - 1) / team + 63) / 64 * 64;
-      if (rows[k] > cap) return (int64_t)-1;
-      sum += (n + rows[k] - 1) / rows[k];
+      const double c = tau > 0.0 ? (tau / iterations(probs[k]) - kFixedUs) / slice_us : kCap;
+      const int32_t want = (int32_t)std::min<double>(kCap, std::max(c, 1.0));
+      // evenly over the team, at most kMaxTeam members
+      const int32_t n = slices(probs[k]), team = std::min((n + want - 1) / want, cus);
+      take[k] = (n + team - 1) / team;
+      if (take[k] > kCap) return (int64_t)-1;
+      sum += (n + take[k] - 1) / take[k];
     }
     return sum;
   };
@@ -768,7 +1048,7 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
   if (all <= cus) {
     double lo = 0.0, hi = 0.0;
     for (const ResidentProblem &q : probs)
-      hi = std::max(hi, iterations(q) * (6.0 + row_us * cap));
+      hi = std::max(hi, iterations(q) * (kFixedUs + slice_us * kCap));
     for (int step = 0; step < 12; ++step) {
       const double mid = 0.5 * (lo + hi);
       const int64_t n = total(mid);
@@ -779,29 +1059,42 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
   }
   std::vector<size_t> order(np);
   for (size_t k = 0; k < np; ++k) order[k] = k;
-  auto cost = [&](size_t k) { return iterations(probs[k]) * (6.0 + row_us * rows[k]); };
+  auto cost = [&](size_t k) { return iterations(probs[k]) * (kFixedUs + slice_us * take[k]); };
   std::stable_sort(order.begin(), order.end(),
                    [&](size_t i, size_t j) { return cost(i) > cost(j); });
-  std::vector<EllJob> jobs(np);
-  std::vector<EllPart> parts;
+  const bool small = *std::max_element(take.begin(), take.end()) <= kSmallCap;
+  // the small kernel if every part's LDS holds what it keeps of the outside rows
+  std::vector<EllJob> jobs;
   std::vector<int2> slots;
-  int32_t most = 0;
-  for (size_t o = 0; o < np; ++o) {
-    const ResidentProblem &q = probs[order[o]];
-    const int32_t R = rows[order[o]], end = q.lo + (q.n + 63) / 64 * 64;
-    EllJob &j = jobs[o];
-    j.index = q.index;
-    j.team = (end - q.lo + R - 1) / R;
-    j.sums_at = (uint32_t)p->sums_words;
-    p->sums_words += part_words(j.team) + kTotalWords;
-    most = std::max(most, R);
-    for (int r = 0; r < j.team; ++r) {
-      parts.push_back(EllPart{q.lo + r * R, std::min(q.lo + (r + 1) * R, end), R, 0, 0});
-      slots.push_back(int2{(int)o, r});
+  bool fits = false;
+  for (const auto &[rpt, windows] : {std::pair<int, bool>{2, true}, {2, false}, {8, false}}) {
+    if (rpt == 2 && !small) continue;
+    Split split;
+    jobs.clear();
+    slots.clear();
+    p->sums_words = 0;
+    for (size_t o = 0; o < np; ++o) {
+      const ResidentProblem &q = probs[order[o]];
+      const int32_t s0 = q.lo / 64, s1 = s0 + slices(q), each = take[order[o]];
+      const size_t had = split.parts.size();
+      if (!windows || !split_windows(split, off, s0, s1, each, cus, A.n))
+        split_runs(split, s0, s1, each, A.n);
+      EllJob j{};
+      j.index = q.index;
+      j.team = (int32_t)(split.parts.size() - had);
+      j.sums_at = (uint32_t)p->sums_words;
+      p->sums_words += part_words(j.team) + kTotalWords;
+      jobs.push_back(j);
+      for (int r = 0; r < j.team; ++r) slots.push_back(int2{(int)o, r});
+    }
+    // (shares of windows may take more workgroups than planned)
+    if (windows && all <= cus && split.parts.size() > (size_t)cus) continue;
+    LFG_TRY(ell_split(s, p, A, split, rpt, &fits));
+    if (fits) {
+      p->rpt = rpt;
+      break;
     }
   }
-  bool fits = false;
-  LFG_TRY(ell_split(s, p, A, parts, &fits));
   if (!fits) return LFGPU_OK;
   LFG_TRY(dalloc(&p->jobs, np, "resident batch jobs"));
   LFG_TRY(dalloc(&p->slots, slots.size(), "resident batch slots"));
@@ -811,7 +1104,6 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
   LFG_HIP(hipMemcpyAsync(p->slots, slots.data(), slots.size() * sizeof(int2),
                          hipMemcpyHostToDevice, s));
   LFG_HIP(hipStreamSynchronize(s));
-  p->rpt = most <= 2 * kThreads ? 2 : 8;
   return LFGPU_OK;
 }
 
@@ -822,8 +1114,9 @@ int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *
   hipStream_t s = ctx->stream;
   EllArgs a{};
   // (the problems' sums have their own words; they are cleared with the rest)
-  const bool fresh = resident_will_clear(bufs, (size_t)4 * A.n, ell_tags(opts));
-  LFG_TRY(resident_prepare(s, bufs, (size_t)4 * A.n, ell_tags(opts), &a.tag0));
+  const size_t words = (size_t)2 * planes(plan->rpt) * A.n;
+  const bool fresh = resident_will_clear(bufs, words, ell_tags(opts));
+  LFG_TRY(resident_prepare(s, bufs, words, ell_tags(opts), &a.tag0));
   if (fresh) LFG_TRY(resident_clear(s, plan->sums, plan->sums_words));
   // the counter and the abort flag
   LFG_TRY(resident_clear(s, reinterpret_cast<unsigned long long *>(plan->ticket), 2));
@@ -838,7 +1131,7 @@ int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *
   a.ticket = plan->ticket;
   return resident_launch_team(s, kEllBatch[plan->rpt == 2 ? 0 : 1][opts.mode],
                               std::min(plan->nparts, std::min(ctx->cus, kMaxTeam)), &a,
-                              (size_t)plan->most * sizeof(double), taken);
+                              plan->lds, taken);
 }
 
 }  // namespace lfgpu

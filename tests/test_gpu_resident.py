@@ -185,6 +185,50 @@ def test_resident_pcg_on_ell(ctx, S, L, mode):
     A.close()
 
 
+def _kinds_system(S, L, seed):
+    """A system with three kinds of rows, numbered kind by kind as third-order
+    DOFs are: the lattice's vertices (up to 24 neighbours), two nodes on every
+    edge and one in every triangle (three each); weights as _lattice_system."""
+    rng = np.random.default_rng(seed)
+    v = np.arange(S * L).reshape(L, S)
+    e = np.concatenate([np.stack([a.ravel(), b.ravel()], 1) for a, b in (
+        (v[:, :-1], v[:, 1:]), (v[:-1], v[1:]), (v[:-1, :-1], v[1:, 1:]))])
+    t = np.concatenate([np.stack([c.ravel() for c in k], 1) for k in (
+        (v[:-1, :-1], v[:-1, 1:], v[1:, 1:]), (v[:-1, :-1], v[1:, :-1], v[1:, 1:]))])
+    one = v.size + 2 * np.arange(len(e))  # an edge's first node
+    mid = v.size + 2 * len(e) + np.arange(len(t))
+    pairs = np.concatenate([e, np.stack([one, one + 1], 1)]
+                           + [np.stack([e[:, k], one + m], 1) for k in (0, 1) for m in (0, 1)]
+                           + [np.stack([t[:, k], mid], 1) for k in (0, 1, 2)])
+    n = v.size + 2 * len(e) + len(t)
+    i, j = pairs.T
+    w = np.exp(rng.standard_normal(i.size))
+    diag = np.full(n, 1e-3)
+    np.add.at(diag, i, w)
+    np.add.at(diag, j, w)
+    k = np.arange(n)
+    return np.concatenate([i, j, k]), np.concatenate([j, i, k]), np.concatenate([-w, -w, diag]), n
+
+
+# rows of several lengths: one part, parts with their share of every length
+# (one to three rows a thread, rows longer than what stays in registers) and
+# runs of rows
+@pytest.mark.parametrize("S, L", [(5, 4), (12, 10), (40, 41), (130, 129), (160, 150), (200, 190),
+                                  (230, 220)])
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_pcg_on_rows_of_several_lengths(ctx, S, L, mode):
+    r, c, v, n = _kinds_system(S, L, S)
+    A = capi.coo_to_csr(ctx, r, c, v, n, n)
+    out = _compare(ctx, A, n, mode, n + 1)
+    assert capi.solver_storage(A)[0] == capi.STORAGE_ELL16 and out[1][0].syncs == 1
+    x0 = np.random.default_rng(5).standard_normal(n)
+    out = _compare(ctx, A, n, mode, n + 2, x0=x0, maxit=3, rtol=1e-14)
+    assert out[0][0].iters == out[1][0].iters == 3
+    eps = 1e-13 if mode == capi.PCG_FP64 else 1e-5 if mode == capi.PCG_MIXED else 1e-12
+    assert np.linalg.norm(out[0][1] - out[1][1]) <= eps * np.linalg.norm(out[0][1])
+    A.close()
+
+
 def test_wrapped_band_matrix_keeps_the_sweeps(ctx):
     # the offsets of a lattice, but entries across the lines' ends
     n, S = 4096, 64
