@@ -49,6 +49,7 @@ struct ResidentDia {
   const int32_t *off = nullptr;
   const double *val = nullptr, *rowsum = nullptr, *dinv = nullptr;
   bool sym = false;  // lower diagonals equal the mirrored upper ones bit for bit
+  bool diag = false;  // 1 / dinv is the row sum less the off-diagonal values, to 1e-13
   // mixed modes: the FP32 copies, D^-1 in bfloat16 (FP32 vectors) or FP32,
   // and the solution's low part
   const float *val32 = nullptr, *rowsum32 = nullptr, *dinv32 = nullptr;

@@ -10,7 +10,7 @@
 // above, the matrix is streamed once an iteration.  Time per iteration, P1,
 // sweeps against this, in us:
 //              64^2   512^2   1023x770   1024^2   2048x256   1400^2   2048^2
-//   FP64     12.6/2.4 17.6/3.4 29.8/4.8 32.0/6.3  20.8/4.0 55.1/20.0  101/43
+//   FP64     12.6/2.4 17.6/3.4 29.8/4.8 32.0/6.3  20.8/4.0 55.1/14.4  101/37
 //   FP32     15.2/3.5 14.4/4.1 19.6/5.3 21.8/6.1  17.0/4.7 31.6/13.9 57.6/28
 //   FP32 mat 17.4/3.8 16.7/4.2 24.3/5.4 30.5/6.4  21.1/4.7 46.6/13.6 85.3/49
 //
@@ -204,6 +204,17 @@ struct Tile {
       }
     }
   }
+  // The same from an array with a value for every slot.
+  template <class VT>
+  __device__ __forceinline__ void publish_slots(const VT *src, int first) const {
+    static_assert(sizeof(VT) == 8, "two words a value");
+    if ((int)threadIdx.x < first) return;
+    word_t *w = words + ((size_t)(tag & 1u) * team + rank) * 2 * slots;
+    for (int32_t s = (int32_t)threadIdx.x - first; s < np; s += kThreads - first) {
+      put(&w[s], low_word(src[s], tag));
+      put(&w[slots + s], high_word(src[s], tag));
+    }
+  }
   // Waits for the halo cells and hands (h, place, value) to fn, two cells per
   // thread in flight, with the threads from `first` on.
   template <class VT, class F>
@@ -261,8 +272,8 @@ struct Tile {
 //     sums and arrives while the team sum runs, which takes the exchange off
 //     the iteration's critical path.
 //   STREAM: the matrix (its upper half: symmetric values) is read from memory
-//     every iteration, the next row's loads in flight while a row is worked
-//     on; p travels between the update and the next product.
+//     every iteration, the next rows' loads in flight while a row is worked
+//     on; in the mixed modes p travels between the update and the next product.
 enum { GHOST, STREAM };
 
 // From this many cells a thread the GHOST variants keep row sums and D^-1 in
@@ -315,18 +326,15 @@ struct TileLds {
   }
 };
 
-// RPT: cells per thread.  XR: the cells j < XR keep their x in a register, the
-// others' is read and written in every update (as many as the registers hold
-// without spills).  AHEAD: rows of a stream in flight.
-template <int KIND, int RPT, int XR, int AHEAD, bool BATCH>
+// GHOST in FP64.  RPT: cells per thread.
+template <int RPT, bool BATCH>
 __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team, double *dyn,
                                            SumLds &sh) {
-  constexpr bool kStream = KIND == STREAM, kGhost = KIND == GHOST;
   const int t = threadIdx.x;
   Tile T(a, rank, team);
-  typedef TileLds<KIND, double, RPT> Lds;
+  typedef TileLds<GHOST, double, RPT> Lds;
   const Lds M(dyn, a, T);
-  constexpr bool kRegDiag = !kStream && !Lds::kDiag;
+  constexpr bool kRegDiag = !Lds::kDiag;
   double *const lp = M.lp;
   // (a batch's smaller tiles leave the last cell numbers empty)
   const int nj = BATCH ? (T.th * T.P + kThreads - 1) / kThreads : RPT;
@@ -335,43 +343,36 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
   T.tables(t);
   const int32_t cells = Lds::cells(a.TW);
   for (int32_t i = t; i < cells; i += kThreads) lp[i] = 0.0;
-  if constexpr (kGhost)
-    for (int32_t h = t; h < T.ng; h += kThreads) M.gr[h] = M.gq[h] = M.gd[h] = 0.0;
+  for (int32_t h = t; h < T.ng; h += kThreads) M.gr[h] = M.gq[h] = M.gd[h] = 0.0;
   const int32_t at0 = T.P + 1 + t;  // LDS place of the thread's first cell
 
-  double x[XR > 0 ? XR : 1], r[RPT], q[RPT];
-  double v[kStream ? 1 : RPT][ND], rs[kRegDiag ? RPT : 1], di[kRegDiag ? RPT : 1];
+  double x[RPT], r[RPT], q[RPT];
+  double v[RPT][ND], rs[kRegDiag ? RPT : 1], di[kRegDiag ? RPT : 1];
   uint64_t live = 0;  // the thread's cells that are rows of the tile
   __syncthreads();
   {
     Tile::Walk w = T.first(t);
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
-      r[j] = q[j] = 0.0;
-      if (j < XR) x[j] = 0.0;
-      if constexpr (!kStream) {
-        if constexpr (kRegDiag) rs[j] = di[j] = 0.0;
-        else M.rs[t + j * kThreads] = M.di[t + j * kThreads] = 0.0;
+      r[j] = q[j] = x[j] = 0.0;
+      if constexpr (kRegDiag) rs[j] = di[j] = 0.0;
+      else M.rs[t + j * kThreads] = M.di[t + j * kThreads] = 0.0;
 #pragma unroll
-        for (int d = 0; d < ND; ++d) v[j][d] = 0.0;
-      }
+      for (int d = 0; d < ND; ++d) v[j][d] = 0.0;
       if (T.alive(w)) {
         live |= 1ull << j;
-        const double xi = a.x[w.g];
-        if (j < XR) x[j] = xi;
-        lp[at0 + j * kThreads] = xi;
-        if constexpr (!kStream) {
-          if constexpr (kRegDiag) {
-            rs[j] = a.rowsum[w.g];
-            di[j] = a.dinv[w.g];
-          } else {
-            M.rs[t + j * kThreads] = a.rowsum[w.g];
-            M.di[t + j * kThreads] = a.dinv[w.g];
-          }
-#pragma unroll
-          for (int d = 0; d < ND; ++d)
-            if (d < a.ndiag) v[j][d] = a.val[(int64_t)d * a.n + w.g];
+        x[j] = a.x[w.g];
+        lp[at0 + j * kThreads] = x[j];
+        if constexpr (kRegDiag) {
+          rs[j] = a.rowsum[w.g];
+          di[j] = a.dinv[w.g];
+        } else {
+          M.rs[t + j * kThreads] = a.rowsum[w.g];
+          M.di[t + j * kThreads] = a.dinv[w.g];
         }
+#pragma unroll
+        for (int d = 0; d < ND; ++d)
+          if (d < a.ndiag) v[j][d] = a.val[(int64_t)d * a.n + w.g];
       }
       T.next(w);
       __builtin_amdgcn_sched_barrier(0);
@@ -388,75 +389,24 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
     const double *bp[ND];
 #pragma unroll
     for (int d = 0; d < ND; ++d) bp[d] = lc + a.shift[d];
-    if constexpr (!kStream) {
-      const double *lrs = M.rs + opaque(t), *ldi = M.di + opaque(t);
+    const double *lrs = M.rs + opaque(t), *ldi = M.di + opaque(t);
 #pragma unroll
-      for (int j = 0; j < RPT; ++j) {
-        if (BATCH && j >= nj) break;
-        // every LDS read of the row before the first use
-        const double pi = lc[j * kThreads];
-        double c[ND], acc = 0.0;
+    for (int j = 0; j < RPT; ++j) {
+      if (BATCH && j >= nj) break;
+      // every LDS read of the row before the first use
+      const double pi = lc[j * kThreads];
+      double c[ND], acc = 0.0;
 #pragma unroll
-        for (int d = 0; d < ND; ++d) c[d] = bp[d][j * kThreads];
-        const double s = kRegDiag ? rs[kRegDiag ? j : 0] : lrs[j * kThreads];
-        const double dv = kRegDiag ? di[kRegDiag ? j : 0] : ldi[j * kThreads];
-        __builtin_amdgcn_sched_barrier(0);
+      for (int d = 0; d < ND; ++d) c[d] = bp[d][j * kThreads];
+      const double s = kRegDiag ? rs[kRegDiag ? j : 0] : lrs[j * kThreads];
+      const double dv = kRegDiag ? di[kRegDiag ? j : 0] : ldi[j * kThreads];
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int d = 0; d < ND; ++d) acc = __builtin_fma(v[j][d], c[d] - pi, acc);
-        q[j] = __builtin_fma(s, pi, acc);
-        pin(q[j]);
-        fn(j, pi, dv);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-      // the next rows of the stream: the diagonals (the lower ones as the
-      // mirrored upper ones: zero before the first row), row sum and D^-1
-      double nv[AHEAD][ND], ns[AHEAD], nd[AHEAD];
-      Tile::Walk w = T.first(opaque(t));
-      auto load_row = [&](int j) {
-        const int k = j % AHEAD;
-        const int32_t g = (live >> j) & 1 ? w.g : T.g0;
-        const uint32_t at = (uint32_t)g * 8u;
-#pragma unroll
-        for (int d = 0; d < ND; ++d) {
-          if (d < ND / 2)
-            nv[k][d] =
-                load_at(a.val + (int64_t)(ND - 1 - d) * a.n, (uint32_t)max(g + a.off[d], 0) * 8u);
-          else
-            nv[k][d] = load_at(a.val + (int64_t)d * a.n, at);
-        }
-        if (T.y0 == 0) {
-#pragma unroll
-          for (int d = 0; d < ND / 2; ++d)
-            if (g + a.off[d] < 0) nv[k][d] = 0.0;
-        }
-        ns[k] = load_at(a.rowsum, at);
-        nd[k] = load_at(a.dinv, at);
-        T.next(w);
-      };
-#pragma unroll
-      for (int j = 0; j < AHEAD; ++j) load_row(j);
-#pragma unroll
-      for (int j = 0; j < RPT; ++j) {
-        double vr[ND];
-#pragma unroll
-        for (int d = 0; d < ND; ++d) vr[d] = nv[j % AHEAD][d];
-        const double s = ns[j % AHEAD], dv = nd[j % AHEAD];
-        const double pi = lc[j * kThreads];
-        double c[ND], acc = 0.0;
-#pragma unroll
-        for (int d = 0; d < ND; ++d) c[d] = bp[d][j * kThreads];
-        if (AHEAD == 1 && j + 1 < RPT) load_row(j + 1);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int d = 0; d < ND; ++d) acc = __builtin_fma(vr[d], c[d] - pi, acc);
-        const double qi = __builtin_fma(s, pi, acc);
-        q[j] = (live >> j) & 1 ? qi : 0.0;
-        pin(q[j]);
-        fn(j, pi, dv);
-        __builtin_amdgcn_sched_barrier(0);
-        if (AHEAD > 1 && j + AHEAD < RPT) load_row(j + AHEAD);
-      }
+      for (int d = 0; d < ND; ++d) acc = __builtin_fma(v[j][d], c[d] - pi, acc);
+      q[j] = __builtin_fma(s, pi, acc);
+      pin(q[j]);
+      fn(j, pi, dv);
+      __builtin_amdgcn_sched_barrier(0);
     }
   };
 
@@ -471,11 +421,9 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
       if ((live >> j) & 1) {
         const double bi = a.b[w.g];
         r[j] = bi - q[j];
-        const double z =
-            (kRegDiag ? di[kRegDiag ? j : 0] : kStream ? a.dinv[w.g] : M.di[t + j * kThreads]) *
-            r[j];
+        const double z = (kRegDiag ? di[kRegDiag ? j : 0] : M.di[t + j * kThreads]) * r[j];
         lp[at0 + j * kThreads] = z;
-        if constexpr (kGhost) M.lq[at0 + j * kThreads] = r[j];
+        M.lq[at0 + j * kThreads] = r[j];
         bb = __builtin_fma(bi, bi, bb);
         rr = __builtin_fma(r[j], r[j], rr);
         rz = __builtin_fma(r[j], z, rz);
@@ -484,20 +432,18 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
       __builtin_amdgcn_sched_barrier(0);
     }
   }
-  if constexpr (kGhost) {
-    // the halo cells' r, D^-1 and p = D^-1 r
-    __syncthreads();
-    ++T.tag;
-    T.template publish<double>(M.lq, 0);
-    T.template fetch<double>(0, &sh.bad, [&](int32_t h, int32_t at, double rv) {
-      const int32_t cell = at - T.P - 1 + T.P;  // from the line above the tile
-      const int32_t line = cell / T.P - 1, c = cell - (line + 1) * T.P;
-      const double d = a.dinv[T.g0 + line * T.S + c - 1];
-      M.gr[h] = rv;
-      M.gd[h] = d;
-      lp[at] = d * rv;
-    });
-  }
+  // the halo cells' r, D^-1 and p = D^-1 r
+  __syncthreads();
+  ++T.tag;
+  T.template publish<double>(M.lq, 0);
+  T.template fetch<double>(0, &sh.bad, [&](int32_t h, int32_t at, double rv) {
+    const int32_t cell = at - T.P - 1 + T.P;  // from the line above the tile
+    const int32_t line = cell / T.P - 1, c = cell - (line + 1) * T.P;
+    const double d = a.dinv[T.g0 + line * T.S + c - 1];
+    M.gr[h] = rv;
+    M.gd[h] = d;
+    lp[at] = d * rv;
+  });
   int iter = 0, converged = 0;
   bool run = true, ok;
   double thr, rr_out;
@@ -518,27 +464,21 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
   for (int k = 0; run && ok; ++k) {
     double s[5] = {0.0, 0.0, 0.0, rr, rz};
     __syncthreads();
-    if constexpr (kStream) {
-      T.template exchange<double>(lp, &sh.bad);
-      __syncthreads();
-    }
     double *lqc = M.lq + opaque(at0);
     sweep([&](int j, double pi, double dv) {
-      if constexpr (kGhost) lqc[j * kThreads] = q[j];
+      lqc[j * kThreads] = q[j];
       const double dq = dv * q[j];
       s[0] = __builtin_fma(pi, q[j], s[0]);
       s[1] = __builtin_fma(dq, r[j], s[1]);
       s[2] = __builtin_fma(dq, q[j], s[2]);
       pin(s[0]), pin(s[1]), pin(s[2]);
     });
-    if constexpr (kGhost) ++T.tag;
+    ++T.tag;
     ok = team_sum(tm, sh, s, [&] {
-      if constexpr (kGhost) {
-        const int first = sums_threads(tm);
-        T.template publish<double>(M.lq, first);
-        T.template fetch<double>(first, &sh.bad,
-                                 [&](int32_t h, int32_t, double qv) { M.gq[h] = qv; });
-      }
+      const int first = sums_threads(tm);
+      T.template publish<double>(M.lq, first);
+      T.template fetch<double>(first, &sh.bad,
+                               [&](int32_t h, int32_t, double qv) { M.gq[h] = qv; });
     });
     if (!ok) break;
     rr_out = s[3];
@@ -554,54 +494,341 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
     const double beta = rho_next / rho;
     rr = rz = 0.0;
     double *lc = lp + opaque(at0);
-    // the next row's streamed values
-    double nd = 0.0, nx = 0.0;
-    Tile::Walk w = T.first(opaque(t));
-    uint32_t xat = 0, nxat = 0;
-    auto load_update = [&](int j) {
-      if constexpr (kStream) {
-        nxat = (uint32_t)((live >> j) & 1 ? w.g : T.g0) * 8u;
-        nd = load_at(a.dinv, nxat);
-        if (j >= XR) nx = load_at(a.x, nxat);
-        T.next(w);
-      }
-    };
-    load_update(0);
     const double *ldi = M.di + opaque(t);
     double np = lc[0];
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
       if (BATCH && j >= nj) break;
-      const double dv = kRegDiag ? di[kRegDiag ? j : 0] : kStream ? nd : ldi[j * kThreads];
-      const double xi = j < XR ? x[j < XR ? j : 0] : nx;
-      xat = nxat;
+      const double dv = kRegDiag ? di[kRegDiag ? j : 0] : ldi[j * kThreads];
       const double pi = np;
-      if (j + 1 < RPT) {
-        load_update(j + 1);
-        np = lc[(j + 1) * kThreads];
-      }
+      if (j + 1 < RPT) np = lc[(j + 1) * kThreads];
       // (cells that are no rows: r, q and so their sums stay zero)
-      const double xn = __builtin_fma(alpha, pi, xi);
-      if (j < XR) x[j < XR ? j : 0] = xn;
+      x[j] = __builtin_fma(alpha, pi, x[j]);
       r[j] = __builtin_fma(-alpha, q[j], r[j]);
       const double z = dv * r[j];
       const double p = __builtin_fma(beta, pi, z);
       rr = __builtin_fma(r[j], r[j], rr);
       rz = __builtin_fma(r[j], z, rz);
-      if ((live >> j) & 1) {
-        lc[j * kThreads] = p;
-        if (j >= XR) *reinterpret_cast<double *>(reinterpret_cast<char *>(a.x) + xat) = xn;
-      }
+      if ((live >> j) & 1) lc[j * kThreads] = p;
       pin(r[j]), pin(rr), pin(rz);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (kGhost) {
-      for (int32_t h = t; h < T.ng; h += kThreads) {
-        const int32_t at = T.gpos[h];
-        const double rn = __builtin_fma(-alpha, M.gq[h], M.gr[h]);
-        M.gr[h] = rn;
-        lp[at] = __builtin_fma(beta, lp[at], M.gd[h] * rn);
+    for (int32_t h = t; h < T.ng; h += kThreads) {
+      const int32_t at = T.gpos[h];
+      const double rn = __builtin_fma(-alpha, M.gq[h], M.gr[h]);
+      M.gr[h] = rn;
+      lp[at] = __builtin_fma(beta, lp[at], M.gd[h] * rn);
+    }
+  }
+  if (ok) {
+    Tile::Walk w = T.first(opaque(t));
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      if ((live >> j) & 1) a.x[w.g] = bb == 0.0 ? 0.0 : x[j];
+      T.next(w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  if (T.rank == 0 && t == 0) {
+    a.st->rr = rr_out;
+    a.st->bb = bb;
+    a.st->iter = iter;
+    a.st->converged = converged;
+    a.st->refinements = 0;
+    a.st->aborted = ok ? 0 : 1;
+  }
+  return ok;
+}
+
+template <int RPT>
+__global__ __launch_bounds__(kThreads) void k_res_tile(TileArgs a) {
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  (void)tile_solve<RPT, false>(a, blockIdx.x, gridDim.x, dyn, sh);
+}
+
+// The streamed solve in FP64.  What bounds it is the matrix's trip through the
+// chip's caches every iteration, so that it reads as little as it can: the
+// three upper diagonals and the row sums (32 B a row), from which the lower
+// ones (symmetric values), the diagonal (row sum minus the others) and D^-1
+// follow.  z = D^-1 r and D^-1 q take the places of r and q, so that the update
+// needs no D^-1: z -= alpha D^-1 q, p = z + beta p; r = D z is formed in the
+// next product, for its sums.  D^-1 q travels during the team sum as GHOST's q
+// does, from an LDS array of the rim.  Against 64 B a row and an exchange of p between update and product:
+// 1400^2 20.0 -> 14.4, 2048^2 43.3 -> 36.6 us an iteration
+// (18 of them the matrix, 9 the trips of x).  One row of the stream in flight
+// a thread: two take 36.7, three spill.
+//
+// 1 / d to rounding, by Newton's iteration
+__device__ __forceinline__ double reciprocal(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+  return __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+}
+
+template <int RPT>
+struct StreamLds {
+  double *lp;         // padded tile of p
+  double *rim;        // D^-1 q of the rim, by slot, and 64 places for the other cells'
+  double *gz, *gdq;   // the halo cells' z and D^-1 q
+  __device__ __forceinline__ StreamLds(double *base, const TileArgs &a, Tile &T) {
+    lp = base;
+    rim = lp + TileLds<STREAM, double, RPT>::cells(a.TW);
+    gz = rim + a.slots + 64;
+    gdq = gz + a.ghosts;
+    T.gpos = reinterpret_cast<int32_t *>(gdq + a.ghosts);
+    T.gsrc = T.gpos + a.ghosts;
+    T.ppos = T.gsrc + a.ghosts;
+  }
+  static size_t bytes(const TileArgs &a) {
+    return (TileLds<STREAM, double, RPT>::cells(a.TW) + (size_t)a.slots + 64 +
+            2 * (size_t)a.ghosts) *
+               8 +
+           4 * (2 * (size_t)a.ghosts + a.slots) + 16;
+  }
+};
+
+// RPT: cells per thread.  XR: the cells j < XR keep their x in a register, the
+// others' is read and written in every update (as many as the registers hold
+// without spills).  AHEAD: rows of a stream in flight.
+template <int RPT, int XR, int AHEAD>
+__global__ __launch_bounds__(kThreads) void k_res_stream(TileArgs a) {
+  extern __shared__ double dyn[];
+  __shared__ SumLds sh;
+  constexpr int NU = ND / 2;  // upper diagonals: ND / 2.. of a.val
+  const int t = threadIdx.x;
+  Tile T(a, blockIdx.x, gridDim.x);
+  const StreamLds<RPT> M(dyn, a, T);
+  double *const lp = M.lp;
+  Team tm{T.rank, T.team, a.part, a.total, a.abort, a.tag0};
+  if (t == 0) sh.bad = 0;
+  T.tables(t);
+  const int32_t cells = TileLds<STREAM, double, RPT>::cells(a.TW);
+  for (int32_t i = t; i < cells; i += kThreads) lp[i] = 0.0;
+  for (int32_t i = t; i < a.slots; i += kThreads) M.rim[i] = 0.0;
+  for (int32_t h = t; h < T.ng; h += kThreads) M.gz[h] = M.gdq[h] = 0.0;
+  const int32_t at0 = T.P + 1 + t;  // LDS place of the thread's first cell
+
+  double x[XR > 0 ? XR : 1], z[RPT], dq[RPT];
+  uint64_t live = 0;  // the thread's cells that are rows of the tile
+  __syncthreads();
+  {
+    Tile::Walk w = T.first(t);
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      z[j] = dq[j] = 0.0;
+      if (j < XR) x[j] = 0.0;
+      if (T.alive(w)) {
+        live |= 1ull << j;
+        const double xi = a.x[w.g];
+        if (j < XR) x[j] = xi;
+        lp[at0 + j * kThreads] = xi;
       }
+      T.next(w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __syncthreads();
+  T.template exchange<double>(lp, &sh.bad);
+  __syncthreads();
+
+  // the next rows of the stream: the upper diagonals, the lower ones as the
+  // mirrored upper ones (before the first row the last row's, which are zero:
+  // a value changed after its load would be waited for at once), and the row
+  // sum
+  double nv[AHEAD][ND], ns[AHEAD];
+  Tile::Walk lw;
+  auto load_row = [&](int j) {
+    const int k = j % AHEAD;
+    const int32_t g = (live >> j) & 1 ? lw.g : T.g0;
+    const uint32_t at = (uint32_t)g * 8u;
+#pragma unroll
+    for (int d = 0; d < NU; ++d) {
+      const int32_t c = g + a.off[d];
+      nv[k][d] = load_at(a.val + (int64_t)(ND - 1 - d) * a.n, (uint32_t)(c < 0 ? a.n - 1 : c) * 8u);
+      nv[k][NU + d] = load_at(a.val + (int64_t)(NU + d) * a.n, at);
+    }
+    ns[k] = load_at(a.rowsum, at);
+    T.next(lw);
+  };
+  auto prefetch = [&] {
+    lw = T.first(opaque(t));
+#pragma unroll
+    for (int j = 0; j < AHEAD; ++j) load_row(j);
+  };
+  // (A p)_i in difference form from LDS, the diagonal and p_i, handed to fn
+  auto sweep = [&](auto &&fn) {
+    // (LDS instructions reach 64 KB from a register: new bases every 16 rows)
+    const double *lc = lp, *bp[ND];
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      if (j % 16 == 0) {
+        lc = lp + opaque(at0 + j * kThreads);
+#pragma unroll
+        for (int d = 0; d < ND; ++d) bp[d] = lc + a.shift[d];
+      }
+      const int in = j % 16 * kThreads;
+      double vr[ND];
+#pragma unroll
+      for (int d = 0; d < ND; ++d) vr[d] = nv[j % AHEAD][d];
+      const double s = ns[j % AHEAD];
+      const double pi = lc[in];
+      double c[ND], acc = 0.0, diag = s;
+#pragma unroll
+      for (int d = 0; d < ND; ++d) c[d] = bp[d][in];
+      if (AHEAD == 1 && j + 1 < RPT) load_row(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < ND; ++d) {
+        acc = __builtin_fma(vr[d], c[d] - pi, acc);
+        diag -= vr[d];
+      }
+      fn(j, __builtin_fma(s, pi, acc), diag, pi);
+      __builtin_amdgcn_sched_barrier(0);
+      if (AHEAD > 1 && j + AHEAD < RPT) load_row(j + AHEAD);
+    }
+  };
+
+  double rr = 0.0, bb = 0.0;
+  prefetch();
+  sweep([&](int j, double qi, double, double) {
+    dq[j] = (live >> j) & 1 ? qi : 0.0;
+    pin(dq[j]);
+  });
+  __syncthreads();
+  // r = b - A x, z = p = D^-1 r
+  {
+    Tile::Walk w = T.first(opaque(t));
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      if ((live >> j) & 1) {
+        const double bi = a.b[w.g];
+        const double ri = bi - dq[j];
+        z[j] = a.dinv[w.g] * ri;
+        lp[at0 + j * kThreads] = z[j];
+        bb = __builtin_fma(bi, bi, bb);
+        rr = __builtin_fma(ri, ri, rr);
+      }
+      T.next(w);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __syncthreads();
+  ++T.tag;
+  T.template publish<double>(lp, 0);
+  T.template fetch<double>(0, &sh.bad, [&](int32_t h, int32_t at, double v) {
+    M.gz[h] = v;
+    lp[at] = v;
+  });
+  int iter = 0, converged = 0;
+  bool run = true, ok;
+  double thr, rr_out;
+  {
+    double s[2] = {bb, rr};
+    ok = team_sum(tm, sh, s, [] {});
+    bb = s[0];
+    rr_out = s[1];
+    thr = a.tol2 * bb;
+    thr = thr > 2.2250738585072014e-308 ? thr : 2.2250738585072014e-308;
+    if (bb == 0.0 || s[1] < thr) {
+      converged = 1;
+      run = false;
+    } else if (a.maxit <= 0) {
+      run = false;
+    }
+  }
+  for (int k = 0; run && ok; ++k) {
+    double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    __syncthreads();
+    {
+      prefetch();
+      Tile::Walk w = T.first(opaque(t));
+      sweep([&](int j, double qi, double diag, double pi) {
+        const bool row = (live >> j) & 1;
+        qi = row ? qi : 0.0;
+        const double d = row ? reciprocal(diag) * qi : 0.0;
+        const double ri = diag * z[j];
+        dq[j] = d;
+        s[0] = __builtin_fma(pi, qi, s[0]);
+        s[1] = __builtin_fma(qi, z[j], s[1]);
+        s[2] = __builtin_fma(d, qi, s[2]);
+        s[3] = __builtin_fma(ri, ri, s[3]);
+        s[4] = __builtin_fma(ri, z[j], s[4]);
+        const int32_t lx = w.c - 1;
+        const int32_t line = w.line;
+        int32_t to = a.slots + (t & 63);  // (no rim: a place that nobody reads)
+        to = lx == T.tw - 1 ? 2 * T.TW + T.TH + line : to;
+        to = lx == 0 ? 2 * T.TW + line : to;
+        to = line == T.th - 1 ? T.TW + lx : to;
+        to = line == 0 ? lx : to;
+        M.rim[row ? to : a.slots + (t & 63)] = d;
+        T.next(w);
+        pin(dq[j]), pin(s[0]), pin(s[1]), pin(s[2]), pin(s[3]), pin(s[4]);
+      });
+    }
+    ++T.tag;
+    ok = team_sum(tm, sh, s, [&] {
+      const int first = sums_threads(tm);
+      T.template publish_slots<double>(M.rim, first);
+      T.template fetch<double>(first, &sh.bad,
+                               [&](int32_t h, int32_t, double v) { M.gdq[h] = v; });
+    });
+    if (!ok) break;
+    rr_out = s[3];
+    if (s[3] < thr) {
+      converged = 1;
+      iter = k > 0 ? k - 1 : 0;
+      break;
+    }
+    iter = k;
+    if (k >= a.maxit) break;
+    const double rho = s[4], alpha = rho / s[0];
+    const double rho_next = rho - 2.0 * alpha * s[1] + alpha * alpha * s[2];
+    const double beta = rho_next / rho;
+    double *lc = lp;
+    // the streamed x: kX rows in flight
+    constexpr int kX = 4;
+    double nx[kX];
+    uint32_t nat[kX];
+    Tile::Walk w = T.first(opaque(t));
+    auto load_x = [&](int j) {
+      nat[j % kX] = (uint32_t)((live >> j) & 1 ? w.g : T.g0) * 8u;
+      nx[j % kX] = load_at(a.x, nat[j % kX]);
+      T.next(w);
+    };
+    // (streamed cells first: their loads run while the others are updated)
+    if constexpr (XR < RPT) {
+#pragma unroll
+      for (int j = 0; j < XR; ++j) T.next(w);
+#pragma unroll
+      for (int j = XR; j < XR + kX && j < RPT; ++j) load_x(j);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int j = 0; j < RPT; ++j) {
+      if (j % 16 == 0) lc = lp + opaque(at0 + j * kThreads);
+      const int in = j % 16 * kThreads;
+      const double pi = lc[in];
+      if (j < XR) {
+        x[j < XR ? j : 0] = __builtin_fma(alpha, pi, x[j < XR ? j : 0]);
+      } else {
+        const double xn = __builtin_fma(alpha, pi, nx[j % kX]);
+        if ((live >> j) & 1)
+          *reinterpret_cast<double *>(reinterpret_cast<char *>(a.x) + nat[j % kX]) = xn;
+        if (j + kX < RPT) load_x(j + kX);
+      }
+      // (cells that are no rows: z and D^-1 q stay zero)
+      z[j] = __builtin_fma(-alpha, dq[j], z[j]);
+      const double p = __builtin_fma(beta, pi, z[j]);
+      if ((live >> j) & 1) lc[in] = p;
+      pin(z[j]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int32_t h = t; h < T.ng; h += kThreads) {
+      const int32_t at = T.gpos[h];
+      const double zn = __builtin_fma(-alpha, M.gdq[h], M.gz[h]);
+      M.gz[h] = zn;
+      lp[at] = __builtin_fma(beta, lp[at], zn);
     }
   }
   if (ok) {
@@ -624,14 +851,6 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
     a.st->refinements = 0;
     a.st->aborted = ok ? 0 : 1;
   }
-  return ok;
-}
-
-template <int KIND, int RPT, int XR, int AHEAD = 1>
-__global__ __launch_bounds__(kThreads) void k_res_tile(TileArgs a) {
-  extern __shared__ double dyn[];
-  __shared__ SumLds sh;
-  (void)tile_solve<KIND, RPT, XR, AHEAD, false>(a, blockIdx.x, gridDim.x, dyn, sh);
 }
 
 // A batch: the workgroups take slots (a problem and a rank in its team) from
@@ -686,7 +905,7 @@ __global__ __launch_bounds__(kThreads) void k_res_tile_batch(TileArgs base) {
   extern __shared__ double dyn[];
   __shared__ SumLds sh;
   batch_loop(base, [&](const TileArgs &a, int rank, int team) {
-    return tile_solve<GHOST, RPT, RPT, 1, true>(a, rank, team, dyn, sh);
+    return tile_solve<RPT, true>(a, rank, team, dyn, sh);
   });
 }
 
@@ -1091,13 +1310,12 @@ struct TileVariant {
   size_t (*lds)(const TileArgs &);
   void (*fn)(TileArgs);
 };
-#define LFG_TILE(K, R, ...) \
-  {K, R, &TileLds<K, double, R>::bytes, &k_res_tile<K, R, __VA_ARGS__>}
+#define LFG_TILE(R) {GHOST, R, &TileLds<GHOST, double, R>::bytes, &k_res_tile<R>}
 #define LFG_TILEM(K, T, R, A) {K, R, &TileLds<K, T, R>::bytes, &k_res_tile_mixed<K, T, R, A>}
+#define LFG_STREAM(R, ...) {STREAM, R, &StreamLds<R>::bytes, &k_res_stream<R, __VA_ARGS__>}
 const std::vector<TileVariant> kTileVariants[3] = {
-    {LFG_TILE(GHOST, 1, 1), LFG_TILE(GHOST, 3, 3), LFG_TILE(GHOST, 5, 5), LFG_TILE(GHOST, 7, 7),
-     LFG_TILE(GHOST, 9, 9), LFG_TILE(STREAM, 17, 17, 2), LFG_TILE(STREAM, 25, 13, 2),
-     LFG_TILE(STREAM, 33, 0, 2)},
+    {LFG_TILE(1), LFG_TILE(3), LFG_TILE(5), LFG_TILE(7), LFG_TILE(9), LFG_STREAM(17, 17, 1),
+     LFG_STREAM(25, 16, 1), LFG_STREAM(33, 0, 1)},
     {LFG_TILEM(GHOST, float, 1, 1), LFG_TILEM(GHOST, float, 3, 1), LFG_TILEM(GHOST, float, 5, 1),
      LFG_TILEM(GHOST, float, 7, 1), LFG_TILEM(GHOST, float, 9, 1), LFG_TILEM(STREAM, float, 17, 4),
      LFG_TILEM(STREAM, float, 25, 4), LFG_TILEM(STREAM, float, 33, 4)},
@@ -1107,6 +1325,7 @@ const std::vector<TileVariant> kTileVariants[3] = {
      LFG_TILEM(STREAM, double, 25, 3), LFG_TILEM(STREAM, double, 33, 2)},
 };
 #undef LFG_TILE
+#undef LFG_STREAM
 #undef LFG_TILEM
 
 // Splits the lattice a.S x a.L into at most `most` tiles of at most cap padded
@@ -1159,9 +1378,9 @@ void tile_shifts(J &a) {
 }
 
 // the first variant that takes the lattice, or nullptr
-const TileVariant *tile_plan(TileArgs &a, int mode, bool sym, int cus, int *team) {
+const TileVariant *tile_plan(TileArgs &a, int mode, bool sym, bool diag, int cus, int *team) {
   for (const TileVariant &v : kTileVariants[mode]) {
-    if (v.kind == STREAM && !(sym && a.ndiag == ND)) continue;
+    if (v.kind == STREAM && !(sym && a.ndiag == ND && (diag || mode != LFGPU_PCG_FP64))) continue;
     const int64_t cap = (int64_t)v.rpt * kThreads;
     if ((int64_t)a.S * a.L > cap * cus) continue;
     *team = tile_split(a, cap, cus, v.kind == STREAM, v.lds);
@@ -1297,7 +1516,7 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
   a.L = A.n / A.width;
   a.ndiag = A.ndiag;
   int team = 0;
-  const TileVariant *v = tile_plan(a, opts.mode, A.sym, std::min(ctx->cus, kMaxTeam), &team);
+  const TileVariant *v = tile_plan(a, opts.mode, A.sym, A.diag, std::min(ctx->cus, kMaxTeam), &team);
   if (!v) return LFGPU_OK;
   for (int d = 0; d < A.ndiag; ++d) a.off[d] = A.off[d];
   tile_shifts(a);

@@ -95,6 +95,7 @@ struct lfgpu_solver_cache {
   // sweep of the PCG then reads the upper diagonals only (measured 7 %
   // faster at 2048^2; the FP32 sweeps measured slower that way)
   bool sym64 = false;
+  bool diag64 = false;  // the diagonal is the row sum less the others (k_dia_sym)
   // work vectors
   double *r = nullptr, *p = nullptr, *q = nullptr;
   float *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *xa32 = nullptr;
@@ -535,10 +536,13 @@ __global__ void k_fill_vals(const int32_t *row_ptr, const int32_t *col, const do
   if (dinv16) dinv16[r] = __float2bfloat16((float)d);
 }
 
-// flag = 1 if a lower-diagonal value differs, bit for bit, from the
+// flag |= 1 if a lower-diagonal value differs, bit for bit, from the
 // mirrored upper-diagonal value (the offsets are ascending and
-// mirror-symmetric: off[d] = -off[nd-1-d])
-__global__ void k_dia_sym(const double *val, int32_t n, int nd, DiagSet ds, int *flag) {
+// mirror-symmetric: off[d] = -off[nd-1-d]); flag |= 2 if the row sum less the
+// off-diagonal values is not the diagonal that dinv inverts, to 1e-13 (a row
+// without a diagonal, or one that the others cancel)
+__global__ void k_dia_sym(const double *val, const double *rowsum, const double *dinv, int32_t n,
+                          int nd, DiagSet ds, int *flag) {
   const int32_t r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
   bool bad = false;
@@ -548,12 +552,15 @@ __global__ void k_dia_sym(const double *val, int32_t n, int nd, DiagSet ds, int 
     const double b = c >= 0 ? val[(int64_t)(nd - 1 - d) * n + c] : 0.0;
     bad = bad || __double_as_longlong(a) != __double_as_longlong(b);
   }
-  if (bad) atomicOr(flag, 1);
+  double diag = rowsum[r];
+  for (int d = 0; d < nd; ++d) diag -= val[(int64_t)d * n + r];
+  const int bits = (bad ? 1 : 0) | (fabs(diag * dinv[r] - 1.0) <= 1e-13 ? 0 : 2);
+  if (bits) atomicOr(flag, bits);
 }
 
-// Sets the cache's sym64 flag for its current values.
+// Sets the cache's sym64 and diag64 flags for its current values.
 int dia_symmetry(lfgpu_ctx *ctx, lfgpu_solver_cache *c, int32_t n) {
-  c->sym64 = false;
+  c->sym64 = c->diag64 = false;
   if (c->fmt != FMT_DIA || c->ndiag % 2 != 0) return LFGPU_OK;
   for (int d = 0; d < c->ndiag; ++d)
     if (c->off[d] != -c->off[c->ndiag - 1 - d] || (2 * d < c->ndiag && c->off[d] >= 0))
@@ -566,16 +573,17 @@ int dia_symmetry(lfgpu_ctx *ctx, lfgpu_solver_cache *c, int32_t n) {
   LFG_TRY(dalloc(&flag, 1, "symmetry flag"));
   hipError_t e = hipMemsetAsync(flag, 0, 4, s);
   if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_dia_sym, dim3(grid_for(n, 256)), dim3(256), 0, s, c->val, n, c->ndiag,
-                       ds, flag);
+    hipLaunchKernelGGL(k_dia_sym, dim3(grid_for(n, 256)), dim3(256), 0, s, c->val, c->rowsum,
+                       c->dinv, n, c->ndiag, ds, flag);
     e = hipGetLastError();
   }
-  int h = 1;
+  int h = 3;
   if (e == hipSuccess) e = hipMemcpyAsync(&h, flag, 4, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   dfree(flag);
   if (e != hipSuccess) return hip_fail(e, "DIA symmetry check");
-  c->sym64 = h == 0;
+  c->sym64 = (h & 1) == 0;
+  c->diag64 = (h & 2) == 0;
   return LFGPU_OK;
 }
 
@@ -3875,6 +3883,7 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       rd.rowsum = c->rowsum;
       rd.dinv = c->dinv;
       rd.sym = c->sym64;
+      rd.diag = c->diag64;
       rd.val32 = c->val32;
       rd.rowsum32 = c->rowsum32;
       rd.dinv32 = c->dinv32;

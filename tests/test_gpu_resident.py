@@ -146,6 +146,18 @@ def test_resident_pcg_on_large_lattices(ctx, S, L, mode):
     A.close()
 
 
+def test_streamed_lattice_without_a_diagonal_entry_keeps_the_sweeps(ctx):
+    # (the streamed solve takes the diagonal from the row sums)
+    S, L = 1141, 1140
+    r, c, v, n = _lattice_system(S, L, P1, 3)
+    k = np.nonzero((r == c) & (r == n // 2))[0]
+    r, c, v = (np.delete(q, k) for q in (r, c, v))
+    A = capi.coo_to_csr(ctx, r, c, v, n, n)
+    out = _compare(ctx, A, n, capi.PCG_FP64, 1, maxit=3, rtol=1e-14)
+    assert np.array_equal(out[0][1], out[1][1])  # graph replay against plain launches
+    A.close()
+
+
 @pytest.mark.parametrize("mode", MODES)
 def test_resident_pcg_is_deterministic_and_zero_rhs(ctx, mode):
     r, c, v, n = _lattice_system(264, 265, P1, 9)
