@@ -60,6 +60,10 @@ int exclusive_scan_i32(hipStream_t s, const int32_t *in, int32_t *out, int64_t n
 
 }  // namespace lfgpu
 
+namespace lfgpu {
+struct Staging;  // pinned buffers of large downloads (lfgpu_core.hip)
+}
+
 struct lfgpu_ctx {
   int device = 0;
   int cus = 0;  // compute units (the largest team of a resident solve)
@@ -72,7 +76,19 @@ struct lfgpu_ctx {
   // reusable device scratch for reductions (partials + scalars)
   double *red = nullptr;
   size_t red_count = 0;
+  lfgpu::Staging *staging = nullptr;
 };
+
+namespace lfgpu {
+// Copies device arrays to host memory, after what is queued on the context's
+// stream, and waits for them.
+struct Download {
+  void *host;
+  const void *dev;
+  size_t bytes;
+};
+int download(lfgpu_ctx *ctx, const Download *what, int n);
+}  // namespace lfgpu
 
 struct lfgpu_vec {
   lfgpu_ctx *ctx = nullptr;

@@ -55,16 +55,12 @@ extern "C" int lfgpu_csr_info(const lfgpu_csr *A, int32_t *nrows, int32_t *ncols
 extern "C" int lfgpu_csr_download(const lfgpu_csr *A, int32_t *row_ptr, int32_t *col,
                                   double *val) {
   LFG_REQUIRE(A, LFGPU_EINVAL, "NULL matrix");
-  hipStream_t s = A->ctx->stream;
-  if (row_ptr)
-    LFG_HIP(hipMemcpyAsync(row_ptr, A->row_ptr, ((size_t)A->nrows + 1) * 4, hipMemcpyDeviceToHost,
-                           s));
-  if (col && A->nnz)
-    LFG_HIP(hipMemcpyAsync(col, A->col, (size_t)A->nnz * 4, hipMemcpyDeviceToHost, s));
-  if (val && A->nnz)
-    LFG_HIP(hipMemcpyAsync(val, A->val, (size_t)A->nnz * 8, hipMemcpyDeviceToHost, s));
-  LFG_HIP(hipStreamSynchronize(s));
-  return LFGPU_OK;
+  Download what[3];
+  int n = 0;
+  if (row_ptr) what[n++] = {row_ptr, A->row_ptr, ((size_t)A->nrows + 1) * 4};
+  if (col && A->nnz) what[n++] = {col, A->col, (size_t)A->nnz * 4};
+  if (val && A->nnz) what[n++] = {val, A->val, (size_t)A->nnz * 8};
+  return download(A->ctx, what, n);
 }
 
 extern "C" int lfgpu_csr_destroy(lfgpu_csr *A) {
