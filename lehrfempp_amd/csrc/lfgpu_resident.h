@@ -60,10 +60,11 @@ struct ResidentDia {
 // Jacobi-PCG in opts.mode on the context stream (rtol, maxit, mode and the
 // refinement options of lfgpu_pcg), queued without synchronisation; *st
 // (pinned) receives the outcome.  *taken = false (and nothing queued) when
-// the system does not fit the chip.
+// the system does not fit the chip; *ask (unless null) is set then if it would
+// with A.sym and A.diag.
 int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
                      const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
-                     bool *taken);
+                     bool *taken, bool *ask);
 
 // The lattice problems of a batch, side by side in one launch.  st (device)
 // receives the outcome of problem `index` at st[index].

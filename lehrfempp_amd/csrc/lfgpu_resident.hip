@@ -999,16 +999,14 @@ __device__ __forceinline__ bool tile_solve_mixed(const TileArgs &a, int rank, in
       const uint32_t at = (uint32_t)g * 4u;
 #pragma unroll
       for (int d = 0; d < ND; ++d) {
+        // (before the first row the last row's upper values, which are zero: a
+        // value changed after its load would be waited for at once)
+        const int32_t c = g + a.off[d];
         if (d < ND / 2)
-          nv[k][d] =
-              load_at(a.val32 + (int64_t)(ND - 1 - d) * a.n, (uint32_t)max(g + a.off[d], 0) * 4u);
+          nv[k][d] = load_at(a.val32 + (int64_t)(ND - 1 - d) * a.n,
+                             (uint32_t)(c < 0 ? a.n - 1 : c) * 4u);
         else
           nv[k][d] = load_at(a.val32 + (int64_t)d * a.n, at);
-      }
-      if (T.y0 == 0) {
-#pragma unroll
-        for (int d = 0; d < ND / 2; ++d)
-          if (g + a.off[d] < 0) nv[k][d] = 0.0f;
       }
       ns[k] = load_at(a.rowsum32, at);
       nd[k] = mixed_dinv<VT>(a, g);
@@ -1507,7 +1505,7 @@ int resident_launch(hipStream_t s, ResidentBufs *bufs, const void *fn, int team,
 
 int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
                      const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
-                     bool *taken) {
+                     bool *taken, bool *ask) {
   *taken = false;
   if (A.n <= 0 || A.width <= 0 || A.ndiag > ND) return LFGPU_OK;
   TileArgs a{};
@@ -1516,7 +1514,9 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
   a.L = A.n / A.width;
   a.ndiag = A.ndiag;
   int team = 0;
-  const TileVariant *v = tile_plan(a, opts.mode, A.sym, A.diag, std::min(ctx->cus, kMaxTeam), &team);
+  const int cus = std::min(ctx->cus, kMaxTeam);
+  const TileVariant *v = tile_plan(a, opts.mode, A.sym, A.diag, cus, &team);
+  if (!v && ask) *ask = tile_plan(a, opts.mode, true, true, cus, &team) != nullptr;
   if (!v) return LFGPU_OK;
   for (int d = 0; d < A.ndiag; ++d) a.off[d] = A.off[d];
   tile_shifts(a);

@@ -96,6 +96,8 @@ struct lfgpu_solver_cache {
   // faster at 2048^2; the FP32 sweeps measured slower that way)
   bool sym64 = false;
   bool diag64 = false;  // the diagonal is the row sum less the others (k_dia_sym)
+  uint64_t sym_version = ~0ull;  // built values that the two are of
+  int *sym_flag = nullptr;
   // work vectors
   double *r = nullptr, *p = nullptr, *q = nullptr;
   float *r32 = nullptr, *p32 = nullptr, *q32 = nullptr, *xa32 = nullptr;
@@ -135,7 +137,8 @@ void solver_cache_free(lfgpu_csr *A) {
   resident_free(&c->res);
   resident_ell_free(c->res_ell);
   for (void *p : {(void *)c->slice_off, (void *)c->s_col, (void *)c->s_dcol, (void *)c->val, (void *)c->val32,
-                  (void *)c->dinv, (void *)c->dinv32, (void *)c->dinv16, (void *)c->rowsum, (void *)c->rowsum32,
+                  (void *)c->dinv, (void *)c->dinv32, (void *)c->dinv16, (void *)c->rowsum,
+                  (void *)c->rowsum32, (void *)c->sym_flag,
                   (void *)c->r, (void *)c->p, (void *)c->q, (void *)c->r32, (void *)c->p32,
                   (void *)c->q32, (void *)c->xa32, (void *)c->xlo, (void *)c->r64, (void *)c->xa64,
                   (void *)c->part, (void *)c->cg1, (void *)c->rpart, (void *)c->st,
@@ -558,8 +561,13 @@ __global__ void k_dia_sym(const double *val, const double *rowsum, const double 
   if (bits) atomicOr(flag, bits);
 }
 
-// Sets the cache's sym64 and diag64 flags for its current values.
+// Sets the cache's sym64 and diag64 flags for its current values, for those
+// who need them: the FP64 sweeps and the streamed resident solve.  (With every
+// refresh, and with a flag of its own each time, the test took 60 us of a
+// solve on 64^2.)
 int dia_symmetry(lfgpu_ctx *ctx, lfgpu_solver_cache *c, int32_t n) {
+  if (c->sym_version == c->built_version) return LFGPU_OK;
+  c->sym_version = c->built_version;
   c->sym64 = c->diag64 = false;
   if (c->fmt != FMT_DIA || c->ndiag % 2 != 0) return LFGPU_OK;
   for (int d = 0; d < c->ndiag; ++d)
@@ -569,8 +577,8 @@ int dia_symmetry(lfgpu_ctx *ctx, lfgpu_solver_cache *c, int32_t n) {
   ds.ndiag = c->ndiag;
   for (int d = 0; d < kMaxDiag; ++d) ds.off[d] = c->off[d];
   hipStream_t s = ctx->stream;
-  int *flag = nullptr;
-  LFG_TRY(dalloc(&flag, 1, "symmetry flag"));
+  if (!c->sym_flag) LFG_TRY(dalloc(&c->sym_flag, 1, "symmetry flag"));
+  int *flag = c->sym_flag;
   hipError_t e = hipMemsetAsync(flag, 0, 4, s);
   if (e == hipSuccess) {
     hipLaunchKernelGGL(k_dia_sym, dim3(grid_for(n, 256)), dim3(256), 0, s, c->val, c->rowsum,
@@ -580,8 +588,10 @@ int dia_symmetry(lfgpu_ctx *ctx, lfgpu_solver_cache *c, int32_t n) {
   int h = 3;
   if (e == hipSuccess) e = hipMemcpyAsync(&h, flag, 4, hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
-  dfree(flag);
-  if (e != hipSuccess) return hip_fail(e, "DIA symmetry check");
+  if (e != hipSuccess) {
+    c->sym_version = ~0ull;
+    return hip_fail(e, "DIA symmetry check");
+  }
   c->sym64 = (h & 1) == 0;
   c->diag64 = (h & 2) == 0;
   return LFGPU_OK;
@@ -933,9 +943,9 @@ int ensure_cache(lfgpu_ctx *ctx, lfgpu_csr *A, bool need32, bool allow_perm) {
   if (c->built_version != A->val_version) {
     fill_vals_enqueue(s, A, c);
     LFG_HIP(hipGetLastError());
-    LFG_TRY(dia_symmetry(ctx, c, n));
     LFG_TRY(block_setup(ctx, A, c));
     c->built_version = A->val_version;
+    c->sym_version = ~0ull;
   }
   return LFGPU_OK;
 }
@@ -3882,14 +3892,20 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       rd.val = c->val;
       rd.rowsum = c->rowsum;
       rd.dinv = c->dinv;
-      rd.sym = c->sym64;
-      rd.diag = c->diag64;
       rd.val32 = c->val32;
       rd.rowsum32 = c->rowsum32;
       rd.dinv32 = c->dinv32;
       rd.dinv16 = c->dinv16;
       rd.xlo = c->xlo;
-      LFG_TRY(resident_pcg_dia(ctx, &c->res, rd, *opts, b->d, x->d, rs, &taken));
+      for (bool known : {false, true}) {
+        bool ask = false;
+        LFG_TRY(resident_pcg_dia(ctx, &c->res, rd, *opts, b->d, x->d, rs, &taken,
+                                 known ? nullptr : &ask));
+        if (!ask) break;
+        LFG_TRY(dia_symmetry(ctx, c, n));
+        rd.sym = c->sym64;
+        rd.diag = c->diag64;
+      }
     } else {
       ResidentEll re;
       re.n = n;
@@ -3910,6 +3926,7 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
     if (taken) return resident_finish(ctx, &c->res, rs, mixed, info);
   }
 
+  if (!mixed) LFG_TRY(dia_symmetry(ctx, c, n));
   if (single && !c->cg1)
     LFG_TRY(dalloc(&c->cg1, (size_t)6 * n, "single-reduction PCG vectors"));
   // sliced ELL: one-row-per-thread sweeps (k_cgr_*, k_mxr_*) in FP64 and
@@ -4897,6 +4914,7 @@ extern "C" int lfgpu_solver_storage(const lfgpu_csr *A, int *storage, int *ndiag
              : c->s_dcol         ? LFGPU_STORAGE_ELL16
                                  : LFGPU_STORAGE_ELL;
   if (ndiag) *ndiag = c ? c->ndiag : 0;
+  if (sym && c) LFG_TRY(dia_symmetry(A->ctx, const_cast<lfgpu_solver_cache *>(c), A->nrows));
   if (sym) *sym = c && c->sym64 ? 1 : 0;
   return LFGPU_OK;
 }
