@@ -11,8 +11,8 @@
 // sweeps against this, in us:
 //              64^2   512^2   1023x770   1024^2   2048x256   1400^2   2048^2
 //   FP64     12.6/2.4 17.6/3.4 29.8/4.8 32.0/6.3  20.8/4.0 55.1/14.4  101/37
-//   FP32     15.2/3.5 14.4/4.1 19.6/5.3 21.8/6.1  17.0/4.7 31.6/13.9 57.6/28
-//   FP32 mat 17.4/3.8 16.7/4.2 24.3/5.4 30.5/6.4  21.1/4.7 46.6/13.6 85.3/49
+//   FP32     15.2/3.4 14.4/3.9 19.6/5.2 21.8/5.9  17.0/4.6 31.6/13.8 57.6/26
+//   FP32 mat 17.4/3.5 16.7/4.1 24.3/5.2 30.5/6.4  21.1/4.5 46.6/13.2 85.3/47
 //
 // One iteration (the recurrences and the stopping test of the two-sweep
 // solver, with one team sum instead of two):
@@ -915,8 +915,8 @@ __global__ __launch_bounds__(kThreads) void k_res_tile_batch(TileArgs base) {
 // in VT (float: D^-1 in bfloat16; double: D^-1 in FP32), row sums and dot
 // products in FP64.  x (high part) and its low part stay in memory: they are
 // touched by the reliable updates only.  A reliable update forms
-// b - A x - A xa - A xlo in FP64 with the FP64 matrix read from memory, the
-// three vectors passing through LDS one after the other (p waits in the
+// b - A x - A (xa + xlo) in FP64 with the FP64 matrix read from memory, the
+// two vectors passing through LDS one after the other (p waits in the
 // registers of q), folds xa into (x, xlo) by TwoSum and replaces r by the
 // true residual, p by p + M (r_true - r).  The first residual b - A x is the
 // same code.
@@ -1127,7 +1127,7 @@ __device__ __forceinline__ bool tile_solve_mixed(const TileArgs &a, int rank, in
       }
       continue;
     }
-    // reliable update (or the first residual): r64 = b - A x - A xa - A xlo
+    // reliable update (or the first residual): r64 = b - A x - A (xa + xlo)
     double r64[RPT];
     {
       Tile::Walk w = T.first(opaque(t));
@@ -1144,16 +1144,28 @@ __device__ __forceinline__ bool tile_solve_mixed(const TileArgs &a, int rank, in
 #pragma unroll
       for (int j = 0; j < RPT; ++j) bb = __builtin_fma(r64[j], r64[j], bb);
     }
-    for (int part = 0; part < (first ? 1 : 3); ++part) {
+    // (values of memory in groups of rows and the next rows' in flight, each
+    // row waits for its own else; with 7 and 9 cells a thread more than this
+    // spills registers of the iterations)
+    constexpr int G = RPT <= 5 ? RPT : kGhost ? 2 : 4;
+    for (int part = 0; part < (first ? 1 : 2); ++part) {
       __syncthreads();  // the last readers of LDS are done
       {
+        const double *const y = part == 0 ? a.x : a.xlo;
         Tile::Walk w = T.first(opaque(t));
 #pragma unroll
-        for (int j = 0; j < RPT; ++j) {
-          if ((live >> j) & 1)
-            lp[at0 + j * kThreads] =
-                part == 0 ? a.x[w.g] : part == 1 ? (double)xa[j] : a.xlo[w.g];
-          T.next(w);
+        for (int j0 = 0; j0 < RPT; j0 += G) {
+          double yi[G];
+#pragma unroll
+          for (int j = j0; j < j0 + G && j < RPT; ++j) {
+            yi[j - j0] = load_at(y, (uint32_t)((live >> j) & 1 ? w.g : T.g0) * 8u);
+            T.next(w);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int j = j0; j < j0 + G && j < RPT; ++j)
+            if ((live >> j) & 1)
+              lp[at0 + j * kThreads] = part == 0 ? yi[j - j0] : yi[j - j0] + (double)xa[j];
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -1161,23 +1173,32 @@ __device__ __forceinline__ bool tile_solve_mixed(const TileArgs &a, int rank, in
       T.template exchange<double>(lp, &sh.bad);
       __syncthreads();
       {
+        constexpr int kNext = RPT <= 5 ? 2 : 1;
+        double nv[kNext][ND], ns[kNext];
         Tile::Walk w = T.first(opaque(t));
+        auto load_row = [&](int j) {
+          const uint32_t g = (uint32_t)((live >> j) & 1 ? w.g : T.g0) * 8u;
+#pragma unroll
+          for (int d = 0; d < ND; ++d)
+            nv[j % kNext][d] = d < a.ndiag ? load_at(a.val + (int64_t)d * a.n, g) : 0.0;
+          ns[j % kNext] = load_at(a.rowsum, g);
+          T.next(w);
+        };
+#pragma unroll
+        for (int j = 0; j < kNext && j < RPT; ++j) load_row(j);
         const double *lc = lp + opaque(at0);
 #pragma unroll
         for (int j = 0; j < RPT; ++j) {
-          const int32_t g = (live >> j) & 1 ? w.g : T.g0;
           const double yi = lc[j * kThreads];
           double acc = 0.0;
 #pragma unroll
           for (int d = 0; d < ND; ++d)
-            if (d < a.ndiag)
-              acc = __builtin_fma(a.val[(int64_t)d * a.n + g], lc[j * kThreads + a.shift[d]] - yi,
-                                  acc);
-          acc = __builtin_fma(a.rowsum[g], yi, acc);
+            acc = __builtin_fma(nv[j % kNext][d], lc[j * kThreads + a.shift[d]] - yi, acc);
+          acc = __builtin_fma(ns[j % kNext], yi, acc);
           if ((live >> j) & 1) r64[j] -= acc;
           pin(r64[j]);
-          T.next(w);
           __builtin_amdgcn_sched_barrier(0);
+          if (j + kNext < RPT) load_row(j + kNext);
         }
       }
     }
@@ -1201,16 +1222,29 @@ __device__ __forceinline__ bool tile_solve_mixed(const TileArgs &a, int rank, in
       stop = converged || itp >= a.maxit;
       Tile::Walk w = T.first(opaque(t));
 #pragma unroll
-      for (int j = 0; j < RPT; ++j) {
-        if ((live >> j) & 1) {
-          const double hi = a.x[w.g], dx = (double)xa[j];
-          const double sm = hi + dx, bp = sm - hi;
-          const double err = (hi - (sm - bp)) + (dx - bp);
-          a.x[w.g] = sm;
-          a.xlo[w.g] += err;
+      for (int j0 = 0; j0 < RPT; j0 += G) {
+        double hi[G], lo[G];
+        uint32_t at[G];
+#pragma unroll
+        for (int j = j0; j < j0 + G && j < RPT; ++j) {
+          at[j - j0] = (uint32_t)((live >> j) & 1 ? w.g : T.g0) * 8u;
+          hi[j - j0] = load_at(a.x, at[j - j0]);
+          lo[j - j0] = load_at(a.xlo, at[j - j0]);
+          T.next(w);
         }
-        xa[j] = (VT)0;
-        T.next(w);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = j0; j < j0 + G && j < RPT; ++j) {
+          const double h = hi[j - j0], dx = (double)xa[j];
+          const double sm = h + dx, bp = sm - h;
+          const double err = (h - (sm - bp)) + (dx - bp);
+          if ((live >> j) & 1) {
+            *reinterpret_cast<double *>(reinterpret_cast<char *>(a.x) + at[j - j0]) = sm;
+            *reinterpret_cast<double *>(reinterpret_cast<char *>(a.xlo) + at[j - j0]) =
+                lo[j - j0] + err;
+          }
+          xa[j] = (VT)0;
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }

@@ -463,7 +463,7 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
         }
       continue;
     }
-    // the first residual b - A x, or a reliable update's b - A x - A xa - A xlo
+    // the first residual b - A x, or a reliable update's b - A x - A (xa + xlo)
     double r64[RPT];
 #pragma unroll
     for (int j = 0; j < RPT; ++j) {
@@ -476,7 +476,7 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
 #pragma unroll
       for (int j = 0; j < RPT; ++j) bb = __builtin_fma(r64[j], r64[j], bb);
     }
-    for (int turn = 0; turn < (first ? 1 : 3); ++turn) {
+    for (int turn = 0; turn < (first ? 1 : 2); ++turn) {
       if (turn == 0) {
         __syncthreads();  // the last readers of LDS are done
       } else {
@@ -493,7 +493,7 @@ __device__ __forceinline__ bool ell_solve(const EllArgs &a, int32_t slot, int ra
         const int32_t i = ti + j * kThreads;
         if ((live >> j) & 1) {
           const int32_t g = 64 * slice(j) + (ti & 63);
-          const double y = turn == 0 ? a.x[at(g)] : turn == 1 ? (double)x[j] : a.xlo[g];
+          const double y = turn == 0 ? a.x[at(g)] : (double)x[j] + a.xlo[g];
           if (!kMixed) x[j] = (VT)y;
           lp[i] = y;
           if ((needed >> j) & 1) publish(g, y, 0);
