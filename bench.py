@@ -12,8 +12,9 @@ and solved per second over the timed steps (Melem/s).
 
 The default line also carries, as extra keys, the P3 workload (c3) and the
 batched workload (c4) below, each precision mode of every solve, the
-roofline of the dominant kernels (every sweep launch of 200 PCG iterations
-timed by its own hipEvent pair), and, after all device work has finished,
+roofline of the swept solver's kernels (every sweep launch of 200 PCG
+iterations timed by its own hipEvent pair; the timed solves run resident, in
+one launch, which has no launches to bracket), and, after all device work has finished,
 the oracle checks at full size: the oracle (CPU restatement of the
 reference pipeline) builds its own mesh, assembles the same problem in the
 reference's cell order, compares the pattern bit for bit and the values
@@ -26,7 +27,7 @@ Other configurations (each prints its own JSON line):
                     U(-0.2h, 0.2h), degree-6 quadrature, PCG in FP64 and mixed
   --config batched  256 independent P1 problems, sides log-uniform in
                     [32, 512], a = exp(N(0,1)), f = 1, one assembly launch and
-                    one graph-replayed batched PCG
+                    one batched PCG
   --config adjoint  1024 x 1024 P1, J = 1/2 (u - u_obs)^T M (u - u_obs), dJ/dtheta
                     by an adjoint solve, checked against central differences
   --config fkpp     Fisher/KPP Strang splitting (SDIRK-2 diffusion + exact
@@ -459,7 +460,7 @@ def run_p1(args, capi, ctx):
     log("assembly: row-owner %.3f ms, MFMA two-phase %.3f ms"
         % (np.median(asm_ms), np.median(asm_mfma)))
 
-    # roofline of the dominant kernels: the two sweeps of the FP64 iteration,
+    # roofline of the swept solver: the two sweeps of the FP64 iteration,
     # each launch timed between its own hipEvents (and the FP32-Krylov sweeps)
     _, _, sym = capi.solver_storage(P.plan.csr)
     t64, _ = capi.pcg_sweep_times(ctx, P.plan.csr, P.b, P.x, iters=args.sweep_iters)
@@ -519,7 +520,9 @@ def run_p1(args, capi, ctx):
             "dia_gbs_in_solve": roof["iteration"]["algorithmic_bytes"]
             / (float(np.median(pcg_ms)) * 1e-3 / max(1, iters[-1])) / 1e9,
             "csr_formula_bytes": spmv_bytes(P.nnz, P.nv) + 80 * P.nv,
-            "note": "dia_bytes: what the DIA sweeps must move (sweep_bytes); csr_formula_bytes: "
+            "note": "dia_bytes: what the DIA sweeps must move (sweep_bytes; the resident solve "
+                    "keeps most of it on the chip, so that dia_gbs_in_solve passes the memory's "
+                    "rate); csr_formula_bytes: "
                     "the CSR storage figure 12 nnz + 4 (N+1) + 16 N + 80 N, for reference"},
         "oracle": None,
         "cpu_baseline": None,
@@ -714,7 +717,7 @@ def run_batched(args, capi, ctx, nprob=256, seed=4):
     per_mode = {}
     for name, md in modes.items():
         x.fill(0.0)
-        # tunes / captures the graph
+        # (storage and plans are built)
         batch.pcg(b, x, rtol=1e-10, maxit=MAXIT, mode=md, graph=args.batch_graph)
         times = []
         for _ in range(max(1, args.batch_steps)):
@@ -740,10 +743,10 @@ def run_batched(args, capi, ctx, nprob=256, seed=4):
         log("batched %s: %.1f ms/step (pcg %.1f ms), iters %d..%d, %d host syncs"
             % (name, 1e3 * wall, per_mode[name]["pcg_ms"], min(it), max(it), summ.syncs))
         if args.batch_graph == 0:
-            # the step as one captured graph (assembly, value refresh, set-up,
-            # first chunk) plus the captured chunks: lfgpu_batch_assemble_pcg
+            # the step as one call (assembly, value refresh, solve):
+            # lfgpu_batch_assemble_pcg
             x.fill(0.0)
-            batch.assemble_pcg(plan, *acoef, x, rtol=1e-10, maxit=MAXIT, mode=md)  # captures
+            batch.assemble_pcg(plan, *acoef, x, rtol=1e-10, maxit=MAXIT, mode=md)
             ftimes = []
             for _ in range(max(1, args.batch_steps)):
                 ctx.sync()
@@ -759,10 +762,10 @@ def run_batched(args, capi, ctx, nprob=256, seed=4):
             per_mode[name].update({
                 "melem_s": ne / fwall / 1e6, "ms_per_step": 1e3 * fwall,
                 "device_ms": float(np.median([t[1] for t in ftimes])),
-                "host_syncs": int(fs.syncs), "path": "one captured graph per step "
-                "(lfgpu_batch_assemble_pcg) and the captured chunks",
+                "host_syncs": int(fs.syncs), "path": "one call per step "
+                "(lfgpu_batch_assemble_pcg)",
                 "bitwise_equal_to_separate_calls": same, "separate_calls": sep})
-            log("batched %s one graph: %.1f ms/step (device %.1f ms), %d host syncs, "
+            log("batched %s one call: %.1f ms/step (device %.1f ms), %d host syncs, "
                 "bitwise equal to the separate calls: %s"
                 % (name, 1e3 * fwall, per_mode[name]["device_ms"], fs.syncs, same))
     plain = (None if args.no_plain else
@@ -813,8 +816,7 @@ def run_batched_p3(args, capi, ctx, nprob=256, seed=6):
     owns a contiguous row range; a = exp(N(0,1)) per cell, f = 1.  The
     batch storage is sliced ELL (the P3 patterns are not banded), tuned by
     the autotuner for this degree.  Each step: the separate calls
-    (assembly, batched PCG) and one captured graph per step
-    (lfgpu_batch_assemble_pcg)."""
+    (assembly, batched PCG) and one call (lfgpu_batch_assemble_pcg)."""
     rng = np.random.default_rng(seed)
     sizes = np.rint(np.exp(rng.uniform(np.log(8), np.log(64), nprob))).astype(int)
     xs, cs, cds, fls, doff, coff, vo = [], [], [], [], [0], [0], 0
@@ -879,14 +881,13 @@ def run_batched_p3(args, capi, ctx, nprob=256, seed=6):
         wall, fwall = float(np.median(times)), float(np.median(ftimes))
         per_mode[name] = {
             "melem_s": ne / fwall / 1e6, "ms_per_step": 1e3 * fwall, "host_syncs": int(fs.syncs),
-            "path": "one captured graph per step (lfgpu_batch_assemble_pcg) and the captured "
-                    "chunks",
+            "path": "one call per step (lfgpu_batch_assemble_pcg)",
             "bitwise_equal_to_separate_calls": same,
             "separate_calls": {"ms_per_step": 1e3 * wall, "host_syncs": int(summ.syncs)},
             "iters_max": int(max(it)), "iters_min": int(min(it)),
             "refinements_sum": int(sum(i.refinements for i in infos)),
             "converged": bool(fs.converged), "worst_relres": fs.relres}
-        log("batched P3 %s: %.1f ms/step one graph (%d syncs), %.1f ms separate (%d syncs), "
+        log("batched P3 %s: %.1f ms/step one call (%d syncs), %.1f ms separate (%d syncs), "
             "iters %d..%d, bitwise equal %s" % (name, 1e3 * fwall, fs.syncs, 1e3 * wall,
                                                 summ.syncs, min(it), max(it), same))
     out = {"metric": "batched P3 assemble + PCG, Melem/s",
@@ -1356,7 +1357,7 @@ def main():
     ap.add_argument("--c2-only", action="store_true",
                     help="default configuration: only the 2048^2 P1 problem (no P3 / batched)")
     ap.add_argument("--batch-graph", type=int, default=0, choices=[0, -1],
-                    help="batched: 0 replays captured chunks, -1 plain launches")
+                    help="batched: 0 the resident solve, -1 the sweeps by plain launches")
     ap.add_argument("--batch-steps", type=int, default=3,
                     help="batched: timed repetitions per precision mode")
     ap.add_argument("--sweep-iters", type=int, default=200,

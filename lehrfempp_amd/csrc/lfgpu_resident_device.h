@@ -15,7 +15,7 @@
 //
 // Every wait is bounded by the real-time clock: a workgroup that waits longer
 // than kWaitTicks raises the team's abort flag and leaves, the others see the
-// flag in their own waits and leave too.
+// flag in their own waits and leave too; the caller then runs the sweeps.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -94,6 +94,7 @@ struct lfgpu_solver_cache {
   // equal the mirrored upper-diagonal values bit for bit: the FP64 SpMV
   // sweep of the PCG then reads the upper diagonals only (measured 7 %
   // faster at 2048^2; the FP32 sweeps measured slower that way)
+  bool no_resident = false;  // a resident solve was aborted
   bool sym64 = false;
   bool diag64 = false;  // the diagonal is the row sum less the others (k_dia_sym)
   uint64_t sym_version = ~0ull;  // built values that the two are of
@@ -3804,15 +3805,22 @@ int pcg_finish(lfgpu_ctx *ctx, const PcgState *hs, bool mixed, lfgpu_pcg_info *i
   return LFGPU_OK;
 }
 
+// One resident solve at a time on a device: it takes the whole chip, and the
+// launches of several host threads would only wait for each other there.
+std::mutex &resident_turn(const lfgpu_ctx *ctx) {
+  static std::mutex turn[64];
+  return turn[ctx->device & 63];
+}
+
 // end of a resident solve: one wait, then as pcg_finish
 int resident_finish(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentState *rs, bool mixed,
-                    lfgpu_pcg_info *info) {
+                    lfgpu_pcg_info *info, bool *aborted) {
   LFG_HIP(hipEventRecord(ctx->ev1, ctx->stream));
   LFG_HIP(hipEventSynchronize(ctx->ev1));
-  if (rs->aborted) {
+  *aborted = rs->aborted != 0;
+  if (*aborted) {
     bufs->epoch = 0xffffffffu;  // the next solve clears the words and the flag
-    set_error("resident PCG: a workgroup waited over 4 s for another one's values");
-    return LFGPU_EHIP;
+    return LFGPU_OK;
   }
   PcgState h{};
   h.bb = rs->bb;
@@ -3879,9 +3887,10 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
 
   // the resident solve (lfgpu_resident*.hip) where the system fits the chip,
   // unless the caller asked for graph replays or plain launches of the sweeps
-  if (!single && c->blk_n == 0 && opts->graph == 0 && !t_timer) {
+  if (!single && c->blk_n == 0 && opts->graph == 0 && !t_timer && !c->no_resident) {
     ResidentState *rs = reinterpret_cast<ResidentState *>(ctx->pinned);
     bool taken = false;
+    std::lock_guard<std::mutex> turn(resident_turn(ctx));
     LFG_HIP(hipEventRecord(ctx->ev0, s));
     if (c->fmt == FMT_DIA) {
       ResidentDia rd;
@@ -3923,7 +3932,12 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       re.xlo = c->xlo;
       LFG_TRY(resident_pcg_ell(ctx, &c->res, &c->res_ell, re, *opts, b->d, x->d, rs, &taken));
     }
-    if (taken) return resident_finish(ctx, &c->res, rs, mixed, info);
+    if (taken) {
+      // (a workgroup waited over 4 s for another one, as when other processes
+      // hold a part of the chip: the sweeps go on from the x reached)
+      const int rc = resident_finish(ctx, &c->res, rs, mixed, info, &c->no_resident);
+      if (!c->no_resident) return rc;
+    }
   }
 
   if (!mixed) LFG_TRY(dia_symmetry(ctx, c, n));
@@ -4547,7 +4561,8 @@ int batch_resident_ready(lfgpu_batch *bt, const lfgpu_pcg_opts *opts, bool *read
 }
 
 // The whole batch in one launch for its lattices and one for the others.
-// *taken = false: the chip does not hold the teams (nothing was run).
+// *taken = false: the chip does not hold the teams (nothing was run), or a
+// workgroup's wait was aborted.
 int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
                        const lfgpu_pcg_opts *opts, lfgpu_pcg_info *infos,
                        lfgpu_pcg_info *summary, bool *taken) {
@@ -4567,6 +4582,7 @@ int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
   for (int p = 0; p < bt->nprob; ++p) R.h_st[p].converged = 1;
   LFG_HIP(hipMemcpyAsync(R.st, R.h_st, bt->nprob * sizeof(ResidentState), hipMemcpyHostToDevice, s));
   *taken = true;
+  std::lock_guard<std::mutex> turn(resident_turn(ctx));
   if (!R.tiles.empty()) {
     ResidentDia rd;
     rd.n = bt->A->nrows;
@@ -4592,8 +4608,8 @@ int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
       for (ResidentTiles *t : R.plan)
         if (t) resident_tiles_reset(t);
       R.bufs.epoch = 0xffffffffu;
-      set_error("resident batch: a workgroup waited over 4 s for another one's values");
-      return LFGPU_EHIP;
+      *taken = false;  // (as in lfgpu_pcg: the sweeps go on from the x reached)
+      return LFGPU_OK;
     }
   return batch_report_of(
       bt,
