@@ -1013,9 +1013,84 @@ int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan
   return resident_launch(s, bufs, v->fn[opts.mode], plan->nparts, &a, plan->lds, st, taken);
 }
 
-// Team sizes as for the lattice problems (resident_tiles_plan): an iteration
-// takes about 6 us and 0.3 ns a slot of a workgroup's rows.
-constexpr double kFixedUs = 6.0, kSlotUs = 0.0003;
+// The two batch kernels: rows a thread, and what an iteration takes (us, and us
+// a slot of a workgroup's rows).
+struct EllBatchKind {
+  int rpt;
+  double fixed, slot;
+};
+constexpr EllBatchKind kEllBatchKinds[2] = {{2, 2.5, 0.00015}, {8, 6.0, 0.0003}};
+
+// Teams of a batch for one of the kernels.
+struct EllTeams {
+  std::vector<int32_t> take;   // slices a workgroup, by problem
+  std::vector<size_t> order;   // longest problems first
+  int64_t workgroups = 0;
+  double span = 0.0;           // when the last problem ends
+};
+
+// Team sizes as for the lattice problems (resident_tiles_plan); false if a
+// problem's team would not fit the chip.
+bool ell_teams(const std::vector<ResidentProblem> &probs, const EllBatchKind &kind,
+               double slots_per_slice, int cus, EllTeams &out) {
+  const size_t np = probs.size();
+  const int cap = kind.rpt * kWaves;
+  const double slice_us = kind.slot * slots_per_slice;
+  auto iterations = [&](const ResidentProblem &q) { return std::sqrt((double)q.n); };
+  out.take.resize(np);
+  auto team_of = [&](size_t k) {
+    return ((probs[k].n + 63) / 64 + out.take[k] - 1) / out.take[k];
+  };
+  auto total = [&](double tau) {
+    int64_t sum = 0;
+    for (size_t k = 0; k < np; ++k) {
+      const double c = tau > 0.0 ? (tau / iterations(probs[k]) - kind.fixed) / slice_us : cap;
+      const int32_t want = (int32_t)std::min<double>(cap, std::max(c, 1.0));
+      // evenly over the team, at most kMaxTeam members
+      const int32_t n = (probs[k].n + 63) / 64, team = std::min((n + want - 1) / want, cus);
+      out.take[k] = (n + team - 1) / team;
+      if (out.take[k] > cap) return (int64_t)-1;
+      sum += team_of(k);
+    }
+    return sum;
+  };
+  out.workgroups = total(0.0);
+  if (out.workgroups < 0) return false;
+  if (out.workgroups <= cus) {
+    double lo = 0.0, hi = 0.0;
+    for (const ResidentProblem &q : probs)
+      hi = std::max(hi, iterations(q) * (kind.fixed + slice_us * cap));
+    for (int step = 0; step < 12; ++step) {
+      const double mid = 0.5 * (lo + hi);
+      const int64_t n = total(mid);
+      if (n >= 0 && n <= cus) hi = mid;
+      else lo = mid;
+    }
+    out.workgroups = total(hi);
+  }
+  auto cost = [&](size_t k) {
+    return iterations(probs[k]) * (kind.fixed + slice_us * out.take[k]);
+  };
+  out.order.resize(np);
+  for (size_t k = 0; k < np; ++k) out.order[k] = k;
+  std::stable_sort(out.order.begin(), out.order.end(),
+                   [&](size_t i, size_t j) { return cost(i) > cost(j); });
+  // the teams in order, each on the workgroups that are free first
+  std::vector<double> until(cus, 0.0);
+  out.span = 0.0;
+  for (size_t k : out.order) {
+    const int team = team_of(k);
+    std::sort(until.begin(), until.end());
+    const double end = until[team - 1] + cost(k);
+    std::fill(until.begin(), until.begin() + team, end);
+    out.span = std::max(out.span, end);
+  }
+  return true;
+}
+
+// The kernel whose teams end first by that model.  64 P3 problems of 8 to 64
+// cells: two rows a thread, the matrix half in registers, in turns 18.5 ms;
+// eight rows, nearly all problems at once with their matrices streamed, 24.5.
 int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
                             const std::vector<ResidentProblem> &probs, ResidentEllPlan **out) {
   ResidentEllPlan *p = *out = new ResidentEllPlan();
@@ -1023,59 +1098,30 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
   const int cus = std::min(ctx->cus, kMaxTeam);
   const size_t np = probs.size();
   if (np == 0 || !A.dcol) return LFGPU_OK;
-  const int kCap = 8 * kWaves, kSmallCap = 2 * kWaves;  // slices
   std::vector<int32_t> off;
   LFG_TRY(slice_offsets(s, A, off));
-  const double slice_us = 64 * kSlotUs * (double)A.slots / std::max(A.n, 1);
-  auto iterations = [&](const ResidentProblem &q) { return std::sqrt((double)q.n); };
-  auto slices = [&](const ResidentProblem &q) { return (q.n + 63) / 64; };
-  std::vector<int32_t> take(np);  // slices a workgroup
-  auto total = [&](double tau) {
-    int64_t sum = 0;
-    for (size_t k = 0; k < np; ++k) {
-      const double c = tau > 0.0 ? (tau / iterations(probs[k]) - kFixedUs) / slice_us : kCap;
-      const int32_t want = (int32_t)std::min<double>(kCap, std::max(c, 1.0));
-      // evenly over the team, at most kMaxTeam members
-      const int32_t n = slices(probs[k]), team = std::min((n + want - 1) / want, cus);
-      take[k] = (n + team - 1) / team;
-      if (take[k] > kCap) return (int64_t)-1;
-      sum += (n + take[k] - 1) / take[k];
-    }
-    return sum;
-  };
-  const int64_t all = total(0.0);
-  if (all < 0) return LFGPU_OK;
-  if (all <= cus) {
-    double lo = 0.0, hi = 0.0;
-    for (const ResidentProblem &q : probs)
-      hi = std::max(hi, iterations(q) * (kFixedUs + slice_us * kCap));
-    for (int step = 0; step < 12; ++step) {
-      const double mid = 0.5 * (lo + hi);
-      const int64_t n = total(mid);
-      if (n >= 0 && n <= cus) hi = mid;
-      else lo = mid;
-    }
-    (void)total(hi);
-  }
-  std::vector<size_t> order(np);
-  for (size_t k = 0; k < np; ++k) order[k] = k;
-  auto cost = [&](size_t k) { return iterations(probs[k]) * (kFixedUs + slice_us * take[k]); };
-  std::stable_sort(order.begin(), order.end(),
-                   [&](size_t i, size_t j) { return cost(i) > cost(j); });
-  const bool small = *std::max_element(take.begin(), take.end()) <= kSmallCap;
-  // the small kernel if every part's LDS holds what it keeps of the outside rows
+  const double per_slice = 64.0 * (double)A.slots / std::max(A.n, 1);
+  EllTeams teams[2];
+  bool can[2];
+  for (int k = 0; k < 2; ++k) can[k] = ell_teams(probs, kEllBatchKinds[k], per_slice, cus, teams[k]);
+  const int better = can[0] && (!can[1] || teams[0].span <= teams[1].span) ? 0 : 1;
   std::vector<EllJob> jobs;
   std::vector<int2> slots;
   bool fits = false;
-  for (const auto &[rpt, windows] : {std::pair<int, bool>{2, true}, {2, false}, {8, false}}) {
-    if (rpt == 2 && !small) continue;
+  // (the small kernel only if every part's LDS holds what it keeps of the
+  // outside rows; with its share of the windows' lengths a part, or runs)
+  for (int turn = 0; turn < 4 && !fits; ++turn) {
+    const int kind = turn < 2 ? better : 1 - better;
+    const bool windows = turn % 2 == 0;
+    if (!can[kind] || (windows && kind == 1)) continue;
+    const EllTeams &t = teams[kind];
     Split split;
     jobs.clear();
     slots.clear();
     p->sums_words = 0;
     for (size_t o = 0; o < np; ++o) {
-      const ResidentProblem &q = probs[order[o]];
-      const int32_t s0 = q.lo / 64, s1 = s0 + slices(q), each = take[order[o]];
+      const ResidentProblem &q = probs[t.order[o]];
+      const int32_t s0 = q.lo / 64, s1 = s0 + (q.n + 63) / 64, each = t.take[t.order[o]];
       const size_t had = split.parts.size();
       if (!windows || !split_windows(split, off, s0, s1, each, cus, A.n))
         split_runs(split, s0, s1, each, A.n);
@@ -1088,12 +1134,10 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
       for (int r = 0; r < j.team; ++r) slots.push_back(int2{(int)o, r});
     }
     // (shares of windows may take more workgroups than planned)
-    if (windows && all <= cus && split.parts.size() > (size_t)cus) continue;
-    LFG_TRY(ell_split(s, p, A, split, rpt, &fits));
-    if (fits) {
-      p->rpt = rpt;
-      break;
-    }
+    if (windows && t.workgroups <= cus && split.parts.size() > (size_t)cus) continue;
+    p->rpt = 0;
+    LFG_TRY(ell_split(s, p, A, split, kEllBatchKinds[kind].rpt, &fits));
+    if (fits) p->rpt = kEllBatchKinds[kind].rpt;
   }
   if (!fits) return LFGPU_OK;
   LFG_TRY(dalloc(&p->jobs, np, "resident batch jobs"));

@@ -297,3 +297,35 @@ def test_resident_batch(ctx, kind, mode):
         assert np.linalg.norm(xa - xb) <= bound, k
     for h in (batch, b, A):
         h.close()
+
+
+# a problem of more rows than two a thread hold beside a small one (the kernel
+# of eight rows a thread), and problems that the small kernel takes in turns
+@pytest.mark.parametrize("make", [
+    lambda: [_flipped_system(520, 521, 1), _kinds_system(40, 41, 2)],
+    lambda: [_kinds_system(70 + k, 60, k) for k in range(12)],
+])
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_batch_of_large_problems(ctx, make, mode):
+    parts, off = [], [0]
+    for r, c, v, n in make():
+        parts.append((r + off[-1], c + off[-1], v))
+        off.append(off[-1] + n)
+    n = off[-1]
+    A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n, n)
+    bh = np.random.default_rng(3).standard_normal(n)
+    b = capi.Vec(ctx, bh)
+    batch = capi.Batch(ctx, A, np.array(off, np.int32))
+    out = []
+    for graph in (1, 0):
+        x = capi.Vec(ctx, n)
+        summ, _ = batch.pcg(b, x, rtol=1e-10, maxit=20000, mode=mode, graph=graph)
+        assert summ.converged
+        out.append(x.numpy())
+        x.close()
+    assert summ.syncs == 1  # the resident solve ran
+    for lo, hi in zip(off, off[1:]):
+        bound = 2.2e-10 * np.linalg.norm(bh[lo:hi]) / 1e-3
+        assert np.linalg.norm(out[0][lo:hi] - out[1][lo:hi]) <= bound
+    for h in (batch, b, A):
+        h.close()
