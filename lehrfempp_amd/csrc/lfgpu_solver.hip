@@ -3252,7 +3252,8 @@ __global__ void k_bdia_fill(const int32_t *row_ptr, const int32_t *col, const do
     const int32_t c = col[q];
     if (c == r) continue;
     int d = 0;
-    while (d < nd - 1 && off[d] != c - r) ++d;
+    while (d < nd && off[d] != c - r) ++d;
+    if (d == nd) continue;  // (a problem that is not read from its diagonals)
     bval[(int64_t)d * n + r] = val[q];
     if (bval32) bval32[(int64_t)d * n + r] = (float)val[q];
   }
@@ -4274,19 +4275,24 @@ int batch_report_of(lfgpu_batch *bt, Get &&get, int syncs, lfgpu_pcg_info *infos
 namespace {
 
 // bad[p] = 1 if some entry of problem p does not couple lattice neighbours
-// (width[p] rows a line; 0: not looked at)
+// (width[p] rows a line; 0: not looked at) or, with sets (those of
+// k_bdia_mid), has an offset that the problem's set lacks: the set is that of
+// 64 rows, and another row may couple to any of its eight neighbours
 __global__ void k_batch_lattice(const int32_t *row_ptr, const int32_t *col, int32_t n,
                                 const int32_t *row_off, int nprob, const int32_t *width,
-                                int32_t *bad) {
+                                const int32_t *sets, int32_t *bad) {
   const int32_t r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= n) return;
   const int p = batch_prob_of(row_off, nprob, r);
   const int32_t w = width[p], lo = row_off[p];
   if (w <= 0) return;
   const int32_t y = (r - lo) / w, x = (r - lo) - y * w;
+  const int32_t *set = sets ? sets + p * (kMaxDiag + 2) : nullptr;
   for (int32_t q = row_ptr[r]; q < row_ptr[r + 1]; ++q) {
     const int32_t c = col[q] - lo, cy = c / w, cx = c - cy * w;
-    if (abs(cx - x) > 1 || abs(cy - y) > 1) {
+    bool known = !set || col[q] == r;
+    for (int d = 0; !known && d < set[0]; ++d) known = set[1 + d] == col[q] - r;
+    if (!known || abs(cx - x) > 1 || abs(cy - y) > 1) {
       bad[p] = 1;
       return;
     }
@@ -4294,8 +4300,9 @@ __global__ void k_batch_lattice(const int32_t *row_ptr, const int32_t *col, int3
 }
 
 // The problems of the batch that are lattices (as dia_lattice, on each
-// problem's own rows, with its offsets from the rows near its middle), in
-// R.tiles with their offsets, the others in R.rest.
+// problem's own rows, with its offsets from the rows near its middle, which
+// have to cover its entries unless the whole matrix is on DIA), in R.tiles
+// with their offsets, the others in R.rest.
 int batch_find_lattices(lfgpu_batch *bt) {
   lfgpu_csr *A = bt->A;
   lfgpu_batch::Resident &R = bt->res;
@@ -4340,7 +4347,8 @@ int batch_find_lattices(lfgpu_batch *bt) {
     if (e == hipSuccess) e = hipMemsetAsync(dbad, 0, (size_t)np * 4, s);
     if (e == hipSuccess) {
       hipLaunchKernelGGL(k_batch_lattice, dim3(grid_for(n, 256)), dim3(256), 0, s, A->row_ptr,
-                         A->col, n, bt->d_row_off, np, dwidth, dbad);
+                         A->col, n, bt->d_row_off, np, dwidth,
+                         bt->fmt == FMT_DIA ? nullptr : dev, dbad);
       e = hipGetLastError();
     }
     if (e == hipSuccess) e = hipMemcpyAsync(bad.data(), dbad, (size_t)np * 4, hipMemcpyDeviceToHost, s);

@@ -329,3 +329,69 @@ def test_resident_batch_of_large_problems(ctx, make, mode):
         assert np.linalg.norm(out[0][lo:hi] - out[1][lo:hi]) <= bound
     for h in (batch, b, A):
         h.close()
+
+
+def _fixed_band(system, first, last):
+    """The system with rows first..last - 1 fixed (identity rows and columns)."""
+    r, c, v, n = system
+    fixed = np.zeros(n, bool)
+    fixed[first:last] = True
+    keep = (~fixed[r] & ~fixed[c]) | (r == c)
+    r, c, v = r[keep], c[keep], v[keep].copy()
+    v[(r == c) & fixed[r]] = 1.0
+    return r, c, v, n
+
+
+def _turned_lattice(S, L, at, seed):
+    """_lattice_system whose squares below line `at` are cut along the other
+    diagonal."""
+    y = np.arange(L * S) // S
+    r, c, v, n = _lattice_system(S, L, ((1, 0), (0, 1), (1, 1)), seed)
+    r2, c2, v2, _ = _lattice_system(S, L, ((1, 0), (0, 1), (-1, 1)), seed + 1)
+    keep = (abs(r - c) != S + 1) | (np.minimum(y[r], y[c]) >= at)
+    turn = (abs(r2 - c2) == S - 1) & (np.minimum(y[r2], y[c2]) < at)
+    r, c, v = (np.concatenate([a[keep], b[turn]]) for a, b in ((r, r2), (c, c2), (v, v2)))
+    off = r != c
+    v[~off] = 1e-3
+    diag = np.zeros(n)
+    np.subtract.at(diag, r[off], v[off])
+    v[~off] += diag[r[~off]]
+    return r, c, v, n
+
+
+# problems with couplings that the 64 rows from the middle on do not show:
+# another diagonal in a part of the lattice, and fixed rows all over the middle
+# (a line, and lines of a lattice); beside them a problem with all six
+@pytest.mark.parametrize("make", [
+    lambda: [_turned_lattice(81, 81, 20, 1), _lattice_system(20, 30, P1, 2)],
+    lambda: [_turned_lattice(81, 81, 70, 3), _turned_lattice(100, 12, 3, 4)],
+    lambda: [_fixed_band(_lattice_system(400, 1, ((1, 0),), 5), 190, 275),
+             _flipped_system(30, 31, 6)],
+    lambda: [_fixed_band(_lattice_system(90, 40, P1, 7), 1790, 1890), _flipped_system(30, 31, 8),
+             _fixed_band(_lattice_system(300, 1, ((1, 0),), 9), 140, 220),
+             _lattice_system(20, 30, P1, 2)],
+])
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_batch_with_couplings_away_from_the_middle(ctx, make, mode):
+    parts, off = [], [0]
+    for r, c, v, n in make():
+        parts.append((r + off[-1], c + off[-1], v))
+        off.append(off[-1] + n)
+    n = off[-1]
+    A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n, n)
+    bh = np.random.default_rng(3).standard_normal(n)
+    b = capi.Vec(ctx, bh)
+    batch = capi.Batch(ctx, A, np.array(off, np.int32))
+    out = []
+    for graph in (-1, 0):
+        x = capi.Vec(ctx, n)
+        summ, _ = batch.pcg(b, x, rtol=1e-10, maxit=20000, mode=mode, graph=graph)
+        assert summ.converged
+        out.append(x.numpy())
+        x.close()
+    assert summ.syncs == 1  # the resident solve ran
+    for lo, hi in zip(off, off[1:]):
+        bound = 2.2e-10 * np.linalg.norm(bh[lo:hi]) / 1e-3
+        assert np.linalg.norm(out[0][lo:hi] - out[1][lo:hi]) <= bound
+    for h in (batch, b, A):
+        h.close()
