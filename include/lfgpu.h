@@ -61,6 +61,12 @@ int lfgpu_ctx_sync(lfgpu_ctx *ctx);
 /* Device time (hipEvent pair on the context stream) of the most recent
  * assembly / SpMV / PCG call, in milliseconds. */
 int lfgpu_ctx_last_ms(lfgpu_ctx *ctx, double *ms);
+/* Longest time a workgroup of a one-launch solve (lfgpu_pcg_opts.graph) of
+ * this context waits for another one before the whole launch gives up and the
+ * swept solver goes on from the x reached (4 s at first; 0: every such solve
+ * ends that way).  Workgroups wait long only where other processes hold a
+ * part of the GPU. */
+int lfgpu_ctx_set_resident_wait(lfgpu_ctx *ctx, double seconds);
 
 /* ---- device vectors ---------------------------------------------------- */
 int lfgpu_vec_create(lfgpu_ctx *ctx, int64_t n, const double *host_init,
@@ -305,7 +311,8 @@ typedef struct lfgpu_pcg_opts {
    * recurrences (default). */
   int single_reduction;
   /* 0 (default) = the whole solve in one launch with the vectors kept on
-   * the chip where the system fits (any mode; info->syncs is 1 then), else
+   * the chip where the system fits (any mode; info->syncs is 1 then, and at
+   * least 2 where the launch gave up and the sweeps went on), else
    * plain launches, or in FP64 below 2^20 rows, where the solve is bound by
    * the launch rate, replays of each chunk of check_every iterations from a
    * captured hipGraph; 1 = always replay chunks (FP64); -1 = plain launches.

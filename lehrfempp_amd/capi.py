@@ -57,6 +57,7 @@ SIGNATURES = {
     "lfgpu_ctx_destroy": (C.c_int, [_P]),
     "lfgpu_ctx_sync": (C.c_int, [_P]),
     "lfgpu_ctx_last_ms": (C.c_int, [_P, _d]),
+    "lfgpu_ctx_set_resident_wait": (C.c_int, [_P, C.c_double]),
     "lfgpu_vec_create": (C.c_int, [_P, C.c_int64, _d, C.POINTER(_P)]),
     "lfgpu_vec_destroy": (C.c_int, [_P]),
     "lfgpu_vec_size": (C.c_int, [_P, _i64]),
@@ -189,6 +190,10 @@ class Context:
         v = C.c_double()
         check(lib().lfgpu_ctx_last_ms(self.h, C.byref(v)))
         return v.value
+
+    def set_resident_wait(self, seconds):
+        """lfgpu_ctx_set_resident_wait."""
+        check(lib().lfgpu_ctx_set_resident_wait(self.h, float(seconds)))
 
     # -- factories ------------------------------------------------------------
     def vec(self, n_or_array):

@@ -331,6 +331,13 @@ extern "C" int lfgpu_ctx_sync(lfgpu_ctx *c) {
   return LFGPU_OK;
 }
 
+extern "C" int lfgpu_ctx_set_resident_wait(lfgpu_ctx *c, double seconds) {
+  LFG_REQUIRE(c, LFGPU_EINVAL, "ctx is NULL");
+  LFG_REQUIRE(seconds >= 0.0, LFGPU_EINVAL, "the wait must not be negative");
+  c->wait_ticks = (uint64_t)std::min(seconds * 1e8, 1e18);
+  return LFGPU_OK;
+}
+
 extern "C" int lfgpu_ctx_last_ms(lfgpu_ctx *c, double *ms) {
   LFG_REQUIRE(c && ms, LFGPU_EINVAL, "NULL argument");
   *ms = c->last_ms;

@@ -67,6 +67,9 @@ struct Staging;  // pinned buffers of large downloads (lfgpu_core.hip)
 struct lfgpu_ctx {
   int device = 0;
   int cus = 0;  // compute units (the largest team of a resident solve)
+  // the longest wait of a workgroup of a resident solve for another one, in
+  // ticks of the 100 MHz real-time clock (lfgpu_ctx_set_resident_wait)
+  uint64_t wait_ticks = 400000000ull;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   hipEvent_t evp[2] = {nullptr, nullptr};  // solver polls (no timing)

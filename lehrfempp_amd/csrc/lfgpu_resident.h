@@ -14,31 +14,53 @@ struct ResidentState {
   int iter, converged, refinements, aborted;
 };
 
+// The bound on the waits of a launch, and the flag by which a workgroup that
+// gave one up ends all teams of the launch.  The flag alone tells whether a
+// solve is whole: a workgroup that gives up in the last sum leaves its part of
+// x unwritten, while the one that reports may have got its total and found
+// convergence.
+struct ResidentAbort {
+  int raised, pad;
+  uint64_t ticks;
+};
+// What the host reads after a solve.
+struct ResidentOutcome {
+  ResidentState solve;
+  ResidentAbort team;
+};
+
 // Communication buffers of the resident solves on one matrix (owned by the
 // solver cache); epoch is the last tag any exchange in them has used.
 struct ResidentBufs {
   unsigned long long *halo = nullptr;
   size_t halo_words = 0;
   unsigned long long *sums = nullptr;  // team sums (fixed size)
-  ResidentState *state = nullptr;      // followed by the abort flag
-  int *abort = nullptr;
+  ResidentOutcome *outcome = nullptr;
+  uint64_t ticks = 0;  // outcome->team.ticks
   uint32_t epoch = 0;
 };
 void resident_free(ResidentBufs *b);
 // Buffers for a solve that exchanges through `words` words and uses at most
 // `need` tags; *tag0 the tag before its first.
-int resident_prepare(hipStream_t s, ResidentBufs *bufs, size_t words, uint64_t need,
+int resident_prepare(lfgpu_ctx *ctx, ResidentBufs *bufs, size_t words, uint64_t need,
                      uint32_t *tag0);
 // Whether resident_prepare would clear the buffers.
 bool resident_will_clear(const ResidentBufs *bufs, size_t words, uint64_t need);
 int resident_clear(hipStream_t s, unsigned long long *words, size_t n);
+// What the workgroups of a batch share: the counter that hands out the slots,
+// and the abort flag; set before every launch.
+struct ResidentControl {
+  int ticket, pad;
+  ResidentAbort abort;
+};
+int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control);
 int resident_launch_team(hipStream_t s, const void *fn, int team, void *args, size_t lds,
                          bool *taken);
 // Queues kernel fn (one argument struct) on `team` workgroups that all run at
 // once, and the copy of its outcome to *st; *taken = false where the chip
 // does not hold them.
 int resident_launch(hipStream_t s, ResidentBufs *bufs, const void *fn, int team, void *args,
-                    size_t lds, ResidentState *st, bool *taken);
+                    size_t lds, ResidentOutcome *out, bool *taken);
 
 // A matrix on DIA storage (val[d * n + row], offsets ascending) whose rows
 // form a lattice: `width` rows a line, n / width lines, no entry but between
@@ -58,16 +80,16 @@ struct ResidentDia {
 };
 
 // Jacobi-PCG in opts.mode on the context stream (rtol, maxit, mode and the
-// refinement options of lfgpu_pcg), queued without synchronisation; *st
+// refinement options of lfgpu_pcg), queued without synchronisation; *out
 // (pinned) receives the outcome.  *taken = false (and nothing queued) when
 // the system does not fit the chip; *ask (unless null) is set then if it would
 // with A.sym and A.diag.
 int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
-                     const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
-                     bool *taken, bool *ask);
+                     const lfgpu_pcg_opts &opts, const double *b, double *x,
+                     ResidentOutcome *out, bool *taken, bool *ask);
 
 // The lattice problems of a batch, side by side in one launch.  st (device)
-// receives the outcome of problem `index` at st[index].
+// receives the outcome of problem `index` at st[index], *ab (pinned) the flag.
 struct ResidentProblem {
   int32_t index, lo, n, width, ndiag;
   int32_t off[8];
@@ -82,7 +104,7 @@ void resident_tiles_reset(ResidentTiles *p);
 // (A.width, A.ndiag and A.off are the problems' own)
 int resident_tiles_run(lfgpu_ctx *ctx, ResidentTiles *p, const ResidentDia &A,
                        const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
-                       bool *taken);
+                       ResidentAbort *ab, bool *taken);
 
 // Sliced-ELL storage split over a team for the resident solves: a workgroup
 // owns a run of storage rows and keeps their p in LDS, with the values of the
@@ -106,13 +128,13 @@ struct ResidentEll {
 // As resident_pcg_dia; *plan is built by the first call.
 int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **plan,
                      const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b, double *x,
-                     ResidentState *st, bool *taken);
+                     ResidentOutcome *out, bool *taken);
 // The problems of a batch that are no lattices: problem q owns the storage
 // rows from q.lo (a multiple of 64) on, q.n of them.
 int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
                             const std::vector<ResidentProblem> &probs, ResidentEllPlan **out);
 int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *plan,
                            const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b,
-                           double *x, ResidentState *st, bool *taken);
+                           double *x, ResidentState *st, ResidentAbort *ab, bool *taken);
 
 }  // namespace lfgpu

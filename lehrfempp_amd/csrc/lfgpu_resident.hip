@@ -72,7 +72,7 @@ struct TileArgs {
   double *x;
   word_t *halo_words;  // [2][team][2][slots]
   word_t *part, *total;
-  int *abort;
+  ResidentAbort *abort;
   uint32_t tag0;
   double tol2;
   int maxit;
@@ -101,7 +101,7 @@ struct Tile {
   int32_t S, P, tw, th, x0, y0, n, g0;
   int32_t rank, team, TW, TH, TX, L, slots;
   word_t *words;
-  int *abort;
+  ResidentAbort *abort;
   uint32_t tag;
   int32_t *gpos, *gsrc, *ppos;  // LDS tables of the exchange
   int32_t ng, np;
@@ -1333,6 +1333,13 @@ __global__ void k_zero_words(word_t *p, size_t n) {
        i += (size_t)gridDim.x * blockDim.x)
     p[i] = 0;
 }
+// (a bound of nothing: the flag is up from the start)
+__global__ void k_set_abort(ResidentAbort *a, uint64_t ticks, int *ticket) {
+  if (threadIdx.x != 0) return;
+  a->raised = ticks == 0;
+  a->ticks = ticks;
+  if (ticket) *ticket = 0;
+}
 
 // The variants in order of preference (the smallest number of cells per
 // thread with which the team and its LDS fit): FP64, FP32 vectors, FP64
@@ -1444,7 +1451,7 @@ namespace lfgpu {
 void resident_free(ResidentBufs *b) {
   dfree(b->halo);
   dfree(b->sums);
-  dfree(b->state);
+  dfree(b->outcome);
   *b = ResidentBufs{};
 }
 
@@ -1478,12 +1485,19 @@ bool resident_will_clear(const ResidentBufs *bufs, size_t words, uint64_t need) 
   return !bufs->sums || words > bufs->halo_words || bufs->epoch + need > 0xfffffff0ull;
 }
 
-int resident_prepare(hipStream_t s, ResidentBufs *bufs, size_t words, uint64_t need,
+int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control) {
+  hipLaunchKernelGGL(k_set_abort, dim3(1), dim3(64), 0, ctx->stream, &control->abort,
+                     ctx->wait_ticks, &control->ticket);
+  LFG_HIP(hipGetLastError());
+  return LFGPU_OK;
+}
+
+int resident_prepare(lfgpu_ctx *ctx, ResidentBufs *bufs, size_t words, uint64_t need,
                      uint32_t *tag0) {
+  hipStream_t s = ctx->stream;
   if (!bufs->sums) {
     LFG_TRY(dalloc(&bufs->sums, kPartWords + kTotalWords, "resident PCG sums"));
-    LFG_TRY(dalloc(&bufs->state, 2, "resident PCG state"));
-    bufs->abort = reinterpret_cast<int *>(bufs->state + 1);
+    LFG_TRY(dalloc(&bufs->outcome, 1, "resident PCG state"));
     bufs->epoch = 0xffffffffu;  // forces the clearing below
   }
   if (words > bufs->halo_words) {
@@ -1494,15 +1508,19 @@ int resident_prepare(hipStream_t s, ResidentBufs *bufs, size_t words, uint64_t n
     bufs->halo_words = words;
     bufs->epoch = 0xffffffffu;
   }
+  bool fresh = false;
   if (bufs->epoch + need > 0xfffffff0ull) {
     hipLaunchKernelGGL(k_zero_words, dim3(256), dim3(256), 0, s, bufs->halo, bufs->halo_words);
     hipLaunchKernelGGL(k_zero_words, dim3(8), dim3(256), 0, s, bufs->sums,
                        kPartWords + kTotalWords);
-    hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s,
-                       reinterpret_cast<word_t *>(bufs->state),
-                       2 * sizeof(ResidentState) / sizeof(word_t));
-    LFG_HIP(hipGetLastError());
     bufs->epoch = 0;
+    fresh = true;
+  }
+  if (fresh || bufs->ticks != ctx->wait_ticks) {
+    bufs->ticks = ctx->wait_ticks;
+    hipLaunchKernelGGL(k_set_abort, dim3(1), dim3(64), 0, s, &bufs->outcome->team,
+                       bufs->ticks, (int *)nullptr);
+    LFG_HIP(hipGetLastError());
   }
   *tag0 = bufs->epoch;
   bufs->epoch = (uint32_t)std::min<uint64_t>(bufs->epoch + need, 0xffffffffull);
@@ -1530,16 +1548,16 @@ int resident_launch_team(hipStream_t s, const void *fn, int team, void *args, si
 }
 
 int resident_launch(hipStream_t s, ResidentBufs *bufs, const void *fn, int team, void *args,
-                    size_t lds, ResidentState *st, bool *taken) {
+                    size_t lds, ResidentOutcome *out, bool *taken) {
   LFG_TRY(resident_launch_team(s, fn, team, args, lds, taken));
   if (*taken)
-    LFG_HIP(hipMemcpyAsync(st, bufs->state, sizeof(ResidentState), hipMemcpyDeviceToHost, s));
+    LFG_HIP(hipMemcpyAsync(out, bufs->outcome, sizeof(ResidentOutcome), hipMemcpyDeviceToHost, s));
   return LFGPU_OK;
 }
 
 int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
-                     const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
-                     bool *taken, bool *ask) {
+                     const lfgpu_pcg_opts &opts, const double *b, double *x,
+                     ResidentOutcome *out, bool *taken, bool *ask) {
   *taken = false;
   if (A.n <= 0 || A.width <= 0 || A.ndiag > ND) return LFGPU_OK;
   TileArgs a{};
@@ -1557,16 +1575,16 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
   // tags of this solve: one exchange and one sum an iteration, six for a
   // reliable update (at most one an iteration), and a few at the start
   hipStream_t s = ctx->stream;
-  LFG_TRY(resident_prepare(s, bufs, (size_t)2 * team * 2 * a.slots,
+  LFG_TRY(resident_prepare(ctx, bufs, (size_t)2 * team * 2 * a.slots,
                            (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 7) + 16,
                            &a.tag0));
   fill_args(a, A, opts, b, x);
   a.halo_words = bufs->halo;
   a.part = bufs->sums;
   a.total = bufs->sums + kPartWords;
-  a.abort = bufs->abort;
-  a.st = bufs->state;
-  return resident_launch(s, bufs, reinterpret_cast<const void *>(v->fn), team, &a, v->lds(a), st,
+  a.abort = &bufs->outcome->team;
+  a.st = &bufs->outcome->solve;
+  return resident_launch(s, bufs, reinterpret_cast<const void *>(v->fn), team, &a, v->lds(a), out,
                          taken);
 }
 
@@ -1582,7 +1600,7 @@ struct ResidentTiles {
   TileJob *jobs = nullptr;
   int2 *slots = nullptr;
   word_t *words = nullptr;  // sums, then halos
-  int *ticket = nullptr;    // followed by the abort flag
+  ResidentControl *control = nullptr;
   uint32_t epoch = 0xffffffffu;
 };
 
@@ -1591,7 +1609,7 @@ void resident_tiles_free(ResidentTiles *p) {
   dfree(p->jobs);
   dfree(p->slots);
   dfree(p->words);
-  dfree(p->ticket);
+  dfree(p->control);
   delete p;
 }
 
@@ -1689,7 +1707,7 @@ int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &prob
   LFG_TRY(dalloc(&p->jobs, np, "resident batch jobs"));
   LFG_TRY(dalloc(&p->slots, slots.size(), "resident batch slots"));
   LFG_TRY(dalloc(&p->words, p->sums_words + p->halo_words, "resident batch words"));
-  LFG_TRY(dalloc(&p->ticket, 4, "resident batch counter"));
+  LFG_TRY(dalloc(&p->control, 1, "resident batch counter"));
   LFG_HIP(hipMemcpyAsync(p->jobs, jobs.data(), np * sizeof(TileJob), hipMemcpyHostToDevice, s));
   LFG_HIP(hipMemcpyAsync(p->slots, slots.data(), slots.size() * sizeof(int2),
                          hipMemcpyHostToDevice, s));
@@ -1704,7 +1722,7 @@ void resident_tiles_reset(ResidentTiles *p) { p->epoch = 0xffffffffu; }
 
 int resident_tiles_run(lfgpu_ctx *ctx, ResidentTiles *p, const ResidentDia &A,
                        const lfgpu_pcg_opts &opts, const double *b, double *x, ResidentState *st,
-                       bool *taken) {
+                       ResidentAbort *ab, bool *taken) {
   *taken = false;
   hipStream_t s = ctx->stream;
   const uint64_t need = (uint64_t)opts.maxit * (opts.mode == LFGPU_PCG_FP64 ? 1 : 7) + 16;
@@ -1713,26 +1731,25 @@ int resident_tiles_run(lfgpu_ctx *ctx, ResidentTiles *p, const ResidentDia &A,
                        p->sums_words + p->halo_words);
     p->epoch = 0;
   }
-  // the counter and the abort flag
-  hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(64), 0, s, reinterpret_cast<word_t *>(p->ticket),
-                     (size_t)2);
-  LFG_HIP(hipGetLastError());
+  LFG_TRY(resident_start_batch(ctx, p->control));
   TileArgs a{};
   fill_args(a, A, opts, b, x);
   a.halo_words = p->words + p->sums_words;
   a.part = p->words;
-  a.abort = p->ticket + 2;
+  a.abort = &p->control->abort;
   a.tag0 = p->epoch;
   a.st = st;
   a.jobs = p->jobs;
   a.job_slots = p->slots;
   a.nslots = p->nslots;
-  a.ticket = p->ticket;
+  a.ticket = &p->control->ticket;
   p->epoch = (uint32_t)std::min<uint64_t>(p->epoch + need, 0xffffffffull);
   const int team = std::min(p->nslots, std::min(ctx->cus, kMaxTeam));
-  return resident_launch_team(
+  LFG_TRY(resident_launch_team(
       s, reinterpret_cast<const void *>(kBatchVariants[opts.mode][p->variant].fn), team, &a,
-      p->lds, taken);
+      p->lds, taken));
+  LFG_HIP(hipMemcpyAsync(ab, a.abort, sizeof(ResidentAbort), hipMemcpyDeviceToHost, s));
+  return LFGPU_OK;
 }
 
 }  // namespace lfgpu

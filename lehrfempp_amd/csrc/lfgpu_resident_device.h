@@ -14,13 +14,15 @@
 // those wrote e + 1 after they had read e.
 //
 // Every wait is bounded by the real-time clock: a workgroup that waits longer
-// than kWaitTicks raises the team's abort flag and leaves, the others see the
+// than ResidentAbort::ticks raises the team's abort flag and leaves, the others see the
 // flag in their own waits and leave too; the caller then runs the sweeps.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+
+#include "lfgpu_resident.h"
 
 namespace lfgpu {
 namespace res {
@@ -42,7 +44,6 @@ constexpr int kSums = 5;       // values of one team sum
 // reads a thread took 3.9).
 constexpr int kFlatTeam = 64;
 constexpr int kLeaders = 8;
-constexpr uint64_t kWaitTicks = 400000000ull;  // 4 s of the 100 MHz real-time clock
 
 __device__ __forceinline__ void put(word_t *p, word_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -82,17 +83,18 @@ __device__ __forceinline__ void pin(T &v) {
 
 // A bounded wait: returns false once the team has been aborted.
 struct Wait {
-  int *abort;
+  ResidentAbort *abort;
   uint64_t t0 = 0;
   uint32_t polls = 0;
-  __device__ __forceinline__ explicit Wait(int *a) : abort(a) {}
+  __device__ __forceinline__ explicit Wait(ResidentAbort *a) : abort(a) {}
   __device__ __forceinline__ bool more() {
     if ((++polls & 255u) != 0) return true;
     const uint64_t now = wall_clock64();
     if (t0 == 0) t0 = now;
-    if (__hip_atomic_load(abort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
-    if (now - t0 > kWaitTicks) {
-      __hip_atomic_store(abort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__hip_atomic_load(&abort->raised, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      return false;
+    if (now - t0 > __hip_atomic_load(&abort->ticks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+      __hip_atomic_store(&abort->raised, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       return false;
     }
     return true;
@@ -185,7 +187,7 @@ struct Team {
   int rank, size;
   word_t *part;   // [2][size][kLine] partial sums of every member
   word_t *total;  // [2][kLeaders][kLine] sums over a leader's group
-  int *abort;
+  ResidentAbort *abort;
   uint32_t tag;   // number of the last team sum
 };
 
@@ -200,7 +202,7 @@ __device__ __forceinline__ int sums_threads(const Team &tm) {
 // poll in flight half a round trip behind gains 1 %.)
 template <int N>
 __device__ __forceinline__ bool poll_words(const word_t *src, int step, bool in, uint32_t tag,
-                                           int *abort, word_t (&a)[N]) {
+                                           ResidentAbort *abort, word_t (&a)[N]) {
   Wait wait(abort);
   for (;;) {
 #pragma unroll

@@ -61,7 +61,7 @@ struct EllArgs {
   double *xlo;  // storage order
   word_t *words;  // [2][planes(rpt)][n]
   word_t *part, *total;
-  int *abort;
+  ResidentAbort *abort;
   uint32_t tag0;
   double tol2;
   int maxit;
@@ -749,7 +749,7 @@ struct ResidentEllPlan {
   int2 *slots = nullptr;
   word_t *sums = nullptr;
   size_t sums_words = 0;
-  int *ticket = nullptr;  // followed by the abort flag
+  ResidentControl *control = nullptr;
 };
 
 void resident_ell_free(ResidentEllPlan *p) {
@@ -762,7 +762,7 @@ void resident_ell_free(ResidentEllPlan *p) {
   dfree(p->jobs);
   dfree(p->slots);
   dfree(p->sums);
-  dfree(p->ticket);
+  dfree(p->control);
   delete p;
 }
 bool resident_ell_fits(const ResidentEllPlan *p) { return p && p->rpt > 0; }
@@ -973,7 +973,7 @@ namespace lfgpu {
 
 int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan,
                      const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b, double *x,
-                     ResidentState *st, bool *taken) {
+                     ResidentOutcome *out, bool *taken) {
   *taken = false;
   if (A.n <= 0 || !A.dcol) return LFGPU_OK;
   hipStream_t s = ctx->stream;
@@ -1002,15 +1002,15 @@ int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan
   for (const EllVariant &k : kEllVariants)
     if (k.rpt == plan->rpt) v = &k;
   EllArgs a{};
-  LFG_TRY(resident_prepare(s, bufs, (size_t)2 * planes(plan->rpt) * A.n, ell_tags(opts),
+  LFG_TRY(resident_prepare(ctx, bufs, (size_t)2 * planes(plan->rpt) * A.n, ell_tags(opts),
                            &a.tag0));
   fill_args(a, plan, A, opts, b, x);
   a.words = bufs->halo;
   a.part = bufs->sums;
   a.total = bufs->sums + kPartWords;
-  a.abort = bufs->abort;
-  a.st = bufs->state;
-  return resident_launch(s, bufs, v->fn[opts.mode], plan->nparts, &a, plan->lds, st, taken);
+  a.abort = &bufs->outcome->team;
+  a.st = &bufs->outcome->solve;
+  return resident_launch(s, bufs, v->fn[opts.mode], plan->nparts, &a, plan->lds, out, taken);
 }
 
 // The two batch kernels: rows a thread, and what an iteration takes (us, and us
@@ -1143,7 +1143,7 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
   LFG_TRY(dalloc(&p->jobs, np, "resident batch jobs"));
   LFG_TRY(dalloc(&p->slots, slots.size(), "resident batch slots"));
   LFG_TRY(dalloc(&p->sums, p->sums_words, "resident batch sums"));
-  LFG_TRY(dalloc(&p->ticket, 4, "resident batch counter"));
+  LFG_TRY(dalloc(&p->control, 1, "resident batch counter"));
   LFG_HIP(hipMemcpyAsync(p->jobs, jobs.data(), np * sizeof(EllJob), hipMemcpyHostToDevice, s));
   LFG_HIP(hipMemcpyAsync(p->slots, slots.data(), slots.size() * sizeof(int2),
                          hipMemcpyHostToDevice, s));
@@ -1153,29 +1153,30 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
 
 int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *plan,
                            const ResidentEll &A, const lfgpu_pcg_opts &opts, const double *b,
-                           double *x, ResidentState *st, bool *taken) {
+                           double *x, ResidentState *st, ResidentAbort *ab, bool *taken) {
   *taken = false;
   hipStream_t s = ctx->stream;
   EllArgs a{};
   // (the problems' sums have their own words; they are cleared with the rest)
   const size_t words = (size_t)2 * planes(plan->rpt) * A.n;
   const bool fresh = resident_will_clear(bufs, words, ell_tags(opts));
-  LFG_TRY(resident_prepare(s, bufs, words, ell_tags(opts), &a.tag0));
+  LFG_TRY(resident_prepare(ctx, bufs, words, ell_tags(opts), &a.tag0));
   if (fresh) LFG_TRY(resident_clear(s, plan->sums, plan->sums_words));
-  // the counter and the abort flag
-  LFG_TRY(resident_clear(s, reinterpret_cast<unsigned long long *>(plan->ticket), 2));
+  LFG_TRY(resident_start_batch(ctx, plan->control));
   fill_args(a, plan, A, opts, b, x);
   a.words = bufs->halo;
   a.part = plan->sums;
-  a.abort = plan->ticket + 2;
+  a.abort = &plan->control->abort;
   a.st = st;
   a.jobs = plan->jobs;
   a.job_slots = plan->slots;
   a.nslots = plan->nparts;
-  a.ticket = plan->ticket;
-  return resident_launch_team(s, kEllBatch[plan->rpt == 2 ? 0 : 1][opts.mode],
-                              std::min(plan->nparts, std::min(ctx->cus, kMaxTeam)), &a,
-                              plan->lds, taken);
+  a.ticket = &plan->control->ticket;
+  LFG_TRY(resident_launch_team(s, kEllBatch[plan->rpt == 2 ? 0 : 1][opts.mode],
+                               std::min(plan->nparts, std::min(ctx->cus, kMaxTeam)), &a,
+                               plan->lds, taken));
+  LFG_HIP(hipMemcpyAsync(ab, a.abort, sizeof(ResidentAbort), hipMemcpyDeviceToHost, s));
+  return LFGPU_OK;
 }
 
 }  // namespace lfgpu

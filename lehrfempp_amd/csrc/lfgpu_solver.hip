@@ -3150,6 +3150,7 @@ struct lfgpu_batch {
     std::vector<ResidentProblem> tiles, rest;
     ResidentTiles *plan[3] = {nullptr, nullptr, nullptr};
     ResidentState *st = nullptr, *h_st = nullptr;  // device, pinned [nprob]
+    ResidentAbort *h_abort = nullptr;  // pinned: tiles', the others'
     // the others
     ResidentEllPlan *eplan = nullptr;
     ResidentBufs bufs;
@@ -3814,11 +3815,12 @@ std::mutex &resident_turn(const lfgpu_ctx *ctx) {
 }
 
 // end of a resident solve: one wait, then as pcg_finish
-int resident_finish(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentState *rs, bool mixed,
+int resident_finish(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentOutcome *out, bool mixed,
                     lfgpu_pcg_info *info, bool *aborted) {
   LFG_HIP(hipEventRecord(ctx->ev1, ctx->stream));
   LFG_HIP(hipEventSynchronize(ctx->ev1));
-  *aborted = rs->aborted != 0;
+  const ResidentState *rs = &out->solve;
+  *aborted = out->team.raised != 0 || rs->aborted != 0;
   if (*aborted) {
     bufs->epoch = 0xffffffffu;  // the next solve clears the words and the flag
     return LFGPU_OK;
@@ -3888,8 +3890,9 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
 
   // the resident solve (lfgpu_resident*.hip) where the system fits the chip,
   // unless the caller asked for graph replays or plain launches of the sweeps
+  int gave_up = 0;  // resident solves that did not end
   if (!single && c->blk_n == 0 && opts->graph == 0 && !t_timer && !c->no_resident) {
-    ResidentState *rs = reinterpret_cast<ResidentState *>(ctx->pinned);
+    ResidentOutcome *rs = reinterpret_cast<ResidentOutcome *>(ctx->pinned);
     bool taken = false;
     std::lock_guard<std::mutex> turn(resident_turn(ctx));
     LFG_HIP(hipEventRecord(ctx->ev0, s));
@@ -3934,10 +3937,11 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       LFG_TRY(resident_pcg_ell(ctx, &c->res, &c->res_ell, re, *opts, b->d, x->d, rs, &taken));
     }
     if (taken) {
-      // (a workgroup waited over 4 s for another one, as when other processes
+      // (a workgroup gave up its wait for another one, as when other processes
       // hold a part of the chip: the sweeps go on from the x reached)
       const int rc = resident_finish(ctx, &c->res, rs, mixed, info, &c->no_resident);
-      if (!c->no_resident) return rc;
+      if (rc != LFGPU_OK || !c->no_resident) return rc;
+      gave_up = 1;
     }
   }
 
@@ -3958,7 +3962,7 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
   // two pinned state slots: the iterations are polled one step behind
   static_assert(2 * sizeof(PcgState) <= 4096, "pinned context buffer holds two states");
   PcgState *hslot = reinterpret_cast<PcgState *>(ctx->pinned);
-  int slot = 0, syncs = 0;
+  int slot = 0, syncs = gave_up;
   PollHist hist;
   auto poll = [&](auto &&launch) {
     return poll_chunks(
@@ -4483,6 +4487,7 @@ void batch_resident_free(lfgpu_batch *bt) {
                   (void *)R.val32, (void *)R.rowsum32, (void *)R.dinv32, (void *)R.dinv16})
     dfree(p);
   if (R.h_st) (void)hipHostFree(R.h_st);
+  if (R.h_abort) (void)hipHostFree(R.h_abort);
   R = lfgpu_batch::Resident{};
 }
 
@@ -4530,6 +4535,7 @@ int batch_resident_setup(lfgpu_batch *bt) {
   }
   LFG_TRY(dalloc(&R.st, (size_t)bt->nprob, "resident batch states"));
   LFG_HIP(hipHostMalloc(&R.h_st, bt->nprob * sizeof(ResidentState), hipHostMallocDefault));
+  LFG_HIP(hipHostMalloc(&R.h_abort, 2 * sizeof(ResidentAbort), hipHostMallocDefault));
   R.state = 1;
   return LFGPU_OK;
 }
@@ -4569,11 +4575,11 @@ int batch_resident_ready(lfgpu_batch *bt, const lfgpu_pcg_opts *opts, bool *read
 }
 
 // The whole batch in one launch for its lattices and one for the others.
-// *taken = false: the chip does not hold the teams (nothing was run), or a
-// workgroup's wait was aborted.
+// *taken = false: the chip does not hold the teams; or (*aborted) a workgroup
+// gave up its wait.
 int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
                        const lfgpu_pcg_opts *opts, lfgpu_pcg_info *infos,
-                       lfgpu_pcg_info *summary, bool *taken) {
+                       lfgpu_pcg_info *summary, bool *taken, bool *aborted) {
   lfgpu_ctx *ctx = bt->ctx;
   lfgpu_batch::Resident &R = bt->res;
   hipStream_t s = ctx->stream;
@@ -4588,6 +4594,7 @@ int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
   // (problems without rows keep this state: converged, nothing done)
   std::memset(R.h_st, 0, bt->nprob * sizeof(ResidentState));
   for (int p = 0; p < bt->nprob; ++p) R.h_st[p].converged = 1;
+  std::memset(R.h_abort, 0, 2 * sizeof(ResidentAbort));
   LFG_HIP(hipMemcpyAsync(R.st, R.h_st, bt->nprob * sizeof(ResidentState), hipMemcpyHostToDevice, s));
   *taken = true;
   std::lock_guard<std::mutex> turn(resident_turn(ctx));
@@ -4602,23 +4609,25 @@ int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
     rd.dinv32 = c->dinv32;
     rd.dinv16 = c->dinv16;
     rd.xlo = c->xlo;
-    LFG_TRY(resident_tiles_run(ctx, R.plan[opts->mode], rd, *opts, b->d, x->d, R.st, taken));
+    LFG_TRY(resident_tiles_run(ctx, R.plan[opts->mode], rd, *opts, b->d, x->d, R.st,
+                               &R.h_abort[0], taken));
   }
   if (*taken && !R.rest.empty())
     LFG_TRY(resident_ell_batch_run(ctx, &R.bufs, R.eplan, batch_rest_view(bt), *opts, b->d, x->d,
-                                   R.st, taken));
+                                   R.st, &R.h_abort[1], taken));
   if (!*taken) return LFGPU_OK;
   LFG_HIP(hipMemcpyAsync(R.h_st, R.st, bt->nprob * sizeof(ResidentState), hipMemcpyDeviceToHost, s));
   LFG_HIP(hipEventRecord(ctx->ev1, s));
   LFG_HIP(hipEventSynchronize(ctx->ev1));
-  for (int p = 0; p < bt->nprob; ++p)
-    if (R.h_st[p].aborted) {
-      for (ResidentTiles *t : R.plan)
-        if (t) resident_tiles_reset(t);
-      R.bufs.epoch = 0xffffffffu;
-      *taken = false;  // (as in lfgpu_pcg: the sweeps go on from the x reached)
-      return LFGPU_OK;
-    }
+  *aborted = R.h_abort[0].raised || R.h_abort[1].raised;
+  for (int p = 0; p < bt->nprob; ++p) *aborted = *aborted || R.h_st[p].aborted;
+  if (*aborted) {
+    for (ResidentTiles *t : R.plan)
+      if (t) resident_tiles_reset(t);
+    R.bufs.epoch = 0xffffffffu;
+    *taken = false;  // (as in lfgpu_pcg: the sweeps go on from the x reached)
+    return LFGPU_OK;
+  }
   return batch_report_of(
       bt,
       [&](int p) {
@@ -4641,11 +4650,11 @@ extern "C" int lfgpu_batch_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, const lfgpu_vec 
               LFGPU_EINVAL, "unknown PCG mode");
   LFG_REQUIRE(opts->rtol >= 0.0 && opts->maxit >= 0, LFGPU_EINVAL, "bad PCG options");
   const bool mixed = opts->mode != LFGPU_PCG_FP64;
-  bool ready = false;
+  bool ready = false, aborted = false;
   LFG_TRY(batch_resident_ready(bt, opts, &ready));
   if (ready) {
     bool taken = false;
-    const int rc = batch_resident_run(bt, b, x, opts, infos, summary, &taken);
+    const int rc = batch_resident_run(bt, b, x, opts, infos, summary, &taken, &aborted);
     if (taken || rc != LFGPU_OK) return rc;
     bt->res.state = -1;
   }
@@ -4663,7 +4672,7 @@ extern "C" int lfgpu_batch_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, const lfgpu_vec 
   }
   int check = opts->check_every > 0 ? opts->check_every : 64;
   check += check & 1;
-  int slot = 0, syncs = 0;
+  int slot = 0, syncs = aborted ? 1 : 0;
   LFG_HIP(hipEventRecord(ctx->ev0, s));
   if (opts->mode == LFGPU_PCG_MIXED) {
     LFG_TRY(batch_run_mixed<float>(bt, b->d, x->d, opts, check, opts->mode, &slot, &syncs));

@@ -395,3 +395,80 @@ def test_resident_batch_with_couplings_away_from_the_middle(ctx, make, mode):
         assert np.linalg.norm(out[0][lo:hi] - out[1][lo:hi]) <= bound
     for h in (batch, b, A):
         h.close()
+
+
+# a context whose resident solves give up their waits at once: the flag is up
+# from the start, whatever the workgroup that reports the outcome has seen, and
+# the sweeps go on; one workgroup, one hop, two hops, the streamed matrix, the
+# three kernels on sliced ELL; then a solve on the same words and a fresh one
+@pytest.mark.parametrize("make", [
+    lambda: _lattice_system(20, 21, P1, 1), lambda: _lattice_system(65, 65, P1, 2),
+    lambda: _lattice_system(362, 363, P1, 3), lambda: _lattice_system(1141, 1140, P1, 3),
+    lambda: _flipped_system(40, 64, 4), lambda: _flipped_system(450, 451, 5),
+    lambda: _kinds_system(130, 129, 6),
+])
+@pytest.mark.parametrize("mode", MODES)
+def test_solve_that_gives_up_its_waits_ends_in_the_sweeps(make, mode):
+    r, c, v, n = make()
+    if n > 10**6:
+        v[-n:] += 1.0
+    bh = np.random.default_rng(1).standard_normal(n)
+    bound = 2.2e-10 * np.linalg.norm(bh) / 1e-3
+    with capi.Context(0) as ctx:
+        A, fresh = (capi.coo_to_csr(ctx, r, c, v, n, n) for _ in range(2))
+        b, x = capi.Vec(ctx, bh), capi.Vec(ctx, n)
+        capi.pcg(ctx, A, b, x, mode=mode, graph=-1)
+        want = x.numpy()
+        x.fill(0.0)
+        ctx.set_resident_wait(0.0)
+        info = capi.pcg(ctx, A, b, x, rtol=1e-10, mode=mode)
+        assert info.converged and info.syncs >= 2
+        assert np.linalg.norm(x.numpy() - want) <= bound
+        ctx.set_resident_wait(4.0)
+        for M in (A, fresh):
+            x.fill(0.0)
+            info = capi.pcg(ctx, M, b, x, rtol=1e-10, mode=mode)
+            assert info.converged and (info.syncs == 1 or M is A)
+            assert np.linalg.norm(x.numpy() - want) <= bound
+        for h in (x, b, A, fresh):
+            h.close()
+
+
+@pytest.mark.parametrize("kind", ["lattice", "flipped", "both"])
+@pytest.mark.parametrize("mode", MODES)
+def test_batch_that_gives_up_its_waits_ends_in_the_sweeps(kind, mode):
+    parts, off = [], [0]
+    for k in range(12):
+        make = _flipped_system if kind == "flipped" or (kind == "both" and k % 2) else (
+            lambda S, L, seed: _lattice_system(S, L, P1, seed))
+        r, c, v, n = make(20 + 11 * k, 30 + 5 * k, k)
+        parts.append((r + off[-1], c + off[-1], v))
+        off.append(off[-1] + n)
+    n = off[-1]
+    bh = np.random.default_rng(3).standard_normal(n)
+    with capi.Context(0) as ctx:
+        A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n, n)
+        b, x = capi.Vec(ctx, bh), capi.Vec(ctx, n)
+        out = []
+        for graph, seconds in ((-1, 4.0), (0, 0.0), (0, 4.0)):
+            batch = capi.Batch(ctx, A, np.array(off, np.int32))
+            ctx.set_resident_wait(seconds)
+            x.fill(0.0)
+            summ, infos = batch.pcg(b, x, rtol=1e-10, maxit=20000, mode=mode, graph=graph)
+            assert summ.converged and all(i.converged for i in infos)
+            out.append((summ.syncs, x.numpy()))
+            batch.close()
+        assert out[1][0] >= 2 and out[2][0] == 1
+        for lo, hi in zip(off, off[1:]):
+            bound = 2.2e-10 * np.linalg.norm(bh[lo:hi]) / 1e-3
+            for _, got in out[1:]:
+                assert np.linalg.norm(got[lo:hi] - out[0][1][lo:hi]) <= bound
+        for h in (x, b, A):
+            h.close()
+
+
+def test_resident_wait_is_checked(ctx):
+    for bad in (-1.0, float("nan")):
+        with pytest.raises(capi.LfgpuError) as e:
+            ctx.set_resident_wait(bad)
+        assert e.value.code == capi.EINVAL
