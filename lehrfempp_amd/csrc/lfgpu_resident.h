@@ -48,12 +48,21 @@ int resident_prepare(lfgpu_ctx *ctx, ResidentBufs *bufs, size_t words, uint64_t 
 bool resident_will_clear(const ResidentBufs *bufs, size_t words, uint64_t need);
 int resident_clear(hipStream_t s, unsigned long long *words, size_t n);
 // What the workgroups of a batch share: the counter that hands out the slots,
-// and the abort flag; set before every launch.
+// the abort flag and, behind them, every problem's number of workgroups that
+// have come to it; set before every launch.
 struct ResidentControl {
   int ticket, pad;
   ResidentAbort abort;
+  int *arrived() { return reinterpret_cast<int *>(this + 1); }
+  static int alloc(ResidentControl **out, size_t jobs) {
+    void *p = nullptr;
+    const int rc = dmalloc(&p, sizeof(ResidentControl) + jobs * sizeof(int),
+                           "resident batch counters");
+    *out = static_cast<ResidentControl *>(p);
+    return rc;
+  }
 };
-int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control);
+int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control, int jobs);
 int resident_launch_team(hipStream_t s, const void *fn, int team, void *args, size_t lds,
                          bool *taken);
 // Queues kernel fn (one argument struct) on `team` workgroups that all run at

@@ -90,7 +90,7 @@ struct TileArgs {
   const TileJob *__restrict__ jobs;
   const int2 *__restrict__ job_slots;
   int nslots;
-  int *ticket;
+  int *ticket, *arrived;
 };
 
 // The workgroup's tile: tw x th cells of the lattice, padded by one halo cell
@@ -859,7 +859,7 @@ __global__ __launch_bounds__(kThreads) void k_res_stream(TileArgs a) {
 // first unfinished problem always gets its team together.
 template <class F>
 __device__ __forceinline__ void batch_loop(const TileArgs &base, F &&solve) {
-  __shared__ int slot;
+  __shared__ int slot, up;
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) slot = atomicAdd(base.ticket, 1);
@@ -867,6 +867,10 @@ __device__ __forceinline__ void batch_loop(const TileArgs &base, F &&solve) {
     const int k = __builtin_amdgcn_readfirstlane(slot);
     if (k >= base.nslots) return;
     const int2 jr = base.job_slots[k];
+    // (the job is read after the wait: held across it, the mixed kernels of 7
+    // cells a thread spill 82 registers instead of 7, and 64 problems of 32 to
+    // 512 lines take 59 ms instead of 46)
+    if (!team_assembles(base.arrived + jr.x, base.jobs[jr.x].team, base.abort, up)) return;
     const TileJob &jb = base.jobs[jr.x];
     TileArgs a = base;
     a.S = jb.S;
@@ -1334,11 +1338,20 @@ __global__ void k_zero_words(word_t *p, size_t n) {
     p[i] = 0;
 }
 // (a bound of nothing: the flag is up from the start)
-__global__ void k_set_abort(ResidentAbort *a, uint64_t ticks, int *ticket) {
-  if (threadIdx.x != 0) return;
+__device__ __forceinline__ void set_abort(ResidentAbort *a, uint64_t ticks) {
   a->raised = ticks == 0;
   a->ticks = ticks;
-  if (ticket) *ticket = 0;
+}
+__global__ void k_set_abort(ResidentAbort *a, uint64_t ticks) {
+  if (threadIdx.x == 0) set_abort(a, ticks);
+}
+__global__ void k_start_batch(ResidentControl *c, int *arrived, int jobs, uint64_t ticks) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < jobs) arrived[i] = 0;
+  if (i == 0) {
+    c->ticket = 0;
+    set_abort(&c->abort, ticks);
+  }
 }
 
 // The variants in order of preference (the smallest number of cells per
@@ -1485,9 +1498,9 @@ bool resident_will_clear(const ResidentBufs *bufs, size_t words, uint64_t need) 
   return !bufs->sums || words > bufs->halo_words || bufs->epoch + need > 0xfffffff0ull;
 }
 
-int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control) {
-  hipLaunchKernelGGL(k_set_abort, dim3(1), dim3(64), 0, ctx->stream, &control->abort,
-                     ctx->wait_ticks, &control->ticket);
+int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control, int jobs) {
+  hipLaunchKernelGGL(k_start_batch, dim3((unsigned)((jobs + 255) / 256)), dim3(256), 0,
+                     ctx->stream, control, control->arrived(), jobs, ctx->wait_ticks);
   LFG_HIP(hipGetLastError());
   return LFGPU_OK;
 }
@@ -1519,7 +1532,7 @@ int resident_prepare(lfgpu_ctx *ctx, ResidentBufs *bufs, size_t words, uint64_t 
   if (fresh || bufs->ticks != ctx->wait_ticks) {
     bufs->ticks = ctx->wait_ticks;
     hipLaunchKernelGGL(k_set_abort, dim3(1), dim3(64), 0, s, &bufs->outcome->team,
-                       bufs->ticks, (int *)nullptr);
+                       bufs->ticks);
     LFG_HIP(hipGetLastError());
   }
   *tag0 = bufs->epoch;
@@ -1594,7 +1607,7 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
 // ---------------------------------------------------------------------------
 struct ResidentTiles {
   bool fits = false;
-  int nslots = 0, variant = 0;
+  int nslots = 0, njobs = 0, variant = 0;
   size_t lds = 0;
   size_t halo_words = 0, sums_words = 0;
   TileJob *jobs = nullptr;
@@ -1707,7 +1720,8 @@ int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &prob
   LFG_TRY(dalloc(&p->jobs, np, "resident batch jobs"));
   LFG_TRY(dalloc(&p->slots, slots.size(), "resident batch slots"));
   LFG_TRY(dalloc(&p->words, p->sums_words + p->halo_words, "resident batch words"));
-  LFG_TRY(dalloc(&p->control, 1, "resident batch counter"));
+  p->njobs = (int)np;
+  LFG_TRY(ResidentControl::alloc(&p->control, np));
   LFG_HIP(hipMemcpyAsync(p->jobs, jobs.data(), np * sizeof(TileJob), hipMemcpyHostToDevice, s));
   LFG_HIP(hipMemcpyAsync(p->slots, slots.data(), slots.size() * sizeof(int2),
                          hipMemcpyHostToDevice, s));
@@ -1731,7 +1745,7 @@ int resident_tiles_run(lfgpu_ctx *ctx, ResidentTiles *p, const ResidentDia &A,
                        p->sums_words + p->halo_words);
     p->epoch = 0;
   }
-  LFG_TRY(resident_start_batch(ctx, p->control));
+  LFG_TRY(resident_start_batch(ctx, p->control, p->njobs));
   TileArgs a{};
   fill_args(a, A, opts, b, x);
   a.halo_words = p->words + p->sums_words;
@@ -1743,6 +1757,7 @@ int resident_tiles_run(lfgpu_ctx *ctx, ResidentTiles *p, const ResidentDia &A,
   a.job_slots = p->slots;
   a.nslots = p->nslots;
   a.ticket = &p->control->ticket;
+  a.arrived = p->control->arrived();
   p->epoch = (uint32_t)std::min<uint64_t>(p->epoch + need, 0xffffffffull);
   const int team = std::min(p->nslots, std::min(ctx->cus, kMaxTeam));
   LFG_TRY(resident_launch_team(

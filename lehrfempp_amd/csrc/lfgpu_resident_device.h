@@ -101,6 +101,27 @@ struct Wait {
   }
 };
 
+// The workgroups of a batch draw their slots in order, so that the first ones
+// of a team find it incomplete until the others have ended the problems that
+// they are at, whatever those take: that wait has no bound of time.  It ends,
+// since the earlier problems' workgroups are all there and end, or raise the
+// flag.  Returns false, in all threads, once it is up.  `scratch` is shared.
+__device__ __forceinline__ bool team_assembles(int *arrived, int team, ResidentAbort *abort,
+                                               int &scratch) {
+  if (threadIdx.x == 0) {
+    int up = 0;
+    __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    while (team > 1 && !up &&
+           __hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < team) {
+      up = __hip_atomic_load(&abort->raised, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __builtin_amdgcn_s_sleep(2);
+    }
+    scratch = up;
+  }
+  __syncthreads();
+  return __builtin_amdgcn_readfirstlane(scratch) == 0;
+}
+
 // Lane l's 32 bits from the lane that the DPP control CTRL names.
 template <int CTRL>
 __device__ __forceinline__ double dpp(double v) {

@@ -72,7 +72,7 @@ struct EllArgs {
   const EllJob *__restrict__ jobs;
   const int2 *__restrict__ job_slots;  // slot (= part) -> job, rank in its team
   int nslots;
-  int *ticket;
+  int *ticket, *arrived;
 };
 
 // the precision modes: FP64; FP32 vectors; FP64 vectors with the FP32 matrix
@@ -611,7 +611,7 @@ template <int MODE, int RPT>
 __global__ __launch_bounds__(kThreads) void k_res_ell_batch(EllArgs base) {
   extern __shared__ double dyn[];
   __shared__ SumLds sh;
-  __shared__ int slot;
+  __shared__ int slot, up;
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) slot = atomicAdd(base.ticket, 1);
@@ -619,6 +619,7 @@ __global__ __launch_bounds__(kThreads) void k_res_ell_batch(EllArgs base) {
     const int k = __builtin_amdgcn_readfirstlane(slot);
     if (k >= base.nslots) return;
     const int2 jr = base.job_slots[k];
+    if (!team_assembles(base.arrived + jr.x, base.jobs[jr.x].team, base.abort, up)) return;
     const EllJob &jb = base.jobs[jr.x];
     EllArgs a = base;
     a.part += jb.sums_at;
@@ -750,6 +751,7 @@ struct ResidentEllPlan {
   word_t *sums = nullptr;
   size_t sums_words = 0;
   ResidentControl *control = nullptr;
+  int njobs = 0;
 };
 
 void resident_ell_free(ResidentEllPlan *p) {
@@ -1143,7 +1145,8 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
   LFG_TRY(dalloc(&p->jobs, np, "resident batch jobs"));
   LFG_TRY(dalloc(&p->slots, slots.size(), "resident batch slots"));
   LFG_TRY(dalloc(&p->sums, p->sums_words, "resident batch sums"));
-  LFG_TRY(dalloc(&p->control, 1, "resident batch counter"));
+  p->njobs = (int)np;
+  LFG_TRY(ResidentControl::alloc(&p->control, np));
   LFG_HIP(hipMemcpyAsync(p->jobs, jobs.data(), np * sizeof(EllJob), hipMemcpyHostToDevice, s));
   LFG_HIP(hipMemcpyAsync(p->slots, slots.data(), slots.size() * sizeof(int2),
                          hipMemcpyHostToDevice, s));
@@ -1162,7 +1165,7 @@ int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *
   const bool fresh = resident_will_clear(bufs, words, ell_tags(opts));
   LFG_TRY(resident_prepare(ctx, bufs, words, ell_tags(opts), &a.tag0));
   if (fresh) LFG_TRY(resident_clear(s, plan->sums, plan->sums_words));
-  LFG_TRY(resident_start_batch(ctx, plan->control));
+  LFG_TRY(resident_start_batch(ctx, plan->control, plan->njobs));
   fill_args(a, plan, A, opts, b, x);
   a.words = bufs->halo;
   a.part = plan->sums;
@@ -1172,6 +1175,7 @@ int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *
   a.job_slots = plan->slots;
   a.nslots = plan->nparts;
   a.ticket = &plan->control->ticket;
+  a.arrived = plan->control->arrived();
   LFG_TRY(resident_launch_team(s, kEllBatch[plan->rpt == 2 ? 0 : 1][opts.mode],
                                std::min(plan->nparts, std::min(ctx->cus, kMaxTeam)), &a,
                                plan->lds, taken));

@@ -472,3 +472,28 @@ def test_resident_wait_is_checked(ctx):
         with pytest.raises(capi.LfgpuError) as e:
             ctx.set_resident_wait(bad)
         assert e.value.code == capi.EINVAL
+
+
+# problems that take more than half of the chip each, one after the other: the
+# workgroups that are first at the second one wait for the rest of its team
+# until the first problem is done, several times the bound of a wait here
+@pytest.mark.parametrize("make", [lambda k: _lattice_system(840, 830, P1, k),
+                                  lambda k: _flipped_system(800, 801, k)])
+def test_batch_waits_for_a_team_as_long_as_the_problem_before_takes(make):
+    parts, off, maxit = [], [0], 8000
+    for k in range(2):
+        r, c, v, n = make(k)
+        parts.append((r + off[-1], c + off[-1], v))
+        off.append(off[-1] + n)
+    n = off[-1]
+    with capi.Context(0) as ctx:
+        A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n, n)
+        b, x = capi.Vec(ctx, np.random.default_rng(3).standard_normal(n)), capi.Vec(ctx, n)
+        batch = capi.Batch(ctx, A, np.array(off, np.int32))
+        batch.pcg(b, x, rtol=0.0, maxit=2, raise_on_noconv=False)  # (builds the plans)
+        ctx.set_resident_wait(0.012)
+        summ, infos = batch.pcg(b, x, rtol=0.0, maxit=maxit, raise_on_noconv=False)
+        assert summ.syncs == 1 and all(i.iters == maxit for i in infos)
+        assert summ.ms > 2 * 2 * 12.0  # (else the bound was not reached)
+        for h in (batch, x, b, A):
+            h.close()
