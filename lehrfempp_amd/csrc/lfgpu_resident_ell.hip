@@ -772,10 +772,12 @@ bool resident_ell_fits(const ResidentEllPlan *p) { return p && p->rpt > 0; }
 
 namespace {
 
-// The parts of a split, their slices one after the other.
+// The parts of a split, their slices one after the other, and each part's
+// problem's number of slices, which bounds the outside rows that it can have
+// (most of a batch's small problems have one part, and none).
 struct Split {
   std::vector<EllPart> parts;
-  std::vector<int32_t> slist;
+  std::vector<int32_t> slist, of;
   void add(const std::vector<int32_t> &slices, int32_t n) {
     EllPart q{};
     q.r0 = 64 * slices.front();
@@ -785,6 +787,8 @@ struct Split {
     slist.insert(slist.end(), slices.begin(), slices.end());
     parts.push_back(q);
   }
+  // the parts added since the last call make up a problem of n slices
+  void problem(int32_t n) { of.resize(parts.size(), n); }
 };
 
 // Splits the slices [s0, s1) into runs of `each` slices.  (Runs of equally
@@ -877,7 +881,7 @@ int ell_split(hipStream_t s, ResidentEllPlan *p, const ResidentEll &A, Split &sp
     EllPart &q = split.parts[g];
     if (64 * q.slices >= room) return LFGPU_OK;
     q.at = at;
-    at += room - 64 * q.slices;
+    at += std::min(room - 64 * q.slices, 64 * (split.of[g] - q.slices));
     span = std::max(span, q.r1 - q.r0);
     for (int32_t k = 0; k < q.slices; ++k)
       home[split.slist[(size_t)q.first + k]] = int2{(int)g, k};
@@ -991,6 +995,7 @@ int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan
       Split split;
       if (v.rpt > kSmallRows || !split_windows(split, off, 0, slices, cap, cus, A.n))
         split_runs(split, 0, slices, (slices + want - 1) / want, A.n);
+      split.problem(slices);
       bool fits = false;
       LFG_TRY(ell_split(s, p, A, split, v.rpt, &fits));
       if (!fits) continue;
@@ -1127,6 +1132,7 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
       const size_t had = split.parts.size();
       if (!windows || !split_windows(split, off, s0, s1, each, cus, A.n))
         split_runs(split, s0, s1, each, A.n);
+      split.problem(s1 - s0);
       EllJob j{};
       j.index = q.index;
       j.team = (int32_t)(split.parts.size() - had);

@@ -10,6 +10,8 @@ matrices here have no eigenvalue below 1e-3, so two converged solutions differ
 by at most 2 rtol ||b|| / 1e-3 (a tenth more for the recurrence residual's
 distance from the true one).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -495,5 +497,36 @@ def test_batch_waits_for_a_team_as_long_as_the_problem_before_takes(make):
         summ, infos = batch.pcg(b, x, rtol=0.0, maxit=maxit, raise_on_noconv=False)
         assert summ.syncs == 1 and all(i.iters == maxit for i in infos)
         assert summ.ms > 2 * 2 * 12.0  # (else the bound was not reached)
+        for h in (batch, x, b, A):
+            h.close()
+
+
+def test_small_unstructured_problems_take_little_memory():
+    # 3000 problems of 64 rows, which read no rows of other workgroups
+    total, now = ctypes.c_size_t(), ctypes.c_size_t()
+
+    def free_bytes():
+        assert capi.lib().hipMemGetInfo(ctypes.byref(now), ctypes.byref(total)) == 0
+        return now.value
+
+    parts, off = [], [0]
+    for k in range(3000):
+        r, c, v, n = _flipped_system(8, 8, k)
+        parts.append((r + off[-1], c + off[-1], v))
+        off.append(off[-1] + n)
+    n = off[-1]
+    with capi.Context(0) as ctx:
+        A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n, n)
+        b, x = capi.Vec(ctx, np.random.default_rng(3).standard_normal(n)), capi.Vec(ctx, n)
+        batch = capi.Batch(ctx, A, np.array(off, np.int32))
+        free = []
+        for graph in (1, 0):
+            x.fill(0.0)
+            summ, _ = batch.pcg(b, x, graph=graph)
+            free.append(free_bytes())
+        assert summ.syncs == 1  # the resident solve ran
+        # its matrix (10 B a slot), places (2 B a slot), team sums (10 KB a
+        # problem of one workgroup at most) and vectors
+        assert free[0] - free[1] < 64 << 20, free
         for h in (batch, x, b, A):
             h.close()
