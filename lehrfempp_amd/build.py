@@ -51,6 +51,8 @@ DEMO_SRC = os.path.join(ROOT, "tests", "cpp", "homdir_demo.cc")
 DEMO_BIN = os.path.join(ROOT, "tests", "cpp", "homdir_demo")
 BINDING_SRC = os.path.join(ROOT, "tests", "cpp", "binding_demo.cc")
 BINDING_BIN = os.path.join(ROOT, "tests", "cpp", "binding_demo")
+ALLOC_SRC = os.path.join(ROOT, "tests", "cpp", "alloc_demo.cc")
+ALLOC_BIN = os.path.join(ROOT, "tests", "cpp", "alloc_demo")
 ORACLE_DIR = os.path.join(ROOT, "oracle")
 
 
@@ -63,16 +65,28 @@ def binding_demo_cmd(out: str) -> list:
             "-llfref", "-Wl,-rpath,$ORIGIN/../../lehrfempp_amd:$ORIGIN/../../oracle", "-o", out]
 
 
+def alloc_demo_cmd(out: str) -> list:
+    """g++ line of the driver whose device allocations fail
+    (tests/cpp/alloc_demo.cc)."""
+    return ["g++", "-std=c++20", "-O2", "-Wall", "-Wextra", "-I", os.path.join(ROOT, "include"),
+            ALLOC_SRC, "-L", HERE, "-llfgpu", "-ldl", "-rdynamic",
+            "-Wl,-rpath,$ORIGIN/../../lehrfempp_amd", "-o", out]
+
+
 def build_cpp_demo() -> str:
     """Compile the C++ drivers with g++ against liblfgpu.so: the facade
-    driver (tests/cpp/homdir_demo.cc) and, when the oracle library is built,
-    the LehrFEM++-binding driver (tests/cpp/binding_demo.cc)."""
+    driver (tests/cpp/homdir_demo.cc), the driver of failing allocations
+    (tests/cpp/alloc_demo.cc) and, when the oracle library is built, the
+    LehrFEM++-binding driver (tests/cpp/binding_demo.cc)."""
     cmd = ["g++", "-std=c++20", "-O2", "-Wall", "-I", ROOT, "-I", os.path.join(ROOT, "include"),
            DEMO_SRC, "-L", HERE, "-llfgpu", "-Wl,-rpath,$ORIGIN/../../lehrfempp_amd",
            "-o", DEMO_BIN]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError("g++ failed for the C++ facade driver:\n%s" % res.stderr[-8000:])
+    res = subprocess.run(alloc_demo_cmd(ALLOC_BIN), capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed for the allocation driver:\n%s" % res.stderr[-8000:])
     if os.path.exists(os.path.join(ORACLE_DIR, "liblfref.so")):
         res = subprocess.run(binding_demo_cmd(BINDING_BIN), capture_output=True, text=True)
         if res.returncode != 0:

@@ -1495,7 +1495,7 @@ int resident_clear(hipStream_t s, unsigned long long *words, size_t n) {
 }
 
 bool resident_will_clear(const ResidentBufs *bufs, size_t words, uint64_t need) {
-  return !bufs->sums || words > bufs->halo_words || bufs->epoch + need > 0xfffffff0ull;
+  return !bufs->outcome || words > bufs->halo_words || bufs->epoch + need > 0xfffffff0ull;
 }
 
 int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control, int jobs) {
@@ -1508,8 +1508,8 @@ int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control, int jobs) {
 int resident_prepare(lfgpu_ctx *ctx, ResidentBufs *bufs, size_t words, uint64_t need,
                      uint32_t *tag0) {
   hipStream_t s = ctx->stream;
-  if (!bufs->sums) {
-    LFG_TRY(dalloc(&bufs->sums, kPartWords + kTotalWords, "resident PCG sums"));
+  if (!bufs->outcome) {
+    if (!bufs->sums) LFG_TRY(dalloc(&bufs->sums, kPartWords + kTotalWords, "resident PCG sums"));
     LFG_TRY(dalloc(&bufs->outcome, 1, "resident PCG state"));
     bufs->epoch = 0xffffffffu;  // forces the clearing below
   }

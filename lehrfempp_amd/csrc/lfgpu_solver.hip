@@ -3814,6 +3814,15 @@ std::mutex &resident_turn(const lfgpu_ctx *ctx) {
   return turn[ctx->device & 63];
 }
 
+// Gives back what the resident solves on a matrix hold, after an allocation
+// among it failed.
+void resident_release(lfgpu_solver_cache *c) {
+  resident_free(&c->res);
+  resident_ell_free(c->res_ell);
+  c->res_ell = nullptr;
+  clear_error();
+}
+
 // end of a resident solve: one wait, then as pcg_finish
 int resident_finish(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentOutcome *out, bool mixed,
                     lfgpu_pcg_info *info, bool *aborted) {
@@ -3894,6 +3903,7 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
   if (!single && c->blk_n == 0 && opts->graph == 0 && !t_timer && !c->no_resident) {
     ResidentOutcome *rs = reinterpret_cast<ResidentOutcome *>(ctx->pinned);
     bool taken = false;
+    int rc = LFGPU_OK;
     std::lock_guard<std::mutex> turn(resident_turn(ctx));
     LFG_HIP(hipEventRecord(ctx->ev0, s));
     if (c->fmt == FMT_DIA) {
@@ -3912,10 +3922,11 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       rd.xlo = c->xlo;
       for (bool known : {false, true}) {
         bool ask = false;
-        LFG_TRY(resident_pcg_dia(ctx, &c->res, rd, *opts, b->d, x->d, rs, &taken,
-                                 known ? nullptr : &ask));
+        rc = resident_pcg_dia(ctx, &c->res, rd, *opts, b->d, x->d, rs, &taken,
+                              known ? nullptr : &ask);
         if (!ask) break;
-        LFG_TRY(dia_symmetry(ctx, c, n));
+        rc = dia_symmetry(ctx, c, n);
+        if (rc != LFGPU_OK) break;
         rd.sym = c->sym64;
         rd.diag = c->diag64;
       }
@@ -3934,12 +3945,18 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       re.dinv32 = c->dinv32;
       re.dinv16 = c->dinv16;
       re.xlo = c->xlo;
-      LFG_TRY(resident_pcg_ell(ctx, &c->res, &c->res_ell, re, *opts, b->d, x->d, rs, &taken));
+      rc = resident_pcg_ell(ctx, &c->res, &c->res_ell, re, *opts, b->d, x->d, rs, &taken);
     }
-    if (taken) {
+    if (rc == LFGPU_EOOM) {
+      // (the sweeps need none of this memory)
+      resident_release(c);
+      c->no_resident = true;
+    } else if (rc != LFGPU_OK) {
+      return rc;
+    } else if (taken) {
       // (a workgroup gave up its wait for another one, as when other processes
       // hold a part of the chip: the sweeps go on from the x reached)
-      const int rc = resident_finish(ctx, &c->res, rs, mixed, info, &c->no_resident);
+      rc = resident_finish(ctx, &c->res, rs, mixed, info, &c->no_resident);
       if (rc != LFGPU_OK || !c->no_resident) return rc;
       gave_up = 1;
     }
@@ -4491,6 +4508,14 @@ void batch_resident_free(lfgpu_batch *bt) {
   R = lfgpu_batch::Resident{};
 }
 
+// The batch keeps the sweeps from here on (which need none of this memory).
+void batch_resident_give_up(lfgpu_batch *bt) {
+  (void)hipStreamSynchronize(bt->ctx->stream);
+  batch_resident_free(bt);
+  bt->res.state = -1;
+  clear_error();
+}
+
 // Decides once per batch whether every problem can run resident in every
 // mode, and builds what that takes.  (The cache and bt->fmt exist.)
 int batch_resident_setup(lfgpu_batch *bt) {
@@ -4569,7 +4594,11 @@ int batch_resident_ready(lfgpu_batch *bt, const lfgpu_pcg_opts *opts, bool *read
   if (bt->fmt < 0 || bt->res.state == 0)
     LFG_TRY(ensure_cache(bt->ctx, bt->A, opts->mode != LFGPU_PCG_FP64, false));
   if (bt->fmt < 0) LFG_TRY(batch_choose_format(bt));
-  if (bt->res.state == 0) LFG_TRY(batch_resident_setup(bt));
+  if (bt->res.state == 0) {
+    const int rc = batch_resident_setup(bt);
+    if (rc == LFGPU_EOOM) batch_resident_give_up(bt);
+    else LFG_TRY(rc);
+  }
   *ready = bt->res.state == 1;
   return LFGPU_OK;
 }
@@ -4655,8 +4684,13 @@ extern "C" int lfgpu_batch_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, const lfgpu_vec 
   if (ready) {
     bool taken = false;
     const int rc = batch_resident_run(bt, b, x, opts, infos, summary, &taken, &aborted);
-    if (taken || rc != LFGPU_OK) return rc;
-    bt->res.state = -1;
+    if (rc == LFGPU_EOOM) {
+      batch_resident_give_up(bt);
+    } else if (taken || rc != LFGPU_OK) {
+      return rc;
+    } else {
+      bt->res.state = -1;
+    }
   }
   LFG_TRY(ensure_cache(ctx, bt->A, mixed, false));
   hipStream_t s = ctx->stream;

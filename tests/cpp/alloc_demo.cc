@@ -1,0 +1,162 @@
+// Solves in one launch while device allocations fail.  The driver's own
+// hipMalloc stands before the runtime's and lets the k-th allocation of a call
+// fail, for every k there is: the call has to end like one that had the memory
+// (the sweeps, whose storage exists by then, need none of it), and so has the
+// next call, whatever the failed one had allocated.
+// Exit status 0 on success.
+#include <dlfcn.h>
+
+#include <cmath>
+#include <cstdio>
+#include <random>
+#include <vector>
+
+#include "lfgpu.h"
+
+namespace {
+long g_calls = 0, g_fail_at = -1;
+}  // namespace
+
+extern "C" int hipMalloc(void **p, size_t bytes) {
+  static auto *real = reinterpret_cast<int (*)(void **, size_t)>(dlsym(RTLD_NEXT, "hipMalloc"));
+  if (g_calls++ == g_fail_at) {
+    *p = nullptr;
+    return 2;  // hipErrorOutOfMemory
+  }
+  return real(p, bytes);
+}
+
+namespace {
+int fails = 0;
+#define EXPECT(cond, ...)                 \
+  do {                                    \
+    if (!(cond)) {                        \
+      std::printf("FAIL: " __VA_ARGS__);  \
+      std::printf("\n");                  \
+      ++fails;                            \
+    }                                     \
+  } while (0)
+#define OK(call) EXPECT((call) == LFGPU_OK, "%s: %s", #call, lfgpu_last_error())
+
+struct System {
+  std::vector<int32_t> row, col, off{0};
+  std::vector<double> val, rhs;
+  int32_t n = 0;
+};
+
+// Adds a lattice Laplacian plus 0.01 (S x L vertices, every square cut along a
+// diagonal, the other one in `turned` of ten squares) as a problem.
+void add_lattice(System &s, int S, int L, int turned, unsigned seed) {
+  std::mt19937 gen(seed);
+  const int32_t base = s.n;
+  std::vector<double> diag((size_t)S * L, 0.01);
+  auto couple = [&](int a, int b) {
+    const double w = 0.5 + gen() % 1000 * 0.002;
+    s.row.insert(s.row.end(), {base + a, base + b});
+    s.col.insert(s.col.end(), {base + b, base + a});
+    s.val.insert(s.val.end(), {-w, -w});
+    diag[a] += w;
+    diag[b] += w;
+  };
+  for (int y = 0; y < L; ++y)
+    for (int x = 0; x < S; ++x) {
+      const int i = y * S + x;
+      if (x + 1 < S) couple(i, i + 1);
+      if (y + 1 < L) couple(i, i + S);
+      if (x + 1 < S && y + 1 < L) {
+        if ((int)(gen() % 10) < turned) couple(i + 1, i + S);
+        else couple(i, i + S + 1);
+      }
+    }
+  for (int i = 0; i < S * L; ++i) {
+    s.row.push_back(base + i);
+    s.col.push_back(base + i);
+    s.val.push_back(diag[i]);
+    s.rhs.push_back(gen() % 1000 * 0.002 - 1.0);
+  }
+  s.n += S * L;
+  s.off.push_back(s.n);
+}
+
+double norm(const std::vector<double> &a, const std::vector<double> *less = nullptr) {
+  double s = 0.0;
+  for (size_t i = 0; i < a.size(); ++i) {
+    const double v = a[i] - (less ? (*less)[i] : 0.0);
+    s += v * v;
+  }
+  return std::sqrt(s);
+}
+
+void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch) {
+  std::vector<double> want((size_t)s.n), got((size_t)s.n);
+  lfgpu_pcg_opts opts{};
+  opts.rtol = 1e-11;
+  opts.maxit = 20000;
+  opts.mode = mode;
+  // two solutions of residuals below rtol ||b||, no eigenvalue below 0.01, and
+  // a tenth for the recurrence residual's distance from the true one
+  const double bound = 2.2 * opts.rtol * norm(s.rhs) / 0.01;
+  for (long k = 0;; ++k) {
+    lfgpu_csr *A = nullptr;
+    lfgpu_vec *b = nullptr, *x = nullptr;
+    lfgpu_batch *bt = nullptr;
+    OK(lfgpu_coo_to_csr(ctx, (int64_t)s.val.size(), s.row.data(), s.col.data(), s.val.data(), s.n,
+                        s.n, &A));
+    OK(lfgpu_vec_create(ctx, s.n, s.rhs.data(), &b));
+    OK(lfgpu_vec_create(ctx, s.n, nullptr, &x));
+    if (batch) OK(lfgpu_batch_create(ctx, A, (int)s.off.size() - 1, s.off.data(), &bt));
+    lfgpu_pcg_info info{};
+    auto solve = [&](int graph, std::vector<double> &to) {
+      OK(lfgpu_vec_fill(x, 0.0));
+      opts.graph = graph;
+      if (batch) OK(lfgpu_batch_pcg(ctx, bt, b, x, &opts, nullptr, &info));
+      else OK(lfgpu_pcg(ctx, A, b, x, &opts, &info));
+      EXPECT(info.converged, "%s, allocation %ld: not converged", name, k);
+      OK(lfgpu_vec_download(x, to.data(), s.n));
+    };
+    solve(1, want);
+    g_calls = 0;
+    g_fail_at = k;
+    solve(0, got);
+    const bool failed = g_calls > k;
+    g_fail_at = -1;
+    EXPECT(norm(got, &want) <= bound, "%s, allocation %ld: %g off", name, k, norm(got, &want));
+    EXPECT(failed || info.syncs == 1, "%s: not in one launch", name);
+    solve(0, got);
+    EXPECT(norm(got, &want) <= bound, "%s, after allocation %ld: %g off", name, k,
+           norm(got, &want));
+    OK(lfgpu_batch_destroy(bt));
+    OK(lfgpu_vec_destroy(x));
+    OK(lfgpu_vec_destroy(b));
+    OK(lfgpu_csr_destroy(A));
+    if (!failed) {
+      std::printf("%s: %ld allocations\n", name, k);
+      std::fflush(stdout);
+      return;
+    }
+  }
+}
+}  // namespace
+
+int main() {
+  lfgpu_ctx *ctx = nullptr;
+  OK(lfgpu_ctx_create(0, &ctx));
+  if (!ctx) return 1;
+  System lattice, ell, equal, bands, both;
+  add_lattice(lattice, 90, 70, 0, 1);
+  add_lattice(ell, 90, 70, 5, 2);
+  for (int k = 0; k < 4; ++k) add_lattice(equal, 24, 30, 0, 3 + k);
+  for (int k = 0; k < 4; ++k) add_lattice(bands, 24 + k, 30, 0, 7 + k);
+  for (int k = 0; k < 6; ++k) add_lattice(both, 40 + k, 50, k % 2 ? 5 : 0, 11 + k);
+  for (int mode : {LFGPU_PCG_FP64, LFGPU_PCG_MIXED, LFGPU_PCG_MIXED_MATRIX}) {
+    run("lattice", ctx, lattice, mode, false);
+    run("sliced ELL", ctx, ell, mode, false);
+    run("batch of equal lattices", ctx, equal, mode, true);
+    run("batch of lattices", ctx, bands, mode, true);
+    run("batch of both", ctx, both, mode, true);
+  }
+  OK(lfgpu_ctx_destroy(ctx));
+  if (fails) return 1;
+  std::printf("OK\n");
+  return 0;
+}
