@@ -754,8 +754,7 @@ struct ResidentEllPlan {
   int njobs = 0;
 };
 
-void resident_ell_free(ResidentEllPlan *p) {
-  if (!p) return;
+static void release(ResidentEllPlan *p) {
   dfree(p->parts);
   dfree(p->slist);
   dfree(p->ext);
@@ -765,6 +764,12 @@ void resident_ell_free(ResidentEllPlan *p) {
   dfree(p->slots);
   dfree(p->sums);
   dfree(p->control);
+  *p = ResidentEllPlan{};
+}
+
+void resident_ell_free(ResidentEllPlan *p) {
+  if (!p) return;
+  release(p);
   delete p;
 }
 bool resident_ell_fits(const ResidentEllPlan *p) { return p && p->rpt > 0; }
@@ -1002,6 +1007,7 @@ int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan
       p->rpt = v.rpt;
       break;
     }
+    if (p->rpt == 0) release(p);  // (it only says that the matrix does not fit)
   }
   const ResidentEllPlan *plan = *pplan;
   if (plan->rpt == 0) return LFGPU_OK;

@@ -3345,7 +3345,11 @@ int batch_choose_format(lfgpu_batch *bt) {
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   dfree(flag);
   if (e != hipSuccess) return hip_fail(e, "batch DIA check");
-  if (hflag != 0) return LFGPU_OK;
+  if (hflag != 0) {
+    dfree(bt->boff);
+    bt->boff = nullptr;
+    return LFGPU_OK;
+  }
   LFG_TRY(dalloc(&bt->bval, (size_t)nd * n, "batch DIA values"));
   bt->bndiag = nd;
   bt->fmt = FMT_BDIA;
@@ -4511,6 +4515,16 @@ void batch_resident_free(lfgpu_batch *bt) {
 // The batch keeps the sweeps from here on (which need none of this memory).
 void batch_resident_give_up(lfgpu_batch *bt) {
   (void)hipStreamSynchronize(bt->ctx->stream);
+  if (bt->res.own_diag) {
+    dfree(bt->boff);
+    dfree(bt->bval);
+    dfree(bt->bval32);
+    bt->boff = nullptr;
+    bt->bval = nullptr;
+    bt->bval32 = nullptr;
+    bt->bndiag = 0;
+    bt->bbuilt = ~0ull;
+  }
   batch_resident_free(bt);
   bt->res.state = -1;
   clear_error();
@@ -4539,12 +4553,12 @@ int batch_resident_setup(lfgpu_batch *bt) {
       nd = std::max(nd, q.ndiag);
       for (int d = 0; d < q.ndiag; ++d) off[(size_t)q.index * kMaxDiag + d] = q.off[d];
     }
+    R.own_diag = true;
     LFG_TRY(dalloc(&bt->boff, off.size(), "batch diagonal offsets"));
     LFG_HIP(hipMemcpyAsync(bt->boff, off.data(), off.size() * 4, hipMemcpyHostToDevice, s));
     LFG_HIP(hipStreamSynchronize(s));
     LFG_TRY(dalloc(&bt->bval, (size_t)nd * A->nrows, "batch DIA values"));
     bt->bndiag = nd;
-    R.own_diag = true;
   }
   if (!R.tiles.empty())
     for (int mode = 0; mode < 3; ++mode) {
@@ -4596,8 +4610,8 @@ int batch_resident_ready(lfgpu_batch *bt, const lfgpu_pcg_opts *opts, bool *read
   if (bt->fmt < 0) LFG_TRY(batch_choose_format(bt));
   if (bt->res.state == 0) {
     const int rc = batch_resident_setup(bt);
-    if (rc == LFGPU_EOOM) batch_resident_give_up(bt);
-    else LFG_TRY(rc);
+    if (bt->res.state != 1) batch_resident_give_up(bt);
+    if (rc != LFGPU_EOOM) LFG_TRY(rc);
   }
   *ready = bt->res.state == 1;
   return LFGPU_OK;
@@ -4684,13 +4698,8 @@ extern "C" int lfgpu_batch_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, const lfgpu_vec 
   if (ready) {
     bool taken = false;
     const int rc = batch_resident_run(bt, b, x, opts, infos, summary, &taken, &aborted);
-    if (rc == LFGPU_EOOM) {
-      batch_resident_give_up(bt);
-    } else if (taken || rc != LFGPU_OK) {
-      return rc;
-    } else {
-      bt->res.state = -1;
-    }
+    if (taken || (rc != LFGPU_OK && rc != LFGPU_EOOM)) return rc;
+    batch_resident_give_up(bt);
   }
   LFG_TRY(ensure_cache(ctx, bt->A, mixed, false));
   hipStream_t s = ctx->stream;

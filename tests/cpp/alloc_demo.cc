@@ -2,19 +2,23 @@
 // hipMalloc stands before the runtime's and lets the k-th allocation of a call
 // fail, for every k there is: the call has to end like one that had the memory
 // (the sweeps, whose storage exists by then, need none of it), and so has the
-// next call, whatever the failed one had allocated.
+// next call, whatever the failed one had allocated.  Nothing stays allocated
+// that the sweeps do not read, nor anything once the handles are gone.
 // Exit status 0 on success.
 #include <dlfcn.h>
 
 #include <cmath>
 #include <cstdio>
 #include <random>
+#include <unordered_map>
 #include <vector>
 
 #include "lfgpu.h"
 
 namespace {
 long g_calls = 0, g_fail_at = -1;
+size_t g_live = 0;  // bytes allocated
+std::unordered_map<void *, size_t> g_size;
 }  // namespace
 
 extern "C" int hipMalloc(void **p, size_t bytes) {
@@ -23,7 +27,18 @@ extern "C" int hipMalloc(void **p, size_t bytes) {
     *p = nullptr;
     return 2;  // hipErrorOutOfMemory
   }
-  return real(p, bytes);
+  const int e = real(p, bytes);
+  if (e == 0) g_live += g_size[*p] = bytes;
+  return e;
+}
+extern "C" int hipFree(void *p) {
+  static auto *real = reinterpret_cast<int (*)(void *)>(dlsym(RTLD_NEXT, "hipFree"));
+  const auto it = g_size.find(p);
+  if (it != g_size.end()) {
+    g_live -= it->second;
+    g_size.erase(it);
+  }
+  return real(p);
 }
 
 namespace {
@@ -45,8 +60,9 @@ struct System {
 };
 
 // Adds a lattice Laplacian plus 0.01 (S x L vertices, every square cut along a
-// diagonal, the other one in `turned` of ten squares) as a problem.
-void add_lattice(System &s, int S, int L, int turned, unsigned seed) {
+// diagonal, the other one in `turned` of ten squares of the first `lines`
+// lines) as a problem.
+void add_lattice(System &s, int S, int L, int turned, unsigned seed, int lines = 1 << 20) {
   std::mt19937 gen(seed);
   const int32_t base = s.n;
   std::vector<double> diag((size_t)S * L, 0.01);
@@ -64,7 +80,7 @@ void add_lattice(System &s, int S, int L, int turned, unsigned seed) {
       if (x + 1 < S) couple(i, i + 1);
       if (y + 1 < L) couple(i, i + S);
       if (x + 1 < S && y + 1 < L) {
-        if ((int)(gen() % 10) < turned) couple(i + 1, i + S);
+        if (y < lines && (int)(gen() % 10) < turned) couple(i + 1, i + S);
         else couple(i, i + S + 1);
       }
     }
@@ -97,6 +113,7 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
   // a tenth for the recurrence residual's distance from the true one
   const double bound = 2.2 * opts.rtol * norm(s.rhs) / 0.01;
   for (long k = 0;; ++k) {
+    const size_t before = g_live;
     lfgpu_csr *A = nullptr;
     lfgpu_vec *b = nullptr, *x = nullptr;
     lfgpu_batch *bt = nullptr;
@@ -115,6 +132,7 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
       OK(lfgpu_vec_download(x, to.data(), s.n));
     };
     solve(1, want);
+    const size_t swept = g_live;
     g_calls = 0;
     g_fail_at = k;
     solve(0, got);
@@ -122,6 +140,8 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
     g_fail_at = -1;
     EXPECT(norm(got, &want) <= bound, "%s, allocation %ld: %g off", name, k, norm(got, &want));
     EXPECT(failed || info.syncs == 1, "%s: not in one launch", name);
+    EXPECT(!failed || g_live == swept, "%s, allocation %ld: %ld bytes kept", name, k,
+           (long)(g_live - swept));
     solve(0, got);
     EXPECT(norm(got, &want) <= bound, "%s, after allocation %ld: %g off", name, k,
            norm(got, &want));
@@ -129,6 +149,8 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
     OK(lfgpu_vec_destroy(x));
     OK(lfgpu_vec_destroy(b));
     OK(lfgpu_csr_destroy(A));
+    EXPECT(g_live == before, "%s, allocation %ld: %ld bytes lost", name, k,
+           (long)(g_live - before));
     if (!failed) {
       std::printf("%s: %ld allocations\n", name, k);
       std::fflush(stdout);
@@ -142,18 +164,22 @@ int main() {
   lfgpu_ctx *ctx = nullptr;
   OK(lfgpu_ctx_create(0, &ctx));
   if (!ctx) return 1;
-  System lattice, ell, equal, bands, both;
+  System lattice, ell, equal, bands, both, mixed;
   add_lattice(lattice, 90, 70, 0, 1);
   add_lattice(ell, 90, 70, 5, 2);
   for (int k = 0; k < 4; ++k) add_lattice(equal, 24, 30, 0, 3 + k);
   for (int k = 0; k < 4; ++k) add_lattice(bands, 24 + k, 30, 0, 7 + k);
   for (int k = 0; k < 6; ++k) add_lattice(both, 40 + k, 50, k % 2 ? 5 : 0, 11 + k);
+  // (what the middle of the turned ones shows does not cover them: no diagonals
+  // for the sweeps, which run on sliced ELL, but for the others' tiles)
+  for (int k = 0; k < 6; ++k) add_lattice(mixed, 70 + k, 50, k % 2 ? 5 : 0, 21 + k, 10);
   for (int mode : {LFGPU_PCG_FP64, LFGPU_PCG_MIXED, LFGPU_PCG_MIXED_MATRIX}) {
     run("lattice", ctx, lattice, mode, false);
     run("sliced ELL", ctx, ell, mode, false);
     run("batch of equal lattices", ctx, equal, mode, true);
     run("batch of lattices", ctx, bands, mode, true);
     run("batch of both", ctx, both, mode, true);
+    run("batch of both, swept on ELL", ctx, mixed, mode, true);
   }
   OK(lfgpu_ctx_destroy(ctx));
   if (fails) return 1;
