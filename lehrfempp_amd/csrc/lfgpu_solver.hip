@@ -578,7 +578,6 @@ int dia_symmetry(lfgpu_ctx *ctx, lfgpu_solver_cache *c, int32_t n) {
   ds.ndiag = c->ndiag;
   for (int d = 0; d < kMaxDiag; ++d) ds.off[d] = c->off[d];
   hipStream_t s = ctx->stream;
-  if (!c->sym_flag) LFG_TRY(dalloc(&c->sym_flag, 1, "symmetry flag"));
   int *flag = c->sym_flag;
   hipError_t e = hipMemsetAsync(flag, 0, 4, s);
   if (e == hipSuccess) {
@@ -875,6 +874,9 @@ int ensure_cache(lfgpu_ctx *ctx, lfgpu_csr *A, bool need32, bool allow_perm) {
       for (int d = 0; d < kMaxDiag; ++d) c->off[d] = d < ds.ndiag ? ds.off[d] : 0;
       c->mlen = (int64_t)ds.ndiag * n;
       LFG_TRY(dia_lattice(ctx, A, c));
+      // (here, where the matrix's device is current: lfgpu_solver_storage may
+      // ask for the test from any thread)
+      LFG_TRY(dalloc(&c->sym_flag, 1, "symmetry flag"));
     } else {
       c->fmt = FMT_ELL;
       if (allow_perm && n > 0) LFG_TRY(ell_locality_order(ctx, A, c));

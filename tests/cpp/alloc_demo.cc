@@ -158,6 +158,27 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
     }
   }
 }
+
+// Asking for the storage allocates nothing (the calling thread's device need
+// not be the matrix's), also where the answer takes the symmetry test first.
+void storage(lfgpu_ctx *ctx, const System &s) {
+  lfgpu_csr *A = nullptr;
+  lfgpu_vec *b = nullptr, *x = nullptr;
+  OK(lfgpu_coo_to_csr(ctx, (int64_t)s.val.size(), s.row.data(), s.col.data(), s.val.data(), s.n,
+                      s.n, &A));
+  OK(lfgpu_vec_create(ctx, s.n, s.rhs.data(), &b));
+  OK(lfgpu_vec_create(ctx, s.n, nullptr, &x));
+  OK(lfgpu_spmv(ctx, A, b, x));
+  const long calls = g_calls;
+  int kind = -1, ndiag = 0, sym = 0;
+  OK(lfgpu_solver_storage(A, &kind, &ndiag, &sym));
+  EXPECT(kind == LFGPU_STORAGE_DIA && ndiag == 6 && sym == 1, "storage %d, %d diagonals, %d", kind,
+         ndiag, sym);
+  EXPECT(g_calls == calls, "lfgpu_solver_storage allocates");
+  OK(lfgpu_vec_destroy(x));
+  OK(lfgpu_vec_destroy(b));
+  OK(lfgpu_csr_destroy(A));
+}
 }  // namespace
 
 int main() {
@@ -181,6 +202,7 @@ int main() {
     run("batch of both", ctx, both, mode, true);
     run("batch of both, swept on ELL", ctx, mixed, mode, true);
   }
+  storage(ctx, lattice);
   OK(lfgpu_ctx_destroy(ctx));
   if (fails) return 1;
   std::printf("OK\n");
