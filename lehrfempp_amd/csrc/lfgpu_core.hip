@@ -144,6 +144,32 @@ using namespace lfgpu;
 // ===========================================================================
 extern "C" const char *lfgpu_last_error(void) { return g_last_error.c_str(); }
 
+// ---------------------------------------------------------------------------
+// downloads: what a context keeps for them
+// ---------------------------------------------------------------------------
+namespace lfgpu {
+
+// Pageable host memory limits a large download, not the link: the runtime
+// copies it out of its own pinned buffers with one thread, which takes the
+// page faults of a fresh destination as well (12 GB/s).  Here the arrays go
+// through a ring of pinned chunks that kCopiers threads empty while the next
+// chunks arrive: a matrix of 31 MB 2.35 -> 1.66 ms, of 190 MB 18.9 -> 6.4 ms
+// (6 or 8 threads, chunks of 1 or 4 MB: the same to 10 % more).
+struct Staging {
+  static constexpr size_t kChunk = (size_t)2 << 20;
+  static constexpr int kSlots = 8;
+  std::mutex busy;  // one download at a time; others take the plain copy
+  char *buf = nullptr;  // (with the first large download)
+  hipEvent_t ev[kSlots] = {};  // of the context's device
+  ~Staging() {
+    for (hipEvent_t e : ev)
+      if (e) (void)hipEventDestroy(e);
+    if (buf) (void)hipHostFree(buf);
+  }
+};
+
+}  // namespace lfgpu
+
 extern "C" int lfgpu_ctx_create(int device, lfgpu_ctx **out) {
   LFG_REQUIRE(out, LFGPU_EINVAL, "out is NULL");
   *out = nullptr;
@@ -161,6 +187,10 @@ extern "C" int lfgpu_ctx_create(int device, lfgpu_ctx **out) {
     e = hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, device);
   for (int k = 0; k < 2 && e == hipSuccess; ++k)
     e = hipEventCreateWithFlags(&c->evp[k], hipEventDisableTiming);
+  // (events go with the device that is current here; a download's need not be)
+  c->staging = new Staging();
+  for (hipEvent_t &ev : c->staging->ev)
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
   if (e == hipSuccess) e = hipHostMalloc(&c->pinned, 4096, hipHostMallocDefault);
   if (e != hipSuccess) {
     lfgpu_ctx_destroy(c);
@@ -175,44 +205,22 @@ extern "C" int lfgpu_ctx_create(int device, lfgpu_ctx **out) {
 // ---------------------------------------------------------------------------
 namespace lfgpu {
 
-// Pageable host memory limits a large download, not the link: the runtime
-// copies it out of its own pinned buffers with one thread, which takes the
-// page faults of a fresh destination as well (12 GB/s).  Here the arrays go
-// through a ring of pinned chunks that kCopiers threads empty while the next
-// chunks arrive: a matrix of 31 MB 2.35 -> 1.66 ms, of 190 MB 18.9 -> 6.4 ms
-// (6 or 8 threads, chunks of 1 or 4 MB: the same to 10 % more).
-struct Staging {
-  static constexpr size_t kChunk = (size_t)2 << 20;
-  static constexpr int kSlots = 8;
-  std::mutex busy;  // one download at a time; others take the plain copy
-  char *buf = nullptr;
-  hipEvent_t ev[kSlots] = {};
-  ~Staging() {
-    for (hipEvent_t e : ev)
-      if (e) (void)hipEventDestroy(e);
-    if (buf) (void)hipHostFree(buf);
-  }
-};
 constexpr int kCopiers = 4;
 // Below this the threads' start (about 20 us each) outweighs the copy.
 constexpr size_t kStageFrom = (size_t)4 << 20;
 
-static std::mutex g_staging;  // guards the contexts' staging pointers
+static std::mutex g_staging;  // guards the contexts' staging buffers
 
 static Staging *staging(lfgpu_ctx *ctx) {
   std::lock_guard<std::mutex> hold(g_staging);
-  if (ctx->staging) return ctx->staging;
-  Staging *s = new Staging();
-  bool ok = hipHostMalloc((void **)&s->buf, Staging::kChunk * Staging::kSlots,
-                          hipHostMallocDefault) == hipSuccess;
-  for (hipEvent_t &e : s->ev)
-    ok = ok && hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
-  if (!ok) {
+  Staging *s = ctx->staging;
+  if (!s->buf && hipHostMalloc((void **)&s->buf, Staging::kChunk * Staging::kSlots,
+                               hipHostMallocPortable) != hipSuccess) {
     (void)hipGetLastError();
-    delete s;
+    s->buf = nullptr;
     return nullptr;
   }
-  return ctx->staging = s;
+  return s;
 }
 
 static int download_plain(lfgpu_ctx *ctx, const Download *what, int n) {

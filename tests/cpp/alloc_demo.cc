@@ -1,5 +1,5 @@
-// Solves in one launch while device allocations fail.  The driver's own
-// hipMalloc stands before the runtime's and lets the k-th allocation of a call
+// Solves in one launch while device allocations fail, and large downloads
+// while host allocations do.  The driver's own hipMalloc stands before the runtime's and lets the k-th allocation of a call
 // fail, for every k there is: the call has to end like one that had the memory
 // (the sweeps, whose storage exists by then, need none of it), and so has the
 // next call, whatever the failed one had allocated.  Nothing stays allocated
@@ -9,6 +9,9 @@
 
 #include <cmath>
 #include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <new>
 #include <random>
 #include <unordered_map>
 #include <vector>
@@ -30,6 +33,13 @@ extern "C" int hipMalloc(void **p, size_t bytes) {
   const int e = real(p, bytes);
   if (e == 0) g_live += g_size[*p] = bytes;
   return e;
+}
+long g_events = 0;
+extern "C" int hipEventCreateWithFlags(void **ev, unsigned flags) {
+  static auto *real = reinterpret_cast<int (*)(void **, unsigned)>(
+      dlsym(RTLD_NEXT, "hipEventCreateWithFlags"));
+  ++g_events;
+  return real(ev, flags);
 }
 extern "C" int hipFree(void *p) {
   static auto *real = reinterpret_cast<int (*)(void *)>(dlsym(RTLD_NEXT, "hipFree"));
@@ -159,6 +169,21 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
   }
 }
 
+// A download through the staging ring creates no event (the context's device
+// need not be current).
+void download(lfgpu_ctx *ctx) {
+  const int64_t n = 3 << 20;
+  std::vector<double> in((size_t)n), out((size_t)n);
+  for (int64_t i = 0; i < n; ++i) in[i] = 1.0 / (1.0 + (double)i);
+  lfgpu_vec *v = nullptr;
+  OK(lfgpu_vec_create(ctx, n, in.data(), &v));
+  const long events = g_events;
+  OK(lfgpu_vec_download(v, out.data(), n));
+  EXPECT(out == in, "download");
+  EXPECT(g_events == events, "the download creates %ld events", g_events - events);
+  OK(lfgpu_vec_destroy(v));
+}
+
 // Asking for the storage allocates nothing (the calling thread's device need
 // not be the matrix's), also where the answer takes the symmetry test first.
 void storage(lfgpu_ctx *ctx, const System &s) {
@@ -203,6 +228,7 @@ int main() {
     run("batch of both, swept on ELL", ctx, mixed, mode, true);
   }
   storage(ctx, lattice);
+  download(ctx);
   OK(lfgpu_ctx_destroy(ctx));
   if (fails) return 1;
   std::printf("OK\n");
