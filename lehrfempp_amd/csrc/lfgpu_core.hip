@@ -261,8 +261,9 @@ static int download_staged(lfgpu_ctx *ctx, Staging *st, const std::vector<Downlo
   team.reserve(kCopiers);
   try {
     for (int k = 0; k < kCopiers; ++k) team.emplace_back(copier);
-  } catch (const std::system_error &) {
-    // (fewer threads)
+  } catch (const std::exception &) {
+    // (no thread, or no memory for one: fewer threads; nothing may leave this
+    // function while one runs)
   }
   *taken = !team.empty();
   if (!*taken) return LFGPU_OK;

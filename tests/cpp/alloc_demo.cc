@@ -41,6 +41,23 @@ extern "C" int hipEventCreateWithFlags(void **ev, unsigned flags) {
   ++g_events;
   return real(ev, flags);
 }
+// this thread's host allocations in the library (the runtime's go as they
+// are), of which the k-th fails
+thread_local long g_news = 0, g_news_fail = -1;
+static bool from_library(void *caller) {
+  Dl_info info;
+  return dladdr(caller, &info) != 0 && info.dli_fname && std::strstr(info.dli_fname, "liblfgpu.so");
+}
+void *operator new(size_t bytes) {
+  void *p = nullptr;
+  if (g_news_fail < 0 || !from_library(__builtin_return_address(0)) || g_news++ != g_news_fail)
+    p = std::malloc(bytes);
+  if (!p) throw std::bad_alloc();
+  return p;
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, size_t) noexcept { std::free(p); }
+
 extern "C" int hipFree(void *p) {
   static auto *real = reinterpret_cast<int (*)(void *)>(dlsym(RTLD_NEXT, "hipFree"));
   const auto it = g_size.find(p);
@@ -170,7 +187,8 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
 }
 
 // A download through the staging ring creates no event (the context's device
-// need not be current).
+// need not be current), and any of its host allocations may fail: the list of
+// chunks, and what a copying thread takes to start.
 void download(lfgpu_ctx *ctx) {
   const int64_t n = 3 << 20;
   std::vector<double> in((size_t)n), out((size_t)n);
@@ -181,6 +199,17 @@ void download(lfgpu_ctx *ctx) {
   OK(lfgpu_vec_download(v, out.data(), n));
   EXPECT(out == in, "download");
   EXPECT(g_events == events, "the download creates %ld events", g_events - events);
+  long k = 0;
+  for (bool failed = true; failed; ++k) {
+    std::fill(out.begin(), out.end(), 0.0);
+    g_news = 0;
+    g_news_fail = k;
+    const int rc = lfgpu_vec_download(v, out.data(), n);
+    failed = g_news > k;
+    g_news_fail = -1;
+    EXPECT(rc == LFGPU_OK && out == in, "download, host allocation %ld", k);
+  }
+  std::printf("download: %ld host allocations\n", k - 1);
   OK(lfgpu_vec_destroy(v));
 }
 
