@@ -69,8 +69,8 @@ def alloc_demo_cmd(out: str) -> list:
     """g++ line of the driver whose device allocations fail
     (tests/cpp/alloc_demo.cc)."""
     return ["g++", "-std=c++20", "-O2", "-Wall", "-Wextra", "-I", os.path.join(ROOT, "include"),
-            ALLOC_SRC, "-L", HERE, "-llfgpu", "-ldl", "-rdynamic",
-            "-Wl,-rpath,$ORIGIN/../../lehrfempp_amd", "-o", out]
+            ALLOC_SRC, "-L", HERE, "-llfgpu", "-L", "/opt/rocm/lib", "-lamdhip64", "-ldl",
+            "-rdynamic", "-Wl,-rpath,$ORIGIN/../../lehrfempp_amd", "-o", out]
 
 
 def build_cpp_demo() -> str:

@@ -291,13 +291,21 @@ int download(lfgpu_ctx *ctx, const Download *what, int n) {
   size_t total = 0;
   for (int k = 0; k < n; ++k) total += what[k].bytes;
   if (total >= kStageFrom) {
-    // (a pinned destination needs no staging)
-    hipPointerAttribute_t attr;
-    const bool known = hipPointerGetAttributes(&attr, what[n - 1].host) == hipSuccess &&
-                       attr.type != hipMemoryTypeUnregistered;
+    // (a pinned destination needs no staging, and no thread may write to one on
+    // a device)
+    bool pageable = false, device = false;
+    for (int k = 0; k < n; ++k) {
+      hipPointerAttribute_t attr;
+      if (what[k].bytes == 0) continue;
+      if (hipPointerGetAttributes(&attr, what[k].host) != hipSuccess ||
+          attr.type == hipMemoryTypeUnregistered)
+        pageable = true;
+      else if (attr.type != hipMemoryTypeHost)
+        device = true;
+    }
     (void)hipGetLastError();
     try {
-      Staging *st = known ? nullptr : staging(ctx);
+      Staging *st = pageable && !device ? staging(ctx) : nullptr;
       if (st && st->busy.try_lock()) {
         std::lock_guard<std::mutex> hold(st->busy, std::adopt_lock);
         std::vector<Download> chunks;

@@ -68,6 +68,10 @@ extern "C" int hipFree(void *p) {
   return real(p);
 }
 
+extern "C" int hipHostMalloc(void **p, size_t bytes, unsigned flags);
+extern "C" int hipHostFree(void *p);
+extern "C" int hipMemcpy(void *to, const void *from, size_t bytes, int kind);
+
 namespace {
 int fails = 0;
 #define EXPECT(cond, ...)                 \
@@ -213,6 +217,33 @@ void download(lfgpu_ctx *ctx) {
   OK(lfgpu_vec_destroy(v));
 }
 
+// The arrays of a matrix may go to different kinds of memory.
+void scattered(lfgpu_ctx *ctx) {
+  System s;
+  add_lattice(s, 500, 400, 0, 1);
+  lfgpu_csr *A = nullptr;
+  OK(lfgpu_coo_to_csr(ctx, (int64_t)s.val.size(), s.row.data(), s.col.data(), s.val.data(), s.n,
+                      s.n, &A));
+  int64_t nnz = 0;
+  OK(lfgpu_csr_info(A, nullptr, nullptr, &nnz));
+  std::vector<int32_t> rp((size_t)s.n + 1), col((size_t)nnz), got((size_t)nnz);
+  std::vector<double> val((size_t)nnz), val2((size_t)nnz);
+  OK(lfgpu_csr_download(A, rp.data(), col.data(), val.data()));
+  void *dev = nullptr, *pinned = nullptr;
+  EXPECT(hipMalloc(&dev, 4 * (size_t)nnz) == 0 && hipHostMalloc(&pinned, 4 * (size_t)nnz, 0) == 0,
+         "memory");
+  for (void *to : {dev, pinned}) {
+    OK(lfgpu_csr_download(A, rp.data(), static_cast<int32_t *>(to), val2.data()));
+    EXPECT(hipMemcpy(got.data(), to, 4 * (size_t)nnz, 4) == 0, "hipMemcpy");
+    EXPECT(got == col && val2 == val, "download to scattered arrays");
+    std::fill(got.begin(), got.end(), 0);
+    std::fill(val2.begin(), val2.end(), 0.0);
+  }
+  hipHostFree(pinned);
+  hipFree(dev);
+  OK(lfgpu_csr_destroy(A));
+}
+
 // Asking for the storage allocates nothing (the calling thread's device need
 // not be the matrix's), also where the answer takes the symmetry test first.
 void storage(lfgpu_ctx *ctx, const System &s) {
@@ -258,6 +289,7 @@ int main() {
   }
   storage(ctx, lattice);
   download(ctx);
+  scattered(ctx);
   OK(lfgpu_ctx_destroy(ctx));
   if (fails) return 1;
   std::printf("OK\n");
