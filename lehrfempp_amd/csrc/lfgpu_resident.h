@@ -1,6 +1,8 @@
 // Resident Jacobi-PCG (lfgpu_resident.hip): the whole solve in one launch.
 #pragma once
 
+#include <algorithm>
+#include <chrono>
 #include <cstdint>
 #include <vector>
 
@@ -27,6 +29,24 @@ struct ResidentAbort {
 struct ResidentOutcome {
   ResidentState solve;
   ResidentAbort team;
+};
+
+// When the resident solves of a matrix or a batch may run again after one that
+// gave up: the sweeps take over for 16 times as long as it cost, twice as long
+// after each further one in a row, so that a lasting cause (a part of the chip
+// held by another process) costs a few per cent and a passing one not the
+// resident solves for good.
+struct ResidentPause {
+  double until = 0.0, times = 16.0;
+  static double now() {
+    return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch())
+        .count();
+  }
+  bool over() const { return until == 0.0 || now() >= until; }
+  void start(double lost) {
+    until = now() + times * lost;
+    times = std::min(2.0 * times, 1e6);
+  }
 };
 
 // Communication buffers of the resident solves on one matrix (owned by the

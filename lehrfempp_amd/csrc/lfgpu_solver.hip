@@ -94,7 +94,7 @@ struct lfgpu_solver_cache {
   // equal the mirrored upper-diagonal values bit for bit: the FP64 SpMV
   // sweep of the PCG then reads the upper diagonals only (measured 7 %
   // faster at 2048^2; the FP32 sweeps measured slower that way)
-  bool no_resident = false;  // a resident solve was aborted
+  ResidentPause pause;  // of the resident solves
   bool sym64 = false;
   bool diag64 = false;  // the diagonal is the row sum less the others (k_dia_sym)
   uint64_t sym_version = ~0ull;  // built values that the two are of
@@ -3148,6 +3148,7 @@ struct lfgpu_batch {
   // whole slice, its rows in the locality order.
   struct Resident {
     int state = 0;  // 0: not looked at, 1: every problem fits, -1: the sweeps
+    ResidentPause pause;
     bool own_diag = false;  // bval is kept for the tiles only
     std::vector<ResidentProblem> tiles, rest;
     ResidentTiles *plan[3] = {nullptr, nullptr, nullptr};
@@ -3831,15 +3832,18 @@ void resident_release(lfgpu_solver_cache *c) {
 
 // end of a resident solve: one wait, then as pcg_finish
 int resident_finish(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentOutcome *out, bool mixed,
-                    lfgpu_pcg_info *info, bool *aborted) {
+                    lfgpu_pcg_info *info, ResidentPause *pause, bool *aborted) {
+  const double from = ResidentPause::now();
   LFG_HIP(hipEventRecord(ctx->ev1, ctx->stream));
   LFG_HIP(hipEventSynchronize(ctx->ev1));
   const ResidentState *rs = &out->solve;
   *aborted = out->team.raised != 0 || rs->aborted != 0;
   if (*aborted) {
     bufs->epoch = 0xffffffffu;  // the next solve clears the words and the flag
+    pause->start(ResidentPause::now() - from);
     return LFGPU_OK;
   }
+  *pause = ResidentPause{};
   PcgState h{};
   h.bb = rs->bb;
   h.rr = rs->rr;
@@ -3906,10 +3910,11 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
   // the resident solve (lfgpu_resident*.hip) where the system fits the chip,
   // unless the caller asked for graph replays or plain launches of the sweeps
   int gave_up = 0;  // resident solves that did not end
-  if (!single && c->blk_n == 0 && opts->graph == 0 && !t_timer && !c->no_resident) {
+  if (!single && c->blk_n == 0 && opts->graph == 0 && !t_timer && c->pause.over()) {
     ResidentOutcome *rs = reinterpret_cast<ResidentOutcome *>(ctx->pinned);
-    bool taken = false;
+    bool taken = false, aborted = false;
     int rc = LFGPU_OK;
+    const double from = ResidentPause::now();
     std::lock_guard<std::mutex> turn(resident_turn(ctx));
     LFG_HIP(hipEventRecord(ctx->ev0, s));
     if (c->fmt == FMT_DIA) {
@@ -3956,14 +3961,14 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
     if (rc == LFGPU_EOOM) {
       // (the sweeps need none of this memory)
       resident_release(c);
-      c->no_resident = true;
+      c->pause.start(ResidentPause::now() - from);
     } else if (rc != LFGPU_OK) {
       return rc;
     } else if (taken) {
       // (a workgroup gave up its wait for another one, as when other processes
       // hold a part of the chip: the sweeps go on from the x reached)
-      rc = resident_finish(ctx, &c->res, rs, mixed, info, &c->no_resident);
-      if (rc != LFGPU_OK || !c->no_resident) return rc;
+      rc = resident_finish(ctx, &c->res, rs, mixed, info, &c->pause, &aborted);
+      if (rc != LFGPU_OK || !aborted) return rc;
       gave_up = 1;
     }
   }
@@ -4615,7 +4620,7 @@ int batch_resident_ready(lfgpu_batch *bt, const lfgpu_pcg_opts *opts, bool *read
     if (bt->res.state != 1) batch_resident_give_up(bt);
     if (rc != LFGPU_EOOM) LFG_TRY(rc);
   }
-  *ready = bt->res.state == 1;
+  *ready = bt->res.state == 1 && bt->res.pause.over();
   return LFGPU_OK;
 }
 
@@ -4661,6 +4666,7 @@ int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
     LFG_TRY(resident_ell_batch_run(ctx, &R.bufs, R.eplan, batch_rest_view(bt), *opts, b->d, x->d,
                                    R.st, &R.h_abort[1], taken));
   if (!*taken) return LFGPU_OK;
+  const double from = ResidentPause::now();
   LFG_HIP(hipMemcpyAsync(R.h_st, R.st, bt->nprob * sizeof(ResidentState), hipMemcpyDeviceToHost, s));
   LFG_HIP(hipEventRecord(ctx->ev1, s));
   LFG_HIP(hipEventSynchronize(ctx->ev1));
@@ -4670,9 +4676,11 @@ int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
     for (ResidentTiles *t : R.plan)
       if (t) resident_tiles_reset(t);
     R.bufs.epoch = 0xffffffffu;
+    R.pause.start(ResidentPause::now() - from);
     *taken = false;  // (as in lfgpu_pcg: the sweeps go on from the x reached)
     return LFGPU_OK;
   }
+  R.pause = ResidentPause{};
   return batch_report_of(
       bt,
       [&](int p) {
@@ -4701,7 +4709,7 @@ extern "C" int lfgpu_batch_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, const lfgpu_vec 
     bool taken = false;
     const int rc = batch_resident_run(bt, b, x, opts, infos, summary, &taken, &aborted);
     if (taken || (rc != LFGPU_OK && rc != LFGPU_EOOM)) return rc;
-    batch_resident_give_up(bt);
+    if (!aborted) batch_resident_give_up(bt);
   }
   LFG_TRY(ensure_cache(ctx, bt->A, mixed, false));
   hipStream_t s = ctx->stream;

@@ -11,6 +11,7 @@ by at most 2 rtol ||b|| / 1e-3 (a tenth more for the recurrence residual's
 distance from the true one).
 """
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -529,4 +530,27 @@ def test_small_unstructured_problems_take_little_memory():
         # problem of one workgroup at most) and vectors
         assert free[0] - free[1] < 64 << 20, free
         for h in (batch, x, b, A):
+            h.close()
+
+
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_solves_come_back_after_one_that_gave_up(mode):
+    r, c, v, n = _flipped_system(60, 61, 1)
+    with capi.Context(0) as ctx:
+        A = capi.coo_to_csr(ctx, r, c, v, n, n)
+        batch = capi.Batch(ctx, A, np.array([0, n], np.int32))
+        b, x = capi.Vec(ctx, np.random.default_rng(1).standard_normal(n)), capi.Vec(ctx, n)
+
+        def batched(*a, **k):
+            return batch.pcg(*a, **k)[0]
+        for solve in (batched, lambda *a, **k: capi.pcg(ctx, A, *a, **k)):
+            for seconds in (0.0, 4.0, 0.0, 0.0, 4.0):
+                # (the sweeps take the next calls for 16, then 32 times what the
+                # lost launches took, a few ms each)
+                time.sleep(0.3)
+                ctx.set_resident_wait(seconds)
+                x.fill(0.0)
+                info = solve(b, x, rtol=1e-10, mode=mode)
+                assert info.converged and (info.syncs == 1) == (seconds > 0.0)
+        for h in (x, b, batch, A):
             h.close()
