@@ -32,7 +32,7 @@ struct ResidentOutcome {
 };
 
 // When the resident solves of a matrix or a batch may run again after one that
-// gave up: the sweeps take over for 16 times as long as it cost, twice as long
+// gave up or was refused: the sweeps take over for 16 times as long as it cost, twice as long
 // after each further one in a row, so that a lasting cause (a part of the chip
 // held by another process) costs a few per cent and a passing one not the
 // resident solves for good.
@@ -83,6 +83,10 @@ struct ResidentControl {
   }
 };
 int resident_start_batch(lfgpu_ctx *ctx, ResidentControl *control, int jobs);
+// Status of a cooperative launch that the runtime refused: while another
+// process that has made such launches lives on the device, they fail with
+// hipErrorIllegalState, and the sweeps have to do.
+constexpr int kResidentRefused = -1;
 int resident_launch_team(hipStream_t s, const void *fn, int team, void *args, size_t lds,
                          bool *taken);
 // Queues kernel fn (one argument struct) on `team` workgroups that all run at

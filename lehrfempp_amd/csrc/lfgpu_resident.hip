@@ -1550,11 +1550,10 @@ int resident_launch_team(hipStream_t s, const void *fn, int team, void *args, si
     // all workgroups of the team must run at once
     const hipError_t e =
         hipLaunchCooperativeKernel(fn, dim3(team), dim3(kThreads), argv, (unsigned)lds, s);
-    if (e == hipErrorCooperativeLaunchTooLarge) {
+    if (e != hipSuccess) {
       (void)hipGetLastError();
-      return LFGPU_OK;
+      return e == hipErrorCooperativeLaunchTooLarge ? LFGPU_OK : kResidentRefused;
     }
-    LFG_HIP(e);
   }
   *taken = true;
   return LFGPU_OK;

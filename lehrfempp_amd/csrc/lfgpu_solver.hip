@@ -3914,8 +3914,8 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
     ResidentOutcome *rs = reinterpret_cast<ResidentOutcome *>(ctx->pinned);
     bool taken = false, aborted = false;
     int rc = LFGPU_OK;
-    const double from = ResidentPause::now();
     std::lock_guard<std::mutex> turn(resident_turn(ctx));
+    const double from = ResidentPause::now();
     LFG_HIP(hipEventRecord(ctx->ev0, s));
     if (c->fmt == FMT_DIA) {
       ResidentDia rd;
@@ -3958,9 +3958,9 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       re.xlo = c->xlo;
       rc = resident_pcg_ell(ctx, &c->res, &c->res_ell, re, *opts, b->d, x->d, rs, &taken);
     }
-    if (rc == LFGPU_EOOM) {
+    if (rc == LFGPU_EOOM || rc == kResidentRefused) {
       // (the sweeps need none of this memory)
-      resident_release(c);
+      if (rc == LFGPU_EOOM) resident_release(c);
       c->pause.start(ResidentPause::now() - from);
     } else if (rc != LFGPU_OK) {
       return rc;
@@ -4625,8 +4625,8 @@ int batch_resident_ready(lfgpu_batch *bt, const lfgpu_pcg_opts *opts, bool *read
 }
 
 // The whole batch in one launch for its lattices and one for the others.
-// *taken = false: the chip does not hold the teams; or (*aborted) a workgroup
-// gave up its wait.
+// *taken = false: the chip does not hold the teams; or (*aborted) the launch
+// was refused, or a workgroup gave up its wait.
 int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
                        const lfgpu_pcg_opts *opts, lfgpu_pcg_info *infos,
                        lfgpu_pcg_info *summary, bool *taken, bool *aborted) {
@@ -4648,6 +4648,8 @@ int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
   LFG_HIP(hipMemcpyAsync(R.st, R.h_st, bt->nprob * sizeof(ResidentState), hipMemcpyHostToDevice, s));
   *taken = true;
   std::lock_guard<std::mutex> turn(resident_turn(ctx));
+  const double from = ResidentPause::now();
+  int rc = LFGPU_OK;
   if (!R.tiles.empty()) {
     ResidentDia rd;
     rd.n = bt->A->nrows;
@@ -4659,14 +4661,20 @@ int batch_resident_run(lfgpu_batch *bt, const lfgpu_vec *b, lfgpu_vec *x,
     rd.dinv32 = c->dinv32;
     rd.dinv16 = c->dinv16;
     rd.xlo = c->xlo;
-    LFG_TRY(resident_tiles_run(ctx, R.plan[opts->mode], rd, *opts, b->d, x->d, R.st,
-                               &R.h_abort[0], taken));
+    rc = resident_tiles_run(ctx, R.plan[opts->mode], rd, *opts, b->d, x->d, R.st, &R.h_abort[0],
+                            taken);
   }
-  if (*taken && !R.rest.empty())
-    LFG_TRY(resident_ell_batch_run(ctx, &R.bufs, R.eplan, batch_rest_view(bt), *opts, b->d, x->d,
-                                   R.st, &R.h_abort[1], taken));
-  if (!*taken) return LFGPU_OK;
-  const double from = ResidentPause::now();
+  if (rc == LFGPU_OK && *taken && !R.rest.empty())
+    rc = resident_ell_batch_run(ctx, &R.bufs, R.eplan, batch_rest_view(bt), *opts, b->d, x->d,
+                                R.st, &R.h_abort[1], taken);
+  if (rc != LFGPU_OK || !*taken) {
+    // (the lattices' launch may be under way)
+    LFG_HIP(hipStreamSynchronize(s));
+    if (rc != kResidentRefused) return rc;
+    R.pause.start(ResidentPause::now() - from);
+    *aborted = true;
+    return LFGPU_OK;
+  }
   LFG_HIP(hipMemcpyAsync(R.h_st, R.st, bt->nprob * sizeof(ResidentState), hipMemcpyDeviceToHost, s));
   LFG_HIP(hipEventRecord(ctx->ev1, s));
   LFG_HIP(hipEventSynchronize(ctx->ev1));

@@ -1,5 +1,5 @@
-// Solves in one launch while device allocations fail, and large downloads
-// while host allocations do.  The driver's own hipMalloc stands before the runtime's and lets the k-th allocation of a call
+// Solves in one launch while device allocations fail or the launch is refused,
+// and large downloads while host allocations fail.  The driver's own hipMalloc stands before the runtime's and lets the k-th allocation of a call
 // fail, for every k there is: the call has to end like one that had the memory
 // (the sweeps, whose storage exists by then, need none of it), and so has the
 // next call, whatever the failed one had allocated.  Nothing stays allocated
@@ -7,12 +7,14 @@
 // Exit status 0 on success.
 #include <dlfcn.h>
 
+#include <chrono>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <new>
 #include <random>
+#include <thread>
 #include <unordered_map>
 #include <vector>
 
@@ -33,6 +35,17 @@ extern "C" int hipMalloc(void **p, size_t bytes) {
   const int e = real(p, bytes);
   if (e == 0) g_live += g_size[*p] = bytes;
   return e;
+}
+struct Grid {
+  uint32_t x, y, z;
+};
+int g_refuse = 0;  // what cooperative launches return
+extern "C" int hipLaunchCooperativeKernel(const void *fn, Grid grid, Grid block, void **args,
+                                          unsigned lds, void *stream) {
+  static auto *real =
+      reinterpret_cast<int (*)(const void *, Grid, Grid, void **, unsigned, void *)>(
+          dlsym(RTLD_NEXT, "hipLaunchCooperativeKernel"));
+  return g_refuse ? g_refuse : real(fn, grid, block, args, lds, stream);
 }
 long g_events = 0;
 extern "C" int hipEventCreateWithFlags(void **ev, unsigned flags) {
@@ -74,6 +87,7 @@ extern "C" int hipMemcpy(void *to, const void *from, size_t bytes, int kind);
 
 namespace {
 int fails = 0;
+bool g_resident = true;  // solves run in one launch where the system fits
 #define EXPECT(cond, ...)                 \
   do {                                    \
     if (!(cond)) {                        \
@@ -170,7 +184,7 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
     const bool failed = g_calls > k;
     g_fail_at = -1;
     EXPECT(norm(got, &want) <= bound, "%s, allocation %ld: %g off", name, k, norm(got, &want));
-    EXPECT(failed || info.syncs == 1, "%s: not in one launch", name);
+    EXPECT(failed || info.syncs == 1 || !g_resident, "%s: not in one launch", name);
     EXPECT(!failed || g_live == swept, "%s, allocation %ld: %ld bytes kept", name, k,
            (long)(g_live - swept));
     solve(0, got);
@@ -188,6 +202,63 @@ void run(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch
       return;
     }
   }
+}
+
+// The device's cooperative queue may belong to another process: its launches
+// then fail with "the operation cannot be performed in the present state".
+void refused(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool batch) {
+  std::vector<double> want((size_t)s.n), got((size_t)s.n);
+  lfgpu_csr *A = nullptr;
+  lfgpu_vec *b = nullptr, *x = nullptr;
+  lfgpu_batch *bt = nullptr;
+  OK(lfgpu_coo_to_csr(ctx, (int64_t)s.val.size(), s.row.data(), s.col.data(), s.val.data(), s.n,
+                      s.n, &A));
+  OK(lfgpu_vec_create(ctx, s.n, s.rhs.data(), &b));
+  OK(lfgpu_vec_create(ctx, s.n, nullptr, &x));
+  if (batch) OK(lfgpu_batch_create(ctx, A, (int)s.off.size() - 1, s.off.data(), &bt));
+  lfgpu_pcg_opts opts{};
+  opts.rtol = 1e-11;
+  opts.maxit = 20000;
+  opts.mode = mode;
+  const double bound = 2.2 * opts.rtol * norm(s.rhs) / 0.01;  // as in run()
+  for (int turn = 0; turn < 4; ++turn) {  // the sweeps, refused twice, then not
+    lfgpu_pcg_info info{};
+    opts.graph = turn == 0 ? 1 : 0;
+    g_refuse = turn < 3 ? 401 : 0;
+    if (turn == 3) std::this_thread::sleep_for(std::chrono::milliseconds(300));
+    OK(lfgpu_vec_fill(x, 0.0));
+    if (batch) OK(lfgpu_batch_pcg(ctx, bt, b, x, &opts, nullptr, &info));
+    else OK(lfgpu_pcg(ctx, A, b, x, &opts, &info));
+    g_refuse = 0;
+    EXPECT(info.converged, "%s, turn %d: not converged", name, turn);
+    EXPECT(turn < 3 || info.syncs == 1 || !g_resident, "%s: not in one launch", name);
+    OK(lfgpu_vec_download(x, got.data(), s.n));
+    if (turn == 0) want = got;
+    EXPECT(norm(got, &want) <= bound, "%s, turn %d: %g off", name, turn, norm(got, &want));
+  }
+  OK(lfgpu_batch_destroy(bt));
+  OK(lfgpu_vec_destroy(x));
+  OK(lfgpu_vec_destroy(b));
+  OK(lfgpu_csr_destroy(A));
+}
+
+// Whether solves run in one launch here: another process may hold the queue.
+bool resident(lfgpu_ctx *ctx, const System &s) {
+  lfgpu_csr *A = nullptr;
+  lfgpu_vec *b = nullptr, *x = nullptr;
+  OK(lfgpu_coo_to_csr(ctx, (int64_t)s.val.size(), s.row.data(), s.col.data(), s.val.data(), s.n,
+                      s.n, &A));
+  OK(lfgpu_vec_create(ctx, s.n, s.rhs.data(), &b));
+  OK(lfgpu_vec_create(ctx, s.n, nullptr, &x));
+  lfgpu_pcg_opts opts{};
+  opts.rtol = 1e-11;
+  opts.maxit = 20000;
+  lfgpu_pcg_info info{};
+  OK(lfgpu_pcg(ctx, A, b, x, &opts, &info));
+  OK(lfgpu_vec_destroy(x));
+  OK(lfgpu_vec_destroy(b));
+  OK(lfgpu_csr_destroy(A));
+  return info.syncs == 1;
 }
 
 // A download through the staging ring creates no event (the context's device
@@ -279,6 +350,8 @@ int main() {
   // (what the middle of the turned ones shows does not cover them: no diagonals
   // for the sweeps, which run on sliced ELL, but for the others' tiles)
   for (int k = 0; k < 6; ++k) add_lattice(mixed, 70 + k, 50, k % 2 ? 5 : 0, 21 + k, 10);
+  g_resident = resident(ctx, lattice);
+  std::printf("solves run in one launch: %s\n", g_resident ? "yes" : "no");
   for (int mode : {LFGPU_PCG_FP64, LFGPU_PCG_MIXED, LFGPU_PCG_MIXED_MATRIX}) {
     run("lattice", ctx, lattice, mode, false);
     run("sliced ELL", ctx, ell, mode, false);
@@ -286,6 +359,9 @@ int main() {
     run("batch of lattices", ctx, bands, mode, true);
     run("batch of both", ctx, both, mode, true);
     run("batch of both, swept on ELL", ctx, mixed, mode, true);
+    refused("lattice", ctx, lattice, mode, false);
+    refused("sliced ELL", ctx, ell, mode, false);
+    refused("batch of both", ctx, both, mode, true);
   }
   storage(ctx, lattice);
   download(ctx);

@@ -1,4 +1,4 @@
-"""Failing device allocations in the one-launch solves
+"""Failing allocations and refused launches in the one-launch solves
 (tests/cpp/alloc_demo.cc)."""
 import os
 import subprocess
@@ -22,3 +22,25 @@ def test_alloc_driver_runs_on_gpu():
     print(res.stdout)
     assert res.returncode == 0, res.stdout + res.stderr
     assert "OK" in res.stdout
+
+
+@pytest.mark.gpu
+def test_alloc_driver_runs_beside_a_process_that_has_solved():
+    # cooperative launches of a second process can be refused as long as the
+    # first one lives
+    import numpy as np
+
+    from lehrfempp_amd import capi
+    n = 4096
+    i = np.arange(n)
+    with capi.Context(0) as ctx:
+        A = capi.coo_to_csr(ctx, np.concatenate([i, i[:-1], i[1:]]),
+                            np.concatenate([i, i[1:], i[:-1]]),
+                            np.concatenate([np.full(n, 2.1), np.full(2 * n - 2, -1.0)]), n, n)
+        b, x = capi.Vec(ctx, np.ones(n)), capi.Vec(ctx, n)
+        assert capi.pcg(ctx, A, b, x).syncs == 1
+        test_alloc_driver_runs_on_gpu()
+        x.fill(0.0)
+        assert capi.pcg(ctx, A, b, x).syncs == 1
+        for h in (x, b, A):
+            h.close()
