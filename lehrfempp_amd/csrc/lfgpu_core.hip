@@ -115,6 +115,20 @@ int exclusive_scan_i32(hipStream_t s, const int32_t *in, int32_t *out, int64_t n
   return LFGPU_OK;
 }
 
+int sort_by_key(hipStream_t s, const uint64_t *keys, uint64_t *keys_s, const int32_t *idx,
+                int32_t *idx_s, int64_t n, int bits) {
+  size_t tmp_bytes = 0;
+  LFG_HIP(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, keys_s, idx, idx_s, (size_t)n, 0,
+                                    bits, s));
+  void *tmp = nullptr;
+  LFG_TRY(dmalloc(&tmp, tmp_bytes, "sort scratch"));
+  hipError_t e = rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys_s, idx, idx_s, (size_t)n, 0,
+                                           bits, s);
+  if (e == hipSuccess) e = hipStreamSynchronize(s);
+  dfree(tmp);
+  return e == hipSuccess ? LFGPU_OK : hip_fail(e, "rocprim::radix_sort_pairs");
+}
+
 static inline unsigned grid_for(int64_t n, int block) {
   int64_t g = (n + block - 1) / block;
   if (g < 1) g = 1;

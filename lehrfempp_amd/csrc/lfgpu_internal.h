@@ -58,6 +58,10 @@ int resolve_coeff(const lfgpu_coeff *c, int64_t ncells, int nqp, bool allow_null
 int exclusive_scan_i32(hipStream_t s, const int32_t *in, int32_t *out, int64_t n,
                        int64_t *total);
 
+// Stable sort of idx by the low `bits` bits of the keys into keys_s, idx_s.
+int sort_by_key(hipStream_t s, const uint64_t *keys, uint64_t *keys_s, const int32_t *idx,
+                int32_t *idx_s, int64_t n, int bits);
+
 }  // namespace lfgpu
 
 namespace lfgpu {

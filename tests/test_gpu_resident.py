@@ -554,3 +554,32 @@ def test_resident_solves_come_back_after_one_that_gave_up(mode):
                 assert info.converged and (info.syncs == 1) == (seconds > 0.0)
         for h in (x, b, batch, A):
             h.close()
+
+
+# a call on a new batch finds the rows' order and splits them over teams: that
+# takes less than the sweeps' own first call (which tunes and captures) and their
+# solve
+@pytest.mark.parametrize("S, count", [(8, 20000), (64, 1000)])
+def test_first_call_on_unstructured_problems(ctx, S, count):
+    some = [_flipped_system(S, S, k) for k in range(8)]
+    n = some[0][3]
+    parts = [(r + k * n, c + k * n, v) for k in range(count) for r, c, v, _ in (some[k % 8],)]
+    A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n * count, n * count)
+    bh = np.random.default_rng(3).standard_normal((count, n))
+    b, x = capi.Vec(ctx, bh), capi.Vec(ctx, n * count)
+    off = np.arange(count + 1, dtype=np.int32) * n
+    best, got = {}, {}
+    for graph in (1, 0, 1, 0, 1, 0):
+        batch = capi.Batch(ctx, A, off)
+        x.fill(0.0)
+        ctx.sync()
+        start = time.perf_counter()
+        batch.pcg(b, x, rtol=1e-10, graph=graph)
+        best[graph] = min(best.get(graph, 1e9), time.perf_counter() - start)
+        got[graph] = x.numpy().reshape(count, n)
+        batch.close()
+    assert best[0] <= best[1], best
+    bound = 2.2e-10 * np.linalg.norm(bh, axis=1) / 1e-3
+    assert (np.linalg.norm(got[0] - got[1], axis=1) <= bound).all()
+    for h in (x, b, A):
+        h.close()
