@@ -633,36 +633,64 @@ __global__ __launch_bounds__(kThreads) void k_res_ell_batch(EllArgs base) {
 // the split, built once per pattern
 // ---------------------------------------------------------------------------
 // One workgroup per part: a bitmap of the outside columns over the window
-// that 16-bit offsets reach, its prefix sums as their places behind the own
-// rows, and every slot's place.  home: every slice's part and number in it.
-// parts[g].outside = number of outside rows; a part with more than `room`
-// places writes nothing else.
+// that 16-bit offsets reach, the number of them before each of its words, which
+// gives a column's place behind the own rows, and every slot's place.  home:
+// every slice's part and number in it.  parts[g].outside = number of outside
+// rows; a part with more than `room` places writes nothing else.  A wavefront
+// takes a slice; those of a long row all of them together, four columns of a
+// lane in flight (one thread a row, its slots and a binary search for each of
+// them one after the other, took 70 ms for a matrix with one row of 20000).
 constexpr int kSplitThreads = 512;
+constexpr int kSplitWaves = kSplitThreads / 64;
+constexpr int32_t kLongSlice = 64;
 __global__ __launch_bounds__(kSplitThreads) void k_ell_split(
     int32_t n, const int32_t *slice_off, const int16_t *dcol, const int32_t *slist,
     const int2 *home, int32_t room, EllPart *parts, int32_t *ext, uint16_t *lcol,
     uint8_t *needed) {
   extern __shared__ uint32_t map[];
   __shared__ int32_t sums[kSplitThreads];
-  const int t = threadIdx.x, me = blockIdx.x;
+  const int t = threadIdx.x, me = blockIdx.x, lane = t & 63, wave = t >> 6;
   EllPart &part = parts[me];
-  const int32_t r0 = part.r0, rows = 64 * part.slices;
+  const int32_t r0 = part.r0, slices = part.slices, rows = 64 * slices;
   slist += part.first;
   int32_t *list = ext + part.at;
   const int32_t words = (part.r1 - r0 + 65567) / 32;
+  uint32_t *const ahead = map + words;  // outside columns before a word
   for (int32_t k = t; k < words; k += kSplitThreads) map[k] = 0;
   __syncthreads();
-  for (int32_t i = t; i < rows; i += kSplitThreads) {
-    const int32_t s = slist[i >> 6], r = 64 * s + (i & 63);
-    const int32_t o = slice_off[s] + (i & 63), w = (slice_off[s + 1] - slice_off[s]) >> 6;
-    for (int32_t k = 0; k < w && r < n; ++k) {
-      const int32_t c = r + dcol[o + 64 * k];
-      if (home[c >> 6].x != me) {
-        const int32_t b = c - r0 + 32768;
-        atomicOr(&map[b >> 5], 1u << (b & 31));
+  // fn(slot, column, its slice's part and number) for the part's slots of rows
+  // below n, and pad(slot) for the others
+  auto slots = [&](auto &&fn, auto &&pad) {
+    for (int longs = 0; longs < 2; ++longs)
+      for (int32_t i = longs ? 0 : wave; i < slices; i += longs ? 1 : kSplitWaves) {
+        const int32_t s = slist[i], r = 64 * s + lane;
+        const int32_t o = slice_off[s], w = (slice_off[s + 1] - o) >> 6;
+        if ((w > kLongSlice) != (longs != 0)) continue;
+        const int32_t step = longs ? kSplitWaves : 1;
+        for (int32_t k0 = longs ? wave : 0; k0 < w; k0 += 4 * step) {
+          int32_t c[4];
+          int2 h[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u)
+            c[u] = r + dcol[o + 64 * min(k0 + u * step, w - 1) + lane];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) h[u] = home[r < n ? c[u] >> 6 : 0];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int32_t k = k0 + u * step;
+            if (k >= w) continue;
+            if (r < n) fn(o + 64 * k + lane, c[u], h[u]);
+            else pad(o + 64 * k + lane);
+          }
+        }
       }
+  };
+  slots([&](int32_t, int32_t c, int2 h) {
+    if (h.x != me) {
+      const int32_t b = c - r0 + 32768;
+      atomicOr(&map[b >> 5], 1u << (b & 31));
     }
-  }
+  }, [](int32_t) {});
   __syncthreads();
   // thread t's run of words and the number of outside rows before it
   const int32_t per = (words + kSplitThreads - 1) / kSplitThreads;
@@ -679,37 +707,23 @@ __global__ __launch_bounds__(kSplitThreads) void k_ell_split(
   if (t == 0) part.outside = all;
   if (all > room - rows) return;
   int32_t e = before;
-  for (int32_t k = k0; k < k1; ++k)
+  for (int32_t k = k0; k < k1; ++k) {
+    ahead[k] = e;
     for (uint32_t m = map[k]; m; m &= m - 1) {
       const int32_t c = r0 - 32768 + 32 * k + (__ffs(m) - 1);
       list[e++] = c;
       needed[c] = 1;
     }
-  __syncthreads();
-  for (int32_t i = t; i < rows; i += kSplitThreads) {
-    const int32_t s = slist[i >> 6], r = 64 * s + (i & 63);
-    const int32_t o = slice_off[s] + (i & 63), w = (slice_off[s + 1] - slice_off[s]) >> 6;
-    for (int32_t k = 0; k < w; ++k) {
-      int32_t at = 0;  // (lanes past the last row)
-      if (r < n) {
-        const int32_t c = r + dcol[o + 64 * k];
-        const int2 h = home[c >> 6];
-        if (h.x == me) {
-          at = 64 * h.y + (c & 63);
-        } else {
-          // place of c among the outside rows: binary search in the list
-          int32_t lo = 0, hi = all - 1;
-          while (lo < hi) {
-            const int32_t m = (lo + hi) >> 1;
-            if (list[m] < c) lo = m + 1;
-            else hi = m;
-          }
-          at = rows + lo;
-        }
-      }
-      lcol[o + 64 * k] = (uint16_t)at;
-    }
   }
+  __syncthreads();
+  slots([&](int32_t at, int32_t c, int2 h) {
+    int32_t place = 64 * h.y + (c & 63);
+    if (h.x != me) {
+      const int32_t b = c - r0 + 32768;
+      place = rows + ahead[b >> 5] + __popc(map[b >> 5] & ((1u << (b & 31)) - 1u));
+    }
+    lcol[at] = (uint16_t)place;
+  }, [&](int32_t at) { lcol[at] = 0; });  // (lanes past the last row)
 }
 
 struct EllVariant {
@@ -867,6 +881,17 @@ bool split_windows(Split &out, const std::vector<int32_t> &off, int32_t s0, int3
   return true;
 }
 
+// places that 16 bits and the LDS of a workgroup hold
+constexpr int32_t kRoom =
+    (int32_t)(kLdsDynamic / sizeof(double) < 65536 ? kLdsDynamic / sizeof(double) : 65536);
+
+// Whether a row couples to more rows than a workgroup has places for.
+bool row_too_long(const std::vector<int32_t> &off) {
+  for (size_t s = 0; s + 1 < off.size(); ++s)
+    if ((off[s + 1] - off[s]) / 64 >= kRoom) return true;
+  return false;
+}
+
 // LDS of a part
 size_t lds_bytes(const EllPart &q, int rpt) {
   const size_t places = 64 * (size_t)q.slices + q.outside;
@@ -877,7 +902,7 @@ size_t lds_bytes(const EllPart &q, int rpt) {
 // Builds the places of a split; *fits tells whether every part fits the LDS.
 int ell_split(hipStream_t s, ResidentEllPlan *p, const ResidentEll &A, Split &split, int rpt,
               bool *fits) {
-  const int32_t room = (int32_t)std::min<size_t>(kLdsDynamic / sizeof(double), 65536);
+  const int32_t room = kRoom;
   *fits = false;
   int64_t at = 0;
   int32_t span = 0;
@@ -916,7 +941,7 @@ int ell_split(hipStream_t s, ResidentEllPlan *p, const ResidentEll &A, Split &sp
                        hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemsetAsync(p->needed, 0, (size_t)A.n, s);
   if (e == hipSuccess) {
-    const size_t map = (size_t)(span + 65567) / 32 * 4;
+    const size_t map = (size_t)(span + 65567) / 32 * 8;
     hipLaunchKernelGGL(k_ell_split, dim3((unsigned)split.parts.size()), dim3(kSplitThreads), map,
                        s, A.n, A.slice_off, A.dcol, p->slist, dhome, room, p->parts, p->ext,
                        p->lcol, p->needed);
@@ -996,7 +1021,7 @@ int resident_pcg_ell(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan **pplan
     const int32_t slices = (int32_t)off.size() - 1;
     for (const EllVariant &v : kEllVariants) {
       const int cap = v.rpt * kWaves, want = (slices + cap - 1) / cap;
-      if (want > cus) continue;
+      if (want > cus || row_too_long(off)) continue;
       Split split;
       if (v.rpt > kSmallRows || !split_windows(split, off, 0, slices, cap, cus, A.n))
         split_runs(split, 0, slices, (slices + want - 1) / want, A.n);
@@ -1115,6 +1140,7 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
   if (np == 0 || !A.dcol) return LFGPU_OK;
   std::vector<int32_t> off;
   LFG_TRY(slice_offsets(s, A, off));
+  if (row_too_long(off)) return LFGPU_OK;
   const double per_slice = 64.0 * (double)A.slots / std::max(A.n, 1);
   EllTeams teams[2];
   bool can[2];

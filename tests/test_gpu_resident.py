@@ -583,3 +583,35 @@ def test_first_call_on_unstructured_problems(ctx, S, count):
     assert (np.linalg.norm(got[0] - got[1], axis=1) <= bound).all()
     for h in (x, b, A):
         h.close()
+
+
+# a line and a row that couples to all: the first call, which gives every slot its
+# place, takes no longer than the sweeps' first call, also where that row does not
+# fit a workgroup
+@pytest.mark.parametrize("n, fits", [(20000, True), (32000, False)])
+def test_first_call_on_a_matrix_with_a_long_row(ctx, n, fits):
+    i = np.arange(1, n)
+    w = np.exp(np.random.default_rng(1).standard_normal(2 * n - 3))
+    r, c = np.concatenate([np.zeros(n - 1, np.int64), i[:-1]]), np.concatenate([i, i[1:]])
+    diag = np.full(n, 1e-1)
+    np.add.at(diag, r, w)
+    np.add.at(diag, c, w)
+    k = np.arange(n)
+    bh = np.random.default_rng(2).standard_normal(n)
+    b, x = capi.Vec(ctx, bh), capi.Vec(ctx, n)
+    best, got = {}, {}
+    for graph in (1, 0, 1, 0):
+        A = capi.coo_to_csr(ctx, np.concatenate([r, c, k]), np.concatenate([c, r, k]),
+                            np.concatenate([-w, -w, diag]), n, n)
+        x.fill(0.0)
+        ctx.sync()
+        start = time.perf_counter()
+        info = capi.pcg(ctx, A, b, x, rtol=1e-10, graph=graph)
+        best[graph] = min(best.get(graph, 1e9), time.perf_counter() - start)
+        assert info.converged and (graph == 1 or (info.syncs == 1) == fits)
+        got[graph] = x.numpy()
+        A.close()
+    assert best[0] <= 1.1 * best[1], best
+    assert np.linalg.norm(got[0] - got[1]) <= 2.2e-10 * np.linalg.norm(bh) / 0.1
+    for h in (x, b):
+        h.close()
