@@ -615,3 +615,38 @@ def test_first_call_on_a_matrix_with_a_long_row(ctx, n, fits):
     assert np.linalg.norm(got[0] - got[1]) <= 2.2e-10 * np.linalg.norm(bh) / 0.1
     for h in (x, b):
         h.close()
+
+
+# many small lattices: the first call plans for its own mode only, and another
+# mode's first call for that one
+def test_first_call_on_many_lattices(ctx):
+    S, count = 9, 40000
+    some = [_lattice_system(S, S, P1, k) for k in range(8)]
+    n = some[0][3]
+    parts = [(r + k * n, c + k * n, v) for k in range(count) for r, c, v, _ in (some[k % 8],)]
+    A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n * count, n * count)
+    bh = np.random.default_rng(3).standard_normal((count, n))
+    b, x = capi.Vec(ctx, bh), capi.Vec(ctx, n * count)
+    off = np.arange(count + 1, dtype=np.int32) * n
+    best, got, summ = {}, [], capi.PcgInfo()
+    for graph in (1, 0, 1, 0, 1, 0):
+        batch = capi.Batch(ctx, A, off)
+        x.fill(0.0)
+        ctx.sync()
+        opts = capi.PcgOpts(1e-10, 100000, capi.PCG_FP64, 64, 0.0, 0, 0, graph)
+        start = time.perf_counter()  # (without 40000 Python objects of the problems)
+        capi.check(capi.lib().lfgpu_batch_pcg(ctx.h, batch.h, b.h, x.h, ctypes.byref(opts), None,
+                                              ctypes.byref(summ)))
+        best[graph] = min(best.get(graph, 1e9), time.perf_counter() - start)
+        assert graph == 1 or summ.syncs == 1
+    got.append(x.numpy().reshape(count, n))
+    for mode in (capi.PCG_MIXED_MATRIX, capi.PCG_FP64):
+        x.fill(0.0)
+        batch.pcg(b, x, rtol=1e-10, mode=mode)
+        got.append(x.numpy().reshape(count, n))
+    assert np.array_equal(got[0], got[2])
+    bound = 2.2e-10 * np.linalg.norm(bh, axis=1) / 1e-3
+    assert (np.linalg.norm(got[0] - got[1], axis=1) <= bound).all()
+    assert best[0] <= best[1], best
+    for h in (batch, x, b, A):
+        h.close()
