@@ -4601,9 +4601,19 @@ void batch_resident_give_up(lfgpu_batch *bt) {
 
 // The tiles' plan of a mode, made by its first call (40000 problems of 9 x 9 rows:
 // 8 ms a plan, with all three the first FP64 call took 42 ms, the sweeps' 39).
+// None where the sweeps are faster, for many small lattices in the mixed modes:
+// a workgroup takes one at a time and widens its matrix first.  8 x 8 rows,
+// FP32 Krylov, sweeps / one launch: 4000 problems 5.0 / 4.8 ms, 8000 8.5 / 9.3,
+// 40000 37 / 46; 16 x 16 rows 4000 8.8 / 7.2, 32000 54 / 57; 24 x 24 rows 16000
+// 58 / 41.  (FP64: 36 / 26 at 32000 of 16 x 16, 18 / 16 at 40000 of 8 x 8.)
 int batch_tiles_plan(lfgpu_batch *bt, int mode) {
   lfgpu_batch::Resident &R = bt->res;
   if (R.tiles.empty() || R.plan[mode]) return LFGPU_OK;
+  int64_t rows = 0;
+  for (const ResidentProblem &q : R.tiles) rows += q.n;
+  const int64_t count = (int64_t)R.tiles.size();
+  if (mode != LFGPU_PCG_FP64 && count > 20 * (int64_t)bt->ctx->cus && rows <= 256 * count)
+    return LFGPU_OK;
   return resident_tiles_plan(bt->ctx, R.tiles, mode, &R.plan[mode]);
 }
 
@@ -4638,7 +4648,7 @@ int batch_resident_setup(lfgpu_batch *bt, int mode) {
     bt->bndiag = nd;
   }
   LFG_TRY(batch_tiles_plan(bt, mode));
-  if (!R.tiles.empty() && !resident_tiles_fit(R.plan[mode])) return LFGPU_OK;
+  if (R.plan[mode] && !resident_tiles_fit(R.plan[mode])) return LFGPU_OK;
   if (!R.rest.empty()) {
     bool fits = false;
     LFG_TRY(batch_rest_storage(bt, &fits));

@@ -650,3 +650,33 @@ def test_first_call_on_many_lattices(ctx):
     assert best[0] <= best[1], best
     for h in (batch, x, b, A):
         h.close()
+
+
+# many small lattices in the mixed modes, where the sweeps are faster: a call
+# takes no longer than they do, and FP64 stays in one launch
+@pytest.mark.parametrize("mode", MODES)
+def test_many_small_lattices(ctx, mode):
+    S, count = 8, 20000
+    some = [_lattice_system(S, S, P1, k) for k in range(8)]
+    n = some[0][3]
+    parts = [(r + k * n, c + k * n, v) for k in range(count) for r, c, v, _ in (some[k % 8],)]
+    A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n * count, n * count)
+    bh = np.random.default_rng(3).standard_normal((count, n))
+    b, x = capi.Vec(ctx, bh), capi.Vec(ctx, n * count)
+    batch = capi.Batch(ctx, A, np.arange(count + 1, dtype=np.int32) * n)
+    best, got, summ = {}, {}, capi.PcgInfo()
+    for graph in (1, 0) * 4:
+        x.fill(0.0)
+        ctx.sync()
+        opts = capi.PcgOpts(1e-10, 100000, mode, 64, 0.0, 0, 0, graph)
+        start = time.perf_counter()
+        capi.check(capi.lib().lfgpu_batch_pcg(ctx.h, batch.h, b.h, x.h, ctypes.byref(opts), None,
+                                              ctypes.byref(summ)))
+        best[graph] = min(best.get(graph, 1e9), time.perf_counter() - start)
+        assert graph == 1 or (summ.syncs == 1) == (mode == capi.PCG_FP64)
+        got[graph] = x.numpy().reshape(count, n)
+    bound = 2.2e-10 * np.linalg.norm(bh, axis=1) / 1e-3
+    assert (np.linalg.norm(got[0] - got[1], axis=1) <= bound).all()
+    assert best[0] <= 1.1 * best[1], best
+    for h in (batch, x, b, A):
+        h.close()
