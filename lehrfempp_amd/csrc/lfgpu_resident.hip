@@ -53,7 +53,7 @@ struct TileJob {
   int32_t index, lo;  // problem number, first row
   int32_t S, L, TW, TH, TX, team, slots, ghosts, ndiag;
   int32_t off[ND], shift[ND];
-  uint32_t halo_at, sums_at;  // words
+  uint64_t halo_at, sums_at;  // words
 };
 
 struct TileArgs {
@@ -1488,6 +1488,7 @@ static void fill_args(TileArgs &a, const ResidentDia &A, const lfgpu_pcg_opts &o
 }
 
 int resident_clear(hipStream_t s, unsigned long long *words, size_t n) {
+  if (n == 0) return LFGPU_OK;
   hipLaunchKernelGGL(k_zero_words, dim3((unsigned)std::min<size_t>(256, (n + 255) / 256)),
                      dim3(256), 0, s, words, n);
   LFG_HIP(hipGetLastError());
@@ -1704,10 +1705,12 @@ int resident_tiles_plan(lfgpu_ctx *ctx, const std::vector<ResidentProblem> &prob
     j.ndiag = q.ndiag;
     for (int d = 0; d < ND; ++d) j.off[d] = d < q.ndiag ? q.off[d] : 0;
     tile_shifts(j);
-    j.halo_at = (uint32_t)p->halo_words;
-    j.sums_at = (uint32_t)p->sums_words;
-    p->halo_words += (size_t)2 * j.team * 2 * j.slots;
-    p->sums_words += part_words(j.team) + kTotalWords;
+    j.halo_at = p->halo_words;
+    j.sums_at = p->sums_words;
+    if (j.team > 1) {  // (a workgroup alone exchanges nothing)
+      p->halo_words += (size_t)2 * j.team * 2 * j.slots;
+      p->sums_words += part_words(j.team) + kTotalWords;
+    }
     most = std::max<int64_t>(most, (int64_t)(g.TW + 2) * g.TH);
     for (int r = 0; r < j.team; ++r) slots.push_back(int2{(int)o, r});
   }

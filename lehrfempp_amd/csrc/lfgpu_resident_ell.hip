@@ -37,7 +37,7 @@ struct EllPart {
 // One problem of a batch.
 struct EllJob {
   int32_t index, team;
-  uint32_t sums_at;
+  uint64_t sums_at;
 };
 
 struct EllArgs {
@@ -1170,8 +1170,8 @@ int resident_ell_batch_plan(lfgpu_ctx *ctx, const ResidentEll &A,
       EllJob j{};
       j.index = q.index;
       j.team = (int32_t)(split.parts.size() - had);
-      j.sums_at = (uint32_t)p->sums_words;
-      p->sums_words += part_words(j.team) + kTotalWords;
+      j.sums_at = p->sums_words;
+      if (j.team > 1) p->sums_words += part_words(j.team) + kTotalWords;
       jobs.push_back(j);
       for (int r = 0; r < j.team; ++r) slots.push_back(int2{(int)o, r});
     }

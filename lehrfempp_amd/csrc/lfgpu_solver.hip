@@ -4513,6 +4513,10 @@ int batch_rest_storage(lfgpu_batch *bt, bool *fits) {
   lfgpu_batch::Resident &R = bt->res;
   hipStream_t s = bt->ctx->stream;
   *fits = false;
+  int64_t rows = 0;  // of the storage, in which a problem starts at a whole slice
+  for (const ResidentProblem &q : R.rest)
+    rows += ((int64_t)q.n + kSlice - 1) / kSlice * kSlice;
+  if (rows > INT32_MAX - kSlice) return LFGPU_OK;
   LFG_TRY(batch_rest_order(bt));
   LFG_TRY(dalloc(&R.slice_off, (size_t)R.nslices + 1, "batch slice offsets"));
   int32_t *w = nullptr;
@@ -4696,7 +4700,8 @@ int batch_resident_ready(lfgpu_batch *bt, const lfgpu_pcg_opts *opts, bool *read
   if (R.state == 0) {
     const int rc = batch_resident_setup(bt, opts->mode);
     if (R.state != 1) batch_resident_give_up(bt);
-    if (rc != LFGPU_EOOM) LFG_TRY(rc);
+    // (ERANGE: too many slots for 32 bits)
+    if (rc != LFGPU_EOOM && rc != LFGPU_ERANGE) LFG_TRY(rc);
   }
   if (R.state != 1 || !R.pause.over()) return LFGPU_OK;
   const int rc = batch_tiles_plan(bt, opts->mode);

@@ -680,3 +680,30 @@ def test_many_small_lattices(ctx, mode):
     assert best[0] <= 1.1 * best[1], best
     for h in (batch, x, b, A):
         h.close()
+
+
+def test_lattices_of_one_workgroup_take_no_words():
+    # 20000 problems of 25 rows, which exchange nothing with other workgroups
+    parts, off = [], [0]
+    for k in range(20000):
+        r, c, v, n = _lattice_system(5, 5, P1, k) if k < 4 else parts[k % 4]
+        parts.append((r, c, v, n))
+        off.append(off[-1] + n)
+    n = off[-1]
+    trip = [(r + o, c + o, v) for (r, c, v, _), o in zip(parts, off)]
+    total, now = ctypes.c_size_t(), ctypes.c_size_t()
+    with capi.Context(0) as ctx:
+        A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*trip)), n, n)
+        b, x = capi.Vec(ctx, np.random.default_rng(3).standard_normal(n)), capi.Vec(ctx, n)
+        batch = capi.Batch(ctx, A, np.array(off, np.int32))
+        free = []
+        for graph in (1, 0):
+            x.fill(0.0)
+            summ, _ = batch.pcg(b, x, graph=graph)
+            assert capi.lib().hipMemGetInfo(ctypes.byref(now), ctypes.byref(total)) == 0
+            free.append(now.value)
+        assert summ.syncs == 1  # the resident solve ran
+        # jobs, slots and outcomes: 200 B a problem
+        assert free[0] - free[1] < 16 << 20, free
+        for h in (batch, x, b, A):
+            h.close()
