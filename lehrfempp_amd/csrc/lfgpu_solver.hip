@@ -3147,7 +3147,9 @@ struct lfgpu_batch {
   // others on a sliced ELL of their own in which every problem starts at a
   // whole slice, its rows in the locality order.
   struct Resident {
-    int state = 0;  // 0: not looked at, 1: every problem fits, -1: the sweeps
+    // 0: not looked at, 2: tiles and rest are known, 1: every problem fits, and
+    // the storage is there, -1: the sweeps
+    int state = 0;
     ResidentPause pause;
     bool own_diag = false;  // bval is kept for the tiles only
     std::vector<ResidentProblem> tiles, rest;
@@ -4605,29 +4607,18 @@ void batch_resident_give_up(lfgpu_batch *bt) {
 
 // The tiles' plan of a mode, made by its first call (40000 problems of 9 x 9 rows:
 // 8 ms a plan, with all three the first FP64 call took 42 ms, the sweeps' 39).
-// None where the sweeps are faster, for many small lattices in the mixed modes:
-// a workgroup takes one at a time and widens its matrix first.  8 x 8 rows,
-// FP32 Krylov, sweeps / one launch: 4000 problems 5.0 / 4.8 ms, 8000 8.5 / 9.3,
-// 40000 37 / 46; 16 x 16 rows 4000 8.8 / 7.2, 32000 54 / 57; 24 x 24 rows 16000
-// 58 / 41.  (FP64: 36 / 26 at 32000 of 16 x 16, 18 / 16 at 40000 of 8 x 8.)
 int batch_tiles_plan(lfgpu_batch *bt, int mode) {
   lfgpu_batch::Resident &R = bt->res;
   if (R.tiles.empty() || R.plan[mode]) return LFGPU_OK;
-  int64_t rows = 0;
-  for (const ResidentProblem &q : R.tiles) rows += q.n;
-  const int64_t count = (int64_t)R.tiles.size();
-  if (mode != LFGPU_PCG_FP64 && count > 20 * (int64_t)bt->ctx->cus && rows <= 256 * count)
-    return LFGPU_OK;
   return resident_tiles_plan(bt->ctx, R.tiles, mode, &R.plan[mode]);
 }
 
 // Decides once per batch whether every problem can run resident, and builds
-// what that takes in the mode.  (The cache and bt->fmt exist.)
+// what that takes in the mode.  (The cache, bt->fmt and the lists exist.)
 int batch_resident_setup(lfgpu_batch *bt, int mode) {
   lfgpu_batch::Resident &R = bt->res;
   lfgpu_csr *A = bt->A;
   R.state = -1;
-  LFG_TRY(batch_find_lattices(bt));
   hipStream_t s = bt->ctx->stream;
   if (!R.tiles.empty() && bt->fmt == FMT_DIA) {
     // one set of diagonals for all problems
@@ -4652,7 +4643,7 @@ int batch_resident_setup(lfgpu_batch *bt, int mode) {
     bt->bndiag = nd;
   }
   LFG_TRY(batch_tiles_plan(bt, mode));
-  if (R.plan[mode] && !resident_tiles_fit(R.plan[mode])) return LFGPU_OK;
+  if (!R.tiles.empty() && !resident_tiles_fit(R.plan[mode])) return LFGPU_OK;
   if (!R.rest.empty()) {
     bool fits = false;
     LFG_TRY(batch_rest_storage(bt, &fits));
@@ -4689,27 +4680,52 @@ int batch_rest_fill(lfgpu_batch *bt, bool need32) {
   return LFGPU_OK;
 }
 
+// Whether the sweeps are faster in a mode (ms of sweeps / one launch):
+// * many small lattices in the mixed modes, since a workgroup takes one at a
+//   time and widens its matrix first.  FP32 vectors, 8 x 8 rows: 4000 problems
+//   5.0 / 4.8, 8000 8.5 / 9.3, 40000 37 / 46; 16 x 16 rows: 4000 8.8 / 7.2, 32000
+//   54 / 57; 24 x 24 rows: 16000 58 / 41.  (FP64: 40000 of 8 x 8 18 / 16.)
+// * with FP32 vectors, large unstructured problems that the chip does not hold
+//   at once (8 * 512 rows a CU), so that they run in turns.  P1 on unstructured
+//   squares, 400 iterations: 700^2 twice 10.1 / 7.9, 900^2 twice 14.5 / 15.9, four
+//   times 27.1 / 31.5; 300^2 22 times 19.1 / 15.3, 40 times 27.9 / 29.7; 181^2 120
+//   times 32.6 / 26.2.  (FP64 300^2 40 times 37 / 25, FP32 matrix 36 / 30.)
+bool batch_swept(const lfgpu_batch *bt, int mode) {
+  if (mode == LFGPU_PCG_FP64) return false;
+  auto rows_of = [](const std::vector<ResidentProblem> &list) {
+    int64_t rows = 0;
+    for (const ResidentProblem &q : list) rows += q.n;
+    return rows;
+  };
+  const lfgpu_batch::Resident &R = bt->res;
+  const int64_t lattices = (int64_t)R.tiles.size(), others = (int64_t)R.rest.size();
+  const int64_t cus = bt->ctx->cus, chip = 8 * 512 * cus, rows = rows_of(R.rest);
+  if (lattices > 20 * cus && rows_of(R.tiles) <= 256 * lattices) return true;
+  return mode == LFGPU_PCG_MIXED && ((rows > chip && rows > 262144 * others) ||
+                                     (rows > 3 * chip && rows > 50000 * others));
+}
+
 // Whether a call runs resident; on the way, the storage and the plans.
 int batch_resident_ready(lfgpu_batch *bt, const lfgpu_pcg_opts *opts, bool *ready) {
   *ready = false;
-  if (opts->graph != 0) return LFGPU_OK;
-  if (bt->fmt < 0 || bt->res.state == 0)
+  lfgpu_batch::Resident &R = bt->res;
+  if (opts->graph != 0 || R.state < 0) return LFGPU_OK;
+  if (bt->fmt < 0 || R.state == 0 || R.state == 2)
     LFG_TRY(ensure_cache(bt->ctx, bt->A, opts->mode != LFGPU_PCG_FP64, false));
   if (bt->fmt < 0) LFG_TRY(batch_choose_format(bt));
-  lfgpu_batch::Resident &R = bt->res;
+  int rc = LFGPU_OK;
   if (R.state == 0) {
-    const int rc = batch_resident_setup(bt, opts->mode);
-    if (R.state != 1) batch_resident_give_up(bt);
-    // (ERANGE: too many slots for 32 bits)
-    if (rc != LFGPU_EOOM && rc != LFGPU_ERANGE) LFG_TRY(rc);
+    rc = batch_find_lattices(bt);
+    R.state = rc == LFGPU_OK ? 2 : -1;
   }
-  if (R.state != 1 || !R.pause.over()) return LFGPU_OK;
-  const int rc = batch_tiles_plan(bt, opts->mode);
-  if (rc == LFGPU_EOOM) {
+  if (R.state > 0 && (!R.pause.over() || batch_swept(bt, opts->mode))) return LFGPU_OK;
+  if (R.state == 2) rc = batch_resident_setup(bt, opts->mode);
+  else if (R.state == 1) rc = batch_tiles_plan(bt, opts->mode);
+  if (R.state != 1 || rc != LFGPU_OK) {
     batch_resident_give_up(bt);
-    return LFGPU_OK;
+    // (ERANGE: too many slots for 32 bits)
+    return rc == LFGPU_EOOM || rc == LFGPU_ERANGE ? LFGPU_OK : rc;
   }
-  LFG_TRY(rc);
   *ready = R.tiles.empty() || resident_tiles_fit(R.plan[opts->mode]);
   return LFGPU_OK;
 }

@@ -707,3 +707,22 @@ def test_lattices_of_one_workgroup_take_no_words():
         assert free[0] - free[1] < 16 << 20, free
         for h in (batch, x, b, A):
             h.close()
+
+
+# a few large unstructured problems, more than the chip holds at once: in the
+# FP32-Krylov mode the sweeps are faster
+def test_few_large_unstructured_problems(ctx):
+    parts, off = [], [0]
+    for k in range(2):
+        r, c, v, n = _flipped_system(760, 761, k)
+        parts.append((r + off[-1], c + off[-1], v))
+        off.append(off[-1] + n)
+    n = off[-1]
+    A = capi.coo_to_csr(ctx, *(np.concatenate(p) for p in zip(*parts)), n, n)
+    b, x = capi.Vec(ctx, np.random.default_rng(3).standard_normal(n)), capi.Vec(ctx, n)
+    batch = capi.Batch(ctx, A, np.array(off, np.int32))
+    for mode in MODES:
+        summ, _ = batch.pcg(b, x, maxit=300, mode=mode, raise_on_noconv=False)
+        assert (summ.syncs == 1) == (mode != capi.PCG_MIXED)
+    for h in (batch, x, b, A):
+        h.close()
