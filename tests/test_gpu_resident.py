@@ -726,3 +726,59 @@ def test_few_large_unstructured_problems(ctx):
         assert (summ.syncs == 1) == (mode != capi.PCG_MIXED)
     for h in (batch, x, b, A):
         h.close()
+
+
+# entries (of value zero) on one side only: a workgroup then reads rows of others
+# that read none of its own; one to three rows a thread, five, and eight
+@pytest.mark.parametrize("S, L", [(40, 64), (181, 182), (363, 362), (512, 513), (800, 801),
+                                  (1025, 1024)])
+@pytest.mark.parametrize("mode", MODES)
+def test_resident_pcg_on_an_unsymmetric_pattern(ctx, S, L, mode):
+    r, c, v, n = _flipped_system(S, L, S)
+    rng = np.random.default_rng(S)
+    i = rng.integers(0, n // 2, n // 4)  # the upper half reads ahead
+    j = np.minimum(i + rng.integers(2, 3 * S, i.size), n - 1)
+    A = capi.coo_to_csr(ctx, np.concatenate([r, i]), np.concatenate([c, j]),
+                        np.concatenate([v, np.zeros(i.size)]), n, n)
+    out = _compare(ctx, A, n, mode, n + 1)
+    assert capi.solver_storage(A)[0] == capi.STORAGE_ELL16 and out[1][0].syncs == 1
+    x0 = np.random.default_rng(5).standard_normal(n)
+    out = _compare(ctx, A, n, mode, n + 2, x0=x0, maxit=3, rtol=1e-14)
+    assert out[0][0].iters == out[1][0].iters == 3
+    eps = 1e-13 if mode == capi.PCG_FP64 else 1e-5 if mode == capi.PCG_MIXED else 1e-12
+    assert np.linalg.norm(out[0][1] - out[1][1]) <= eps * np.linalg.norm(out[0][1])
+    A.close()
+
+
+# the three modes in turn on one matrix (other teams and layouts in the same
+# words), with caps that use up the exchanges' numbers, so that the words are
+# cleared, and with small ones: every solve like the first of its mode on a matrix
+# of its own
+@pytest.mark.parametrize("make", [
+    lambda: _lattice_system(65, 65, P1, 2), lambda: _lattice_system(362, 363, P1, 3),
+    lambda: _flipped_system(40, 64, 4), lambda: _flipped_system(363, 362, 5),
+])
+def test_resident_solves_share_their_words(ctx, make):
+    r, c, v, n = make()
+    A = capi.coo_to_csr(ctx, r, c, v, n, n)
+    batch = capi.Batch(ctx, A, np.array([0, n], np.int32))
+    b, x = capi.Vec(ctx, np.random.default_rng(1).standard_normal(n)), capi.Vec(ctx, n)
+    for call in (lambda M, B, **k: capi.pcg(ctx, M, b, x, **k),
+                 lambda M, B, **k: B.pcg(b, x, **k)[0]):
+        want = {}
+        for maxit in (20000, 2**31 - 1, 20000, 6 * 10**8, 6 * 10**8, 2**31 - 1):
+            for mode in MODES:
+                if mode not in want:
+                    M = capi.coo_to_csr(ctx, r, c, v, n, n)
+                    B = capi.Batch(ctx, M, np.array([0, n], np.int32))
+                    x.fill(0.0)
+                    call(M, B, mode=mode, maxit=20000)
+                    want[mode] = x.numpy()
+                    B.close()
+                    M.close()
+                x.fill(0.0)
+                info = call(A, batch, mode=mode, maxit=maxit)
+                assert info.converged and info.syncs == 1
+                assert np.array_equal(x.numpy(), want[mode])
+    for h in (batch, x, b, A):
+        h.close()
