@@ -68,10 +68,10 @@ int resident_prepare(lfgpu_ctx *ctx, ResidentBufs *bufs, size_t words, uint64_t 
 bool resident_will_clear(const ResidentBufs *bufs, size_t words, uint64_t need);
 int resident_clear(hipStream_t s, unsigned long long *words, size_t n);
 // What the workgroups of a batch share: the counter that hands out the slots,
-// the abort flag and, behind them, every problem's number of workgroups that
-// have come to it; set before every launch.
+// the number of workgroups that run, the abort flag and, behind them, every
+// problem's number of workgroups that have come to it; set before every launch.
 struct ResidentControl {
-  int ticket, pad;
+  int ticket, running;
   ResidentAbort abort;
   int *arrived() { return reinterpret_cast<int *>(this + 1); }
   static int alloc(ResidentControl **out, size_t jobs) {

@@ -90,7 +90,7 @@ struct TileArgs {
   const TileJob *__restrict__ jobs;
   const int2 *__restrict__ job_slots;
   int nslots;
-  int *ticket, *arrived;
+  int *ticket, *running, *arrived;
 };
 
 // The workgroup's tile: tw x th cells of the lattice, padded by one halo cell
@@ -866,6 +866,7 @@ __global__ __launch_bounds__(kThreads) void k_res_stream(TileArgs a) {
 template <class F>
 __device__ __forceinline__ void batch_loop(const TileArgs &base, F &&solve) {
   __shared__ int slot, up;
+  if (threadIdx.x == 0) atomicAdd(base.running, 1);
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) slot = atomicAdd(base.ticket, 1);
@@ -876,7 +877,8 @@ __device__ __forceinline__ void batch_loop(const TileArgs &base, F &&solve) {
     // (the job is read after the wait: held across it, the mixed kernels of 7
     // cells a thread spill 82 registers instead of 7, and 64 problems of 32 to
     // 512 lines take 59 ms instead of 46)
-    if (!team_assembles(base.arrived + jr.x, base.jobs[jr.x].team, base.abort, up)) return;
+    if (!team_assembles(base.arrived + jr.x, base.jobs[jr.x].team, base.running, base.abort, up))
+      return;
     const TileJob &jb = base.jobs[jr.x];
     TileArgs a = base;
     a.S = jb.S;
@@ -1355,7 +1357,7 @@ __global__ void k_start_batch(ResidentControl *c, int *arrived, int jobs, uint64
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < jobs) arrived[i] = 0;
   if (i == 0) {
-    c->ticket = 0;
+    c->ticket = c->running = 0;
     set_abort(&c->abort, ticks);
   }
 }
@@ -1765,6 +1767,7 @@ int resident_tiles_run(lfgpu_ctx *ctx, ResidentTiles *p, const ResidentDia &A,
   a.job_slots = p->slots;
   a.nslots = p->nslots;
   a.ticket = &p->control->ticket;
+  a.running = &p->control->running;
   a.arrived = p->control->arrived();
   p->epoch = (uint32_t)std::min<uint64_t>(p->epoch + need, 0xffffffffull);
   const int team = std::min(p->nslots, std::min(ctx->cus, kMaxTeam));

@@ -103,17 +103,27 @@ struct Wait {
 
 // The workgroups of a batch draw their slots in order, so that the first ones
 // of a team find it incomplete until the others have ended the problems that
-// they are at, whatever those take: that wait has no bound of time.  It ends,
-// since the earlier problems' workgroups are all there and end, or raise the
-// flag.  Returns false, in all threads, once it is up.  `scratch` is shared.
-__device__ __forceinline__ bool team_assembles(int *arrived, int team, ResidentAbort *abort,
-                                               int &scratch) {
+// they are at, whatever those take: that wait has no bound of time once all
+// workgroups of the launch run (`running` says how many do).  It ends, since the
+// earlier problems' workgroups are all there and end, or raise the flag.  Before
+// that the bound holds, as a workgroup may never come while others hold its CU.
+// Returns false, in all threads, once the flag is up.  `scratch` is shared.
+__device__ __forceinline__ bool team_assembles(int *arrived, int team, const int *running,
+                                               ResidentAbort *abort, int &scratch) {
   if (threadIdx.x == 0) {
     int up = 0;
+    const uint64_t from = wall_clock64();
     __hip_atomic_fetch_add(arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     while (team > 1 && !up &&
            __hip_atomic_load(arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < team) {
       up = __hip_atomic_load(&abort->raised, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (!up &&
+          __hip_atomic_load(running, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < (int)gridDim.x &&
+          wall_clock64() - from >
+              __hip_atomic_load(&abort->ticks, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        __hip_atomic_store(&abort->raised, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        up = 1;
+      }
       __builtin_amdgcn_s_sleep(2);
     }
     scratch = up;

@@ -72,7 +72,7 @@ struct EllArgs {
   const EllJob *__restrict__ jobs;
   const int2 *__restrict__ job_slots;  // slot (= part) -> job, rank in its team
   int nslots;
-  int *ticket, *arrived;
+  int *ticket, *running, *arrived;
 };
 
 // the precision modes: FP64; FP32 vectors; FP64 vectors with the FP32 matrix
@@ -612,6 +612,7 @@ __global__ __launch_bounds__(kThreads) void k_res_ell_batch(EllArgs base) {
   extern __shared__ double dyn[];
   __shared__ SumLds sh;
   __shared__ int slot, up;
+  if (threadIdx.x == 0) atomicAdd(base.running, 1);
   for (;;) {
     __syncthreads();
     if (threadIdx.x == 0) slot = atomicAdd(base.ticket, 1);
@@ -619,7 +620,8 @@ __global__ __launch_bounds__(kThreads) void k_res_ell_batch(EllArgs base) {
     const int k = __builtin_amdgcn_readfirstlane(slot);
     if (k >= base.nslots) return;
     const int2 jr = base.job_slots[k];
-    if (!team_assembles(base.arrived + jr.x, base.jobs[jr.x].team, base.abort, up)) return;
+    if (!team_assembles(base.arrived + jr.x, base.jobs[jr.x].team, base.running, base.abort, up))
+      return;
     const EllJob &jb = base.jobs[jr.x];
     EllArgs a = base;
     a.part += jb.sums_at;
@@ -1215,6 +1217,7 @@ int resident_ell_batch_run(lfgpu_ctx *ctx, ResidentBufs *bufs, ResidentEllPlan *
   a.job_slots = plan->slots;
   a.nslots = plan->nparts;
   a.ticket = &plan->control->ticket;
+  a.running = &plan->control->running;
   a.arrived = plan->control->arrived();
   LFG_TRY(resident_launch_team(s, kEllBatch[plan->rpt == 2 ? 0 : 1][opts.mode],
                                std::min(plan->nparts, std::min(ctx->cus, kMaxTeam)), &a,
