@@ -311,11 +311,15 @@ typedef struct lfgpu_pcg_opts {
    * recurrences (default). */
   int single_reduction;
   /* 0 (default) = the whole solve in one launch with the vectors kept on
-   * the chip where the system fits (any mode; info->syncs is 1 then, and at
-   * least 2 where the launch gave up and the sweeps went on), else
+   * the chip where the system fits (any mode; info->syncs is 1 then), else
    * plain launches, or in FP64 below 2^20 rows, where the solve is bound by
    * the launch rate, replays of each chunk of check_every iterations from a
    * captured hipGraph; 1 = always replay chunks (FP64); -1 = plain launches.
+   * The sweeps also take a call for which memory for the one launch cannot be
+   * had, which the runtime refuses to launch (while another process that has
+   * launched cooperatively lives on the GPU) or in which a workgroup gave up
+   * its wait (lfgpu_ctx_set_resident_wait; info->syncs is at least 2 then), and
+   * the next ones for some time.
    * 1 and -1 give the same iterates; the one-launch solve runs the same
    * recurrences and stopping test with its sums in another order.  Up to two
    * captured chunks are kept per matrix, keyed by the solution vector. */
@@ -376,27 +380,30 @@ int lfgpu_pcg_noalloc(lfgpu_ctx *ctx, const lfgpu_csr *A, const lfgpu_vec *b,
  * plan of a mesh that is the disjoint union of the problems' meshes, so one
  * assembly launch assembles all of them).  row_offsets [nprob+1] (host)
  * partitions the rows; problem p owns rows [row_offsets[p], row_offsets[p+1])
- * and gets its own Jacobi-PCG (Eigen semantics per problem).  All problems
- * advance together, one pair of sweeps per iteration; chunks of iterations
- * are captured into a hipGraph once and replayed, and the workgroup tile is
- * chosen by timing candidates on the first solve.  No reference
+ * and gets its own Jacobi-PCG (Eigen semantics per problem).  No reference
  * counterpart: a batch replaces nprob separate solve calls.
  * lfgpu_batch_create checks on the device that every entry of A lies inside
  * its row's problem block and returns LFGPU_EINVAL otherwise.
  * opts->graph: 0 (default) solves all problems in one launch, and one more for
  * those that are no structured P1 meshes, with their vectors kept on the chip
  * (see lfgpu_pcg_opts.graph; summary->syncs is 1 then), where every problem
- * fits; else, and with 1, replays the captured chunk; -1 launches each
- * chunk's kernels directly (the same iterates as 1, no graph is captured). */
+ * fits and the sweeps are not faster (they are in the mixed modes for thousands
+ * of small structured meshes, and with FP32 vectors for a few large
+ * unstructured ones); else, and with 1, runs sweeps in which all problems
+ * advance together, one pair an iteration, in chunks captured into a hipGraph
+ * once and replayed, with the workgroup tile chosen by timing candidates on the
+ * first such solve; -1 launches each chunk's kernels directly (the same iterates
+ * as 1, no graph is captured). */
 typedef struct lfgpu_batch lfgpu_batch;
 int lfgpu_batch_create(lfgpu_ctx *ctx, lfgpu_csr *A, int nprob,
                        const int32_t *row_offsets, lfgpu_batch **out);
 int lfgpu_batch_destroy(lfgpu_batch *bt);
 /* infos: nprob entries (or NULL); summary: iters = max over problems,
  * converged = all converged, relres = worst, refinements = the tuned rows
- * per workgroup (0 while only one-launch solves have run), ms = device time.  All three modes of lfgpu_pcg: in the
- * mixed modes every problem runs its own reliable updates and stops on its
- * FP64 true residual (infos[p].refinements counts them). */
+ * per workgroup (0 while only one-launch solves have run), ms = device time.
+ * All three modes of lfgpu_pcg: in the mixed modes every problem runs its own
+ * reliable updates and stops on its FP64 true residual (infos[p].refinements
+ * counts them). */
 int lfgpu_batch_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, const lfgpu_vec *b,
                     lfgpu_vec *x, const lfgpu_pcg_opts *opts,
                     lfgpu_pcg_info *infos, lfgpu_pcg_info *summary);
@@ -422,7 +429,7 @@ int lfgpu_batch_storage(const lfgpu_batch *bt, int *storage);
  * coefficient data may change) replay it as one launch and continue with the
  * captured chunks, polled as in
  * lfgpu_batch_pcg (summary->syncs).  summary->ms covers assembly and solve.
- * The batched form of the north-star pipeline (assemble, then solve, per
+ * The batched form of the pipeline (assemble, then solve, per
  * problem; no single reference counterpart: AssembleMatrixLocally +
  * AssembleVectorLocally + the solve of homDir_linfe_demo.cc:130-174). */
 int lfgpu_batch_assemble_pcg(lfgpu_ctx *ctx, lfgpu_batch *bt, lfgpu_plan *p,

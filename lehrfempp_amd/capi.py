@@ -449,8 +449,9 @@ def spmv_timed(ctx, A: Csr, x: Vec, y: Vec, reps: int):
 def pcg(ctx, A: Csr, b: Vec, x: Vec, rtol=1e-10, maxit=None, mode=PCG_FP64, check_every=64,
         raise_on_noconv=True, refine_delta=0.0, refine_max_interval=0, single_reduction=False,
         graph=0):
-    """lfgpu_pcg.  graph: 0 = replay captured FP64 iteration chunks below 2^20
-    rows, 1 = always, -1 = never."""
+    """lfgpu_pcg.  graph: 0 = one launch where the system fits the chip, else
+    replay captured FP64 iteration chunks below 2^20 rows; 1 = replay chunks, -1 =
+    plain launches."""
     n = A.info()[0]
     opts = PcgOpts(rtol, int(2 * n if maxit is None else maxit), mode, check_every,
                    float(refine_delta), int(refine_max_interval), int(bool(single_reduction)),
@@ -513,8 +514,8 @@ class Batch:
     def pcg(self, b: Vec, x: Vec, rtol=1e-10, maxit=100000, check_every=64,
             raise_on_noconv=True, mode=PCG_FP64, refine_delta=0.0, refine_max_interval=0,
             graph=0):
-        """lfgpu_batch_pcg.  graph: 0 = replay the captured chunk, -1 = plain
-        launches."""
+        """lfgpu_batch_pcg.  graph: 0 = one launch where every problem fits, else
+        as 1 = replay the captured chunk; -1 = plain launches."""
         opts = PcgOpts(rtol, int(maxit), mode, check_every, refine_delta, refine_max_interval, 0,
                        int(graph))
         infos = (PcgInfo * self.nprob)()
@@ -529,8 +530,9 @@ class Batch:
                      maxit=100000, check_every=64, raise_on_noconv=True, mode=PCG_FP64,
                      refine_delta=0.0, refine_max_interval=0):
         """lfgpu_batch_assemble_pcg: plan.assemble(fe, alpha, gamma, f, rhs) and
-        pcg(rhs, x), replayed as one captured graph from the second call with
-        the same arguments on."""
+        pcg(rhs, x); where that takes more than one launch a kind of problem,
+        replayed as one captured graph from the second call with the same
+        arguments on."""
         opts = PcgOpts(rtol, int(maxit), mode, check_every, refine_delta, refine_max_interval, 0,
                        0)
         infos = (PcgInfo * self.nprob)()

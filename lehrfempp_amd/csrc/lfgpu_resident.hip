@@ -596,7 +596,9 @@ struct StreamLds {
 
 // RPT: cells per thread.  XR: the cells j < XR keep their x in a register, the
 // others' is read and written in every update (as many as the registers hold
-// without spills).  AHEAD: rows of a stream in flight.
+// and LDS leave room for: all 17; 16 of 25, with 21 registers spilled; none of
+// 33, with 4, since more of them spill more and take longer).  AHEAD: rows of a
+// stream in flight.
 template <int RPT, int XR, int AHEAD>
 __global__ __launch_bounds__(kThreads) void k_res_stream(TileArgs a) {
   extern __shared__ double dyn[];
@@ -1364,7 +1366,11 @@ __global__ void k_start_batch(ResidentControl *c, int *arrived, int jobs, uint64
 
 // The variants in order of preference (the smallest number of cells per
 // thread with which the team and its LDS fit): FP64, FP32 vectors, FP64
-// vectors with the FP32 matrix.
+// vectors with the FP32 matrix.  Registers that they spill: 29, 12 and 28 with 9
+// cells; streamed, 0, 21, 4 in FP64, 0, 16, 92 with FP32 vectors and 0, 166, 368
+// with FP64 ones, which is why the FP32 matrix is the slowest mode at 2048^2
+// (47 us an iteration; FP64 37, FP32 vectors 26): its update reads D^-1 a second
+// time and waits for p's exchange between update and product.
 struct TileVariant {
   int kind, rpt;
   size_t (*lds)(const TileArgs &);
@@ -1450,7 +1456,8 @@ const TileVariant *tile_plan(TileArgs &a, int mode, bool sym, bool diag, int cus
 }
 
 // Batches: up to 3 and up to 7 cells a thread (with 9 FP32 cells 55 registers
-// spill and 64 problems of 32 to 512 lines take 59 ms instead of 46).
+// spill and 64 problems of 32 to 512 lines take 59 ms instead of 46; with 7, 7 of
+// the FP32 and 18 of the FP64 vectors' kernel do, and none in FP64).
 struct BatchVariant {
   int rpt;
   size_t (*lds)(const TileArgs &);
