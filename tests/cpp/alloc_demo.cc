@@ -225,7 +225,7 @@ void refused(const char *name, lfgpu_ctx *ctx, const System &s, int mode, bool b
     lfgpu_pcg_info info{};
     opts.graph = turn == 0 ? 1 : 0;
     g_refuse = turn < 3 ? 401 : 0;
-    if (turn == 3) std::this_thread::sleep_for(std::chrono::milliseconds(300));
+    if (turn == 3) std::this_thread::sleep_for(std::chrono::milliseconds(600));
     OK(lfgpu_vec_fill(x, 0.0));
     if (batch) OK(lfgpu_batch_pcg(ctx, bt, b, x, &opts, nullptr, &info));
     else OK(lfgpu_pcg(ctx, A, b, x, &opts, &info));
