@@ -57,6 +57,7 @@ struct ResidentBufs {
   unsigned long long *sums = nullptr;  // team sums (fixed size)
   ResidentOutcome *outcome = nullptr;
   uint64_t ticks = 0;  // outcome->team.ticks
+  bool kept = false;   // the last solve's start is in its ResidentDia::keep
   uint32_t epoch = 0;
 };
 void resident_free(ResidentBufs *b);
@@ -110,6 +111,11 @@ struct ResidentDia {
   const float *val32 = nullptr, *rowsum32 = nullptr, *dinv32 = nullptr;
   const void *dinv16 = nullptr;
   double *xlo = nullptr;
+  // n values for the start of the streamed FP64 solve, which updates x in memory.
+  // A workgroup that gives up in a team sum still sends what it has, and the
+  // others may take one step with that before they see the flag; the other
+  // solves write x only after a later sum, which then does not come.
+  double *keep = nullptr;
 };
 
 // Jacobi-PCG in opts.mode on the context stream (rtol, maxit, mode and the

@@ -1612,6 +1612,9 @@ int resident_pcg_dia(lfgpu_ctx *ctx, ResidentBufs *bufs, const ResidentDia &A,
   a.total = bufs->sums + kPartWords;
   a.abort = &bufs->outcome->team;
   a.st = &bufs->outcome->solve;
+  bufs->kept = v->kind == STREAM && opts.mode == LFGPU_PCG_FP64;
+  if (bufs->kept)
+    LFG_HIP(hipMemcpyAsync(A.keep, x, (size_t)A.n * 8, hipMemcpyDeviceToDevice, s));
   return resident_launch(s, bufs, reinterpret_cast<const void *>(v->fn), team, &a, v->lds(a), out,
                          taken);
 }

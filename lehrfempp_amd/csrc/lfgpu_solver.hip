@@ -3933,6 +3933,7 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       rd.dinv32 = c->dinv32;
       rd.dinv16 = c->dinv16;
       rd.xlo = c->xlo;
+      rd.keep = c->r;
       for (bool known : {false, true}) {
         bool ask = false;
         rc = resident_pcg_dia(ctx, &c->res, rd, *opts, b->d, x->d, rs, &taken,
@@ -3968,10 +3969,12 @@ extern "C" int lfgpu_pcg(lfgpu_ctx *ctx, const lfgpu_csr *Ac, const lfgpu_vec *b
       return rc;
     } else if (taken) {
       // (a workgroup gave up its wait for another one, as when other processes
-      // hold a part of the chip: the sweeps go on from the x reached)
+      // hold a part of the chip: the sweeps go on from the x reached, or the start)
       rc = resident_finish(ctx, &c->res, rs, mixed, info, &c->pause, &aborted);
       if (rc != LFGPU_OK || !aborted) return rc;
       gave_up = 1;
+      if (c->fmt == FMT_DIA && c->res.kept)
+        LFG_HIP(hipMemcpyAsync(x->d, c->r, (size_t)n * 8, hipMemcpyDeviceToDevice, s));
     }
   }
 

@@ -775,3 +775,25 @@ def test_resident_solves_share_their_words(ctx, make):
                 assert np.array_equal(x.numpy(), want[mode])
     for h in (batch, x, b, A):
         h.close()
+
+
+# the streamed FP64 solve updates x in memory, the last time perhaps by a sum
+# that a workgroup took for whole: where it gives up, the sweeps begin at the
+# caller's x
+def test_streamed_solve_that_gives_up_leaves_the_start(ctx):
+    r, c, v, n = _lattice_system(1141, 1140, P1, 3)
+    v[-n:] += 1.0
+    start = np.random.default_rng(2).standard_normal(n)
+    with capi.Context(0) as own:
+        A = capi.coo_to_csr(own, r, c, v, n, n)
+        b = capi.Vec(own, np.random.default_rng(1).standard_normal(n))
+        x = capi.Vec(own, start)
+        swept = capi.pcg(own, A, b, x, graph=-1)
+        want = x.numpy()
+        own.set_resident_wait(0.0)
+        x.upload(start)
+        info = capi.pcg(own, A, b, x)
+        assert info.syncs >= 2 and info.iters == swept.iters
+        assert np.array_equal(x.numpy(), want)
+        for h in (x, b, A):
+            h.close()
