@@ -63,8 +63,8 @@ int lfgpu_ctx_sync(lfgpu_ctx *ctx);
 int lfgpu_ctx_last_ms(lfgpu_ctx *ctx, double *ms);
 /* Longest time a workgroup of a one-launch solve (lfgpu_pcg_opts.graph) of
  * this context waits for another one before the whole launch gives up and the
- * swept solver goes on from the x reached (4 s at first; 0: every such solve
- * ends that way).  Workgroups wait long only where other processes hold a
+ * swept solver goes on, from the x reached or from the caller's (4 s at first;
+ * 0: every such solve ends that way).  Workgroups wait long only where other processes hold a
  * part of the GPU. */
 int lfgpu_ctx_set_resident_wait(lfgpu_ctx *ctx, double seconds);
 

@@ -341,10 +341,11 @@ __device__ __forceinline__ bool tile_solve(const TileArgs &a, int rank, int team
   Team tm{T.rank, T.team, a.part, a.total, a.abort, a.tag0};
   if (t == 0) sh.bad = 0;
   // Moves the loops by 48 B.  The kernel of one cell a thread waits in short
-  // poll loops most of the time, and where they lie in the lines of the
-  // instruction cache decides: 65 x 65 rows 2.30 us an iteration this way, 2.52
-  // without, 2.58 with all loops on 32 or 64 B.  (To be measured again when
-  // that kernel's code changes.)
+  // poll loops most of the time, and the same code takes 2.30 us an iteration on
+  // 65 x 65 rows this way, 2.52 without, 2.58 with all loops on 32 or 64 B.  Why
+  // is not established (the loops' place in the instruction cache, or the phase
+  // in which their polls meet the words); to be measured again when that kernel's
+  // code changes.
   if constexpr (RPT == 1 && !BATCH) asm volatile(".rept 12\n s_nop 0\n .endr");
   T.tables(t);
   const int32_t cells = Lds::cells(a.TW);
